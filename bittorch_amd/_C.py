@@ -722,3 +722,39 @@ def unpack_dequant(W_T: Tensor, in_features: int, scale: Optional[Tensor] = None
                                      0 if scale_f is None else scale_f.numel(), out.data_ptr(), odt,
                                      N, in_features, _stream(W_T)))
     return out
+
+
+def linear_grad_input(dY: Tensor, W_T: Tensor, scale: Tensor, in_features: int) -> Tensor:
+    """Input gradient of an fp32 packed layer, ``(dY * scale) @ decode(W_T)`` ``[M, K]`` (``dY`` ``[M, N]`` fp32,
+    ``scale`` fp32 ``[N]`` or one entry)."""
+    _check(dY.dim() == 2 and dY.dtype == torch.float32 and dY.numel() > 0, "dY must be 2D fp32")
+    _check(W_T.dim() == 2 and W_T.dtype == torch.uint8 and W_T.shape[0] == (in_features + 3) // 4
+           and W_T.shape[1] == dY.shape[1], "W_T must be uint8 [ceil(K/4), N]")
+    _check(scale.dtype == torch.float32 and scale.numel() in (dY.shape[1], 1), "scale must be fp32 [N] or one entry")
+    _check(_all_cuda(dY, W_T, scale), "All tensors must be CUDA")
+    dY, W_T, scale = dY.contiguous(), W_T.contiguous(), scale.contiguous()
+    M, N = dY.shape
+    out = torch.empty((M, in_features), dtype=torch.float32, device=dY.device)
+    with torch.cuda.device(dY.device):
+        _status(_L.bt_ternary_linear_grad_input(dY.data_ptr(), W_T.data_ptr(), scale.data_ptr(), scale.numel(),
+                                                out.data_ptr(), M, N, in_features, _stream(dY)))
+    return out
+
+
+def linear_grad_weight(dY: Tensor, X: Tensor, scale: Tensor, want_bias: bool = False) -> Tuple[Tensor, Optional[Tensor]]:
+    """Weight gradient under the straight-through estimator, ``scale[:, None] * (dY.T @ X)`` ``[N, K]``, and with
+    ``want_bias`` the bias gradient ``dY.sum(0)`` from the same pass (all fp32, N and K at least 4)."""
+    _check(dY.dim() == 2 and X.dim() == 2 and dY.shape[0] == X.shape[0] and dY.numel() > 0 and X.numel() > 0,
+           "dY [M, N] and X [M, K] must be 2D with the same rows")
+    _check(dY.dtype == X.dtype == scale.dtype == torch.float32, "dY, X and scale must be fp32")
+    _check(scale.numel() in (dY.shape[1], 1), "scale size doesn't match N")
+    _check(_all_cuda(dY, X, scale), "All tensors must be CUDA")
+    dY, X, scale = dY.contiguous(), X.contiguous(), scale.contiguous()
+    (M, N), K = dY.shape, X.shape[1]
+    dW = torch.empty((N, K), dtype=torch.float32, device=dY.device)
+    dB = torch.empty((N,), dtype=torch.float32, device=dY.device) if want_bias else None
+    with torch.cuda.device(dY.device):
+        ws = _workspace(_L.bt_linear_grad_weight_workspace_bytes(M, N, K), dY.device)
+        _status(_L.bt_linear_grad_weight(dY.data_ptr(), X.data_ptr(), scale.data_ptr(), scale.numel(), dW.data_ptr(), _ptr(dB),
+                                         M, N, K, _ptr(ws), 0 if ws is None else ws.numel(), _stream(dY)))
+    return dW, dB

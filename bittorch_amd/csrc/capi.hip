@@ -86,7 +86,11 @@ int launch_row_op(int op, int dtype, const void* A, int64_t lda, const void* Bv,
 bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, const void* Y);
 bool gemm_f16_supported_tiled(int64_t N, int64_t K, const void* X, const void* Y);
 int launch_gemm_f16(int mode, const void* X, const uint8_t* W_T, int w_layout, const Epilogue& epi, void* Y, int y_dtype,
-                    int64_t M, int64_t N, int64_t K, int planes, hipStream_t st);
+                    int64_t M, int64_t N, int64_t K, hipStream_t st);
+bool gemm_f32_supported(int64_t N, int64_t K, const void* X, const void* Y);
+double gemm_f32_cost(int64_t M, int64_t N, int64_t K);
+int launch_gemm_f32(const void* X, const uint8_t* W, int w_layout, const Epilogue& epi, void* Y, int64_t M, int64_t N,
+                    int64_t K, hipStream_t st);
 bool planes_supported(int x_dtype, int y_dtype, int64_t B, int64_t N, int64_t K, const void* X, const void* W, const void* Y,
                       int w_layout);
 int launch_planes(const void* X, const uint8_t* W, int w_layout, const Epilogue& epi, void* Y, int64_t N, int64_t K,
@@ -184,6 +188,18 @@ static bool prefers_stream(int64_t B, int64_t N, int64_t K, bool int8, bool tile
     const double t_stream = 4.0 + work * (int8 ? 2.2e-9 : 5.0e-9) + wgs * (int8 ? 0.003 : 0.004);
     const double t_gemm = rounds * (int8 ? 8.6 + 0.0044 * (double)K : 6.9 + 0.010 * (double)K);
     return t_stream < t_gemm;
+}
+
+// The same choice for fp32 activations: the streaming kernel on three bf16 planes (split in a launch of its own, about 3 us)
+// or gemm_f32_kernel, which splits in registers.
+static bool prefers_stream_f32(int64_t B, int64_t N, int64_t K) {
+    if (const char* env = option(OPT_STREAM_MAX_ROWS)) {
+        const long v = atol(env);
+        if (v >= 1) return B <= v;
+    }
+    if (B <= 32) return true;
+    const double wgs = (double)(ceil_div(B, 16) * ceil_div(N, 64));
+    return 7.0 + (double)B * (double)N * 3.0 * (double)K * 5.0e-9 + wgs * 0.004 < gemm_f32_cost(B, N, K);
 }
 
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -308,7 +324,7 @@ static int packed_forward_impl(const char* who, const void* X, int x_dtype, cons
             const int mode = (x_dtype == BT_F16) ? MODE_F16 : MODE_BF16;
             // tall batches: the tiled matrix-core GEMM reads the copy too (not with the SwiGLU output stage)
             if (!prefers_stream(B, N, K, false, true) && epi_op == 0 && gemm_f16_supported_tiled(N, K, X, Y))
-                return launch_gemm_f16(mode, X, W_T, w_layout, epi, Y, x_dtype, B, N, K, 1, st);
+                return launch_gemm_f16(mode, X, W_T, w_layout, epi, Y, x_dtype, B, N, K, st);
             return launch_stream(mode, X, 2, nullptr, W_T, w_layout, epi, Y, x_dtype, nullptr, B, N, K, 1,
                                  Q_ROW_MAJOR, 0, nullptr, 0.0f, epi_op, st);
         }
@@ -318,10 +334,10 @@ static int packed_forward_impl(const char* who, const void* X, int x_dtype, cons
             return BT_ERR_INVALID;
         }
         const int64_t Kp = plane_len(K);
+        if (!prefers_stream_f32(B, N, K) && epi_op == 0 && gemm_f32_supported(N, K, X, Y))
+            return launch_gemm_f32(X, W_T, w_layout, epi, Y, B, N, K, st);
         rc = launch_split_f32_planes(X, B, K, Kp, workspace, st);
         if (rc) return rc;
-        if (!prefers_stream(B, N, 3 * Kp, false, K % 64 == 0) && epi_op == 0 && gemm_f16_supported_tiled(N, 3 * Kp, workspace, Y))
-            return launch_gemm_f16(MODE_BF16, workspace, W_T, w_layout, epi, Y, BT_F32, B, N, K, 3, st);
         return launch_stream(MODE_BF16, workspace, 2, nullptr, W_T, w_layout, epi, Y, BT_F32, nullptr, B, N, K, 3,
                              Q_ROW_MAJOR, 0, nullptr, 0.0f, epi_op, st);
     }
@@ -331,17 +347,17 @@ static int packed_forward_impl(const char* who, const void* X, int x_dtype, cons
         const int mode = (x_dtype == BT_F16) ? MODE_F16 : MODE_BF16;
         // tall batches go to the tiled matrix-core kernel, decode shapes stream the weights
         if (!prefers_stream(B, N, K, false) && gemm_f16_supported(N, K, X, W_T, Y))
-            return launch_gemm_f16(mode, X, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, x_dtype, B, N, K, 1, st);
+            return launch_gemm_f16(mode, X, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, x_dtype, B, N, K, st);
         return launch_stream(mode, X, 2, nullptr, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, x_dtype, nullptr, B, N, K, 1, Q_ROW_MAJOR, 0, nullptr, 0.0f, 0, st);
     }
     if (x_dtype == BT_F32 && packed_uses_f32_planes(W_T, Y, N, K) && workspace &&
         workspace_bytes >= f32_planes_bytes(B, K) && ((uintptr_t)workspace) % 256 == 0) {
         // (without a workspace the call still succeeds, on the generic kernel)
         const int64_t Kp = plane_len(K);
+        if (!prefers_stream_f32(B, N, K) && gemm_f32_supported(N, K, X, Y))
+            return launch_gemm_f32(X, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, B, N, K, st);
         rc = launch_split_f32_planes(X, B, K, Kp, workspace, st);
         if (rc) return rc;
-        if (!prefers_stream(B, N, 3 * Kp, false) && gemm_f16_supported(N, 3 * Kp, workspace, W_T, Y))
-            return launch_gemm_f16(MODE_BF16, workspace, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, BT_F32, B, N, K, 3, st);
         return launch_stream(MODE_BF16, workspace, 2, nullptr, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, BT_F32, nullptr, B, N, K, 3, Q_ROW_MAJOR, 0, nullptr, 0.0f, 0, st);
     }
     return launch_packed_generic(X, x_dtype, W_T, epi, Y, B, N, K, st);

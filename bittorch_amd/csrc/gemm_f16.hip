@@ -40,14 +40,13 @@ struct GemmFParams {
     int64_t K, M, N;      // K: length of an activation row
     int tiles_m, tiles_n;
     int per_xcd;          // workgroups per XCD (grid = 8 * per_xcd)
-    int wstages;          // 64-wide stages of W_T; a stage index beyond it wraps (see launch_gemm_f16)
+    int wstages;          // 64-wide stages of W_T
     int tiles16;          // WT: 16-column tiles of the decode-tiled weight copy (its 16-row steps are the stages; < 0: stored_tile16)
     int tile_n0;          // first column tile of this launch (tiles_n counts the launch's own column tiles)
     // ---- needed later
     void* Y;              // [M, N]
     int64_t Kb;           // packed weight rows
     int y_dtype;
-    int prehalved;        // MODE_BF16: the activations already carry the factor 1/2 of the +-2.0 weight decode
     Epilogue epi;
 };
 static_assert(offsetof(GemmFParams, Y) == 64, "first argument line as laid out above");
@@ -92,7 +91,7 @@ __device__ __forceinline__ void gemm_f_epilogue(const GemmFParams& p, const v4f 
 #pragma unroll
             for (int t = 0; t < 4; t++) {
                 float a = acc[MB0 + mbi][t][r];
-                if constexpr (MODE == MODE_BF16) a *= (p.prehalved ? 1.0f : 0.5f);  // weights were decoded as +-2.0
+                if constexpr (MODE == MODE_BF16) a *= 0.5f;  // weights were decoded as +-2.0
                 y[t] = epi_float(a, ws[t], bs[t]);
             }
             if constexpr (RES && YDT != BT_F32) {  // what add_residual4 does, on the bits already here
@@ -225,24 +224,11 @@ __global__ __launch_bounds__(512) void gemm_f16_kernel(GemmFParams p) {
             a_reg[1] = *(const uint4*)(ab + 16 + a_off);
         }
         if (part & 2) {
-            // the activation row may hold several planes of K values, all multiplied with the
-            // same weights: the weight stage wraps (uniform)
-            int ws = st;
-            if (ws >= p.wstages) ws -= p.wstages;
-            if (ws >= p.wstages) ws -= p.wstages;
             if constexpr (WT) {
-                const uint4 v = *(const uint4*)(b_base + (size_t)ws * 256 + b_off);
+                const uint4 v = *(const uint4*)(b_base + (size_t)st * 256 + b_off);
                 b_reg[0] = v.x; b_reg[1] = v.y; b_reg[2] = v.z; b_reg[BR - 1] = v.w;
-            } else if constexpr (TAIL) {
-                // zero-padded activation planes with K % 64 != 0: the last weight stage of a plane runs past W_T
-#pragma unroll
-                for (int r = 0; r < 2; r++) {
-                    int64_t kb = (int64_t)ws * (F_BK / 4) + 8 * kgrp + 2 * g + r;
-                    kb = kb < p.Kb ? kb : p.Kb - 1;
-                    b_reg[r] = *(const uint32_t*)(b_base + kb * N + (col_ok ? ncol : 0));
-                }
             } else {
-                const uint8_t* bb = b_base + (int64_t)ws * (F_BK / 4) * N;
+                const uint8_t* bb = b_base + (int64_t)st * (F_BK / 4) * N;
                 b_reg[0] = *(const uint32_t*)(bb + b_off);
                 b_reg[1] = *(const uint32_t*)(bb + N + b_off);
             }
@@ -261,7 +247,7 @@ __global__ __launch_bounds__(512) void gemm_f16_kernel(GemmFParams p) {
             }
         }
         if constexpr (WT) {
-            if (part & 2) {  // the copy is zero-padded to whole steps; this is the last step (no planes with a tail)
+            if (part & 2) {  // the copy is zero-padded to whole steps; this is the last step
                 const uint4 v = *(const uint4*)(b_base + (size_t)min((int)(k0 >> 6), p.wstages - 1) * 256 + b_off);
                 b_reg[0] = v.x; b_reg[1] = v.y; b_reg[2] = v.z; b_reg[BR - 1] = v.w;
             }
@@ -494,9 +480,6 @@ bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, co
            ((uintptr_t)Y) % 16 == 0 && (F_BM + 1) * K * 2 < (1ll << 32) && ceil_div(K, 4) * N < (1ll << 32);
 }
 
-// planes = 1: X is [M, K].  planes = 3: X is [M, 3*Kp], Kp = K rounded up to 64, three zero-padded planes of K
-// values per row whose products with the same weights are summed (fp32 activations split into three bf16 terms).
-// With K % 64 != 0 the last weight stage of every plane runs past W_T's rows: the TAIL instantiation clamps them.
 // One launch over column tiles [tile_n0, tile_n0 + tiles_n) in tiles of 32 * NB rows.
 template <int NB>
 static int launch_gemm_f16_part(GemmFParams p, int mode, int tile_n0, int tiles_n, bool tiled, bool tail, hipStream_t st) {
@@ -535,12 +518,11 @@ static int launch_gemm_f16_part(GemmFParams p, int mode, int tile_n0, int tiles_
 }
 
 int launch_gemm_f16(int mode, const void* X, const uint8_t* W_T, int w_layout, const Epilogue& epi, void* Y, int y_dtype,
-                    int64_t M, int64_t N, int64_t K, int planes, hipStream_t st) {
+                    int64_t M, int64_t N, int64_t K, hipStream_t st) {
     GemmFParams p = {};
     p.X = (const uint16_t*)X; p.W_T = W_T; p.Y = Y; p.epi = epi;
-    p.M = M; p.N = N; p.K = (planes == 3) ? 3 * ceil_div(K, F_BK) * F_BK : K; p.Kb = ceil_div(K, 4);
+    p.M = M; p.N = N; p.K = K; p.Kb = ceil_div(K, 4);
     p.wstages = (int)ceil_div(K, F_BK);
-    p.prehalved = planes == 3;
     p.y_dtype = y_dtype;
     p.tiles16 = tiles16_arg(N, w_layout);
     const bool tail = K % F_BK != 0, tiled = layout_tiled(w_layout);

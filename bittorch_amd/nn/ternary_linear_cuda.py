@@ -3,9 +3,10 @@
 API mirror of ``bittorch/nn/ternary_linear_cuda.py:23-228``.  Forward: one fused
 HIP kernel quantizes and packs the master weights, a second one multiplies the
 activations with the packed weights (fp32 accumulation).  Backward is the
-straight-through estimator with torch matmuls, as in the reference
-(``:73-111``); the dense effective weights it needs are rebuilt from the packed
-bytes instead of being kept alive from the forward.
+straight-through estimator, as in the reference (``:73-111``): fp32 layers run on
+the library's gradient kernels, which read the packed bytes; the other dtypes use torch
+matmuls on dense effective weights rebuilt from the packed bytes instead of being
+kept alive from the forward.
 """
 
 from __future__ import annotations
@@ -20,6 +21,17 @@ from torch import Tensor
 from ..quant.ternary import ternary_quantize
 from ._packed_cache import PackedWeightCache, cache_usable
 from .ternary_linear import _init_linear_params
+
+
+def _fp32_kernels_serve(g2: Tensor, x2: Tensor, packed: Optional[Tensor], scale: Tensor) -> bool:
+    """Whether this backward runs on the library's gradient kernels: fp32 throughout, and no graph of the backward itself
+    wanted (``create_graph=True``: the torch products below are differentiable)."""
+    if packed is None or torch.is_grad_enabled() or g2.numel() == 0:
+        return False
+    if not (g2.dtype == x2.dtype == scale.dtype == torch.float32 and g2.is_cuda):
+        return False
+    n, k = g2.shape[1], x2.shape[1]
+    return 4 <= n < 2 ** 23 and 4 <= k < 2 ** 23 and packed.numel() < 2 ** 32
 
 
 class TernaryLinearCUDAFunction(torch.autograd.Function):
@@ -67,10 +79,19 @@ class TernaryLinearCUDAFunction(torch.autograd.Function):
         from .. import _C
 
         x, packed, scale = ctx.saved_tensors
-        scale_col = scale.reshape(-1, 1)
         g2 = grad_output.reshape(-1, grad_output.shape[-1])
         x2 = x.reshape(-1, x.shape[-1])
         grad_x = grad_w = grad_b = None
+        want_bias = ctx.has_bias and ctx.needs_input_grad[2]
+        if _fp32_kernels_serve(g2, x2, packed, scale):
+            if ctx.needs_input_grad[0]:
+                grad_x = _C.linear_grad_input(g2, packed, scale.reshape(-1), ctx.in_features).reshape(x.shape)
+            if ctx.needs_input_grad[1]:
+                grad_w, grad_b = _C.linear_grad_weight(g2, x2, scale.reshape(-1), want_bias)
+            elif want_bias:
+                grad_b = g2.sum(dim=0)
+            return grad_x, grad_w, grad_b, None, None, None
+        scale_col = scale.reshape(-1, 1)
         if ctx.needs_input_grad[0]:
             if packed is not None:
                 w_eff = _C.unpack_dequant(packed, ctx.in_features, scale.reshape(-1),
@@ -81,7 +102,7 @@ class TernaryLinearCUDAFunction(torch.autograd.Function):
         if ctx.needs_input_grad[1]:
             # d(w_eff)/d(weight) = scale under the straight-through estimator
             grad_w = (g2.t() @ x2) * scale_col.to(g2.dtype)
-        if ctx.has_bias and ctx.needs_input_grad[2]:
+        if want_bias:
             grad_b = g2.sum(dim=0)
         return grad_x, grad_w, grad_b, None, None, None
 

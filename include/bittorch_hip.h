@@ -405,6 +405,21 @@ int bt_unpack_dequant(const uint8_t* W_T, const float* scale, int64_t scale_len,
                       int out_dtype, int64_t N, int64_t K, void* stream);
 
 /*
+ * The backward of an fp32 layer (bittorch/nn/ternary_linear_cuda.py:73-111, straight-through estimator), on the packed
+ * weights and without a dense copy of them:
+ *   bt_ternary_linear_grad_input   dX [M,K] = (dY [M,N] * scale) decode(W_T); dX 16-byte aligned
+ *   bt_linear_grad_weight          dW [N,K] = scale[n] * sum_m dY[m,n] X[m,k] and, if dBias is not NULL,
+ *                                  dBias [N] = sum_m dY[m,n]; N and K at least 4; workspace as described above
+ * Everything is fp32 (scale_len: N, or 1 for a per-tensor scale); products are formed from exact bf16 terms of the
+ * operands and summed in fp32.
+ */
+int bt_ternary_linear_grad_input(const float* dY, const uint8_t* W_T, const float* scale, int64_t scale_len, float* dX,
+                                 int64_t M, int64_t N, int64_t K, void* stream);
+size_t bt_linear_grad_weight_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int bt_linear_grad_weight(const float* dY, const float* X, const float* scale, int64_t scale_len, float* dW, float* dBias,
+                          int64_t M, int64_t N, int64_t K, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Dense ternary weights -> packed transposed layout, on the device.
  * Replaces pack_ternary_transposed (bittorch/quant/ternary_packed.py:174-206) for weights
  * that are already ternary: W_tern [N,K] int8 in {-1,0,+1} -> packed_T [ceil(K/4),N] uint8.

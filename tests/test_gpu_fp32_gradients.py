@@ -1,0 +1,101 @@
+"""GPU: the fp32 matrix-core kernels of ``csrc/gemm_f32.hip`` (forward on row-major and tiled weights, input gradient,
+weight and bias gradient) against float64.
+
+Every product is formed from exact bf16 terms (weight gradient: up to terms below 2^-25 of it) and added in fp32, at most
+six terms per product: the error of a sum of C products is at most 6 (C + 8) 2^-24 of the sum of the products' magnitudes.
+"""
+import pytest
+import torch
+
+from conftest import announce
+
+gpu = pytest.mark.gpu
+EPS = 2.0 ** -24
+
+# edges of the tiles (64, 128, 256 outputs; contraction steps of 32, split over 4 or 8 waves), remainders, the smallest
+SHAPES = [(1, 4, 4), (33, 4, 5), (40, 20, 33), (65, 64, 31), (64, 256, 32), (129, 132, 77), (200, 300, 258), (300, 100, 1000),
+          (513, 1028, 96), (1000, 36, 2048), (2100, 768, 260), (4099, 516, 516), (16384, 192, 130)]
+
+
+def _close(got, a, b, scale=1.0):
+    """got against a @ b in float64, by the bound above; scale: a factor of the rows or columns that is rounded too"""
+    ref = (a.double() @ b.double()) * scale
+    bound = 6 * (a.shape[1] + 8) * EPS * ((a.double().abs() @ b.double().abs()) * scale) + 1e-37
+    assert torch.isfinite(got).all()
+    err = (got.double() - ref).abs()
+    assert bool((err <= bound).all()), float((err / bound).max())
+
+
+def _case(m, n, k, per_channel=True):
+    from bittorch_amd import _C
+    g = torch.Generator("cuda").manual_seed(m * 7 + n * 3 + k)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    w = r(n, k) * 0.02
+    packed, scale, tern = _C.ternary_quantize_pack(w, 0.05, per_channel, True, True)
+    return r(m, k), r(m, n) * 0.01, packed, scale.reshape(-1), tern.float()
+
+
+@gpu
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_fp32_products_against_float64(m, n, k):
+    from bittorch_amd import _C
+    announce("fp32 gradients", m, n, k)
+    x, dy, packed, scale, tern = _case(m, n, k)
+    _close(_C.linear_grad_input(dy, packed, scale, k), dy, tern * scale[:, None])
+    dw, db = _C.linear_grad_weight(dy, x, scale, True)
+    _close(dw, dy.t(), x, scale.double()[:, None])
+    _close(db[:, None], dy.t(), torch.ones(m, 1, device="cuda"))
+    assert torch.equal(_C.linear_grad_weight(dy, x, scale, True)[0], dw)  # a fixed order of the sums
+    if m > 32 and n % 4 == 0:
+        y = _C.ternary_linear_packed_forward(x, packed, scale, None, k)
+        _close(y, x, tern.t(), scale.double()[None, :])
+        _close(_C.ternary_linear_tiled_forward(x, _C.retile_weights(packed, k), scale, None, k, n), x, tern.t(),
+               scale.double()[None, :])
+
+
+@gpu
+@pytest.mark.parametrize("m,n,k", [(70, 24, 40), (1500, 130, 70)])
+def test_fp32_gradients_one_scale_strides_and_alignment(m, n, k):
+    """A per-tensor scale; operands that start 4 bytes into a buffer; an expanded (stride 0) output gradient."""
+    from bittorch_amd import _C
+    announce("fp32 gradients, views", m, n, k)
+    x, dy, packed, scale, tern = _case(m, n, k, per_channel=False)
+    off = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view_as(t)
+    _close(_C.linear_grad_input(off(dy), packed, scale, k), dy, tern * scale)
+    _close(_C.linear_grad_weight(off(dy), off(x), scale)[0], dy.t(), x, float(scale))
+    wide = dy[:, :1].expand(m, n)
+    _close(_C.linear_grad_weight(wide, x, scale)[0], wide.t(), x, float(scale))
+
+
+@gpu
+def test_fp32_gradients_of_non_finite_values():
+    """An infinity or NaN in the output gradient (an overflown loss) leaves what the fp32 products leave: the same
+    elements non-finite, infinities with their sign, everything else untouched."""
+    from bittorch_amd import _C
+    m, n, k = 300, 64, 96
+    announce("fp32 gradients, non-finite", m, n, k)
+    x, dy, packed, scale, tern = _case(m, n, k)
+    dy[7, 5], dy[90, 11], dy[200, 40] = float("inf"), float("-inf"), float("nan")
+    x[120, 3] = float("inf")
+    for got, ref in ((_C.linear_grad_input(dy, packed, scale, k), dy.double() @ (tern * scale[:, None]).double()),
+                     (_C.linear_grad_weight(dy, x, scale)[0], (dy.double().t() @ x.double()) * scale.double()[:, None])):
+        assert torch.equal(torch.isnan(got), torch.isnan(ref))
+        inf = torch.isinf(ref)
+        assert torch.equal(got[inf].double(), ref[inf]) and inf.any()
+        fin = torch.isfinite(ref)
+        assert torch.allclose(got[fin].double(), ref[fin], rtol=1e-4, atol=1e-6)
+
+
+@gpu
+def test_fp32_layer_backward_uses_the_kernels_and_keeps_double_backward():
+    from bittorch_amd import nn
+    announce("fp32 layer backward")
+    layer = nn.TernaryLinear(96, 40).cuda()
+    x = torch.randn(70, 96, device="cuda", requires_grad=True)
+    gy = torch.randn(70, 40, device="cuda")
+    plain = torch.autograd.grad(layer(x), (x, layer.weight, layer.bias), gy)
+    gy2 = gy.clone().requires_grad_()
+    graphed = torch.autograd.grad(layer(x), (x, layer.weight, layer.bias), gy2, create_graph=True)
+    for a, b in zip(plain, graphed):
+        assert torch.allclose(a, b, rtol=1e-4, atol=1e-5 * float(b.detach().abs().max()))
+    assert torch.autograd.grad(graphed[0].sum(), gy2)[0].shape == gy.shape
