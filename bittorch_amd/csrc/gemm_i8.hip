@@ -26,209 +26,9 @@
 #include <cstddef>
 #include <cstdlib>
 
-#include "bt_common.h"
+#include "gemm_i8_common.h"
 
 namespace bt {
-
-constexpr int G_BM = 128;
-constexpr int G_BN = 256;
-constexpr int G_BK = 128;           // k per LDS stage (two k64 MFMA sub-steps)
-constexpr int G_MB = G_BM / 16;     // 16-row blocks per tile
-constexpr int G_STAGE_BYTES = G_BM * G_BK;  // 16 KiB
-
-struct GemmParams {
-    // The first 64 bytes hold what a workgroup needs to find its tile and request its first operands: the kernel
-    // arguments come through the scalar cache a 64-byte line at a time.
-    const int8_t* Q;      // [M, K]
-    const uint8_t* W_T;   // [Kb, N]
-    int64_t K, M, N;
-    int tiles_m, tiles_n;
-    int per_xcd;          // workgroups per XCD (grid = 8 * per_xcd)
-    int wsteps, tiles16;  // WT: 16-row steps and 16-column tiles of the decode-tiled weight copy (tiles16 < 0: stored_tile16)
-    int tile_n0;          // first column tile of this launch (tiles_n counts the launch's own column tiles)
-    // ---- needed later
-    const float* s_x;     // [M]
-    void* Y;              // [M, N]
-    int32_t* acc_out;     // optional [M, N]
-    int64_t Kb;
-    int y_dtype;
-    int long_epilogue;    // A/B runs and tests (option GEMM_LONG_EPILOGUE): never the short epilogue
-    const int32_t* q_rowsum;  // FL kernels: sum of each row of Q over K (what the codes w + 1 of the field layout add)
-    Epilogue epi;
-};
-static_assert(offsetof(GemmParams, s_x) == 64, "first argument line as laid out above");
-
-__device__ __forceinline__ void store4(void* Y, int dt, int64_t idx, const float (&v)[4]) {
-    if (dt == BT_F32) {
-        st4_nt((float*)Y + idx, __builtin_bit_cast(uint32_t, v[0]), __builtin_bit_cast(uint32_t, v[1]),
-               __builtin_bit_cast(uint32_t, v[2]), __builtin_bit_cast(uint32_t, v[3]));
-    } else {
-        uint16_t h[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) h[i] = (dt == BT_F16) ? f32_to_f16_bits(v[i]) : f32_to_bf16_bits(v[i]);
-        st2_nt((uint16_t*)Y + idx, (uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
-    }
-}
-
-// Finishes NB 16-row blocks (acc[MB0 .. MB0+NB-1]) of the tile: NB = 4 in a tile of 128 rows, 2 or 1 in the tiles of
-// 64 and 32 rows a launch's remainder is cut into.
-// The epilogue's operands (row scales of the wave's rows, column scales and biases as raw bits)
-// are requested before the K-half exchange, whose LDS round trips cover their latency.
-template <int NB>
-struct EpiOperands {
-    float sx[NB][4];  // [row block within the half][r]
-    uint32_t ws_bits[4], bs_bits[4];
-    uint2 res[NB][4]; // 16-bit residual of the lane's four columns in each of its rows (short epilogue only)
-};
-// The residual of a 16-bit output for the short epilogue (full tile): all 16 rows requested at once, next to the
-// other epilogue operands, so that the hand-over of the K halves covers their latency.  (One load per row right
-// before its use, as the long epilogue does, leaves a memory round trip per row exposed: 5 us per tile.)
-template <int NB>
-__device__ __forceinline__ void load_epi_residual(const GemmParams& p, int64_t m0, int mb0, int g, int64_t ncol, EpiOperands<NB>& e) {
-    const uint16_t* base = (const uint16_t*)p.epi.residual + (m0 + 16 * mb0 + 4 * g) * p.N + ncol;
-#pragma unroll
-    for (int mbi = 0; mbi < NB; mbi++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) e.res[mbi][r] = *(const uint2*)(base + (int64_t)(16 * mbi + r) * p.N);
-}
-template <int NB>
-__device__ __forceinline__ void load_epi_operands(const GemmParams& p, int64_t m0, int mb0, int g, int64_t ncol,
-                                                  bool col_ok, EpiOperands<NB>& e) {
-#pragma unroll
-    for (int mbi = 0; mbi < NB; mbi++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int64_t m = m0 + 16 * (mb0 + mbi) + 4 * g + r;
-            e.sx[mbi][r] = p.s_x[m < p.M ? m : p.M - 1];
-        }
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        const int64_t n = col_ok ? ncol + t : 0;
-        e.ws_bits[t] = load_bits_rt(p.epi.scale, p.epi.scale_dtype, p.epi.scale_bcast ? 0 : n);
-        e.bs_bits[t] = p.epi.bias ? load_bits_rt(p.epi.bias, p.epi.bias_dtype, n) : 0u;
-    }
-}
-
-// The field layout (W_LAYOUT_TILED_FIELDS, FL = true) leaves column block t of a lane scaled by 4^t (64 for t = 3):
-// float(acc) * (127 / 4^t) is the same real number as float(acc / 4^t) * 127 -- the scaled accumulator has the
-// significant bits of the true one and the factor is a power of two apart from 127 -- so the epilogue takes the
-// scale out in the multiplication it already has.
-template <bool FL>
-__device__ __forceinline__ constexpr float k127(int t) {
-    return FL ? (t == 0 ? 127.0f : t == 1 ? 127.0f / 4.0f : t == 2 ? 127.0f / 16.0f : 127.0f / 64.0f) : 127.0f;
-}
-template <bool FL>
-__device__ __forceinline__ constexpr int field_shift(int t) { return FL ? 2 * t : 0; }
-
-template <int YDT, int MB0, int NB, bool FL = false>
-__device__ __forceinline__ void gemm_epilogue(const GemmParams& p, const v4i (&acc)[2 * NB][4], int64_t m0, int g,
-                                              int64_t ncol, const EpiOperands<NB>& e) {
-    float ws[4], bs[4];
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        ws[t] = bits_to_f32_rt(e.ws_bits[t], p.epi.scale_dtype);
-        bs[t] = p.epi.bias ? bits_to_f32_rt(e.bs_bits[t], p.epi.bias_dtype) : 0.0f;
-    }
-#pragma unroll
-    for (int mbi = 0; mbi < NB; mbi++) {
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int64_t m = m0 + 16 * (MB0 + mbi) + 4 * g + r;
-            if (m >= p.M) continue;
-            const float sx = e.sx[mbi][r];
-            float y[4];
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                // float(127 a) = float(a) * 127 rounded once: |a| <= 127 K < 2^24 (checked by the host), so float(a)
-                // is exact and the product rounds the same integer the reference converts (one operation less than
-                // 127 a in integers first)
-                const float a127f = __fmul_rn((float)acc[MB0 + mbi][t][r], k127<FL>(t));
-                y[t] = epi_int8_f(a127f, sx, ws[t], bs[t]);
-            }
-            if (p.epi.residual) add_residual4(y, p.epi.residual, YDT, m * p.N + ncol);
-            store4(p.Y, YDT, m * p.N + ncol, y);
-            if (p.acc_out) {
-                uint32_t a127[4];
-#pragma unroll
-                for (int t = 0; t < 4; t++) a127[t] = (uint32_t)times127(acc[MB0 + mbi][t][r] >> field_shift<FL>(t));
-                st4_nt(p.acc_out + m * p.N + ncol, a127[0], a127[1], a127[2], a127[3]);
-            }
-        }
-    }
-}
-// The same for the common case, with the bookkeeping taken out of the per-row work: every row of the tile exists,
-// no residual, no accumulator output, and every row scale large enough for the two-operation division
-// (all wave-uniform, checked by the caller).  A row's address is a uniform base plus a 32-bit lane offset fixed
-// for the whole epilogue.  Same bits as gemm_epilogue.
-template <int YDT, int MB0, int NB, bool RES = false, bool FL = false>
-__device__ __forceinline__ void gemm_epilogue_fast(const GemmParams& p, const v4i (&acc)[2 * NB][4], int64_t m0, int g,
-                                                   int64_t ncol, const EpiOperands<NB>& e) {
-    float ws[4], bs[4];
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        ws[t] = bits_to_f32_rt(e.ws_bits[t], p.epi.scale_dtype);
-        bs[t] = p.epi.bias ? bits_to_f32_rt(e.bs_bits[t], p.epi.bias_dtype) : 0.0f;
-    }
-    constexpr int ES = (YDT == BT_F32) ? 4 : 2;
-    const int64_t ncol0 = (int64_t)__builtin_amdgcn_readfirstlane((int)(ncol / G_BN)) * G_BN;  // the tile's first column
-    const uint32_t lane_off = ((uint32_t)(4 * g) * (uint32_t)p.N + (uint32_t)(ncol - ncol0)) * ES;
-    char* const base = (char*)p.Y + ((m0 + 16 * MB0) * p.N + ncol0) * ES;  // uniform
-    const int64_t row_bytes = p.N * ES;
-#pragma unroll
-    for (int mbi = 0; mbi < NB; mbi++) {
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const float sx = e.sx[mbi][r];
-            float y[4];
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const float a127f = __fmul_rn((float)acc[MB0 + mbi][t][r], k127<FL>(t));
-                const float q = div127_fast(__fmul_rn(a127f, sx));
-                y[t] = __fadd_rn(__fmul_rn(q, ws[t]), bs[t]);
-            }
-            if constexpr (RES && YDT != BT_F32) {  // linear rounded to the output's dtype, then + residual (add_residual4)
-                const uint32_t d[2] = {e.res[mbi][r].x, e.res[mbi][r].y};
-#pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    const uint32_t h = (d[t >> 1] >> (16 * (t & 1))) & 0xffffu;
-                    const float rv = (YDT == BT_F16) ? f16_bits_to_f32((uint16_t)h) : bf16_bits_to_f32((uint16_t)h);
-                    y[t] = sum_in_dtype(round_to_dtype(y[t], YDT), rv, YDT);
-                }
-            }
-            char* const dst = base + (int64_t)(16 * mbi + r) * row_bytes + lane_off;
-            if constexpr (YDT == BT_F32) {
-                st4_nt((float*)dst, __builtin_bit_cast(uint32_t, y[0]), __builtin_bit_cast(uint32_t, y[1]),
-                       __builtin_bit_cast(uint32_t, y[2]), __builtin_bit_cast(uint32_t, y[3]));
-            } else {
-                uint16_t h[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) h[i] = (YDT == BT_F16) ? f32_to_f16_bits(y[i]) : f32_to_bf16_bits(y[i]);
-                st2_nt((uint16_t*)dst, (uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
-            }
-        }
-    }
-}
-template <int MB0, int NB, bool FL = false>
-__device__ __forceinline__ void gemm_epilogue_dt(const GemmParams& p, const v4i (&acc)[2 * NB][4], int64_t m0, int g,
-                                                 int64_t ncol, const EpiOperands<NB>& e) {
-    if (p.y_dtype == BT_BF16) gemm_epilogue<BT_BF16, MB0, NB, FL>(p, acc, m0, g, ncol, e);
-    else if (p.y_dtype == BT_F16) gemm_epilogue<BT_F16, MB0, NB, FL>(p, acc, m0, g, ncol, e);
-    else gemm_epilogue<BT_F32, MB0, NB, FL>(p, acc, m0, g, ncol, e);
-}
-template <int MB0, int NB, bool FL = false>
-__device__ __forceinline__ void gemm_epilogue_dt(const GemmParams& p, const v4i (&acc)[2 * NB][4], int64_t m0, int g,
-                                                 int64_t ncol, const EpiOperands<NB>& e, bool fast) {
-    if (fast) {  // wave-uniform
-        if (p.epi.residual) {  // (16-bit outputs only: checked by the caller)
-            if (p.y_dtype == BT_BF16) gemm_epilogue_fast<BT_BF16, MB0, NB, true, FL>(p, acc, m0, g, ncol, e);
-            else gemm_epilogue_fast<BT_F16, MB0, NB, true, FL>(p, acc, m0, g, ncol, e);
-        } else if (p.y_dtype == BT_BF16) gemm_epilogue_fast<BT_BF16, MB0, NB, false, FL>(p, acc, m0, g, ncol, e);
-        else if (p.y_dtype == BT_F16) gemm_epilogue_fast<BT_F16, MB0, NB, false, FL>(p, acc, m0, g, ncol, e);
-        else gemm_epilogue_fast<BT_F32, MB0, NB, false, FL>(p, acc, m0, g, ncol, e);
-        return;
-    }
-    gemm_epilogue_dt<MB0, NB, FL>(p, acc, m0, g, ncol, e);
-}
 
 // Adding the two K halves: waves (wn, 0) and (wn, 1) hold partial sums of the same outputs.  K half 1 hands over row
 // blocks 0..3 and finishes 4..7, K half 0 the other way round, through one 64 KiB area of LDS (the stage buffers, dead
@@ -687,15 +487,20 @@ __global__ __launch_bounds__(512) void gemm_i8_kernel(GemmParams p) {
 
 // the same kernel on the decode-tiled weight copy (256-byte aligned, below 4 GiB: checked by the caller)
 bool gemm_i8_supported_tiled(int64_t N, int64_t K, const void* Q) {
-    return N % 4 == 0 && K % 16 == 0 && ((uintptr_t)Q) % 16 == 0 && (G_BM + 1) * K < (1ll << 32);
+    // (N: 32-bit byte offsets within 16 rows of a 32-bit output)
+    return N % 4 == 0 && N < (1ll << 26) && K % 16 == 0 && ((uintptr_t)Q) % 16 == 0 && (G_BM + 1) * K < (1ll << 32);
 }
 
 // the tiled kernel reads Q with 16-byte loads and W_T / Y with 4-column vectors
 bool gemm_i8_supported(int64_t N, int64_t K, const void* Q, const void* W_T) {
     // 32-bit per-lane offsets: a row tile of Q and the whole of W_T stay below 4 GiB
-    return N % 4 == 0 && K % 16 == 0 && ((uintptr_t)W_T) % 4 == 0 && ((uintptr_t)Q) % 16 == 0 &&
+    return N % 4 == 0 && N < (1ll << 26) && K % 16 == 0 && ((uintptr_t)W_T) % 4 == 0 && ((uintptr_t)Q) % 16 == 0 &&
            (G_BM + 1) * K < (1ll << 32) && ceil_div(K, 4) * N < (1ll << 32);
 }
+
+// gemm_i8_dma.hip
+int gemm_i8_dma_rows(int64_t M, int64_t N, int64_t K, bool tiled);
+int launch_gemm_i8_dma(const GemmParams& p, int rows, bool tiled, bool fields, hipStream_t st);
 
 // One launch over column tiles [tile_n0, tile_n0 + tiles_n) in tiles of 32 * NB rows.
 template <int NB>
@@ -717,20 +522,14 @@ static int launch_gemm_i8_part(GemmParams p, int tile_n0, int tiles_n, bool qoo,
     } else if constexpr (NB != 4) {  // (only where launch_gemm_i8 cuts finer: tiled weights, whole stages)
         if (qoo) hipLaunchKernelGGL((gemm_i8_kernel<false, true, true, true, NB>), grid, block, 0, st, p);
         else hipLaunchKernelGGL((gemm_i8_kernel<false, false, true, true, NB>), grid, block, 0, st, p);
+    } else if (tiled && qoo) {  // (whole stages: gemm_i8_dma_rows takes the others)
+        if (tuning_env("BITTORCH_GEMM_INPHASE")) hipLaunchKernelGGL((gemm_i8_kernel<false, true, true, false>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((gemm_i8_kernel<false, true, true>), grid, block, 0, st, p);
     } else if (tiled) {
-        if (!tail) {
-            if (qoo && tuning_env("BITTORCH_GEMM_INPHASE")) hipLaunchKernelGGL((gemm_i8_kernel<false, true, true, false>), grid, block, 0, st, p);
-            else if (qoo) hipLaunchKernelGGL((gemm_i8_kernel<false, true, true>), grid, block, 0, st, p);
-            else hipLaunchKernelGGL((gemm_i8_kernel<false, false, true>), grid, block, 0, st, p);
-        } else {
-            if (qoo) hipLaunchKernelGGL((gemm_i8_kernel<true, true, true>), grid, block, 0, st, p);
-            else hipLaunchKernelGGL((gemm_i8_kernel<true, false, true>), grid, block, 0, st, p);
-        }
-    } else if (!tail) {
-        if (qoo) hipLaunchKernelGGL((gemm_i8_kernel<false, true>), grid, block, 0, st, p);
-        else hipLaunchKernelGGL((gemm_i8_kernel<false, false>), grid, block, 0, st, p);
+        if (!tail) hipLaunchKernelGGL((gemm_i8_kernel<false, false, true>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((gemm_i8_kernel<true, false, true>), grid, block, 0, st, p);
     } else {
-        if (qoo) hipLaunchKernelGGL((gemm_i8_kernel<true, true>), grid, block, 0, st, p);
+        if (!tail) hipLaunchKernelGGL((gemm_i8_kernel<false, false>), grid, block, 0, st, p);
         else hipLaunchKernelGGL((gemm_i8_kernel<true, false>), grid, block, 0, st, p);
     }
     return check_launch("bt_ternary_gemm_i8");
@@ -749,6 +548,8 @@ int launch_gemm_i8(const int8_t* Q, int q_layout, const float* s_x, const int32_
     p.tiles16 = tiles16_arg(N, w_layout);
     const bool qoo = q_layout == Q_OPERAND_ORDER, tiled = layout_tiled(w_layout), fields = layout_fields(w_layout);
     const int64_t tiles_n = ceil_div(N, G_BN);
+    const int dma_nb = qoo ? gemm_i8_dma_rows(M, N, K, tiled) : 0;  // (gemm_i8_dma.hip)
+    if (dma_nb) return launch_gemm_i8_dma(p, dma_nb, tiled, fields, st);
     // the column tiles of a mostly empty last round in finer tiles, a launch of their own behind the whole tiles
     // (gemm_split; same sums, same bits)
     const GemmSplit sp = gemm_split(M, N, tiled && K % G_BK == 0 && !tuning_env("BITTORCH_GEMM_INPHASE"));

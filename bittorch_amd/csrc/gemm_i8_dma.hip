@@ -1,0 +1,455 @@
+// Tiled int8 x packed-ternary GEMM on activations in operand order: two independent workgroups per compute unit.
+// Arithmetic as in gemm_i8.hip (csrc/kernels/ternary_gemm_tensor_core.cu:73-75, :343-347, :583-589, :652).
+//
+// A 256-thread workgroup (4 waves) owns a tile of 32 NB x 256 outputs; wave w works on columns 64 w .. +63 over the whole of
+// K, so nothing has to be added up at the end, and two workgroups share a compute unit: while one waits, starts, drains or
+// stores, the other one's MFMAs run.  Bound by the issue of a stage: 32 MFMAs (512 cycles) and some 60 other instructions;
+// 2.2 to 2.9 POPS at K = 2560 .. 8192 (4096 x 8192 x 8192 192 us, 207 with the K halves of gemm_i8_kernel).
+//   * Everything that comes from memory goes to LDS without passing through registers (global_load_lds, 16 bytes a lane):
+//     the activations in the operand order the quantizer wrote them in, and each wave's packed weights (1 KiB a stage).  A
+//     stage is 64 k; five stages are in LDS, so a load has three stages (1500 to 4000 cycles) to arrive.
+//   * A stage: 16 MFMAs of row blocks 0..3 with the decode of the next stage's weights behind them, the one barrier, 16
+//     MFMAs of row blocks 4..7 under which the fragments of the next stage's row blocks 0..3 arrive.
+// The loads are counted by hand (the compiler does not see them): `vmcnt` in front of the barrier of stage s leaves the
+// loads of stages s + 3 and s + 4 in flight, so stage s + 1 (fragments) and s + 2 (the weights decoded one stage ahead) are
+// complete; that barrier also stands between the last read of stage s's buffer and the loads of stage s + 5 into it.
+#include "gemm_i8_common.h"
+
+namespace bt {
+
+constexpr int D_BK = 64;   // k per stage
+constexpr int D_NST = 5;   // stages in LDS (60 KiB: what M0's 16-bit byte offset reaches)
+
+// 16 (4) bytes a lane from sbase + voff to LDS byte lds_off + 16 (4) * lane
+__device__ __forceinline__ void dma16(uint32_t lds_off, uint32_t voff, const void* sbase) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_off)), "v"(voff), "s"(sbase) : "memory");
+}
+__device__ __forceinline__ void dma4(uint32_t lds_off, uint32_t voff, const void* sbase) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_off)), "v"(voff), "s"(sbase) : "memory");
+}
+
+enum { W_ROWS = 0, W_TILES = 1, W_FIELDS = 2 };  // row-major W_T, the decode-tiled copy, its field layout
+
+// Output stage: row block by row block, addresses as a uniform row base plus a lane offset fixed for the whole tile.  The
+// empty asm statements keep a row's address from being computed ahead of its turn (left alone, the compiler holds all 32
+// row addresses and residual values at once and spills).
+template <int NB, bool FL>
+__device__ __forceinline__ void dma_store_acc(const GemmParams& p, const v4i (&acc)[2 * NB][4], int64_t m0, int g, int64_t ncol,
+                                              int rows_left) {
+    const uint32_t lane_off = (uint32_t)(4 * g) * (uint32_t)p.N * 4u + (uint32_t)(ncol & (G_BN - 1)) * 4u;
+    char* row = (char*)p.acc_out + (m0 * p.N + (int64_t)__builtin_amdgcn_readfirstlane((int)(ncol / G_BN)) * G_BN) * 4;
+#pragma unroll
+    for (int mb = 0; mb < 2 * NB; mb++) {
+        if (16 * mb >= rows_left) return;  // (uniform)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            asm volatile("" : "+s"(row));
+            if (16 * mb + 4 * g + r < rows_left) {
+                uint32_t a[4];
+#pragma unroll
+                for (int t = 0; t < 4; t++) a[t] = (uint32_t)times127(acc[mb][t][r] >> field_shift<FL>(t));
+                st4_nt(row + lane_off, a[0], a[1], a[2], a[3]);
+            }
+            row += p.N * 4;
+        }
+        row += 12 * p.N * 4;
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+template <int YDT, bool RES, int NB, bool FL>
+__device__ __forceinline__ void dma_epilogue(const GemmParams& p, const v4i (&acc)[2 * NB][4], int64_t m0, int g, int64_t ncol,
+                                             int rows_left, const float* sx_lds, const float (&ws)[4], const float (&bs)[4]) {
+    constexpr int ES = (YDT == BT_F32) ? 4 : 2;
+    const uint32_t lane_off = ((uint32_t)(4 * g) * (uint32_t)p.N + (uint32_t)(ncol & (G_BN - 1))) * ES;
+    const int64_t first = (m0 * p.N + (int64_t)__builtin_amdgcn_readfirstlane((int)(ncol / G_BN)) * G_BN) * ES;
+    const int64_t row_bytes = p.N * ES;
+    char* row = (char*)p.Y + first;
+    const char* res = (const char*)p.epi.residual + first;
+#pragma unroll
+    for (int mb = 0; mb < 2 * NB; mb++) {
+        if (16 * mb >= rows_left) return;  // (uniform)
+        const float4 s4 = *(const float4*)(sx_lds + 16 * mb + 4 * g);
+        const float sx[4] = {s4.x, s4.y, s4.z, s4.w};
+        uint4 rv[4];
+        if constexpr (RES) {  // the block's four rows at once
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                asm volatile("" : "+s"(res));
+                const char* src = res + (16 * mb + 4 * g + r < rows_left ? lane_off : 0u);
+                if constexpr (YDT == BT_F32) rv[r] = *(const uint4*)src;
+                else { const uint2 v = *(const uint2*)src; rv[r] = make_uint4(v.x, v.y, 0u, 0u); }
+                res += (16 * mb + r + 1 < rows_left) ? row_bytes : 0;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            asm volatile("" : "+s"(row));
+            if (16 * mb + 4 * g + r < rows_left) {
+                float y[4];
+#pragma unroll
+                for (int t = 0; t < 4; t++) y[t] = epi_int8_f(__fmul_rn((float)acc[mb][t][r], k127<FL>(t)), sx[r], ws[t], bs[t]);
+                if constexpr (RES) {
+                    const uint32_t d[4] = {rv[r].x, rv[r].y, rv[r].z, rv[r].w};
+#pragma unroll
+                    for (int t = 0; t < 4; t++) {
+                        const uint32_t bits = YDT == BT_F32 ? d[t] : (d[t >> 1] >> (16 * (t & 1))) & 0xffffu;
+                        y[t] = sum_in_dtype(round_to_dtype(y[t], YDT), bits_to_f32_rt(bits, YDT), YDT);
+                    }
+                }
+                store4(row + lane_off, YDT, 0, y);
+            }
+            row += row_bytes;
+        }
+        row += 12 * row_bytes;
+        if constexpr (RES) res = row - (char*)p.Y + (const char*)p.epi.residual;
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+constexpr int dma_lds_bytes(int NB) { return D_NST * (2 * NB * 1024 + 4096); }
+
+// One tile of 32 NB rows.  TAIL: K is not a multiple of the stage.  The activations past the end of K are some of the same
+// row's and meet weights of zero: the tiled copy is padded with them, raw row-major dwords are masked.
+template <int SRC, int NB, bool TAIL>
+__device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int64_t m0, const int tile_n, uint8_t* lds) {
+    constexpr int BM = 32 * NB;
+    constexpr int A_BYTES = 2 * NB * 1024, STAGE = A_BYTES + 4096;
+    constexpr int A_LOADS = NB == 4 ? 2 : 1, W_LOADS = SRC == W_ROWS ? 4 : 1, LOADS = A_LOADS + W_LOADS;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int j = lane & 15, g = lane >> 4;
+    const int64_t ncol = (int64_t)tile_n * G_BN + 64 * wave + 4 * j;
+    const bool col_ok = ncol < p.N;
+    const int nst = (int)((p.K + D_BK - 1) / D_BK);
+    const int64_t k_last = (int64_t)(nst - 1) * D_BK;
+
+    // Lane (i, c = lane / 16) loads 16 bytes of row i of its row block at k = 16 c: LDS then holds slot (block, lane) as
+    // the MFMA lane reads it.  Rows past M repeat the last one (their outputs are never stored); columns past N read
+    // column 0 of row-major weights and the last tile of the copy.
+    const int64_t rows_left = (p.M - m0 < BM) ? p.M - m0 : BM;
+    uint32_t a_off[A_LOADS], a_tail[A_LOADS];
+#pragma unroll
+    for (int b = 0; b < A_LOADS; b++) {
+        const int row = 16 * ((A_LOADS * wave + b) % (2 * NB)) + j;
+        const uint32_t r = (uint32_t)(row < rows_left ? row : rows_left - 1);
+        a_off[b] = r * (uint32_t)p.K + 16u * g;
+        a_tail[b] = r * (uint32_t)p.K + (k_last + 16 * g < p.K ? 16u * g : 0u);
+    }
+    uint32_t w_off[W_LOADS], w_tail[W_LOADS];
+    const bool w_in = !TAIL || SRC != W_ROWS || k_last + 16 * g < p.K;  // this lane's rows of the last stage exist
+    if constexpr (SRC == W_ROWS) {
+#pragma unroll
+        for (int r = 0; r < W_LOADS; r++) {
+            w_off[r] = (uint32_t)(col_ok ? ncol : 0) + (uint32_t)(4 * g + r) * (uint32_t)p.N;
+            w_tail[r] = (uint32_t)(col_ok ? ncol : 0) + (w_in ? (uint32_t)(4 * g + r) * (uint32_t)p.N : 0u);
+        }
+    } else {
+        const int tt = stored_tile16((int)(ncol >> 4), p.tiles16);
+        w_off[0] = ((uint32_t)tt * (uint32_t)p.wsteps * 64u + (uint32_t)(16 * g + 4 * (j & 3))) * 4u;
+    }
+    const int8_t* const a_base = p.Q + m0 * p.K;  // uniform
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+
+    // the next stage to load: its global addresses, and the byte offset of its buffer
+    const int8_t* a_next = a_base;
+    const uint8_t* w_next = p.W_T;
+    uint32_t into = 0;
+    int st_next = 0;
+    const int64_t w_step = SRC == W_ROWS ? 16 * p.N : 256;
+    auto issue_a = [&](int b) {
+        const bool last = TAIL && st_next >= nst - 1;
+        dma16(lds0 + into + (uint32_t)((A_LOADS * wave + b) % (2 * NB)) * 1024u, last ? a_tail[b] : a_off[b], a_next);
+    };
+    auto issue_w = [&](int r) {
+        const bool last = TAIL && st_next >= nst - 1;
+        const uint32_t wd = lds0 + into + A_BYTES + (uint32_t)wave * 1024u;
+        if constexpr (SRC == W_ROWS) dma4(wd + 256u * r, last ? w_tail[r] : w_off[r], w_next);
+        else dma16(wd, w_off[0], w_next);
+    };
+    auto next_buf = [](uint32_t b) { return b + STAGE == D_NST * STAGE ? 0u : b + STAGE; };
+    auto advance = [&]() {  // past the end: the last stage again, never read
+        st_next++;
+        a_next += st_next < nst ? D_BK : 0;
+        w_next += st_next < nst ? w_step : 0;
+        into = next_buf(into);
+    };
+
+    v4i acc[2 * NB][4];
+#pragma unroll
+    for (int mb = 0; mb < 2 * NB; mb++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) acc[mb][t] = v4i{0, 0, 0, 0};
+    if constexpr (SRC == W_FIELDS) {  // lane (j, g) holds rows 16 mb + 4 g + r of its columns
+#pragma unroll
+        for (int mb = 0; mb < 2 * NB; mb++) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int64_t m = m0 + 16 * mb + 4 * g + r;
+                const int32_t rs = p.q_rowsum[m < p.M ? m : p.M - 1];
+                acc[mb][0][r] = -rs;
+                acc[mb][1][r] = -(rs << 2);
+                acc[mb][2][r] = -(rs << 4);
+            }
+        }
+    }
+
+    uint4 a_lo[NB], a_hi[NB];
+    v4i b_dec[2][4];
+    uint32_t raw[4];
+    auto read_raw = [&](int s, uint32_t buf) {
+        const uint8_t* src = lds + buf + A_BYTES + wave * 1024;
+        if constexpr (SRC == W_ROWS) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) raw[r] = *(const uint32_t*)(src + 256 * r + 4 * lane);
+            if (TAIL && s >= nst - 1) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) raw[r] = w_in ? raw[r] : 0u;
+            }
+        } else {
+            const uint4 v = *(const uint4*)(src + 16 * lane);
+            raw[0] = v.x; raw[1] = v.y; raw[2] = v.z; raw[3] = v.w;
+        }
+    };
+    auto read_a = [&](uint32_t buf, int mb0, uint4 (&dst)[NB]) {
+        const uint8_t* src = lds + buf + 16 * lane;
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            dst[i] = *(const uint4*)(src + (mb0 + i) * 1024);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // the decode of one stage's weights in 16 slices, one behind each MFMA of a half
+    uint32_t d_t[4], d_G[4], d_H[4];
+    auto decode_slice = [&](int c, v4i (&out)[4]) {
+        const uint32_t lutA_lo = 0x00FF0100u, lutB_lo = 0x0000FF00u, lutB_hi = 0x00000001u;
+        if constexpr (SRC == W_FIELDS) {
+            out[c >> 2][c & 3] = (int)(raw[c & 3] & (0x03030303u << (2 * (c >> 2))));
+            return;
+        }
+        if constexpr (SRC == W_TILES) {
+            const int t = c >> 2;
+            switch (c & 3) {
+                case 0: d_G[t] = raw[t]; d_H[t] = d_G[t] >> 4; out[t][0] = (int)perm(0u, lutA_lo, d_G[t] & 0x03030303u); break;
+                case 1: out[t][1] = (int)perm(lutB_hi, lutB_lo, d_G[t] & 0x0C0C0C0Cu); break;
+                case 2: out[t][2] = (int)perm(0u, lutA_lo, d_H[t] & 0x03030303u); break;
+                default: out[t][3] = (int)perm(lutB_hi, lutB_lo, d_H[t] & 0x0C0C0C0Cu); break;
+            }
+            return;
+        }
+        // row-major dwords: the 4x4 byte transpose in slices 2 and 3, then three slices per column
+        if (c == 2) {
+            d_t[0] = perm(raw[1], raw[0], 0x05010400u);
+            d_t[1] = perm(raw[1], raw[0], 0x07030602u);
+            d_t[2] = perm(raw[3], raw[2], 0x05010400u);
+            d_t[3] = perm(raw[3], raw[2], 0x07030602u);
+        } else if (c == 3) {
+            d_G[0] = perm(d_t[2], d_t[0], 0x05040100u);
+            d_G[1] = perm(d_t[2], d_t[0], 0x07060302u);
+            d_G[2] = perm(d_t[3], d_t[1], 0x05040100u);
+            d_G[3] = perm(d_t[3], d_t[1], 0x07060302u);
+        } else if (c >= 4) {
+            const int t = (c - 4) / 3;
+            switch ((c - 4) % 3) {
+                case 0: d_H[t] = d_G[t] >> 4; out[t][0] = (int)perm(0u, lutA_lo, d_G[t] & 0x03030303u); break;
+                case 1:
+                    out[t][1] = (int)perm(lutB_hi, lutB_lo, d_G[t] & 0x0C0C0C0Cu);
+                    out[t][2] = (int)perm(0u, lutA_lo, d_H[t] & 0x03030303u);
+                    break;
+                default: out[t][3] = (int)perm(lutB_hi, lutB_lo, d_H[t] & 0x0C0C0C0Cu); break;
+            }
+        }
+    };
+
+    uint32_t buf = 0;
+#pragma unroll
+    for (int s = 0; s < D_NST; s++) {
+#pragma unroll
+        for (int b = 0; b < A_LOADS; b++) issue_a(b);
+#pragma unroll
+        for (int r = 0; r < W_LOADS; r++) issue_w(r);
+        advance();
+    }
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((D_NST - 2) * LOADS) : "memory");  // stages 0 and 1
+    read_raw(0, 0);
+    read_a(0, 0, a_lo);
+#pragma unroll
+    for (int c = 0; c < 16; c++) decode_slice(c, b_dec[0]);
+    read_raw(1, STAGE);
+
+    // Everything but the MFMAs is dealt out between them, two or three instructions behind each: an MFMA occupies the
+    // matrix pipe for 16 cycles, the wave's own issue for 4, and instructions in a row of their own would leave the pipe idle.
+    auto stage = [&](int s, const v4i (&b_cur)[4], v4i (&b_nxt)[4]) {
+        constexpr int SL = 4 / NB;  // slots per MFMA
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int c = 0; c < 16; c++) {
+            if (c % SL == 0) {
+                const int i = (c / SL) >> 2, t = (c / SL) & 3;
+                const v4i a = {(int)a_lo[i].x, (int)a_lo[i].y, (int)a_lo[i].z, (int)a_lo[i].w};
+                acc[i][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b_cur[t], acc[i][t], 0, 0, 0);
+            }
+            if (c < NB) a_hi[c] = *(const uint4*)(lds + buf + 16 * lane + (NB + c) * 1024);
+            decode_slice(c, b_nxt);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((D_NST - 3) * LOADS) : "memory");
+        const uint32_t nxt = next_buf(buf), nxt2 = next_buf(nxt);
+#pragma unroll
+        for (int c = 0; c < 16; c++) {
+            if (c % SL == 0) {
+                const int i = (c / SL) >> 2, t = (c / SL) & 3;
+                const v4i a = {(int)a_hi[i].x, (int)a_hi[i].y, (int)a_hi[i].z, (int)a_hi[i].w};
+                acc[NB + i][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b_cur[t], acc[NB + i][t], 0, 0, 0);
+            }
+            if (c < NB) a_lo[c] = *(const uint4*)(lds + nxt + 16 * lane + c * 1024);
+            if (c == 4) read_raw(s + 2, nxt2);
+            // stage s + 5 over stage s
+            if (c >= 6 && c < 6 + A_LOADS) issue_a(c - 6);
+            if (c >= 8 && c < 8 + W_LOADS) issue_w(c - 8);
+            if (c == 13) advance();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        buf = nxt;
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the fragments arrived under these MFMAs (see gemm_i8_kernel)
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int s = 0;
+    for (; s + 1 < nst; s += 2) {
+        stage(s, b_dec[0], b_dec[1]);
+        stage(s + 1, b_dec[1], b_dec[0]);
+    }
+    if (s < nst) stage(s, b_dec[0], b_dec[1]);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (no load may reach LDS that another workgroup owns by then)
+
+    // ---- output.  The row scales of the tile pass through the wave's own weight area in LDS (nobody else's loads reach it),
+    // so that a row block's four come with one read. ----
+    float* const sx_lds = (float*)(lds + A_BYTES + wave * 1024);
+    uint32_t ws_bits[4], bs_bits[4];
+#pragma unroll
+    for (int q = 0; q < (NB == 4 ? 2 : 1); q++) {
+        const int64_t m = m0 + 64 * q + lane;
+        sx_lds[64 * q + lane] = p.s_x[m < p.M ? m : p.M - 1];
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int64_t n = col_ok ? ncol + t : 0;
+        ws_bits[t] = load_bits_rt(p.epi.scale, p.epi.scale_dtype, p.epi.scale_bcast ? 0 : n);
+        bs_bits[t] = p.epi.bias ? load_bits_rt(p.epi.bias, p.epi.bias_dtype, n) : 0u;
+    }
+    float ws[4], bs[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        ws[t] = bits_to_f32_rt(ws_bits[t], p.epi.scale_dtype);
+        bs[t] = p.epi.bias ? bits_to_f32_rt(bs_bits[t], p.epi.bias_dtype) : 0.0f;
+    }
+    if (!col_ok) return;
+    if (p.acc_out) dma_store_acc<NB, SRC == W_FIELDS>(p, acc, m0, g, ncol, (int)rows_left);
+    if (p.y_dtype == BT_BF16) {
+        if (p.epi.residual) dma_epilogue<BT_BF16, true, NB, SRC == W_FIELDS>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
+        else dma_epilogue<BT_BF16, false, NB, SRC == W_FIELDS>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
+    } else if (p.y_dtype == BT_F16) {
+        if (p.epi.residual) dma_epilogue<BT_F16, true, NB, SRC == W_FIELDS>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
+        else dma_epilogue<BT_F16, false, NB, SRC == W_FIELDS>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
+    } else {
+        if (p.epi.residual) dma_epilogue<BT_F32, true, NB, SRC == W_FIELDS>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
+        else dma_epilogue<BT_F32, false, NB, SRC == W_FIELDS>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
+    }
+}
+
+// NB: tiles of 32 NB rows.  NF > 0: the last p.fine_from .. of an XCD's tiles are computed in tiles of 32 NF rows.
+template <int SRC, int NB, int NF, bool TAIL>
+__global__ __launch_bounds__(256, NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_i8_dma_kernel(GemmParams p) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds[dma_lds_bytes(NB)];
+    // XCD-aware tile order, as in gemm_i8_kernel
+    const uint32_t idx = blockIdx.x >> 3;
+    const bool fine = NF > 0 && idx >= (uint32_t)p.fine_from;  // (uniform)
+    const uint32_t parts = NF > 0 ? NB / (NF > 0 ? NF : 1) : 1, f = fine ? idx - (uint32_t)p.fine_from : 0u;
+    const uint32_t in_xcd = fine ? (uint32_t)p.fine_from + f / parts : idx;
+    const uint32_t lin = (blockIdx.x & 7u) * (uint32_t)p.per_xcd + in_xcd;
+    const uint32_t tiles_m = (uint32_t)p.tiles_m, tiles_n = (uint32_t)p.tiles_n;
+    if (lin >= tiles_m * tiles_n) return;
+    constexpr uint32_t GM = 4;
+    const uint32_t group = lin / (GM * tiles_n);
+    const uint32_t first_m = group * GM;
+    const uint32_t gm = (tiles_m - first_m < GM) ? tiles_m - first_m : GM;
+    const uint32_t in_group = lin - group * GM * tiles_n;
+    const uint32_t tn = (gm == GM) ? in_group / GM : in_group / gm;
+    const int64_t m0 = (int64_t)(first_m + (in_group - tn * gm)) * (32 * NB);
+    if constexpr (NF > 0) {
+        if (fine) {
+            const int64_t mf = m0 + (int64_t)(f % parts) * (32 * NF);
+            if (mf < p.M) gemm_i8_dma_tile<SRC, NF, TAIL>(p, mf, (int)tn, lds);
+            return;
+        }
+    }
+    gemm_i8_dma_tile<SRC, NB, TAIL>(p, m0, (int)tn, lds);
+}
+
+// Into how many finer ones the last, incomplete round of an XCD's 128-row tiles is cut.  Two workgroups that end together
+// free their compute unit for the next two, so a remainder of whole tiles runs in pairs on a part of the chip.  Measured
+// (row-major weights, us, whole / halves / quarters; remainder of 64): 2048 x 11008 x 4096 (22) 104 / 97 / 111; 2900 x 6400 x
+// 6400 (8) 136 / 120 / 122, tiled 120 / 112 / 106; 4096 x 4100 x 4096 (4) 98 / 88 / 86; 2304 x 4096 x 4096 (36) 56 / 63 / 80.
+static int gemm_i8_dma_parts(int64_t tiles) {
+    const int64_t slots = 2 * gemm_compute_units() / 8, rem = ceil_div(tiles, 8) % slots;
+    return rem == 0 || 2 * rem > slots ? 1 : 5 * rem > slots ? 2 : 4;
+}
+// Rows of the tiles in units of 32 (4, 2 or 1), or 0 where gemm_i8_kernel is the better one: tiled weights in whole stages
+// with at most one tile of 128 x 256 for each compute unit.  There a second workgroup has nothing to do, and splitting K
+// over the two waves of a SIMD halves the one tile's chain (K = N = 4096: M = 2048 28.3 us against 30.5 here, M = 512 in its
+// tiles of 32 rows 15.9 against 18.5).  With more tiles (tiled / row-major weights, us, that kernel first): 4096 x 13824 x
+// 2560 133 -> 122 / 148 -> 134; 2048 x 11008 x 4096 93 -> 82 / 104 -> 88; 4096 x 2560 x 6912 (64-row tiles) 67 -> 65 / 85 ->
+// 73; 4096 x 8192 x 8192 207 -> 192 / 250 -> 208; 3000 x 1008 x 1040, K not in whole stages, 38 -> 13 / 16 -> 14.
+// Row-major weights of few tiles: M = 1024, 512 (N = K = 4096) 27.3 -> 25.2, 22.9.
+// The prices are microseconds of a compute unit's run of tiles, fitted to the same runs.
+int gemm_i8_dma_rows(int64_t M, int64_t N, int64_t K, bool tiled) {
+    const int64_t C = gemm_compute_units(), tn = ceil_div(N, G_BN);
+    const int64_t t4 = ceil_div(M, 128) * tn, t2 = ceil_div(M, 64) * tn, t1 = ceil_div(M, 32) * tn;
+    if (tiled && K % 128 == 0 && t4 <= C) return 0;
+    if (t1 <= C) return 1;
+    if (t2 <= C) return 2;
+    const int parts = gemm_i8_dma_parts(t4);
+    const double n4 = parts == 1 ? (double)ceil_div(t4, C) : (double)(2 * (t4 / (2 * C))) + (parts == 2 ? 1.2 : 0.6);
+    return (double)ceil_div(t2, C) * (2.2 + 0.0029 * (double)K) < n4 * (3.5 + 0.0055 * (double)K) ? 2 : 4;
+}
+
+template <int SRC, int NB, bool TAIL>
+static int launch_gemm_i8_dma_src(GemmParams p, hipStream_t st) {
+    p.tile_n0 = 0;
+    p.tiles_n = (int)ceil_div(p.N, G_BN);
+    p.tiles_m = (int)ceil_div(p.M, 32 * NB);
+    const int64_t total = (int64_t)p.tiles_m * p.tiles_n;
+    if (total >= (1ll << 29)) {
+        set_error("bt_ternary_gemm_i8: %lld tiles of %d x 256 outputs are more than one launch takes", (long long)total, 32 * NB);
+        return BT_ERR_INVALID;
+    }
+    p.per_xcd = (int)ceil_div(total, 8);
+    p.fine_from = p.per_xcd;
+    const dim3 block(256);
+    if constexpr (NB == 4) {
+        const int parts = gemm_i8_dma_parts(total);
+        if (parts > 1) {
+            const int rem = p.per_xcd % (int)(2 * gemm_compute_units() / 8);
+            p.fine_from = p.per_xcd - rem;
+            const dim3 grid((unsigned)(8 * (p.fine_from + parts * rem)));
+            if (parts == 2) hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, 4, 2, TAIL>), grid, block, 0, st, p);
+            else hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, 4, 1, TAIL>), grid, block, 0, st, p);
+            return check_launch("bt_ternary_gemm_i8");
+        }
+    }
+    hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, NB, 0, TAIL>), dim3((unsigned)(8 * p.per_xcd)), block, 0, st, p);
+    return check_launch("bt_ternary_gemm_i8");
+}
+template <int NB>
+static int launch_gemm_i8_dma_rows(const GemmParams& p, bool tiled, bool fields, hipStream_t st) {
+    const bool tail = p.K % D_BK != 0;
+    if (fields) return launch_gemm_i8_dma_src<W_FIELDS, NB, false>(p, st);
+    if (tiled) return tail ? launch_gemm_i8_dma_src<W_TILES, NB, true>(p, st) : launch_gemm_i8_dma_src<W_TILES, NB, false>(p, st);
+    return tail ? launch_gemm_i8_dma_src<W_ROWS, NB, true>(p, st) : launch_gemm_i8_dma_src<W_ROWS, NB, false>(p, st);
+}
+int launch_gemm_i8_dma(const GemmParams& p, int rows, bool tiled, bool fields, hipStream_t st) {
+    return rows == 4 ? launch_gemm_i8_dma_rows<4>(p, tiled, fields, st)
+         : rows == 2 ? launch_gemm_i8_dma_rows<2>(p, tiled, fields, st) : launch_gemm_i8_dma_rows<1>(p, tiled, fields, st);
+}
+
+}  // namespace bt
