@@ -37,7 +37,6 @@ EXTRA_FLAGS = {
     # the iterative ILP scheduler keeps the MFMA accumulators in place across the
     # software-pipelined main loop (the default strategy permutes them every iteration)
     "gemm_i8.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
-    "gemm_f16.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
 }
 
 

@@ -55,7 +55,7 @@ static inline const char* tuning_env(const char* name) { return getenv(name); }
 static inline const char* tuning_env(const char*) { return nullptr; }
 #endif
 
-// ---- the remainder of a tiled GEMM launch (gemm_i8.hip, gemm_f16.hip, and the rule that routes a batch to them) ------
+// ---- the remainder of a tiled GEMM launch (gemm_i8.hip, and the rule that routes a batch to it) ------
 // Workgroups take 128 x 256 tiles in rounds of one per compute unit.  When the last round holds tiles for at most half
 // of the compute units, the column tiles of that remainder are computed in tiles of 64 or 32 rows instead (nb = 2 or 1
 // row blocks per K half and wave), two or four workgroups where there was one, in a launch of their own behind the

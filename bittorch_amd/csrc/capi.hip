@@ -84,9 +84,9 @@ int launch_row_op(int op, int dtype, const void* A, int64_t lda, const void* Bv,
                   int64_t K, void* H, int8_t* Q, float* s_x, int q_layout, int32_t* rowsum, hipStream_t st,
                   const char* who);
 bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, const void* Y);
-bool gemm_f16_supported_tiled(int64_t N, int64_t K, const void* X, const void* Y);
-int launch_gemm_f16(int mode, const void* X, const uint8_t* W_T, int w_layout, const Epilogue& epi, void* Y, int y_dtype,
-                    int64_t M, int64_t N, int64_t K, hipStream_t st);
+double gemm_f16_cost(int64_t M, int64_t N, int64_t K);
+int launch_gemm_f16(int mode, const void* X, const uint8_t* W_T, int w_layout, const Epilogue& epi, void* Y, int64_t M,
+                    int64_t N, int64_t K, hipStream_t st);
 bool gemm_f32_supported(int64_t N, int64_t K, const void* X, const void* Y);
 double gemm_f32_cost(int64_t M, int64_t N, int64_t K);
 int launch_gemm_f32(const void* X, const uint8_t* W, int w_layout, const Epilogue& epi, void* Y, int64_t M, int64_t N,
@@ -107,6 +107,7 @@ bool planes_bf16_shape_ok(int64_t N, int64_t K);
 bool planes_bf16_wide(int64_t N, int64_t K);
 int launch_planes_bf16_wide(const void* X, const uint8_t* W, const Epilogue& epi, void* Y, int64_t N, int64_t K, hipStream_t st);
 bool gemm_i8_supported_tiled(int64_t N, int64_t K, const void* Q);
+double gemm_i8_cost(int64_t M, int64_t N, int64_t K, bool tiled, bool operand_order);
 int launch_gemm_i8(const int8_t* Q, int q_layout, const float* s_x, const int32_t* q_rowsum, const uint8_t* W_T, int w_layout,
                    const Epilogue& epi, void* Y, int y_dtype, int32_t* acc_out, int64_t M, int64_t N, int64_t K,
                    hipStream_t st);
@@ -171,23 +172,20 @@ static const int64_t kMaxKInt8 = 132096;
 // chip (five layer shapes, narrow and shallow ones besides, both weight layouts), in microseconds:
 //   streaming  4 + B N K * 2.2e-9 + 0.003 workgroups (int8),  4 + B N K * 5.0e-9 + 0.004 workgroups (16-bit),
 //              workgroups = 16-row blocks x 128- resp. 64-column tiles
-//   GEMM       rounds * (8.6 + 0.0044 K) (int8),  rounds * (6.9 + 0.010 K) (16-bit)
-// which puts the crossover at 1.5 .. 2 M outputs for K = 2560 .. 4096 (the GEMM would occupy under a fifth of
-// the compute units there) and later for shallow layers.  The option STREAM_MAX_ROWS = n replaces the rule by
-// "B <= n" (tuning and test runs).
-static bool prefers_stream(int64_t B, int64_t N, int64_t K, bool int8, bool tiled = false) {
+//   GEMM       gemm_f16_cost (16-bit), gemm_i8_cost (int8): the launch's plan, priced where it is made
+// e.g. M x 7680 x 2560 on row-major weights, streaming / GEMM: 16-bit M = 77 17 / 20, 200 28 / 22; int8 128 14 / 15, 200 22 / 15;
+// 128 x 16384 x 1024 17 / 12 and 16.5 / 9.7; 512 x 512 x 8192 16.5 / 55 and 11 / 34.
+// The option STREAM_MAX_ROWS = n replaces the rule by "B <= n" (tuning and test runs).
+static bool prefers_stream(int64_t B, int64_t N, int64_t K, bool int8, bool tiled = false, bool operand_order = false) {
     if (const char* env = option(OPT_STREAM_MAX_ROWS)) {
         const long v = atol(env);
         if (v >= 1) return B <= v;
     }
     if (B <= 32) return true;
     const double work = (double)B * (double)N * (double)K;
-    // (rounds of whole tiles, or what the finer tiles of a small launch's remainder cost in them)
-    const double rounds = gemm_split(B, N, tiled && K % (int8 ? 128 : 64) == 0).rounds;
     const double wgs = (double)(ceil_div(B, 16) * ceil_div(N, int8 ? 128 : 64));
     const double t_stream = 4.0 + work * (int8 ? 2.2e-9 : 5.0e-9) + wgs * (int8 ? 0.003 : 0.004);
-    const double t_gemm = rounds * (int8 ? 8.6 + 0.0044 * (double)K : 6.9 + 0.010 * (double)K);
-    return t_stream < t_gemm;
+    return t_stream < (int8 ? gemm_i8_cost(B, N, K, tiled, operand_order) : gemm_f16_cost(B, N, K));
 }
 
 // The same choice for fp32 activations: the streaming kernel on three bf16 planes (split in a launch of its own, about 3 us)
@@ -323,8 +321,8 @@ static int packed_forward_impl(const char* who, const void* X, int x_dtype, cons
         if (x_dtype != BT_F32) {
             const int mode = (x_dtype == BT_F16) ? MODE_F16 : MODE_BF16;
             // tall batches: the tiled matrix-core GEMM reads the copy too (not with the SwiGLU output stage)
-            if (!prefers_stream(B, N, K, false, true) && epi_op == 0 && gemm_f16_supported_tiled(N, K, X, Y))
-                return launch_gemm_f16(mode, X, W_T, w_layout, epi, Y, x_dtype, B, N, K, st);
+            if (!prefers_stream(B, N, K, false, true) && epi_op == 0 && gemm_f16_supported(N, K, X, W_T, Y))
+                return launch_gemm_f16(mode, X, W_T, w_layout, epi, Y, B, N, K, st);
             return launch_stream(mode, X, 2, nullptr, W_T, w_layout, epi, Y, x_dtype, nullptr, B, N, K, 1,
                                  Q_ROW_MAJOR, 0, nullptr, 0.0f, epi_op, st);
         }
@@ -347,7 +345,7 @@ static int packed_forward_impl(const char* who, const void* X, int x_dtype, cons
         const int mode = (x_dtype == BT_F16) ? MODE_F16 : MODE_BF16;
         // tall batches go to the tiled matrix-core kernel, decode shapes stream the weights
         if (!prefers_stream(B, N, K, false) && gemm_f16_supported(N, K, X, W_T, Y))
-            return launch_gemm_f16(mode, X, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, x_dtype, B, N, K, st);
+            return launch_gemm_f16(mode, X, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, B, N, K, st);
         return launch_stream(mode, X, 2, nullptr, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, x_dtype, nullptr, B, N, K, 1, Q_ROW_MAJOR, 0, nullptr, 0.0f, 0, st);
     }
     if (x_dtype == BT_F32 && packed_uses_f32_planes(W_T, Y, N, K) && workspace &&
@@ -466,14 +464,14 @@ static int gemm_i8_impl(const char* who, const int8_t* Q, int q_layout, const fl
             set_error("%s: tiled weights must be 256-byte aligned and below 4 GiB", who);
             return BT_ERR_INVALID;
         }
-        if (!prefers_stream(B, N, K, true, true) && gemm_i8_supported_tiled(N, K, Q))
+        if (!prefers_stream(B, N, K, true, true, q_layout == Q_OPERAND_ORDER) && gemm_i8_supported_tiled(N, K, Q))
             return launch_gemm_i8(Q, q_layout, s_x, nullptr, W_T, w_layout, epi, Y, y_dtype, acc_out, B, N, K, st);
         return launch_stream(MODE_I8, Q, 1, s_x, W_T, w_layout, epi, Y, y_dtype, acc_out, B, N, K, 1, q_layout, 0, nullptr,
                              0.0f, 0, st);
     }
     // decode-shape batches, and any batch whose N the tiled kernel's 4-column
     // vector accesses cannot take, stream the weights once per 16 rows
-    if (prefers_stream(B, N, K, true) || !gemm_i8_supported(N, K, Q, W_T)) {
+    if (prefers_stream(B, N, K, true, false, q_layout == Q_OPERAND_ORDER) || !gemm_i8_supported(N, K, Q, W_T)) {
         if (!stream_supported(N, K, W_T)) {
             set_error("%s: packed weight matrix of %lld x %lld bytes exceeds the 4 GiB the kernels address", who,
                       (long long)ceil_div(K, 4), (long long)N);

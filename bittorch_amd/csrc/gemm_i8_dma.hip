@@ -14,21 +14,12 @@
 // loads of stages s + 3 and s + 4 in flight, so stage s + 1 (fragments) and s + 2 (the weights decoded one stage ahead) are
 // complete; that barrier also stands between the last read of stage s's buffer and the loads of stage s + 5 into it.
 #include "gemm_i8_common.h"
+#include "lds_dma.h"
 
 namespace bt {
 
 constexpr int D_BK = 64;   // k per stage
 constexpr int D_NST = 5;   // stages in LDS (60 KiB: what M0's 16-bit byte offset reaches)
-
-// 16 (4) bytes a lane from sbase + voff to LDS byte lds_off + 16 (4) * lane
-__device__ __forceinline__ void dma16(uint32_t lds_off, uint32_t voff, const void* sbase) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_off)), "v"(voff), "s"(sbase) : "memory");
-}
-__device__ __forceinline__ void dma4(uint32_t lds_off, uint32_t voff, const void* sbase) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_off)), "v"(voff), "s"(sbase) : "memory");
-}
-
-enum { W_ROWS = 0, W_TILES = 1, W_FIELDS = 2 };  // row-major W_T, the decode-tiled copy, its field layout
 
 // Output stage: row block by row block, addresses as a uniform row base plus a lane offset fixed for the whole tile.  The
 // empty asm statements keep a row's address from being computed ahead of its turn (left alone, the compiler holds all 32
@@ -136,13 +127,17 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
         a_tail[b] = r * (uint32_t)p.K + (k_last + 16 * g < p.K ? 16u * g : 0u);
     }
     uint32_t w_off[W_LOADS], w_tail[W_LOADS];
-    const bool w_in = !TAIL || SRC != W_ROWS || k_last + 16 * g < p.K;  // this lane's rows of the last stage exist
+    const bool w_in = !TAIL || SRC > W_ROWS16 || k_last + 16 * g < p.K;  // this lane's rows of the last stage exist
     if constexpr (SRC == W_ROWS) {
 #pragma unroll
         for (int r = 0; r < W_LOADS; r++) {
             w_off[r] = (uint32_t)(col_ok ? ncol : 0) + (uint32_t)(4 * g + r) * (uint32_t)p.N;
             w_tail[r] = (uint32_t)(col_ok ? ncol : 0) + (w_in ? (uint32_t)(4 * g + r) * (uint32_t)p.N : 0u);
         }
+    } else if constexpr (SRC == W_ROWS16) {
+        const int64_t col = (int64_t)tile_n * G_BN + 64 * wave + 16 * (lane & 3);
+        w_off[0] = (uint32_t)(col < p.N ? col : 0) + (uint32_t)(lane >> 2) * (uint32_t)p.N;
+        w_tail[0] = k_last + 4 * (lane >> 2) < p.K ? w_off[0] : (uint32_t)(col < p.N ? col : 0);
     } else {
         const int tt = stored_tile16((int)(ncol >> 4), p.tiles16);
         w_off[0] = ((uint32_t)tt * (uint32_t)p.wsteps * 64u + (uint32_t)(16 * g + 4 * (j & 3))) * 4u;
@@ -155,7 +150,7 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
     const uint8_t* w_next = p.W_T;
     uint32_t into = 0;
     int st_next = 0;
-    const int64_t w_step = SRC == W_ROWS ? 16 * p.N : 256;
+    const int64_t w_step = SRC <= W_ROWS16 ? 16 * p.N : 256;
     auto issue_a = [&](int b) {
         const bool last = TAIL && st_next >= nst - 1;
         dma16(lds0 + into + (uint32_t)((A_LOADS * wave + b) % (2 * NB)) * 1024u, last ? a_tail[b] : a_off[b], a_next);
@@ -164,7 +159,7 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
         const bool last = TAIL && st_next >= nst - 1;
         const uint32_t wd = lds0 + into + A_BYTES + (uint32_t)wave * 1024u;
         if constexpr (SRC == W_ROWS) dma4(wd + 256u * r, last ? w_tail[r] : w_off[r], w_next);
-        else dma16(wd, w_off[0], w_next);
+        else dma16(wd, SRC == W_ROWS16 && last ? w_tail[0] : w_off[0], w_next);
     };
     auto next_buf = [](uint32_t b) { return b + STAGE == D_NST * STAGE ? 0u : b + STAGE; };
     auto advance = [&]() {  // past the end: the last stage again, never read
@@ -198,9 +193,9 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
     uint32_t raw[4];
     auto read_raw = [&](int s, uint32_t buf) {
         const uint8_t* src = lds + buf + A_BYTES + wave * 1024;
-        if constexpr (SRC == W_ROWS) {
+        if constexpr (SRC <= W_ROWS16) {
 #pragma unroll
-            for (int r = 0; r < 4; r++) raw[r] = *(const uint32_t*)(src + 256 * r + 4 * lane);
+            for (int r = 0; r < 4; r++) raw[r] = *(const uint32_t*)(src + (SRC == W_ROWS16 ? 64 * (4 * g + r) + 4 * j : 256 * r + 4 * lane));
             if (TAIL && s >= nst - 1) {
 #pragma unroll
                 for (int r = 0; r < 4; r++) raw[r] = w_in ? raw[r] : 0u;
@@ -386,14 +381,6 @@ __global__ __launch_bounds__(256, NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_i8_dm
     gemm_i8_dma_tile<SRC, NB, TAIL>(p, m0, (int)tn, lds);
 }
 
-// Into how many finer ones the last, incomplete round of an XCD's 128-row tiles is cut.  Two workgroups that end together
-// free their compute unit for the next two, so a remainder of whole tiles runs in pairs on a part of the chip.  Measured
-// (row-major weights, us, whole / halves / quarters; remainder of 64): 2048 x 11008 x 4096 (22) 104 / 97 / 111; 2900 x 6400 x
-// 6400 (8) 136 / 120 / 122, tiled 120 / 112 / 106; 4096 x 4100 x 4096 (4) 98 / 88 / 86; 2304 x 4096 x 4096 (36) 56 / 63 / 80.
-static int gemm_i8_dma_parts(int64_t tiles) {
-    const int64_t slots = 2 * gemm_compute_units() / 8, rem = ceil_div(tiles, 8) % slots;
-    return rem == 0 || 2 * rem > slots ? 1 : 5 * rem > slots ? 2 : 4;
-}
 // Rows of the tiles in units of 32 (4, 2 or 1), or 0 where gemm_i8_kernel is the better one: tiled weights in whole stages
 // with at most one tile of 128 x 256 for each compute unit.  There a second workgroup has nothing to do, and splitting K
 // over the two waves of a SIMD halves the one tile's chain (K = N = 4096: M = 2048 28.3 us against 30.5 here, M = 512 in its
@@ -402,15 +389,27 @@ static int gemm_i8_dma_parts(int64_t tiles) {
 // 73; 4096 x 8192 x 8192 207 -> 192 / 250 -> 208; 3000 x 1008 x 1040, K not in whole stages, 38 -> 13 / 16 -> 14.
 // Row-major weights of few tiles: M = 1024, 512 (N = K = 4096) 27.3 -> 25.2, 22.9.
 // The prices are microseconds of a compute unit's run of tiles, fitted to the same runs.
-int gemm_i8_dma_rows(int64_t M, int64_t N, int64_t K, bool tiled) {
+static int gemm_i8_dma_plan(int64_t M, int64_t N, int64_t K, bool tiled, double* us) {
     const int64_t C = gemm_compute_units(), tn = ceil_div(N, G_BN);
     const int64_t t4 = ceil_div(M, 128) * tn, t2 = ceil_div(M, 64) * tn, t1 = ceil_div(M, 32) * tn;
     if (tiled && K % 128 == 0 && t4 <= C) return 0;
-    if (t1 <= C) return 1;
-    if (t2 <= C) return 2;
-    const int parts = gemm_i8_dma_parts(t4);
+    if (t1 <= C) { *us = 5.2 + 0.0035 * (double)K; return 1; }
+    if (t2 <= C) { *us = 5.2 + 0.0045 * (double)K; return 2; }
+    const int parts = gemm_dma_parts(t4);
     const double n4 = parts == 1 ? (double)ceil_div(t4, C) : (double)(2 * (t4 / (2 * C))) + (parts == 2 ? 1.2 : 0.6);
-    return (double)ceil_div(t2, C) * (2.2 + 0.0029 * (double)K) < n4 * (3.5 + 0.0055 * (double)K) ? 2 : 4;
+    const double p4 = n4 * (3.5 + 0.0055 * (double)K), p2 = (double)ceil_div(t2, C) * (2.2 + 0.0029 * (double)K);
+    *us = 2.0 + (p2 < p4 ? p2 : p4);
+    return p2 < p4 ? 2 : 4;
+}
+int gemm_i8_dma_rows(int64_t M, int64_t N, int64_t K, bool tiled) {
+    double us;
+    return gemm_i8_dma_plan(M, N, K, tiled, &us);
+}
+// microseconds of launch_gemm_i8: this file's plan, or gemm_i8_kernel's rounds of whole tiles (of finer ones at their price)
+double gemm_i8_cost(int64_t M, int64_t N, int64_t K, bool tiled, bool operand_order) {
+    double us;
+    if (operand_order && gemm_i8_dma_plan(M, N, K, tiled, &us)) return us;
+    return gemm_split(M, N, tiled && K % 128 == 0).rounds * (8.6 + 0.0044 * (double)K);
 }
 
 template <int SRC, int NB, bool TAIL>
@@ -427,7 +426,7 @@ static int launch_gemm_i8_dma_src(GemmParams p, hipStream_t st) {
     p.fine_from = p.per_xcd;
     const dim3 block(256);
     if constexpr (NB == 4) {
-        const int parts = gemm_i8_dma_parts(total);
+        const int parts = gemm_dma_parts(total);
         if (parts > 1) {
             const int rem = p.per_xcd % (int)(2 * gemm_compute_units() / 8);
             p.fine_from = p.per_xcd - rem;
@@ -441,15 +440,17 @@ static int launch_gemm_i8_dma_src(GemmParams p, hipStream_t st) {
     return check_launch("bt_ternary_gemm_i8");
 }
 template <int NB>
-static int launch_gemm_i8_dma_rows(const GemmParams& p, bool tiled, bool fields, hipStream_t st) {
+static int launch_gemm_i8_dma_rows(const GemmParams& p, int src, hipStream_t st) {
     const bool tail = p.K % D_BK != 0;
-    if (fields) return launch_gemm_i8_dma_src<W_FIELDS, NB, false>(p, st);
-    if (tiled) return tail ? launch_gemm_i8_dma_src<W_TILES, NB, true>(p, st) : launch_gemm_i8_dma_src<W_TILES, NB, false>(p, st);
+    if (src == W_FIELDS) return launch_gemm_i8_dma_src<W_FIELDS, NB, false>(p, st);
+    if (src == W_TILES) return tail ? launch_gemm_i8_dma_src<W_TILES, NB, true>(p, st) : launch_gemm_i8_dma_src<W_TILES, NB, false>(p, st);
+    if (src == W_ROWS16) return tail ? launch_gemm_i8_dma_src<W_ROWS16, NB, true>(p, st) : launch_gemm_i8_dma_src<W_ROWS16, NB, false>(p, st);
     return tail ? launch_gemm_i8_dma_src<W_ROWS, NB, true>(p, st) : launch_gemm_i8_dma_src<W_ROWS, NB, false>(p, st);
 }
 int launch_gemm_i8_dma(const GemmParams& p, int rows, bool tiled, bool fields, hipStream_t st) {
-    return rows == 4 ? launch_gemm_i8_dma_rows<4>(p, tiled, fields, st)
-         : rows == 2 ? launch_gemm_i8_dma_rows<2>(p, tiled, fields, st) : launch_gemm_i8_dma_rows<1>(p, tiled, fields, st);
+    const int src = w_source(tiled, fields, p.W_T, p.N);
+    return rows == 4 ? launch_gemm_i8_dma_rows<4>(p, src, st)
+         : rows == 2 ? launch_gemm_i8_dma_rows<2>(p, src, st) : launch_gemm_i8_dma_rows<1>(p, src, st);
 }
 
 }  // namespace bt
