@@ -18,6 +18,7 @@ tiled copy) runs as single calls, same results as ``layer(x)``.
 
 from __future__ import annotations
 
+import os
 from collections import OrderedDict
 from typing import List, Optional, Sequence, Union
 
@@ -38,18 +39,13 @@ class _Plan:
         self.tiled = [L.tiled_weights() for L in layers]       # keeps the copies alive
         self.scales = [L.scale.contiguous() for L in layers]
         self.biases = None if layers[0].bias is None else [L.bias.contiguous() for L in layers]
-        self.key = self.fingerprint(layers)
+        self.held = [(L.scale, L.bias) for L in layers]        # (no other tensor takes their addresses meanwhile)
+        self.key = _fingerprint(layers)
         self.w_tab = _C.pointer_table(self.tiled)
         self.s_tab = _C.pointer_table(self.scales)
         self.b_tab = None if self.biases is None else _C.pointer_table(self.biases)
         self.io_tabs: "OrderedDict[tuple, tuple]" = OrderedDict()
         self.i8_tabs: "OrderedDict[tuple, tuple]" = OrderedDict()
-
-    @staticmethod
-    def fingerprint(layers):
-        return tuple((L._tiled.data_ptr() if L._tiled is not None else 0, L.scale.data_ptr(), L.scale._version,
-                      0 if L.bias is None else L.bias.data_ptr(), 0 if L.bias is None else L.bias._version)
-                     for L in layers)
 
     def io_tab(self, x: Tensor, y: Tensor, shared_x: bool):
         """Tables of the G row addresses of x [G, K] (or of one shared row) and y [G, N]; cached by address, so a
@@ -89,17 +85,57 @@ class _Plan:
         return self.i8_tabs[key]
 
 
-def _plan_for(layers) -> _Plan:
-    ident = tuple(id(L) for L in layers)
-    plan = _PLANS.get(ident)
-    if plan is not None and plan.key == _Plan.fingerprint(layers):
+def _fingerprint(layers):
+    """Everything about the layers that the checks below and a plan's tables depend on, read past ``nn.Module``'s
+    attribute lookup: with 128 layers the checks one by one took 1.2 ms of host time around a kernel of 87 us, comparing
+    this takes a tenth of it."""
+    key = []
+    for L in layers:
+        d = L.__dict__
+        buffers = d["_buffers"]
+        s, b, t = buffers["scale"], buffers["bias"], d["_tiled"]
+        key.append((type(L), d["in_features"], d["out_features"], d["decode_tiled"], d["_tile_order"],
+                    0 if t is None else t.data_ptr(), s.data_ptr(), s._version, s.numel(), s.dtype,
+                    None if b is None else (b.data_ptr(), b._version, b.numel(), b.dtype)))
+    return key
+
+
+def _known_plan(layers) -> Optional[_Plan]:
+    """The plan of exactly these layers if nothing about them has changed since it was made (the layers then passed every
+    check), or None."""
+    try:
+        ident = tuple(map(id, layers))
+        plan = _PLANS.get(ident)
+        if plan is None or plan.key != _fingerprint(layers):
+            return None
         _PLANS.move_to_end(ident)
         return plan
+    except (KeyError, AttributeError):  # (not an inference layer: the checks say so)
+        return None
+
+
+def _plan_for(layers) -> _Plan:
+    plan = _known_plan(layers)
+    if plan is not None:
+        return plan
     plan = _Plan(layers)
-    _PLANS[ident] = plan
+    _PLANS[tuple(map(id, layers))] = plan
     if len(_PLANS) > _MAX_PLANS:
         _PLANS.popitem(last=False)
     return plan
+
+
+def _check_layers(who: str, layers) -> None:
+    from ..nn.ternary_linear_infer import TernaryLinearInference
+    for L in layers:
+        if not isinstance(L, TernaryLinearInference):
+            raise TypeError(f"{who} takes TernaryLinearInference layers")
+    k, n = layers[0].in_features, layers[0].out_features
+    for L in layers:
+        if (L.in_features, L.out_features) != (k, n):
+            raise ValueError(f"{who}: every layer must have the same in_features and out_features")
+        if (L.bias is None) != (layers[0].bias is None) or L.scale.numel() != layers[0].scale.numel():
+            raise ValueError(f"{who}: layers must agree on having a bias and on the scale's length")
 
 
 def _groupable(layers, x: Tensor) -> bool:
@@ -118,7 +154,10 @@ def _groupable(layers, x: Tensor) -> bool:
             return False
         if L._tiled is None and torch.cuda.is_current_stream_capturing():
             return False  # (a capture never builds the tiled copy)
-    import os
+    return _kernels_allowed()
+
+
+def _kernels_allowed() -> bool:
     return os.environ.get("BITTORCH_KERNEL", "auto") != "generic"
 
 
@@ -131,16 +170,10 @@ def ternary_linear_grouped(layers: Sequence, xs: Union[Tensor, Sequence[Tensor]]
     layers = list(layers)
     if not layers:
         raise ValueError("ternary_linear_grouped: no layers")
-    from ..nn.ternary_linear_infer import TernaryLinearInference
-    for L in layers:
-        if not isinstance(L, TernaryLinearInference):
-            raise TypeError("ternary_linear_grouped takes TernaryLinearInference layers")
+    plan = _known_plan(layers)
+    if plan is None:
+        _check_layers("ternary_linear_grouped", layers)
     g, k, n = len(layers), layers[0].in_features, layers[0].out_features
-    for L in layers:
-        if (L.in_features, L.out_features) != (k, n):
-            raise ValueError("ternary_linear_grouped: every layer must have the same in_features and out_features")
-        if (L.bias is None) != (layers[0].bias is None) or L.scale.numel() != layers[0].scale.numel():
-            raise ValueError("ternary_linear_grouped: layers must agree on having a bias and on the scale's length")
     if not isinstance(xs, Tensor):
         xs = torch.stack([t.reshape(-1) for t in xs])
     shared = xs.numel() == k
@@ -150,18 +183,20 @@ def ternary_linear_grouped(layers: Sequence, xs: Union[Tensor, Sequence[Tensor]]
         if xs.dim() != 2 or xs.shape != (g, k):
             raise RuntimeError(f"input K doesn't match in_features: expected [{g}, {k}] or one row of {k}, got {tuple(xs.shape)}")
         x = xs
-    if any(t is not None and t.is_cuda != x.is_cuda for L in layers for t in (L.scale,)):
+    if plan is not None and not (x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and _kernels_allowed()):
+        plan = None  # (a call the grouped kernel does not take)
+    if plan is None and any(L.scale.is_cuda != x.is_cuda for L in layers):
         raise RuntimeError("All tensors must be CUDA")
     if out is not None and (out.shape != (g, n) or out.dtype != x.dtype or out.device != x.device or out.stride(1) != 1):
         raise ValueError("ternary_linear_grouped: out must be [G, N] in the rows' dtype on their device, rows contiguous")
-    if not _groupable(layers, x):
+    if plan is None and not _groupable(layers, x):
         ys = [L(x if shared else x[u:u + 1]) for u, L in enumerate(layers)]
         y = torch.cat(ys, dim=0)
         return y if out is None else out.copy_(y)
     from .. import _C
     if x.stride(-1) != 1 or (x.data_ptr() % 16) or (not shared and (x.stride(0) * x.element_size()) % 16):
         x = x.contiguous()
-    plan = _plan_for(layers)
+    plan = plan or _plan_for(layers)
     y = out if out is not None else torch.empty((g, n), dtype=x.dtype, device=x.device)
     xt, yt = plan.io_tab(x, y, shared)
     _C.ternary_gemv_grouped(xt, plan.w_tab, plan.s_tab, plan.b_tab, yt, k, n,
@@ -188,17 +223,11 @@ def ternary_linear_int8_grouped(layers: Sequence, xs: Optional[Tensor] = None, q
     layers = list(layers)
     if not layers:
         raise ValueError("ternary_linear_int8_grouped: no layers")
-    from ..nn.ternary_linear_infer import TernaryLinearInference
     from .. import _C
-    for L in layers:
-        if not isinstance(L, TernaryLinearInference):
-            raise TypeError("ternary_linear_int8_grouped takes TernaryLinearInference layers")
+    plan = _known_plan(layers)
+    if plan is None:
+        _check_layers("ternary_linear_int8_grouped", layers)
     g, k, n = len(layers), layers[0].in_features, layers[0].out_features
-    for L in layers:
-        if (L.in_features, L.out_features) != (k, n):
-            raise ValueError("ternary_linear_int8_grouped: every layer must have the same in_features and out_features")
-        if (L.bias is None) != (layers[0].bias is None) or L.scale.numel() != layers[0].scale.numel():
-            raise ValueError("ternary_linear_int8_grouped: layers must agree on having a bias and on the scale's length")
     if (xs is None) == (q is None) or (q is not None and s_x is None):
         raise ValueError("ternary_linear_int8_grouped: give xs, or q together with s_x")
     src = xs if xs is not None else q
@@ -217,15 +246,14 @@ def ternary_linear_int8_grouped(layers: Sequence, xs: Optional[Tensor] = None, q
         if q.dtype != torch.int8 or s_x.shape != (g, m) or s_x.dtype != torch.float32:
             raise RuntimeError("q must be int8 [G, M, K] and s_x fp32 [G, M]")
         q, s_x = q.contiguous(), s_x.contiguous()
-    kinds = (torch.float32, torch.float16, torch.bfloat16)
-    groupable = (g >= _MIN_G_I8 and m <= 16 and k % 16 == 0 and k <= _MAX_K_I8 and _groupable(layers, torch.empty(0, dtype=torch.float16, device=q.device))
-                 and all(L.scale.dtype in kinds for L in layers))
+    groupable = g >= _MIN_G_I8 and m <= 16 and k % 16 == 0 and k <= _MAX_K_I8 and (
+        _kernels_allowed() if plan is not None else _groupable(layers, torch.empty(0, dtype=torch.float16, device=q.device)))
     if out is not None and (out.shape != (g, m, n) or out.dtype != out_dtype or not out.is_contiguous()):
         raise ValueError("ternary_linear_int8_grouped: out must be a contiguous [G, M, N] tensor of out_dtype")
     if not groupable:
         y = torch.stack([L.forward_int8(q[u], s_x[u], out_dtype, None, q_operand_order) for u, L in enumerate(layers)])
         return y if out is None else out.copy_(y)
-    plan = _plan_for(layers)
+    plan = plan or _plan_for(layers)
     y = out if out is not None else torch.empty((g, m, n), dtype=out_dtype, device=q.device)
     qt, st, yt = plan.i8_tab(q, s_x, y)
     _C.ternary_gemm_int8_grouped(qt, st, plan.w_tab, plan.s_tab, plan.b_tab, yt, m, k, n,

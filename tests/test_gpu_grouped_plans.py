@@ -1,0 +1,54 @@
+"""GPU: a grouped call on layers it has seen before notices whatever has changed about them since."""
+import pytest
+import torch
+
+from conftest import announce
+
+pytestmark = pytest.mark.gpu
+
+
+def _layers(n=64, k=128, count=5, bias=True):
+    from bittorch_amd import nn
+    g = torch.Generator("cuda").manual_seed(3)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    return [nn.create_ternary_linear_inference(k, n, r(n, k) * 0.02, r(n) * 0.01 if bias else None).prepare_decode()
+            for _ in range(count)]
+
+
+def _check(layers, x, int8):
+    from bittorch_amd import ops
+    if int8:
+        got = ops.ternary_linear_int8_grouped(layers, x[:, None])
+        want = torch.stack([L.forward_int8(*ops.act_quant_int8(x[u:u + 1]), x.dtype) for u, L in enumerate(layers)])
+    else:
+        got = ops.ternary_linear_grouped(layers, x)
+        want = torch.cat([L(x[u:u + 1]) for u, L in enumerate(layers)])
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("int8", [False, True])
+def test_changes_between_calls_are_seen(int8):
+    from bittorch_amd import ops
+    announce("grouped plans", int8)
+    layers = _layers()
+    x = torch.randn(5, 128, device="cuda").half()
+    for change in (lambda: None, lambda: layers[3].scale.mul_(2), lambda: setattr(layers[1], "bias", layers[1].bias + 1),
+                   lambda: layers[0].bias.zero_(), lambda: setattr(layers[2], "scale", layers[2].scale.clone() * 3),
+                   lambda: layers.reverse(), lambda: layers.__setitem__(4, _layers(count=6)[5])):
+        change()
+        _check(layers, x, int8)
+        _check(layers, x * 2, int8)
+    call = ops.ternary_linear_int8_grouped if int8 else ops.ternary_linear_grouped
+    xs = x[:, None] if int8 else x
+    layers[2].bias = None
+    with pytest.raises(ValueError):
+        call(layers, xs)
+    layers[2].bias = layers[1].bias
+    _check(layers, x, int8)
+    layers[2].scale = layers[2].scale[:1]
+    with pytest.raises(ValueError):
+        call(layers, xs)
+    with pytest.raises(TypeError):
+        call(layers[:2] + [torch.nn.Linear(128, 64)], xs[:3])
+    with pytest.raises((RuntimeError, TypeError)):
+        call(_layers(), xs.cpu())
