@@ -97,8 +97,7 @@ __global__ __launch_bounds__(256) void row_op_kernel(RowOpParams p) {
             const int kc = min(k, K - 8);
             float u[8];
             load8<DT>(p.Bv, row * p.ldb + kc, u);
-#pragma unroll
-            for (int e = 0; e < 8; e++) v[i][e] = swiglu_value(v[i][e], u[e], DT);
+            swiglu8<DT>(v[i], u);
         }
     } else {
         double ss = 0.0;
@@ -153,7 +152,7 @@ __global__ __launch_bounds__(256) void row_op_kernel(RowOpParams p) {
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             const int8_t qv = quant_i8(v[i][e], inv);
-            if (k < K) qsum += (int)qv;
+            if (p.rowsum && k < K) qsum += (int)qv;
             const uint32_t byte = (uint32_t)(uint8_t)qv;
             if (e < 4) lo |= byte << (8 * e);
             else hi |= byte << (8 * (e - 4));
@@ -192,8 +191,7 @@ __global__ __launch_bounds__(256) void row_op_wave_kernel(RowOpParams p, int64_t
             const int k = (i * 64 + lane) * 8;
             float u[8];
             load8<DT>(p.Bv, row * p.ldb + min(k, K - 8), u);
-#pragma unroll
-            for (int e = 0; e < 8; e++) v[i][e] = swiglu_value(v[i][e], u[e], DT);
+            swiglu8<DT>(v[i], u);
         }
     } else {
         double ss = 0.0;
@@ -240,7 +238,7 @@ __global__ __launch_bounds__(256) void row_op_wave_kernel(RowOpParams p, int64_t
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             const int8_t qv = quant_i8(v[i][e], inv);
-            if (k < K) qsum += (int)qv;
+            if (p.rowsum && k < K) qsum += (int)qv;
             const uint32_t byte = (uint32_t)(uint8_t)qv;
             if (e < 4) lo |= byte << (8 * e);
             else hi |= byte << (8 * (e - 4));

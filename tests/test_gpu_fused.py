@@ -70,6 +70,22 @@ def test_swiglu_against_torch_ops(dtype):
     assert torch.equal(q, q_ref) and torch.equal(s, s_ref)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_swiglu_of_every_16_bit_gate_value(oracle, dtype):
+    """The 16-bit row kernels form silu with the hardware's exp2 / reciprocal and a corrected quotient: the oracle's bits for
+    every finite gate value, in ascending order (eight values share a path) and shuffled."""
+    bits = torch.arange(65536, dtype=torch.int32).to(torch.uint16).view(dtype)
+    finite = torch.nan_to_num(bits.float(), nan=1.0, posinf=2.0, neginf=-2.0).to(dtype)
+    announce("swiglu of every gate value", dtype)
+    from bittorch_amd import ops
+    order = torch.randperm(65536, generator=torch.Generator().manual_seed(1))
+    for g in (finite.view(256, 256), finite[order].view(256, 256), finite.view(32, 2048)):
+        u = seeded_acts(*g.shape, seed=2, dtype=dtype)
+        for up in (torch.ones_like(g), u):
+            h = ops.swiglu(g.cuda(), up.cuda())
+            np.testing.assert_array_equal(f32np(h), oracle.swiglu(f32np(g), f32np(up), BT_DT[dtype])[0])
+
+
 def test_swiglu_special_values():
     from bittorch_amd import _C
     g = torch.tensor([[0.0, -0.0, 100.0, -100.0, 1e-30, float("inf"), -float("inf"), float("nan")]]).cuda()
