@@ -25,8 +25,11 @@ from .ternary_linear import _init_linear_params
 
 def _fp32_kernels_serve(g2: Tensor, x2: Tensor, packed: Optional[Tensor], scale: Tensor) -> bool:
     """Whether this backward runs on the library's gradient kernels: fp32 throughout, and no graph of the backward itself
-    wanted (``create_graph=True``: the torch products below are differentiable)."""
+    wanted (``create_graph=True``: the torch products below are differentiable).  A batched gradient
+    (``is_grads_batched=True``, a vectorized Jacobian) has no memory of its own to hand to a kernel."""
     if packed is None or torch.is_grad_enabled() or g2.numel() == 0:
+        return False
+    if torch._C._functorch.is_functorch_wrapped_tensor(g2) or torch._C._functorch.is_legacy_batchedtensor(g2):
         return False
     if not (g2.dtype == x2.dtype == scale.dtype == torch.float32 and g2.is_cuda):
         return False

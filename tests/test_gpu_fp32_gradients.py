@@ -99,3 +99,18 @@ def test_fp32_layer_backward_uses_the_kernels_and_keeps_double_backward():
     for a, b in zip(plain, graphed):
         assert torch.allclose(a, b, rtol=1e-4, atol=1e-5 * float(b.detach().abs().max()))
     assert torch.autograd.grad(graphed[0].sum(), gy2)[0].shape == gy.shape
+
+
+@gpu
+def test_fp32_layer_batched_gradients():
+    """Several output gradients in one backward (``is_grads_batched=True``): as one backward each."""
+    from bittorch_amd import nn
+    announce("fp32 layer, batched gradients")
+    layer = nn.TernaryLinear(96, 40).cuda()
+    x = torch.randn(70, 96, device="cuda", requires_grad=True)
+    y, leaves = layer(x), (x, layer.weight, layer.bias)
+    gys = torch.randn(3, 70, 40, device="cuda")
+    batched = torch.autograd.grad(y, leaves, gys, retain_graph=True, is_grads_batched=True)
+    for i in range(3):
+        for a, b in zip(batched, torch.autograd.grad(y, leaves, gys[i], retain_graph=True)):
+            assert torch.allclose(a[i], b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))
