@@ -758,3 +758,16 @@ def linear_grad_weight(dY: Tensor, X: Tensor, scale: Tensor, want_bias: bool = F
         _status(_L.bt_linear_grad_weight(dY.data_ptr(), X.data_ptr(), scale.data_ptr(), scale.numel(), dW.data_ptr(), _ptr(dB),
                                          M, N, K, _ptr(ws), 0 if ws is None else ws.numel(), _stream(dY)))
     return dW, dB
+
+
+def scale_grad_weight(G: Tensor, scale: Tensor) -> Tensor:
+    """``(G * scale[:, None].to(G.dtype)).float()`` in one pass (``G`` ``[N, K]`` fp16 or bf16, ``scale`` ``[N]`` or one entry)."""
+    _check(G.dim() == 2 and G.dtype in (torch.float16, torch.bfloat16) and G.numel() > 0, "G must be 2D fp16 or bf16")
+    _check(scale.numel() in (G.shape[0], 1), "scale size doesn't match N")
+    _check(_all_cuda(G, scale), "All tensors must be CUDA")
+    G, scale = G.contiguous(), scale.reshape(-1).to(torch.float32).contiguous()
+    out = torch.empty(G.shape, dtype=torch.float32, device=G.device)
+    with torch.cuda.device(G.device):
+        _status(_L.bt_scale_grad_weight(G.data_ptr(), _DT[G.dtype], scale.data_ptr(), scale.numel(), out.data_ptr(),
+                                        G.shape[0], G.shape[1], _stream(G)))
+    return out

@@ -29,12 +29,26 @@ def _fp32_kernels_serve(g2: Tensor, x2: Tensor, packed: Optional[Tensor], scale:
     (``is_grads_batched=True``, a vectorized Jacobian) has no memory of its own to hand to a kernel."""
     if packed is None or torch.is_grad_enabled() or g2.numel() == 0:
         return False
-    if torch._C._functorch.is_functorch_wrapped_tensor(g2) or torch._C._functorch.is_legacy_batchedtensor(g2):
+    if _batched(g2):
         return False
     if not (g2.dtype == x2.dtype == scale.dtype == torch.float32 and g2.is_cuda):
         return False
     n, k = g2.shape[1], x2.shape[1]
     return 4 <= n < 2 ** 23 and 4 <= k < 2 ** 23 and packed.numel() < 2 ** 32
+
+
+def _batched(t: Tensor) -> bool:
+    return torch._C._functorch.is_functorch_wrapped_tensor(t) or torch._C._functorch.is_legacy_batchedtensor(t)
+
+
+def _scale_to_master(g: Tensor, scale: Tensor, master_dtype: Optional[torch.dtype]) -> Tensor:
+    """The 16-bit product ``dY^T X`` times its scale.  For fp32 masters (autocast) the scale and the widening that autograd
+    would do next are one pass, with the same bits; a differentiated or batched backward stays on torch."""
+    if (master_dtype == torch.float32 and g.dtype in (torch.float16, torch.bfloat16) and g.is_cuda and g.numel() > 0
+            and g.shape[0] * ((g.shape[1] + 2047) // 2048) < 2 ** 30 and not torch.is_grad_enabled() and not _batched(g)):
+        from .. import _C
+        return _C.scale_grad_weight(g, scale)
+    return g * scale.reshape(-1, 1).to(g.dtype)
 
 
 class TernaryLinearCUDAFunction(torch.autograd.Function):
@@ -43,9 +57,10 @@ class TernaryLinearCUDAFunction(torch.autograd.Function):
     @staticmethod
     @torch.amp.custom_fwd(device_type="cuda", cast_inputs=torch.float16)
     def forward(ctx, x: Tensor, weight: Tensor, bias: Optional[Tensor], threshold_factor: float,
-                per_channel: bool, cached=None) -> Tensor:
+                per_channel: bool, cached=None, master_dtype: Optional[torch.dtype] = None) -> Tensor:
         """``cached``: optional ``(packed_T, scale, tiled copy or None)`` of exactly these weights (see
-        ``_packed_cache.py``); the quantize+pack kernel is skipped when it is given."""
+        ``_packed_cache.py``); the quantize+pack kernel is skipped when it is given.  ``master_dtype``: the dtype
+        ``weight`` had before autocast, in which its gradient is wanted."""
         from .. import _C
 
         if weight.dtype == torch.float64 or x.dtype == torch.float64:
@@ -73,6 +88,7 @@ class TernaryLinearCUDAFunction(torch.autograd.Function):
         ctx.save_for_backward(x, packed, scale)
         ctx.in_features = weight.shape[1]
         ctx.weight_dtype = weight.dtype
+        ctx.master_dtype = master_dtype
         ctx.has_bias = bias is not None
         return out
 
@@ -93,8 +109,7 @@ class TernaryLinearCUDAFunction(torch.autograd.Function):
                 grad_w, grad_b = _C.linear_grad_weight(g2, x2, scale.reshape(-1), want_bias)
             elif want_bias:
                 grad_b = g2.sum(dim=0)
-            return grad_x, grad_w, grad_b, None, None, None
-        scale_col = scale.reshape(-1, 1)
+            return grad_x, grad_w, grad_b, None, None, None, None
         if ctx.needs_input_grad[0]:
             if packed is not None:
                 w_eff = _C.unpack_dequant(packed, ctx.in_features, scale.reshape(-1),
@@ -104,10 +119,10 @@ class TernaryLinearCUDAFunction(torch.autograd.Function):
             grad_x = (g2 @ w_eff.to(g2.dtype)).reshape(x.shape)
         if ctx.needs_input_grad[1]:
             # d(w_eff)/d(weight) = scale under the straight-through estimator
-            grad_w = (g2.t() @ x2) * scale_col.to(g2.dtype)
+            grad_w = _scale_to_master(g2.t() @ x2, scale, ctx.master_dtype)
         if want_bias:
             grad_b = g2.sum(dim=0)
-        return grad_x, grad_w, grad_b, None, None, None
+        return grad_x, grad_w, grad_b, None, None, None, None
 
 
 class TernaryLinearCUDA(nn.Module):
@@ -138,7 +153,7 @@ class TernaryLinearCUDA(nn.Module):
         if cache_usable(x, self.weight):
             cached = self._packed.get(self.weight, self.threshold_factor, self.per_channel)
         return TernaryLinearCUDAFunction.apply(x, self.weight, self.bias, self.threshold_factor,
-                                               self.per_channel, cached)
+                                               self.per_channel, cached, self.weight.dtype)
 
     def invalidate_packed_cache(self) -> None:
         """Forget the cached packed weights (needed only after an evaluation-time write through ``weight.data``,

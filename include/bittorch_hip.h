@@ -419,6 +419,11 @@ size_t bt_linear_grad_weight_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int bt_linear_grad_weight(const float* dY, const float* X, const float* scale, int64_t scale_len, float* dW, float* dBias,
                           int64_t M, int64_t N, int64_t K, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The weight gradient of a 16-bit product (dY^T X, [N,K] fp16 or bf16) as fp32 masters receive it: each entry times its
+ * row's scale (rounded to the dtype; scale_len: N, or 1), rounded to the dtype, then widened. */
+int bt_scale_grad_weight(const void* G, int dtype, const float* scale, int64_t scale_len, float* dW, int64_t N, int64_t K,
+                         void* stream);
+
 /*
  * Dense ternary weights -> packed transposed layout, on the device.
  * Replaces pack_ternary_transposed (bittorch/quant/ternary_packed.py:174-206) for weights
