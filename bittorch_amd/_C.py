@@ -25,6 +25,7 @@ _L = _lib.load()  # ImportError here == "extension not available"
 
 _DT = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 _INT8_OUT = 3
+_F32_AS_F16 = 4  # bt_quantize_pack: fp32 weights quantized as their fp16 copy
 
 
 def _check(cond: bool, msg: str) -> None:
@@ -516,20 +517,22 @@ def ternary_linear_tensor_core_forward(X: Tensor, W_T: Tensor, scale: Tensor,
 
 
 def ternary_quantize_pack(weight: Tensor, threshold_factor: float = 0.05, per_channel: bool = True,
-                          want_packed: bool = True, want_tern: bool = False
+                          want_packed: bool = True, want_tern: bool = False, as_half: bool = False
                           ) -> Tuple[Optional[Tensor], Tensor, Optional[Tensor]]:
     """Fused quantize + pack of master weights ``[N, K]`` on the GPU.
 
     Returns ``(packed_T uint8 [ceil(K/4), N] | None, scale, w_tern int8 [N, K] | None)``;
     ``scale`` has the weight dtype and shape ``(N,)`` (per channel) or ``()`` (per tensor),
-    exactly what ``quant.ternary_quantize`` returns.
+    exactly what ``quant.ternary_quantize`` returns.  ``as_half=True`` (fp32 weights): the results for ``weight.half()``,
+    rounded as the weights are read.
     """
     _check(weight.dim() == 2, "weight must be 2D [N, K]")
+    _check(not as_half or weight.dtype == torch.float32, "as_half takes fp32 weights")
     _check(weight.is_cuda, "All tensors must be CUDA")
     w = weight.detach().contiguous()
     N, K = w.shape
     _check(N > 0 and K > 0, "weight is empty")
-    wdt = _dt(w, "weight")
+    wdt = _F32_AS_F16 if as_half else _dt(w, "weight")
     dev = w.device
     packed = torch.empty(((K + 3) // 4, N), dtype=torch.uint8, device=dev) if want_packed else None
     tern = torch.empty((N, K), dtype=torch.int8, device=dev) if want_tern else None
@@ -538,7 +541,7 @@ def ternary_quantize_pack(weight: Tensor, threshold_factor: float = 0.05, per_ch
         _status(_L.bt_quantize_pack(w.data_ptr(), wdt, N, K, float(threshold_factor),
                                     int(bool(per_channel)), _ptr(packed), scale.data_ptr(),
                                     _ptr(tern), _stream(w)))
-    scale = scale.to(weight.dtype)
+    scale = scale.to(torch.float16 if as_half else weight.dtype)
     if not per_channel:
         scale = scale.squeeze(0)
     return packed, scale, tern

@@ -109,7 +109,7 @@ class TernaryLinear(nn.Module):
             if cache_usable(x, self.weight):  # packed weights are kept until the masters change
                 cached = self._packed.get(self.weight, self.threshold_factor, self.per_channel)
             return TernaryLinearCUDAFunction.apply(x, self.weight, self.bias, self.threshold_factor,
-                                                   self.per_channel, cached, self.weight.dtype)
+                                                   self.per_channel, cached)
         # plain torch path (reference :194-213): the scale is folded into the
         # weights, which are rounded to the activation dtype before the product
         w_q, scale = ternary_quantize_ste(self.weight, self.threshold_factor, self.per_channel)

@@ -41,7 +41,12 @@ def _batched(t: Tensor) -> bool:
     return torch._C._functorch.is_functorch_wrapped_tensor(t) or torch._C._functorch.is_legacy_batchedtensor(t)
 
 
-def _scale_to_master(g: Tensor, scale: Tensor, master_dtype: Optional[torch.dtype]) -> Tensor:
+def _to_half(t: Optional[Tensor]) -> Optional[Tensor]:
+    """What autocast does with an argument: floating-point GPU tensors other than float64 become fp16."""
+    return t.half() if t is not None and t.is_cuda and t.is_floating_point() and t.dtype != torch.float64 else t
+
+
+def _scale_to_master(g: Tensor, scale: Tensor, master_dtype: torch.dtype) -> Tensor:
     """The 16-bit product ``dY^T X`` times its scale.  For fp32 masters (autocast) the scale and the widening that autograd
     would do next are one pass, with the same bits; a differentiated or batched backward stays on torch."""
     if (master_dtype == torch.float32 and g.dtype in (torch.float16, torch.bfloat16) and g.is_cuda and g.numel() > 0
@@ -55,12 +60,21 @@ class TernaryLinearCUDAFunction(torch.autograd.Function):
     """``y = x @ (ternary(weight) * scale).T + bias`` with STE gradients."""
 
     @staticmethod
-    @torch.amp.custom_fwd(device_type="cuda", cast_inputs=torch.float16)
     def forward(ctx, x: Tensor, weight: Tensor, bias: Optional[Tensor], threshold_factor: float,
-                per_channel: bool, cached=None, master_dtype: Optional[torch.dtype] = None) -> Tensor:
+                per_channel: bool, cached=None) -> Tensor:
         """``cached``: optional ``(packed_T, scale, tiled copy or None)`` of exactly these weights (see
-        ``_packed_cache.py``); the quantize+pack kernel is skipped when it is given.  ``master_dtype``: the dtype
-        ``weight`` had before autocast, in which its gradient is wanted."""
+        ``_packed_cache.py``); the quantize+pack kernel is skipped when it is given.  Under autocast the layer runs in
+        fp16 with autocast off; fp32 masters are rounded as the quantizer reads them."""
+        ctx.master_dtype = weight.dtype
+        if not torch.is_autocast_enabled("cuda"):
+            return TernaryLinearCUDAFunction._forward(ctx, x, weight, bias, threshold_factor, per_channel, cached, False)
+        as_half = (cached is None and x.dtype != torch.float64 and weight.dtype == torch.float32 and weight.is_cuda)
+        with torch.autocast("cuda", enabled=False):
+            return TernaryLinearCUDAFunction._forward(ctx, _to_half(x), weight if as_half else _to_half(weight),
+                                                      _to_half(bias), threshold_factor, per_channel, cached, as_half)
+
+    @staticmethod
+    def _forward(ctx, x, weight, bias, threshold_factor, per_channel, cached, as_half) -> Tensor:
         from .. import _C
 
         if weight.dtype == torch.float64 or x.dtype == torch.float64:
@@ -75,7 +89,7 @@ class TernaryLinearCUDAFunction(torch.autograd.Function):
             if cached is not None:
                 packed, scale, tiled = cached
             else:
-                packed, scale, _ = _C.ternary_quantize_pack(weight, threshold_factor, per_channel)
+                packed, scale, _ = _C.ternary_quantize_pack(weight, threshold_factor, per_channel, as_half=as_half)
             b = None if bias is None else bias.to(x.dtype).contiguous()
             if (tiled is not None and x.dtype in (torch.float16, torch.bfloat16, torch.float32)
                     and os.environ.get("BITTORCH_KERNEL") != "generic"):  # (the shape-generic kernel reads packed_T)
@@ -87,14 +101,17 @@ class TernaryLinearCUDAFunction(torch.autograd.Function):
             ctx.w_eff = None
         ctx.save_for_backward(x, packed, scale)
         ctx.in_features = weight.shape[1]
-        ctx.weight_dtype = weight.dtype
-        ctx.master_dtype = master_dtype
+        ctx.weight_dtype = torch.float16 if as_half else weight.dtype
         ctx.has_bias = bias is not None
         return out
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
     def backward(ctx, grad_output: Tensor):
+        with torch.autocast("cuda", enabled=False):  # (as the forward)
+            return TernaryLinearCUDAFunction._backward(ctx, grad_output)
+
+    @staticmethod
+    def _backward(ctx, grad_output: Tensor):
         from .. import _C
 
         x, packed, scale = ctx.saved_tensors
@@ -109,7 +126,7 @@ class TernaryLinearCUDAFunction(torch.autograd.Function):
                 grad_w, grad_b = _C.linear_grad_weight(g2, x2, scale.reshape(-1), want_bias)
             elif want_bias:
                 grad_b = g2.sum(dim=0)
-            return grad_x, grad_w, grad_b, None, None, None, None
+            return grad_x, grad_w, grad_b, None, None, None
         if ctx.needs_input_grad[0]:
             if packed is not None:
                 w_eff = _C.unpack_dequant(packed, ctx.in_features, scale.reshape(-1),
@@ -122,7 +139,7 @@ class TernaryLinearCUDAFunction(torch.autograd.Function):
             grad_w = _scale_to_master(g2.t() @ x2, scale, ctx.master_dtype)
         if want_bias:
             grad_b = g2.sum(dim=0)
-        return grad_x, grad_w, grad_b, None, None, None, None
+        return grad_x, grad_w, grad_b, None, None, None
 
 
 class TernaryLinearCUDA(nn.Module):
@@ -153,7 +170,7 @@ class TernaryLinearCUDA(nn.Module):
         if cache_usable(x, self.weight):
             cached = self._packed.get(self.weight, self.threshold_factor, self.per_channel)
         return TernaryLinearCUDAFunction.apply(x, self.weight, self.bias, self.threshold_factor,
-                                               self.per_channel, cached, self.weight.dtype)
+                                               self.per_channel, cached)
 
     def invalidate_packed_cache(self) -> None:
         """Forget the cached packed weights (needed only after an evaluation-time write through ``weight.data``,

@@ -29,7 +29,8 @@ extern "C" {
 #define BT_ABI_VERSION 2
 
 /* element types of activations / scales / biases / outputs */
-typedef enum { BT_F32 = 0, BT_F16 = 1, BT_BF16 = 2, BT_I8 = 3 /* bt_unpack_dequant output only */ } bt_dtype;
+typedef enum { BT_F32 = 0, BT_F16 = 1, BT_BF16 = 2, BT_I8 = 3 /* bt_unpack_dequant output only */,
+               BT_F32_AS_F16 = 4 /* bt_quantize_pack input only: fp32 weights, quantized as their fp16 copy is */ } bt_dtype;
 
 typedef enum {
     BT_OK = 0,

@@ -46,3 +46,21 @@ def test_autocast_layer_gradients(per_channel, amp):
     assert torch.equal(gw, want)
     graphed = torch.autograd.grad(y, layer.weight, gy.clone().requires_grad_(), retain_graph=True, create_graph=True)[0]
     assert torch.equal(graphed, want)
+
+
+@pytest.mark.parametrize("per_channel", [True, False])
+@pytest.mark.parametrize("n,k", [(1, 1), (5, 7), (17, 130), (64, 256), (16, 4096), (48, 11008), (32, 5120), (300, 260), (8, 9000)])
+def test_fp32_masters_quantized_as_their_fp16_copy(n, k, per_channel):
+    """Rounded as they are read (both kernels, the tensor-wide maximum too): the bytes and scales of ``weight.half()``."""
+    from bittorch_amd import _C
+    announce("quantize as half", n, k, per_channel)
+    gen = torch.Generator("cuda").manual_seed(n * 31 + k)
+    w = torch.randn(n * k + 1, generator=gen, device="cuda") * 0.02
+    w[::7] *= 1e-5                       # fp16 subnormals
+    for rows in (w[:-1].view(n, k), w[1:].view(n, k), (w[:-1] * 1e-7).view(n, k), (w[:-1] * 3e5).view(n, k),
+                 torch.full((n, k), 1e6, device="cuda")):  # (the last two overflow to infinities)
+        for want_tern in (True, False):                    # (dense values come from the generic kernel only)
+            got, want = (_C.ternary_quantize_pack(t, 0.05, per_channel, True, want_tern, as_half=half)
+                         for t, half in ((rows, True), (rows.half(), False)))
+            for a, b in zip(got, want):
+                assert a is b is None or (a.dtype == b.dtype and torch.equal(a, b))
