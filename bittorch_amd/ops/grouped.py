@@ -48,41 +48,32 @@ class _Plan:
         self.i8_tabs: "OrderedDict[tuple, tuple]" = OrderedDict()
 
     def io_tab(self, x: Tensor, y: Tensor, shared_x: bool):
-        """Tables of the G row addresses of x [G, K] (or of one shared row) and y [G, N]; cached by address, so a
-        decode loop whose buffers repeat (and a captured graph, whose buffers are fixed) builds them once."""
-        key = (x.data_ptr(), y.data_ptr(), shared_x)
-        hit = self.io_tabs.get(key)
-        if hit is not None:
-            self.io_tabs.move_to_end(key)
-            return hit
-        g = y.shape[0]
-        step = 0 if shared_x else x.stride(0) * x.element_size()
-        xt = torch.tensor([x.data_ptr() + u * step for u in range(g)], dtype=torch.int64, device=x.device)
-        yt = torch.tensor([y.data_ptr() + u * y.stride(0) * y.element_size() for u in range(g)], dtype=torch.int64,
-                          device=x.device)
-        self.io_tabs[key] = (xt, yt)
-        if len(self.io_tabs) > 8:
-            self.io_tabs.popitem(last=False)
-        return xt, yt
-
+        """Tables of the G row addresses of x [G, K] (or of one shared row) and y [G, N]."""
+        return self._tables(self.io_tabs, y.shape[0], y.device, ((x.data_ptr(), 0 if shared_x else _unit_bytes(x)),
+                                                                 (y.data_ptr(), _unit_bytes(y))))
 
     def i8_tab(self, q: Tensor, s_x: Tensor, y: Tensor):
-        """Tables of the G units' addresses inside q [G, M, K], s_x [G, M] and y [G, M, N]; cached by address."""
-        key = (q.data_ptr(), s_x.data_ptr(), y.data_ptr())
-        hit = self.i8_tabs.get(key)
+        """Tables of the G units' addresses inside q [G, M, K], s_x [G, M] and y [G, M, N]."""
+        return self._tables(self.i8_tabs, q.shape[0], q.device, tuple((t.data_ptr(), _unit_bytes(t)) for t in (q, s_x, y)))
+
+    @staticmethod
+    def _tables(held, g: int, device, key):
+        """One table of G addresses for each (first address, bytes from one unit to the next) of ``key``; kept by the whole
+        key (the same buffers may hold units of another size on the next call), so a decode loop whose buffers repeat (and
+        a captured graph, whose buffers are fixed) builds them once."""
+        hit = held.get(key)
         if hit is not None:
-            self.i8_tabs.move_to_end(key)
+            held.move_to_end(key)
             return hit
-        g = q.shape[0]
+        tabs = tuple(torch.tensor([base + u * step for u in range(g)], dtype=torch.int64, device=device) for base, step in key)
+        held[key] = tabs
+        if len(held) > 8:
+            held.popitem(last=False)
+        return tabs
 
-        def tab(t):
-            step = t.stride(0) * t.element_size()
-            return torch.tensor([t.data_ptr() + u * step for u in range(g)], dtype=torch.int64, device=t.device)
 
-        self.i8_tabs[key] = (tab(q), tab(s_x), tab(y))
-        if len(self.i8_tabs) > 8:
-            self.i8_tabs.popitem(last=False)
-        return self.i8_tabs[key]
+def _unit_bytes(t: Tensor) -> int:
+    return t.stride(0) * t.element_size()
 
 
 def _fingerprint(layers):

@@ -52,3 +52,26 @@ def test_changes_between_calls_are_seen(int8):
         call(layers[:2] + [torch.nn.Linear(128, 64)], xs[:3])
     with pytest.raises((RuntimeError, TypeError)):
         call(_layers(), xs.cpu())
+
+
+def test_other_rows_types_and_strides_in_the_same_buffers():
+    """A held plan whose next call finds other units at the addresses of the call before."""
+    from bittorch_amd import _C, ops
+    n, k, g = 64, 128, 5
+    announce("grouped plans, same buffers", g, n, k)
+    layers = _layers(n, k, g)
+    xs, outs = torch.randn(g * 16 * k, device="cuda"), torch.empty(g * 16 * n, device="cuda")
+    q, s = torch.empty(g * 16 * k, device="cuda", dtype=torch.int8), torch.empty(g * 16, device="cuda")
+    for m, dtype in ((16, torch.float32), (5, torch.float32), (5, torch.bfloat16), (1, torch.float16), (16, torch.float32)):
+        q1, s1 = _C.act_quant_int8(xs[:g * m * k].view(g * m, k))
+        qv, sv = q[:g * m * k].view(g, m, k), s[:g * m].view(g, m)
+        qv.copy_(q1.view(g, m, k))
+        sv.copy_(s1.view(g, m))
+        out = outs.view(dtype)[:g * m * n].view(g, m, n)
+        want = torch.stack([L.forward_int8(qv[u], sv[u], dtype) for u, L in enumerate(layers)])
+        assert torch.equal(ops.ternary_linear_int8_grouped(layers, q=qv, s_x=sv, out_dtype=dtype, out=out), want)
+    h, outs = xs.half(), outs.view(torch.float16)
+    for wide_x, wide_y in ((1, 1), (2, 1), (1, 2), (2, 2), (1, 1)):
+        x, out = h[:g * wide_x * k].view(g, wide_x * k)[:, :k], outs[:g * wide_y * n].view(g, wide_y * n)[:, :n]
+        want = torch.cat([L(x[u:u + 1]) for u, L in enumerate(layers)])
+        assert torch.equal(ops.ternary_linear_grouped(layers, x, out=out), want)

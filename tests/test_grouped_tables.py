@@ -1,0 +1,38 @@
+"""CPU: the address tables of the grouped calls (``ops/grouped.py``) follow the sizes, types and strides of a call's buffers,
+also where a buffer's address is one seen before."""
+from collections import OrderedDict
+
+import pytest
+import torch
+
+
+def _plan():
+    grouped = pytest.importorskip("bittorch_amd.ops.grouped")
+    plan = object.__new__(grouped._Plan)  # (a plan's other tables hold device addresses of layers)
+    plan.io_tabs, plan.i8_tabs = OrderedDict(), OrderedDict()
+    return plan
+
+
+def _addresses(t):
+    return [t[u].data_ptr() for u in range(t.shape[0])]
+
+
+def test_int8_tables_of_other_rows_and_types_at_the_same_addresses():
+    plan, g, k, n = _plan(), 3, 64, 32
+    q, s, y = torch.zeros(g * 16 * k, dtype=torch.int8), torch.zeros(g * 16), torch.zeros(g * 16 * n)
+    for m, dtype in ((16, torch.float32), (5, torch.float32), (5, torch.bfloat16), (16, torch.bfloat16), (16, torch.float32)):
+        views = (q[:g * m * k].view(g, m, k), s[:g * m].view(g, m), y.view(dtype)[:g * m * n].view(g, m, n))
+        for tab, t in zip(plan.i8_tab(*views), views):
+            assert tab.tolist() == _addresses(t)
+
+
+def test_float_tables_of_other_strides_at_the_same_addresses():
+    plan, g, k, n = _plan(), 4, 64, 32
+    x, y = torch.zeros(g * 2 * k, dtype=torch.float16), torch.zeros(g * 2 * n, dtype=torch.float16)
+    xs = [x[:g * k].view(g, k), x.view(g, 2 * k)[:, :k]]
+    ys = [y[:g * n].view(g, n), y.view(g, 2 * n)[:, :n]]
+    for i, j in ((0, 0), (1, 0), (0, 1), (1, 1), (0, 0)):
+        xt, yt = plan.io_tab(xs[i], ys[j], False)
+        assert xt.tolist() == _addresses(xs[i]) and yt.tolist() == _addresses(ys[j])
+    row = x[:k].view(1, k)
+    assert plan.io_tab(row, ys[0], True)[0].tolist() == [x.data_ptr()] * g
