@@ -84,7 +84,10 @@ def _fingerprint(layers):
     for L in layers:
         d = L.__dict__
         buffers = d["_buffers"]
-        s, b, t = buffers["scale"], buffers["bias"], d["_tiled"]
+        # (a scale or bias that was made a Parameter is found by the ordinary lookup)
+        s = buffers["scale"] if "scale" in buffers else L.scale
+        b = buffers["bias"] if "bias" in buffers else L.bias
+        t = d["_tiled"]
         key.append((type(L), d["in_features"], d["out_features"], d["decode_tiled"], d["_tile_order"],
                     0 if t is None else t.data_ptr(), s.data_ptr(), s._version, s.numel(), s.dtype,
                     None if b is None else (b.data_ptr(), b._version, b.numel(), b.dtype)))

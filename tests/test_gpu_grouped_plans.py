@@ -75,3 +75,17 @@ def test_other_rows_types_and_strides_in_the_same_buffers():
         x, out = h[:g * wide_x * k].view(g, wide_x * k)[:, :k], outs[:g * wide_y * n].view(g, wide_y * n)[:, :n]
         want = torch.cat([L(x[u:u + 1]) for u, L in enumerate(layers)])
         assert torch.equal(ops.ternary_linear_grouped(layers, x, out=out), want)
+
+
+@pytest.mark.parametrize("int8", [False, True])
+def test_layers_whose_scales_and_biases_are_parameters(int8):
+    announce("grouped plans, parameters", int8)
+    layers = _layers()
+    x = torch.randn(5, 128, device="cuda").half()
+    for L in layers[1:3]:
+        L.scale, L.bias = torch.nn.Parameter(L.scale.clone()), torch.nn.Parameter(L.bias.clone())
+    with torch.no_grad():
+        for change in (lambda: None, lambda: layers[1].scale.mul_(2), lambda: layers[2].bias.add_(1)):
+            change()
+            _check(layers, x, int8)
+            _check(layers, x, int8)

@@ -36,3 +36,19 @@ def test_float_tables_of_other_strides_at_the_same_addresses():
         assert xt.tolist() == _addresses(xs[i]) and yt.tolist() == _addresses(ys[j])
     row = x[:k].view(1, k)
     assert plan.io_tab(row, ys[0], True)[0].tolist() == [x.data_ptr()] * g
+
+
+def test_fingerprint_of_a_layer_whose_scale_and_bias_are_parameters():
+    grouped = pytest.importorskip("bittorch_amd.ops.grouped")
+    from bittorch_amd import nn
+    layer = nn.create_ternary_linear_inference(64, 32, torch.randn(32, 64), torch.randn(32))
+    before = grouped._fingerprint([layer])
+    layer.scale, layer.bias = torch.nn.Parameter(layer.scale.clone()), torch.nn.Parameter(layer.bias.clone())
+    keys = [before, grouped._fingerprint([layer])]
+    with torch.no_grad():
+        layer.bias.add_(1)
+        keys.append(grouped._fingerprint([layer]))
+        layer.scale.mul_(2)
+        keys.append(grouped._fingerprint([layer]))
+    assert all(a != b for i, a in enumerate(keys) for b in keys[:i])
+    assert grouped._fingerprint([layer]) == keys[-1]
