@@ -121,19 +121,25 @@ class TernaryLinearInference(nn.Module):
         self._tile_order = order
 
     # ---- decode-tiled copy of the weights ---------------------------------------------------
+    def _tiled_fresh(self) -> bool:
+        """Whether the layer has its tiled copy, of the bytes a held ``weight_packed`` has now."""
+        if not self._has_row_major():
+            return self._tiled is not None
+        wp = self._buffers["weight_packed"]
+        return self._tiled is not None and self._tiled_key == (wp.data_ptr(), wp._version, wp.device, self._tile_order)
+
     def tiled_weights(self) -> Tensor:
         """The decode-tiled copy of the weights (GPU only).  Built on first use from ``weight_packed``, which is
         then released unless ``keep_row_major``; rebuilt when a held ``weight_packed`` has moved or been written."""
         if not self._has_row_major():
             return self._tiled
-        wp = self._buffers["weight_packed"]
-        key = (wp.data_ptr(), wp._version, wp.device, self._tile_order)
-        if self._tiled is None or self._tiled_key != key:
+        if not self._tiled_fresh():
             from .. import _C
+            wp = self._buffers["weight_packed"]
             self._tiled = _C.retile_weights(wp, self.in_features, self._tile_order == "gate_up_pairs")
             # built once on the current stream; later calls may come from any stream
             torch.cuda.current_stream(wp.device).synchronize()
-            self._tiled_key = key
+            self._tiled_key = (wp.data_ptr(), wp._version, wp.device, self._tile_order)
         if not self.keep_row_major and not torch.cuda.is_current_stream_capturing():
             del self._buffers["weight_packed"]  # one resident copy
         return self._tiled
@@ -231,9 +237,7 @@ class TernaryLinearInference(nn.Module):
             return None
         if not self._has_row_major():
             return self._tiled
-        wp = self._buffers["weight_packed"]
-        fresh = self._tiled is not None and self._tiled_key == (wp.data_ptr(), wp._version, wp.device, self._tile_order)
-        if not fresh and torch.cuda.is_current_stream_capturing():
+        if not self._tiled_fresh() and torch.cuda.is_current_stream_capturing():
             return None
         return self.tiled_weights()
 

@@ -88,9 +88,11 @@ def _fingerprint(layers):
         s = buffers["scale"] if "scale" in buffers else L.scale
         b = buffers["bias"] if "bias" in buffers else L.bias
         t = d["_tiled"]
+        w = buffers.get("weight_packed")  # (held beside the tiled copy: written or replaced, the copy is made again)
         key.append((type(L), d["in_features"], d["out_features"], d["decode_tiled"], d["_tile_order"],
-                    0 if t is None else t.data_ptr(), s.data_ptr(), s._version, s.numel(), s.dtype,
-                    None if b is None else (b.data_ptr(), b._version, b.numel(), b.dtype)))
+                    0 if t is None else t.data_ptr(), s.data_ptr(), s._version, s.stride(), s.numel(), s.dtype,
+                    None if b is None else (b.data_ptr(), b._version, b.stride(), b.numel(), b.dtype),
+                    None if w is None else (w.data_ptr(), w._version)))
     return key
 
 
@@ -146,7 +148,7 @@ def _groupable(layers, x: Tensor) -> bool:
             return False
         if L.bias is not None and (L.bias.dtype != L0.bias.dtype or L.bias.dtype not in kinds):
             return False
-        if L._tiled is None and torch.cuda.is_current_stream_capturing():
+        if not L._tiled_fresh() and torch.cuda.is_current_stream_capturing():
             return False  # (a capture never builds the tiled copy)
     return _kernels_allowed()
 

@@ -89,3 +89,36 @@ def test_layers_whose_scales_and_biases_are_parameters(int8):
             change()
             _check(layers, x, int8)
             _check(layers, x, int8)
+
+
+@pytest.mark.parametrize("int8", [False, True])
+def test_packed_weights_written_in_place_or_replaced(int8):
+    from bittorch_amd import ops
+    announce("grouped plans, packed weights", int8)
+    layers = _layers()
+    x = torch.randn(5, 128, device="cuda").half()
+    wide = torch.rand(128, device="cuda")
+
+    def scale_view(step):
+        layers[4].scale = wide[:64 * step:step]
+
+    for change in (lambda: None, lambda: layers[1].weight_packed.zero_(), lambda: layers[1].weight_packed[3].fill_(0x55),
+                   lambda: layers[2].weight_packed, lambda: setattr(layers[2], "weight_packed", layers[1].weight_packed.clone()),
+                   lambda: layers[2].drop_row_major(), lambda: scale_view(1), lambda: scale_view(2)):
+        change()
+        _check(layers, x, int8)
+        _check(layers, x, int8)
+    # written just before a capture: the captured call runs on the bytes as they are, copy or not
+    call = (lambda: ops.ternary_linear_int8_grouped(layers, x[:, None])) if int8 else (lambda: ops.ternary_linear_grouped(layers, x))
+    layers[1].weight_packed[5].fill_(0x11)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        got = call()
+    want = call()
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.allclose(got.float(), want.float(), rtol=2e-3, atol=1e-4)  # (fp16 of fp32 sums in another order)

@@ -52,3 +52,18 @@ def test_fingerprint_of_a_layer_whose_scale_and_bias_are_parameters():
         keys.append(grouped._fingerprint([layer]))
     assert all(a != b for i, a in enumerate(keys) for b in keys[:i])
     assert grouped._fingerprint([layer]) == keys[-1]
+
+
+def test_fingerprint_sees_packed_weights_and_strides():
+    """A held ``weight_packed`` written in place or replaced; a scale or bias that is another view of the same address."""
+    grouped = pytest.importorskip("bittorch_amd.ops.grouped")
+    from bittorch_amd import nn
+    layer = nn.create_ternary_linear_inference(64, 32, torch.randn(32, 64), torch.randn(64)[:32])
+    wide = torch.rand(64)
+    layer.scale = wide[:32]
+    keys = [grouped._fingerprint([layer])]
+    for change in (lambda: layer.weight_packed.bitwise_xor_(1), lambda: setattr(layer, "weight_packed", layer.weight_packed.clone()),
+                   lambda: setattr(layer, "scale", wide[::2]), lambda: setattr(layer, "bias", torch.as_strided(layer.bias, (32,), (2,)))):
+        change()
+        keys.append(grouped._fingerprint([layer]))
+    assert all(a != b for i, a in enumerate(keys) for b in keys[:i])
