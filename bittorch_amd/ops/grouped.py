@@ -20,6 +20,7 @@ from __future__ import annotations
 
 import os
 from collections import OrderedDict
+from operator import attrgetter, itemgetter
 from typing import List, Optional, Sequence, Union
 
 import torch
@@ -39,7 +40,7 @@ class _Plan:
         self.tiled = [L.tiled_weights() for L in layers]       # keeps the copies alive
         self.scales = [L.scale.contiguous() for L in layers]
         self.biases = None if layers[0].bias is None else [L.bias.contiguous() for L in layers]
-        self.held = [(L.scale, L.bias) for L in layers]        # (no other tensor takes their addresses meanwhile)
+        self.held = [(L.scale, L.bias) for L in layers]        # (no other tensor takes their place in the key meanwhile)
         self.key = _fingerprint(layers)
         self.w_tab = _C.pointer_table(self.tiled)
         self.s_tab = _C.pointer_table(self.scales)
@@ -76,24 +77,30 @@ def _unit_bytes(t: Tensor) -> int:
     return t.stride(0) * t.element_size()
 
 
+_data_ptr, _numel, _is_contiguous = Tensor.data_ptr, Tensor.numel, Tensor.is_contiguous
+_own_dict = attrgetter("__dict__")
+_settings = itemgetter("_buffers", "_tiled", "in_features", "out_features", "decode_tiled", "_tile_order")
+_vectors = itemgetter("scale", "bias")
+
+
 def _fingerprint(layers):
     """Everything about the layers that the checks below and a plan's tables depend on, read past ``nn.Module``'s
-    attribute lookup: with 128 layers the checks one by one took 1.2 ms of host time around a kernel of 87 us, comparing
-    this takes a tenth of it."""
-    key = []
-    for L in layers:
-        d = L.__dict__
-        buffers = d["_buffers"]
-        # (a scale or bias that was made a Parameter is found by the ordinary lookup)
-        s = buffers["scale"] if "scale" in buffers else L.scale
-        b = buffers["bias"] if "bias" in buffers else L.bias
-        t = d["_tiled"]
-        w = buffers.get("weight_packed")  # (held beside the tiled copy: written or replaced, the copy is made again)
-        key.append((type(L), d["in_features"], d["out_features"], d["decode_tiled"], d["_tile_order"],
-                    0 if t is None else t.data_ptr(), s.data_ptr(), s._version, s.stride(), s.numel(), s.dtype,
-                    None if b is None else (b.data_ptr(), b._version, b.stride(), b.numel(), b.dtype),
-                    None if w is None else (w.data_ptr(), w._version)))
-    return key
+    attribute lookup and one property of all layers at a time (with 128 layers the checks one by one took 1.2 ms of host
+    time around a kernel of 87 us, this takes about as long as the kernel).  Tensors count as themselves, which fixes
+    dtype and device (a plan keeps them alive); scales and biases may still be pointed elsewhere or shortened.  What is
+    written into one is read where it lies, except where the tables hold a contiguous copy of it."""
+    buffers, tiled, *settings = zip(*map(_settings, map(_own_dict, layers)))
+    try:
+        scales, biases = zip(*map(_vectors, buffers))
+    except KeyError:  # (made Parameters)
+        scales, biases = [L.scale for L in layers], [L.bias for L in layers]
+    vectors = [*scales, *(b for b in biases if b is not None)]
+    contiguous = list(map(_is_contiguous, vectors))
+    return [list(map(type, layers)), settings, list(map(id, tiled)),
+            # (weight_packed held beside the tiled copy: written or replaced, the copy is made again)
+            [(i, w.data_ptr(), w._version) for i, b in enumerate(buffers) if (w := b.get("weight_packed")) is not None],
+            list(map(id, vectors)), list(map(_data_ptr, vectors)), list(map(_numel, vectors)),
+            contiguous if all(contiguous) else [(v.stride(), v._version) for v in vectors]]
 
 
 def _known_plan(layers) -> Optional[_Plan]:

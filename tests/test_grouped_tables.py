@@ -42,28 +42,32 @@ def test_fingerprint_of_a_layer_whose_scale_and_bias_are_parameters():
     grouped = pytest.importorskip("bittorch_amd.ops.grouped")
     from bittorch_amd import nn
     layer = nn.create_ternary_linear_inference(64, 32, torch.randn(32, 64), torch.randn(32))
-    before = grouped._fingerprint([layer])
-    layer.scale, layer.bias = torch.nn.Parameter(layer.scale.clone()), torch.nn.Parameter(layer.bias.clone())
-    keys = [before, grouped._fingerprint([layer])]
-    with torch.no_grad():
-        layer.bias.add_(1)
-        keys.append(grouped._fingerprint([layer]))
-        layer.scale.mul_(2)
+    held = [layer.scale, layer.bias]  # (as a plan does)
+    keys = [grouped._fingerprint([layer])]
+    for name in ("scale", "bias"):
+        setattr(layer, name, torch.nn.Parameter(getattr(layer, name).clone()))
+        held.append(getattr(layer, name))
         keys.append(grouped._fingerprint([layer]))
     assert all(a != b for i, a in enumerate(keys) for b in keys[:i])
     assert grouped._fingerprint([layer]) == keys[-1]
 
 
-def test_fingerprint_sees_packed_weights_and_strides():
-    """A held ``weight_packed`` written in place or replaced; a scale or bias that is another view of the same address."""
+def test_fingerprint_sees_packed_weights_and_views():
+    """A held ``weight_packed`` written in place or replaced; a scale or bias that is another view of the same address, that
+    is shortened or pointed elsewhere, or that is written where the tables hold a contiguous copy of it."""
     grouped = pytest.importorskip("bittorch_amd.ops.grouped")
     from bittorch_amd import nn
     layer = nn.create_ternary_linear_inference(64, 32, torch.randn(32, 64), torch.randn(64)[:32])
-    wide = torch.rand(64)
+    wide, held = torch.rand(64), []
     layer.scale = wide[:32]
     keys = [grouped._fingerprint([layer])]
-    for change in (lambda: layer.weight_packed.bitwise_xor_(1), lambda: setattr(layer, "weight_packed", layer.weight_packed.clone()),
-                   lambda: setattr(layer, "scale", wide[::2]), lambda: setattr(layer, "bias", torch.as_strided(layer.bias, (32,), (2,)))):
-        change()
-        keys.append(grouped._fingerprint([layer]))
+    with torch.no_grad():
+        for change in (lambda: layer.weight_packed.bitwise_xor_(1), lambda: setattr(layer, "weight_packed", layer.weight_packed.clone()),
+                       lambda: setattr(layer, "bias", torch.as_strided(layer.bias, (32,), (2,))), lambda: layer.bias.add_(1),
+                       lambda: setattr(layer.bias, "data", layer.bias.clone()), lambda: setattr(layer, "scale", wide[::2]),
+                       lambda: setattr(layer.scale, "data", wide[:32]), lambda: setattr(layer.scale, "data", wide[:1]),
+                       lambda: setattr(layer, "bias", None)):
+            held += [layer.scale, layer.bias]
+            change()
+            keys.append(grouped._fingerprint([layer]))
     assert all(a != b for i, a in enumerate(keys) for b in keys[:i])
