@@ -53,23 +53,11 @@ def _dt(t: Tensor, what: str) -> int:
         raise RuntimeError(f"{what} must be float32, float16 or bfloat16, got {t.dtype}") from None
 
 
-_ws_cache = {}
-
-
 def _workspace(nbytes: int, device) -> Optional[Tensor]:
-    """Scratch buffer for the current stream of ``device``, kept between calls (the library
-    needs no initialisation of it).  One buffer per (device, stream): calls on one stream
-    run in order."""
-    if nbytes <= 0:
-        return None
-    key = (device.index if device.index is not None else torch.cuda.current_device(),
-           torch.cuda.current_stream(device).cuda_stream)
-    buf = _ws_cache.get(key)
-    if buf is None or buf.numel() < nbytes:
-        size = max(nbytes, 1 << 20)
-        buf = torch.empty(size, dtype=torch.uint8, device=device)
-        _ws_cache[key] = buf
-    return buf
+    """Scratch of one library call (the library needs no initialisation of it), its own: a call makes several launches and
+    ctypes lets go of the interpreter lock, so calls of other host threads can come between them on the same stream; and a
+    captured graph's launches keep addressing theirs, which the graph's pool then holds."""
+    return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes > 0 else None
 
 
 def _all_cuda(*ts: Optional[Tensor]) -> bool:
