@@ -14,6 +14,7 @@
 // the order of k inside an MFMA is free, so a lane loads the fp32 values themselves, splits them in registers (11 VALU
 // operations per pair) and decodes the weights in the matching order.  The split of one wave's rows is hidden behind the
 // MFMAs of the other wave of its SIMD: a tile of 64 x 128 needs 270 VALU operations (1080 cycles) per 96 MFMAs (1536).
+#include <cfloat>
 #include <cstddef>
 
 #include "bt_common.h"
@@ -35,14 +36,15 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint3
     const float la = ra - u2f(f2u(ra) & 0xFFFF0000u), lb = rb - u2f(f2u(rb) & 0xFFFF0000u);
     lo = perm(f2u(lb), f2u(la), 0x07060302u);
 }
-// The same with the middle term rounded to nearest, so that what it leaves has either sign (still exact: 16 bits remain
-// below hi, the rounded term takes 8 and the signed rest fits in 8).
+// The same with hi and mid rounded to nearest: hi leaves at most 2^-8 of x's power of two and mid at most 2^-17, and what is
+// left after each has either sign (still exact: 24 bits are 8, a sign and 8, a sign and 8).  Beyond the largest bf16 value hi
+// becomes an infinity and the other terms NaN.
 __device__ __forceinline__ void split_pair_rn(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-    hi = perm(f2u(b), f2u(a), 0x07060302u);
-    const float ra = a - u2f(f2u(a) & 0xFFFF0000u), rb = b - u2f(f2u(b) & 0xFFFF0000u);
     typedef float v2f __attribute__((ext_vector_type(2)));
     typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-    mid = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{ra, rb}), v2bf));  // v_cvt_pk_bf16_f32
+    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{a, b}), v2bf));  // v_cvt_pk_bf16_f32
+    const float ra = a - u2f(hi << 16), rb = b - u2f(hi & 0xFFFF0000u);
+    mid = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{ra, rb}), v2bf));
     const float la = ra - u2f(mid << 16), lb = rb - u2f(mid & 0xFFFF0000u);
     lo = perm(f2u(lb), f2u(la), 0x07060302u);
 }
@@ -436,8 +438,11 @@ struct GradWParams {
 
 // A wave owns a 64 x 64 tile of dW over its part of the rows.  Lane (i, g) loads columns 4i .. 4i+3 of rows 8g .. 8g+7 of
 // both matrices: component t of those eight float4 is its operand of the MFMA whose row (column) i is matrix column 4i + t,
-// so the transposition costs nothing.  Both operands are split, and of the nine products of terms the six whose weight
-// is at least 2^-17 are formed (the rest are below 2^-25 of a product and have either sign).
+// so the transposition costs nothing.  Both operands are split, and of the nine products of terms six are formed: mid lo and
+// lo mid are at most 2^-25 of the product each and have either sign.  Sums of up to 8 products are formed as fp32 products
+// instead: an MFMA's sums are fewer but not rounded to nearest.  Relative error of 1 / 2 / 4 / 16 rows: MFMAs of all terms
+// 4.3e-8 / 4.2e-8 / 4.1e-8 / 4.2e-8, the vendor's fp32 product 3.6e-8 / 4.1e-8 / 4.8e-8 / 7.8e-8.
+constexpr int GRAD_W_FEW_ROWS = 8;
 template <bool DIRECT>
 __global__ __launch_bounds__(256, 2) void grad_w_f32_kernel(GradWParams p) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -499,6 +504,18 @@ __global__ __launch_bounds__(256, 2) void grad_w_f32_kernel(GradWParams p) {
     const int kt = (int)(k0 >> 6), nkt = (int)((p.K + 63) >> 6);
     float bsum[4] = {0.f, 0.f, 0.f, 0.f};
     int turn = DIRECT ? (kt == 0 ? 0 : -1) : (int)((kt + nkt - (int)(s0 % nkt)) % nkt);
+    auto add_bias = [&](const f32x4_u (&cur)[8]) {
+        if (turn == 0) {
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                float v = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; e++) v += cur[e][t];
+                bsum[t] += v;
+            }
+        }
+        if constexpr (!DIRECT) turn = (turn == 0) ? nkt - 1 : turn - 1;
+    };
 
     u32x4 pg[2][3];
     auto split_g = [&](int t, const f32x4_u (&src)[8]) {
@@ -521,18 +538,7 @@ __global__ __launch_bounds__(256, 2) void grad_w_f32_kernel(GradWParams p) {
                 px[0][t][c] = h; px[1][t][c] = m; px[2][t][c] = l;
             }
         if (more) load_x(nx, false);
-        if (p.bias_out) {  // uniform
-            if (turn == 0) {
-#pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    float v = 0.0f;
-#pragma unroll
-                    for (int e = 0; e < 8; e++) v += cur[e][t];
-                    bsum[t] += v;
-                }
-            }
-            if constexpr (!DIRECT) turn = (turn == 0) ? nkt - 1 : turn - 1;
-        }
+        if (p.bias_out) add_bias(cur);  // uniform
         split_g(0, cur);
         __builtin_amdgcn_sched_barrier(0);
         constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};  // smallest terms first
@@ -546,8 +552,31 @@ __global__ __launch_bounds__(256, 2) void grad_w_f32_kernel(GradWParams p) {
             __builtin_amdgcn_sched_barrier(0);
         }
     };
+    // the tile's sums over rows m .. m1 - 1 as fp32 forms the products
+    auto sum_fp32 = [&](int64_t m, int64_t m1) {
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int u = 0; u < 4; u++) acc[t][u] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (; m < m1; m++) {
+            const f32x4_u xv = *(const f32x4_u*)(p.X + m * p.K + col_x(i));
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const f32x4_u gv = *(const f32x4_u*)(p.G + m * p.N + col_g(4 * g + r));
+#pragma unroll
+                for (int t = 0; t < 4; t++)
+#pragma unroll
+                    for (int u = 0; u < 4; u++) acc[t][u][r] = __builtin_fmaf(gv[t], xv[u], acc[t][u][r]);
+            }
+        }
+    };
     const int64_t sf = s1 < nfull ? s1 : nfull;  // whole steps of this part
-    if (s0 < sf) {
+    const bool few = p.M <= GRAD_W_FEW_ROWS;     // (a single partial step)
+    if (few) {
+        sum_fp32(0, p.M);
+        load_g(0, gr[0], true);
+        if (p.bias_out) add_bias(gr[0]);
+    } else if (s0 < sf) {
         load_g(s0, gr[0], false);
         load_x(s0, false);
         int64_t s = s0;
@@ -557,21 +586,22 @@ __global__ __launch_bounds__(256, 2) void grad_w_f32_kernel(GradWParams p) {
         }
         if (s < sf) step(0, gr[0], gr[1], false);
     }
-    if (s1 > nfull) {  // the last part's partial step
+    if (!few && s1 > nfull) {  // the last part's partial step
         load_g(nfull, gr[0], true);
         load_x(nfull, true);
         step(0, gr[0], gr[1], false);
     }
 
-    // A non-finite operand has no finite terms and left a NaN in every sum it meets: such a tile is summed again as fp32
-    // forms the products.
+    // A non-finite operand has no finite terms and left a NaN in every sum it meets, one beyond the largest bf16 value likewise,
+    // and a product of rounded terms may overflow where the product does not: such a tile is summed again as fp32 forms the
+    // products.
     bool bad = false;
 #pragma unroll
     for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int u = 0; u < 4; u++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) bad |= acc[t][u][r] != acc[t][u][r];
+            for (int r = 0; r < 4; r++) bad |= !(fabsf(acc[t][u][r]) <= FLT_MAX);
     if (bad) {
         const int64_t m1 = s1 * 32 < p.M ? s1 * 32 : p.M;
         for (int t = 0; t < 4; t++)

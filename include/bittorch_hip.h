@@ -411,8 +411,10 @@ int bt_unpack_dequant(const uint8_t* W_T, const float* scale, int64_t scale_len,
  *   bt_ternary_linear_grad_input   dX [M,K] = (dY [M,N] * scale) decode(W_T); dX 16-byte aligned
  *   bt_linear_grad_weight          dW [N,K] = scale[n] * sum_m dY[m,n] X[m,k] and, if dBias is not NULL,
  *                                  dBias [N] = sum_m dY[m,n]; N and K at least 4; workspace as described above
- * Everything is fp32 (scale_len: N, or 1 for a per-tensor scale); products are formed from exact bf16 terms of the
- * operands and summed in fp32.
+ * Everything is fp32 (scale_len: N, or 1 for a per-tensor scale).  An operand is split into three bf16 terms that are its value
+ * exactly (down to 2^-109; smaller ones lose bits below 2^-133) and the products of terms are summed in fp32: all of them for
+ * dX, six of nine for dW over more than 8 rows (the two largest of the rest are at most 2^-25 of a product each).  Over up to
+ * 8 rows dW is formed of fp32 products.
  */
 int bt_ternary_linear_grad_input(const float* dY, const uint8_t* W_T, const float* scale, int64_t scale_len, float* dX,
                                  int64_t M, int64_t N, int64_t K, void* stream);

@@ -1,8 +1,11 @@
 """GPU: the fp32 matrix-core kernels of ``csrc/gemm_f32.hip`` (forward on row-major and tiled weights, input gradient,
 weight and bias gradient) against float64.
 
-Every product is formed from exact bf16 terms (weight gradient: up to terms below 2^-25 of it) and added in fp32, at most
-six terms per product: the error of a sum of C products is at most 6 (C + 8) 2^-24 of the sum of the products' magnitudes.
+Every product is formed from bf16 terms that are the operands exactly, and they are added in fp32.  With ``C`` products in
+steps of 32, the largest terms of all products and, once a step each, the sums of the smaller ones are added to a sum of full
+size: at most ``C + (kinds of terms - 1) ceil(C / 32)`` roundings of 2^-24 of the sum of the products' magnitudes, and as many
+more as parts of the sum are added up or factors multiplied.  The weight gradient leaves out two kinds of terms of at most
+2^-25 of a product each; over up to 8 rows it is formed of fp32 products.
 """
 import pytest
 import torch
@@ -17,13 +20,23 @@ SHAPES = [(1, 4, 4), (33, 4, 5), (40, 20, 33), (65, 64, 31), (64, 256, 32), (129
           (513, 1028, 96), (1000, 36, 2048), (2100, 768, 260), (4099, 516, 516), (16384, 192, 130)]
 
 
-def _close(got, a, b, scale=1.0):
+def _close(got, a, b, roundings, scale=1.0):
     """got against a @ b in float64, by the bound above; scale: a factor of the rows or columns that is rounded too"""
     ref = (a.double() @ b.double()) * scale
-    bound = 6 * (a.shape[1] + 8) * EPS * ((a.double().abs() @ b.double().abs()) * scale) + 1e-37
+    bound = roundings * EPS * ((a.double().abs() @ b.double().abs()) * scale) + 1e-37
     assert torch.isfinite(got).all()
     err = (got.double() - ref).abs()
     assert bool((err <= bound).all()), float((err / bound).max())
+
+
+def _three_terms(c):
+    """Of a sum of c products with a ternary operand: up to 8 parts, a rounded factor before and after, the last rounding."""
+    return c + 2 * ((c + 31) // 32) + 11
+
+
+def _six_terms(m):
+    """Of a weight gradient over m rows (up to 8: fp32 products): parts of 256 rows or more, the scale."""
+    return m + 1 if m <= 8 else m + 5 * ((m + 31) // 32) + (m + 255) // 256 + 2
 
 
 def _case(m, n, k, per_channel=True):
@@ -41,16 +54,16 @@ def test_fp32_products_against_float64(m, n, k):
     from bittorch_amd import _C
     announce("fp32 gradients", m, n, k)
     x, dy, packed, scale, tern = _case(m, n, k)
-    _close(_C.linear_grad_input(dy, packed, scale, k), dy, tern * scale[:, None])
+    _close(_C.linear_grad_input(dy, packed, scale, k), dy, tern * scale[:, None], _three_terms(n))
     dw, db = _C.linear_grad_weight(dy, x, scale, True)
-    _close(dw, dy.t(), x, scale.double()[:, None])
-    _close(db[:, None], dy.t(), torch.ones(m, 1, device="cuda"))
+    _close(dw, dy.t(), x, _six_terms(m), scale.double()[:, None])
+    _close(db[:, None], dy.t(), torch.ones(m, 1, device="cuda"), m)
     assert torch.equal(_C.linear_grad_weight(dy, x, scale, True)[0], dw)  # a fixed order of the sums
     if m > 32 and n % 4 == 0:
         y = _C.ternary_linear_packed_forward(x, packed, scale, None, k)
-        _close(y, x, tern.t(), scale.double()[None, :])
+        _close(y, x, tern.t(), _three_terms(k), scale.double()[None, :])
         _close(_C.ternary_linear_tiled_forward(x, _C.retile_weights(packed, k), scale, None, k, n), x, tern.t(),
-               scale.double()[None, :])
+               _three_terms(k), scale.double()[None, :])
 
 
 @gpu
@@ -61,10 +74,45 @@ def test_fp32_gradients_one_scale_strides_and_alignment(m, n, k):
     announce("fp32 gradients, views", m, n, k)
     x, dy, packed, scale, tern = _case(m, n, k, per_channel=False)
     off = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view_as(t)
-    _close(_C.linear_grad_input(off(dy), packed, scale, k), dy, tern * scale)
-    _close(_C.linear_grad_weight(off(dy), off(x), scale)[0], dy.t(), x, float(scale))
+    _close(_C.linear_grad_input(off(dy), packed, scale, k), dy, tern * scale, _three_terms(n))
+    _close(_C.linear_grad_weight(off(dy), off(x), scale)[0], dy.t(), x, _six_terms(m), float(scale))
     wide = dy[:, :1].expand(m, n)
-    _close(_C.linear_grad_weight(wide, x, scale)[0], wide.t(), x, float(scale))
+    _close(_C.linear_grad_weight(wide, x, scale)[0], wide.t(), x, _six_terms(m), float(scale))
+
+
+@gpu
+@pytest.mark.parametrize("m", [1, 2, 8, 9, 31, 32, 33, 300])
+def test_weight_gradient_of_few_rows(m):
+    """Sums of few products, whose terms left out would show: operands over the whole range of significands, those with the
+    largest terms behind the first (next to 1 + 2^-7 and 1 + 2^-8) among them."""
+    from bittorch_amd import _C
+    n, k = 260, 520
+    announce("fp32 weight gradient, few rows", m)
+    g = torch.Generator("cuda").manual_seed(m)
+    values = lambda *s: torch.where(torch.rand(*s, generator=g, device="cuda") < 0.5, 1 + torch.rand(*s, generator=g, device="cuda"),
+                                    1 + torch.rand(*s, generator=g, device="cuda") * 2.0 ** -6)
+    dy, x, scale = values(m, n), values(m, k), torch.rand(n, generator=g, device="cuda") + 0.5
+    x[:, :4], dy[:, :4] = 1.0077972, 1.0077972
+    for sign in (1.0, -1.0):
+        dy[:, 1::2] *= sign
+        _close(_C.linear_grad_weight(dy, x, scale)[0], dy.t(), x, _six_terms(m), scale.double()[:, None])
+
+
+@gpu
+def test_weight_gradient_of_the_largest_values():
+    """Next to the largest float, where an operand's first term or a product of terms is an infinity and the product is not."""
+    from bittorch_amd import _C
+    announce("fp32 weight gradient, largest values")
+    m, n, k, top = 40, 36, 68, 3.4028234663852886e38
+    dy, x, scale = torch.zeros(m, n, device="cuda"), torch.zeros(m, k, device="cuda"), torch.ones(n, device="cuda")
+    dy[3], x[3] = 1.0, 1.0
+    dy[3, 5], x[3, 7] = top, -top * (1 - 2.0 ** -12)       # beyond the largest bf16 value
+    dy[3, 9], x[3, 11] = 1.9985 * 2.0 ** 63, 1.9985 * 2.0 ** 63  # (their first terms are 2^64)
+    got = _C.linear_grad_weight(dy, x, scale)[0].double()
+    want = (dy.double().t() @ x.double())
+    want[want.abs() > top] *= float("inf")
+    fin = torch.isfinite(want)
+    assert torch.equal(got[~fin], want[~fin]) and bool(((got - want)[fin].abs() <= 2.0 ** -24 * want[fin].abs()).all())
 
 
 @gpu
