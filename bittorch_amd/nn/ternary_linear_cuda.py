@@ -27,14 +27,17 @@ def _fp32_kernels_serve(g2: Tensor, x2: Tensor, packed: Optional[Tensor], scale:
     """Whether this backward runs on the library's gradient kernels: fp32 throughout, and no graph of the backward itself
     wanted (``create_graph=True``: the torch products below are differentiable).  A batched gradient
     (``is_grads_batched=True``, a vectorized Jacobian) has no memory of its own to hand to a kernel."""
-    if packed is None or torch.is_grad_enabled() or g2.numel() == 0:
-        return False
-    if _batched(g2):
+    if packed is None or torch.is_grad_enabled() or g2.numel() == 0 or _batched(g2) or _generic_forced():
         return False
     if not (g2.dtype == x2.dtype == scale.dtype == torch.float32 and g2.is_cuda):
         return False
     n, k = g2.shape[1], x2.shape[1]
     return 4 <= n < 2 ** 23 and 4 <= k < 2 ** 23 and packed.numel() < 2 ** 32
+
+
+def _generic_forced() -> bool:
+    """``BITTORCH_KERNEL=generic``: no kernel but the shape-generic ones, in the backward either (read on every call)."""
+    return os.environ.get("BITTORCH_KERNEL") == "generic"
 
 
 def _batched(t: Tensor) -> bool:
@@ -50,7 +53,7 @@ def _scale_to_master(g: Tensor, scale: Tensor, master_dtype: torch.dtype) -> Ten
     """The 16-bit product ``dY^T X`` times its scale.  For fp32 masters (autocast) the scale and the widening that autograd
     would do next are one pass, with the same bits; a differentiated or batched backward stays on torch."""
     if (master_dtype == torch.float32 and g.dtype in (torch.float16, torch.bfloat16) and g.is_cuda and g.numel() > 0
-            and g.shape[0] * ((g.shape[1] + 2047) // 2048) < 2 ** 30 and not torch.is_grad_enabled() and not _batched(g)):
+            and not _generic_forced() and g.shape[0] * ((g.shape[1] + 2047) // 2048) < 2 ** 30 and not torch.is_grad_enabled() and not _batched(g)):
         from .. import _C
         return _C.scale_grad_weight(g, scale)
     return g * scale.reshape(-1, 1).to(g.dtype)
@@ -92,7 +95,7 @@ class TernaryLinearCUDAFunction(torch.autograd.Function):
                 packed, scale, _ = _C.ternary_quantize_pack(weight, threshold_factor, per_channel, as_half=as_half)
             b = None if bias is None else bias.to(x.dtype).contiguous()
             if (tiled is not None and x.dtype in (torch.float16, torch.bfloat16, torch.float32)
-                    and os.environ.get("BITTORCH_KERNEL") != "generic"):  # (the shape-generic kernel reads packed_T)
+                    and not _generic_forced()):  # (the shape-generic kernel reads packed_T)
                 out = _C.ternary_linear_tiled_forward(x.contiguous(), tiled, scale.reshape(-1).to(x.dtype), b,
                                                       weight.shape[1], weight.shape[0])
             else:

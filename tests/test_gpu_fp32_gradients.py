@@ -162,3 +162,22 @@ def test_fp32_layer_batched_gradients():
     for i in range(3):
         for a, b in zip(batched, torch.autograd.grad(y, leaves, gys[i], retain_graph=True)):
             assert torch.allclose(a[i], b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))
+
+
+@gpu
+def test_generic_kernels_forced_in_the_backward(monkeypatch):
+    """``BITTORCH_KERNEL=generic`` keeps the backward off the matrix-core kernels too: the torch products, bit for bit."""
+    from bittorch_amd import _C, nn
+    announce("fp32 layer backward, generic")
+    monkeypatch.setenv("BITTORCH_KERNEL", "generic")
+    for name in ("linear_grad_input", "linear_grad_weight", "scale_grad_weight"):
+        monkeypatch.setattr(_C, name, None)
+    layer = nn.TernaryLinear(96, 40).cuda()
+    x, gy = torch.randn(70, 96, device="cuda", requires_grad=True), torch.randn(70, 40, device="cuda")
+    gx, gw, gb = torch.autograd.grad(layer(x), (x, layer.weight, layer.bias), gy)
+    packed, scale, _ = _C.ternary_quantize_pack(layer.weight.detach(), layer.threshold_factor, True)
+    assert torch.equal(gx, gy @ _C.unpack_dequant(packed, 96, scale, torch.float32))
+    assert torch.equal(gw, (gy.t() @ x.detach()) * scale[:, None]) and torch.equal(gb, gy.sum(0))
+    with torch.autocast("cuda", dtype=torch.float16):
+        y = layer(x)
+    assert torch.autograd.grad(y, layer.weight, gy.half())[0].dtype == torch.float32
