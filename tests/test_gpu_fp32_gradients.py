@@ -181,3 +181,19 @@ def test_generic_kernels_forced_in_the_backward(monkeypatch):
     with torch.autocast("cuda", dtype=torch.float16):
         y = layer(x)
     assert torch.autograd.grad(y, layer.weight, gy.half())[0].dtype == torch.float32
+
+
+@gpu
+@pytest.mark.parametrize("n", [1, 4, 7, 8, 9])
+def test_input_gradient_of_few_outputs(n):
+    """Of a layer with few outputs: up to 7 the product of exact factors, from 8 on each product may have a rounding of its own."""
+    from bittorch_amd import _C, nn
+    announce("fp32 layer backward, few outputs", n)
+    g = torch.Generator("cuda").manual_seed(n)
+    layer = nn.TernaryLinear(260, n, bias=False).cuda()
+    x, gy = torch.ones(600, 260, device="cuda", requires_grad=True), torch.randn(600, n, generator=g, device="cuda")
+    got = torch.autograd.grad(layer(x), x, gy)[0]
+    packed, scale, tern = _C.ternary_quantize_pack(layer.weight.detach(), layer.threshold_factor, True, True, True)
+    _close(got, gy, tern.float() * scale[:, None], _three_terms(n))
+    if n < 8:
+        assert torch.equal(got, gy @ _C.unpack_dequant(packed, 260, scale, torch.float32))
