@@ -36,7 +36,12 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint3
     const float la = ra - u2f(f2u(ra) & 0xFFFF0000u), lb = rb - u2f(f2u(rb) & 0xFFFF0000u);
     lo = perm(f2u(lb), f2u(la), 0x07060302u);
 }
-// The same with hi and mid rounded to nearest: hi leaves at most 2^-8 of x's power of two and mid at most 2^-17, and what is
+// The same for any value: the smaller terms of an infinity or NaN are zero, so that it meets a weight as fp32 has it.
+__device__ __forceinline__ void split_pair_any(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+    split_pair(fabsf(a) <= FLT_MAX ? a : 0.0f, fabsf(b) <= FLT_MAX ? b : 0.0f, hi, mid, lo);
+    hi = perm(f2u(__builtin_canonicalizef(b)), f2u(__builtin_canonicalizef(a)), 0x07060302u);  // (a quiet NaN's top half is one)
+}
+// The same as the first with hi and mid rounded to nearest: hi leaves at most 2^-8 of x's power of two and mid at most 2^-17, and what is
 // left after each has either sign (still exact: 24 bits are 8, a sign and 8, a sign and 8).  Beyond the largest bf16 value hi
 // becomes an infinity and the other terms NaN.
 __device__ __forceinline__ void split_pair_rn(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
@@ -199,13 +204,8 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
     };
 
     v4f acc[4][4 * NG];
-#pragma unroll
-    for (int b = 0; b < 4; b++)
-#pragma unroll
-        for (int t = 0; t < 4 * NG; t++) acc[b][t] = v4f{0.f, 0.f, 0.f, 0.f};
-
     u32x4 pl[2][3];  // the planes of two row blocks: one in the MFMAs, the next being split
-    auto split = [&](int b, const f32x4_u (&scn)[2]) {
+    auto split = [&](int b, const f32x4_u (&scn)[2], auto any) __attribute__((always_inline)) {
         float x[8];
 #pragma unroll
         for (int e = 0; e < 8; e++) x[e] = raw[b][e >> 2][e & 3];
@@ -220,12 +220,13 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
             const int e0 = (SRC == B_TRANSPOSED) ? (4 * (c >> 1) + 1 - (c & 1)) : c;
             const int e1 = (SRC == B_TRANSPOSED) ? e0 + 2 : 4 + c;
             uint32_t h, m, l;
-            split_pair(x[e0], x[e1], h, m, l);
+            if constexpr (decltype(any)::value) split_pair_any(x[e0], x[e1], h, m, l);
+            else split_pair(x[e0], x[e1], h, m, l);
             pl[b & 1][0][c] = l; pl[b & 1][1][c] = m; pl[b & 1][2][c] = h;
         }
     };
 
-    auto step = [&](int nx, bool more) {  // nx: the step whose operands are requested behind this one's use (uniform)
+    auto step = [&](int nx, bool more, auto any) __attribute__((always_inline)) {  // nx: the step whose operands are requested behind this one's use (uniform)
         u32x4 w[4 * NG];
 #pragma unroll
         for (int q = 0; q < NG; q++)
@@ -246,13 +247,13 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
             }
         const f32x4_u scn[2] = {sc[0], sc[1]};
         if (more) load_w(nx, false);
-        split(0, scn);
+        split(0, scn, any);
         if (more) load_a(0, nx, false);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int b = 0; b < 4; b++) {
             if (b < 3) {
-                split(b + 1, scn);
+                split(b + 1, scn, any);
                 if (more) load_a(b + 1, nx, false);
             }
 #pragma unroll
@@ -262,17 +263,35 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    if (st0 < st1) {
-        load_w(st0, false);
+    auto contract = [&](auto any) __attribute__((always_inline)) {
 #pragma unroll
-        for (int b = 0; b < 4; b++) load_a(b, st0, false);
-        for (int s = st0; s < st1; s++) step(s + 1 < st1 ? s + 1 : s, true);  // (past the end: the last one again, never used)
-    }
-    if (last && nfull < steps) {
-        load_w(nfull, true);
+        for (int b = 0; b < 4; b++)
 #pragma unroll
-        for (int b = 0; b < 4; b++) load_a(b, nfull, true);
-        step(0, false);
+            for (int t = 0; t < 4 * NG; t++) acc[b][t] = v4f{0.f, 0.f, 0.f, 0.f};
+        if (st0 < st1) {
+            load_w(st0, false);
+#pragma unroll
+            for (int b = 0; b < 4; b++) load_a(b, st0, false);
+            for (int s = st0; s < st1; s++) step(s + 1 < st1 ? s + 1 : s, true, any);  // (past the end: the last one again, never used)
+        }
+        if (last && nfull < steps) {
+            load_w(nfull, true);
+#pragma unroll
+            for (int b = 0; b < 4; b++) load_a(b, nfull, true);
+            step(0, false, any);
+        }
+    };
+    contract(std::false_type{});
+    if constexpr (SRC == B_TRANSPOSED) {
+        // a non-finite value has no finite terms and left a NaN in its row: once more, with such values as they are
+        bool bad = false;
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+#pragma unroll
+            for (int t = 0; t < 4 * NG; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) bad |= acc[b][t][r] != acc[b][t][r];
+        if (__any(bad)) contract(std::true_type{});
     }
     if constexpr (KS > 1) {
         // the upper half of the waves hands its sums to the lower half, until wave 0 has them all; NG words of 16 KiB each
@@ -321,19 +340,6 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
 #pragma unroll
                 for (int t = 0; t < 4; t++) y[t] = acc[b][4 * q + t][r] * 2.0f;
                 if constexpr (SRC == B_TRANSPOSED) {
-                    bool bad = false;
-#pragma unroll
-                    for (int t = 0; t < 4; t++) bad |= y[t] != y[t];
-                    if (bad) {  // a non-finite value has no finite terms: the products as fp32 forms them
-#pragma unroll
-                        for (int t = 0; t < 4; t++) y[t] = 0.0f;
-                        const uint8_t* wr = p.W + (int64_t)(col >> 2) * p.ldw;
-                        for (int64_t n = 0; n < p.C; n++) {
-                            const float v = SC ? __fmul_rn(p.X[m * p.C + n], p.a_scale[n]) : p.X[m * p.C + n];
-#pragma unroll
-                            for (int t = 0; t < 4; t++) y[t] += v * (float)decode2((wr[n] >> (2 * t)) & 3u);
-                        }
-                    }
                     if (p.y_scale) {
 #pragma unroll
                         for (int t = 0; t < 4; t++) y[t] = __fmul_rn(y[t], p.y_scale[0]);
@@ -558,6 +564,7 @@ __global__ __launch_bounds__(256, 2) void grad_w_f32_kernel(GradWParams p) {
         for (int t = 0; t < 4; t++)
 #pragma unroll
             for (int u = 0; u < 4; u++) acc[t][u] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4  // (the loads of four rows at once; a backward of 16384 x 768 x 768 full of NaN 730 -> 590 us)
         for (; m < m1; m++) {
             const f32x4_u xv = *(const f32x4_u*)(p.X + m * p.K + col_x(i));
 #pragma unroll
@@ -602,24 +609,7 @@ __global__ __launch_bounds__(256, 2) void grad_w_f32_kernel(GradWParams p) {
         for (int u = 0; u < 4; u++)
 #pragma unroll
             for (int r = 0; r < 4; r++) bad |= !(fabsf(acc[t][u][r]) <= FLT_MAX);
-    if (bad) {
-        const int64_t m1 = s1 * 32 < p.M ? s1 * 32 : p.M;
-        for (int t = 0; t < 4; t++)
-            for (int r = 0; r < 4; r++) {
-                float v[4] = {0.f, 0.f, 0.f, 0.f};
-                for (int64_t m = s0 * 32; m < m1; m++) {
-                    const float gv = p.G[m * p.N + col_g(4 * g + r) + t];
-                    for (int u = 0; u < 4; u++) v[u] = __builtin_fmaf(gv, p.X[m * p.K + col_x(i) + u], v[u]);
-                }
-                // (registers are not addressed by loop variables: selects)
-#pragma unroll
-                for (int tt = 0; tt < 4; tt++)
-#pragma unroll
-                    for (int rr = 0; rr < 4; rr++)
-#pragma unroll
-                        for (int u = 0; u < 4; u++) acc[tt][u][rr] = (tt == t && rr == r) ? v[u] : acc[tt][u][rr];
-            }
-    }
+    if (bad) sum_fp32(s0 * 32, s1 * 32 < p.M ? s1 * 32 : p.M);
 
     float* out = p.out + (DIRECT ? 0 : (int64_t)split * p.N * p.K);
 #pragma unroll

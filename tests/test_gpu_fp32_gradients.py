@@ -116,22 +116,48 @@ def test_weight_gradient_of_the_largest_values():
 
 
 @gpu
-def test_fp32_gradients_of_non_finite_values():
+@pytest.mark.parametrize("per_channel", [True, False])
+@pytest.mark.parametrize("m,n,k", [(300, 64, 96), (7, 100, 96), (16384, 100, 256), (1000, 1100, 640), (130, 4128, 516)])
+def test_fp32_gradients_of_non_finite_values(m, n, k, per_channel):
     """An infinity or NaN in the output gradient (an overflown loss) leaves what the fp32 products leave: the same
     elements non-finite, infinities with their sign, everything else untouched."""
     from bittorch_amd import _C
-    m, n, k = 300, 64, 96
-    announce("fp32 gradients, non-finite", m, n, k)
-    x, dy, packed, scale, tern = _case(m, n, k)
-    dy[7, 5], dy[90, 11], dy[200, 40] = float("inf"), float("-inf"), float("nan")
-    x[120, 3] = float("inf")
+    announce("fp32 gradients, non-finite", m, n, k, per_channel)
+    x, dy, packed, scale, tern = _case(m, n, k, per_channel)
+    dy[1, 5], dy[m // 3, 11], dy[m // 2, 40], dy[5, n - 1] = float("inf"), float("-inf"), float("nan"), float("inf")
+    dy[m - 1, 3] = torch.tensor(0x7F800001).int().view(torch.float32).cuda()  # (a NaN whose upper half is an infinity's)
+    x[m // 4, 3] = float("inf")
     for got, ref in ((_C.linear_grad_input(dy, packed, scale, k), dy.double() @ (tern * scale[:, None]).double()),
                      (_C.linear_grad_weight(dy, x, scale)[0], (dy.double().t() @ x.double()) * scale.double()[:, None])):
         assert torch.equal(torch.isnan(got), torch.isnan(ref))
         inf = torch.isinf(ref)
         assert torch.equal(got[inf].double(), ref[inf]) and inf.any()
         fin = torch.isfinite(ref)
-        assert torch.allclose(got[fin].double(), ref[fin], rtol=1e-4, atol=1e-6)
+        assert torch.allclose(got[fin].double(), ref[fin], rtol=1e-4, atol=1e-5 * float(ref[fin].abs().max()))
+
+
+@gpu
+def test_non_finite_gradients_take_the_time_of_a_few_products():
+    """A diverged step is no hundred times slower than the others (a tile is computed again, not element by element)."""
+    from bittorch_amd import _C
+    m, n, k = 4096, 768, 768
+    announce("fp32 gradients, non-finite, time", m, n, k)
+    x, dy, packed, scale, _ = _case(m, n, k)
+
+    def microseconds(g):
+        times = []
+        for _ in range(7):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            _C.linear_grad_input(g, packed, scale, k)
+            _C.linear_grad_weight(g, x, scale, True)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(end) * 1e3)
+        return sorted(times)[3]
+
+    finite, nan = microseconds(dy), microseconds(torch.full_like(dy, float("nan")))
+    assert nan < 12 * finite, (finite, nan)  # (element by element: 60 times)
 
 
 @gpu
