@@ -87,6 +87,7 @@ bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, co
 double gemm_f16_cost(int64_t M, int64_t N, int64_t K);
 int launch_gemm_f16(int mode, const void* X, const uint8_t* W_T, int w_layout, const Epilogue& epi, void* Y, int64_t M,
                     int64_t N, int64_t K, hipStream_t st);
+bool gemm_f32_shape_ok(int64_t N, int64_t K);
 bool gemm_f32_supported(int64_t N, int64_t K, const void* X, const void* Y);
 double gemm_f32_cost(int64_t M, int64_t N, int64_t K);
 int launch_gemm_f32(const void* X, const uint8_t* W, int w_layout, const Epilogue& epi, void* Y, int64_t M, int64_t N,
@@ -259,8 +260,9 @@ static bool packed_uses_stream(int x_dtype, const void* W_T, const void* Y, int6
     return x_dtype != BT_F32 && stream_supported(N, K, W_T) && fast_path_ok(Y, N, K);
 }
 
-// fp32 activations run on the bf16 matrix-core kernels as three exact bf16 planes (hi, mid, lo), each
-// zero-padded to the kernels' 64-wide step; the planes live in the workspace.
+// fp32 activations run on the bf16 matrix cores as three exact bf16 terms (hi, mid, lo): split in registers by
+// gemm_f32_kernel, or, for the streaming kernel and its output stage, into planes in the workspace, each zero-padded to
+// the kernels' 64-wide step.
 static int64_t plane_len(int64_t K) { return ceil_div(K, 64) * 64; }
 static size_t f32_planes_bytes(int64_t B, int64_t K) { return align256((size_t)B * 3 * plane_len(K) * 2); }
 static bool packed_uses_f32_planes(const void* W_T, const void* Y, int64_t N, int64_t K) {
@@ -270,7 +272,7 @@ static bool packed_uses_f32_planes(const void* W_T, const void* Y, int64_t N, in
 
 extern "C" size_t bt_packed_forward_workspace_bytes(int64_t B, int64_t N, int64_t K, int x_dtype) {
     if (B <= 0 || N <= 0 || K <= 0) return 0;
-    if (x_dtype == BT_F32) return f32_planes_bytes(B, K);
+    if (x_dtype == BT_F32) return !prefers_stream_f32(B, N, K) && gemm_f32_shape_ok(N, K) ? 0 : f32_planes_bytes(B, K);
     return stream_workspace_bytes(x_dtype == BT_F16 ? MODE_F16 : MODE_BF16, B, N, ceil_div(K, 4));
 }
 
@@ -326,15 +328,14 @@ static int packed_forward_impl(const char* who, const void* X, int x_dtype, cons
             return launch_stream(mode, X, 2, nullptr, W_T, w_layout, epi, Y, x_dtype, nullptr, B, N, K, 1,
                                  Q_ROW_MAJOR, 0, nullptr, 0.0f, epi_op, st);
         }
+        if (!prefers_stream_f32(B, N, K) && epi_op == 0 && gemm_f32_supported(N, K, X, Y))
+            return launch_gemm_f32(X, W_T, w_layout, epi, Y, B, N, K, st);
         if (!workspace || workspace_bytes < f32_planes_bytes(B, K) || ((uintptr_t)workspace) % 256 != 0) {
             set_error("%s: fp32 activations on tiled weights need a workspace of %zu bytes (256-byte aligned)", who,
                       f32_planes_bytes(B, K));
             return BT_ERR_INVALID;
         }
-        const int64_t Kp = plane_len(K);
-        if (!prefers_stream_f32(B, N, K) && epi_op == 0 && gemm_f32_supported(N, K, X, Y))
-            return launch_gemm_f32(X, W_T, w_layout, epi, Y, B, N, K, st);
-        rc = launch_split_f32_planes(X, B, K, Kp, workspace, st);
+        rc = launch_split_f32_planes(X, B, K, plane_len(K), workspace, st);
         if (rc) return rc;
         return launch_stream(MODE_BF16, workspace, 2, nullptr, W_T, w_layout, epi, Y, BT_F32, nullptr, B, N, K, 3,
                              Q_ROW_MAJOR, 0, nullptr, 0.0f, epi_op, st);
@@ -348,15 +349,15 @@ static int packed_forward_impl(const char* who, const void* X, int x_dtype, cons
             return launch_gemm_f16(mode, X, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, B, N, K, st);
         return launch_stream(mode, X, 2, nullptr, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, x_dtype, nullptr, B, N, K, 1, Q_ROW_MAJOR, 0, nullptr, 0.0f, 0, st);
     }
-    if (x_dtype == BT_F32 && packed_uses_f32_planes(W_T, Y, N, K) && workspace &&
-        workspace_bytes >= f32_planes_bytes(B, K) && ((uintptr_t)workspace) % 256 == 0) {
-        // (without a workspace the call still succeeds, on the generic kernel)
-        const int64_t Kp = plane_len(K);
+    if (x_dtype == BT_F32 && packed_uses_f32_planes(W_T, Y, N, K)) {
         if (!prefers_stream_f32(B, N, K) && gemm_f32_supported(N, K, X, Y))
             return launch_gemm_f32(X, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, B, N, K, st);
-        rc = launch_split_f32_planes(X, B, K, Kp, workspace, st);
-        if (rc) return rc;
-        return launch_stream(MODE_BF16, workspace, 2, nullptr, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, BT_F32, nullptr, B, N, K, 3, Q_ROW_MAJOR, 0, nullptr, 0.0f, 0, st);
+        // (without a workspace the call still succeeds, on the generic kernel)
+        if (workspace && workspace_bytes >= f32_planes_bytes(B, K) && ((uintptr_t)workspace) % 256 == 0) {
+            rc = launch_split_f32_planes(X, B, K, plane_len(K), workspace, st);
+            if (rc) return rc;
+            return launch_stream(MODE_BF16, workspace, 2, nullptr, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, BT_F32, nullptr, B, N, K, 3, Q_ROW_MAJOR, 0, nullptr, 0.0f, 0, st);
+        }
     }
     return launch_packed_generic(X, x_dtype, W_T, epi, Y, B, N, K, st);
 }
@@ -745,8 +746,10 @@ extern "C" int bt_rmsnorm_rowsum(const void* X, int64_t ld_x, const void* weight
 // ---- packed forward with an activation prologue -----------------------------------------------
 extern "C" size_t bt_packed_forward_fused_workspace_bytes(int64_t B, int64_t N, int64_t K, int x_dtype) {
     if (B <= 0 || N <= 0 || K <= 0 || !valid_dtype(x_dtype)) return 0;
-    // [the prologue's output, B x K in x_dtype, when it runs as its own kernel][the forward's own scratch]
-    return align256((size_t)B * K * dtype_size(x_dtype)) + bt_packed_forward_workspace_bytes(B, N, K, x_dtype);
+    // [the prologue's output, B x K in x_dtype, when it runs as its own kernel][the forward's own scratch: with the SwiGLU
+    // output stage fp32 rows take the planes at any size]
+    return align256((size_t)B * K * dtype_size(x_dtype)) +
+           (x_dtype == BT_F32 ? f32_planes_bytes(B, K) : bt_packed_forward_workspace_bytes(B, N, K, x_dtype));
 }
 
 static int fused_forward_impl(const char* who, const void* X, int64_t ld_x, int x_dtype, int pro_op, const void* pro_b,

@@ -408,10 +408,13 @@ static int launch_gemm_f32_src(const GemmF32Params& p, const char* who, hipStrea
     }
 }
 
-// X 4-byte, Y (and the residual) 16-byte aligned; the kernel's 32-bit offsets span 64 rows of X and the whole of W
+// the kernel's 32-bit offsets span 64 rows of X and the whole of W
+bool gemm_f32_shape_ok(int64_t N, int64_t K) {
+    return N % 4 == 0 && K < (1ll << 23) && N < (1ll << 30) && ceil_div(K, 4) * N < (1ll << 32);
+}
+// X 4-byte, Y (and the residual) 16-byte aligned
 bool gemm_f32_supported(int64_t N, int64_t K, const void* X, const void* Y) {
-    return N % 4 == 0 && ((uintptr_t)X) % 4 == 0 && ((uintptr_t)Y) % 16 == 0 && K < (1ll << 23) && N < (1ll << 30) &&
-           ceil_div(K, 4) * N < (1ll << 32);
+    return gemm_f32_shape_ok(N, K) && ((uintptr_t)X) % 4 == 0 && ((uintptr_t)Y) % 16 == 0;
 }
 
 int launch_gemm_f32(const void* X, const uint8_t* W, int w_layout, const Epilogue& epi, void* Y, int64_t M, int64_t N,

@@ -47,9 +47,11 @@ typedef enum {
  * from one call to the next; two calls that may run concurrently (different
  * streams) need different workspaces.  Workspaces must be 256-byte aligned.
  * At present bt_ternary_linear_tensor_core_forward uses one (the int8 activations
- * and their row scales) and bt_ternary_linear_packed_forward uses one for fp32
- * activations (three bf16 planes); bt_ternary_gemm_i8 keeps the argument so that a
- * kernel that needs scratch can be introduced without an ABI change.
+ * and their row scales), bt_ternary_linear_packed_forward uses one for small
+ * batches of fp32 activations (three bf16 planes), its fused and tiled forms also
+ * one for a prologue that runs as its own kernel, and bt_linear_grad_weight one for
+ * partial sums; bt_ternary_gemm_i8 keeps the argument so that a kernel that needs
+ * scratch can be introduced without an ABI change.
  */
 /* ABI version of the loaded library (BT_ABI_VERSION at build time). */
 int bt_abi_version(void);
@@ -109,13 +111,14 @@ int bt_ternary_linear_forward(const void* X, int x_dtype, const int8_t* W_tern, 
  *   matrix-core GEMM beyond (crossover near 1.5-2 M outputs for K = 2560..4096;
  *   the option STREAM_MAX_ROWS = n replaces the rule by "B <= n").  A single fp16 row (K % 16 == 0,
  *   K <= 16384, N % 4 == 0) runs the exact GEMV on the int8 matrix cores: the dot products are summed
- *   without rounding and rounded to fp32 once.  fp32 activations (any K) are first split into
- *   three bf16 planes (x = hi + mid + lo exactly), each zero-padded to a multiple of 64 values, in
- *   the workspace and run on the same bf16 kernels with exact products and fp32 accumulation.
- *   Unaligned operands, a missing workspace and BITTORCH_KERNEL=generic run a generic
- *   kernel that accumulates in the reference's k order.
- *   workspace: at least bt_packed_forward_workspace_bytes(B,N,K,x_dtype) bytes
- *   (6*B*Kp rounded up to 256 for fp32, Kp = K rounded up to 64; 0 otherwise: may be NULL).
+ *   without rounding and rounded to fp32 once.  fp32 activations (any K) are split into three bf16
+ *   terms (x = hi + mid + lo exactly) that the bf16 matrix cores multiply, products exact, sums in
+ *   fp32: in registers by a GEMM of its own, or, for the streaming kernel (up to 32 rows, and small
+ *   products beyond), into planes in the workspace, each zero-padded to a multiple of 64 values.
+ *   Unaligned operands, a workspace missing where the planes need one and BITTORCH_KERNEL=generic run
+ *   a generic kernel that accumulates in the reference's k order.
+ *   workspace: at least bt_packed_forward_workspace_bytes(B,N,K,x_dtype) bytes (6*B*Kp rounded up to
+ *   256, Kp = K rounded up to 64, for fp32 on the streaming kernel; 0 otherwise: may be NULL).
  */
 size_t bt_packed_forward_workspace_bytes(int64_t B, int64_t N, int64_t K, int x_dtype);
 int bt_ternary_linear_packed_forward(const void* X, int x_dtype, const uint8_t* W_T,
@@ -253,7 +256,8 @@ int bt_ternary_linear_packed_forward_fused(const void* X, int64_t ld_x, int x_dt
  *     N/32 + P, so that one workgroup holds column h of both halves.
  *   bt_ternary_linear_tiled_forward: bt_ternary_linear_packed_forward_fused on the tiled copy, with
  *     pro_op = BT_PRO_NONE allowed (then ld_x must equal K); the weights are streamed once per 16
- *     rows of X, so it is meant for decode shapes; fp32 X needs the workspace.
+ *     rows of X, so it is meant for decode shapes.  workspace: without a prologue and with epi_op
+ *     BT_EPI_NONE or BT_EPI_NATURAL_FROM_PAIRS, bt_packed_forward_workspace_bytes(...) bytes do.
  *     Results equal those of the row-major entry points bit for bit wherever both layouts take the same kernel
  *     (always up to 32 rows); a larger batch near the crossover between the streaming kernel and the tiled GEMM
  *     may be routed differently on the tiled copy (its remainder tiles are cheaper), and the two kernels add the

@@ -11,6 +11,7 @@ import pytest
 import torch
 
 from conftest import announce
+from _util import set_option
 
 gpu = pytest.mark.gpu
 EPS = 2.0 ** -24
@@ -59,7 +60,8 @@ def test_fp32_products_against_float64(m, n, k):
     _close(dw, dy.t(), x, _six_terms(m), scale.double()[:, None])
     _close(db[:, None], dy.t(), torch.ones(m, 1, device="cuda"), m)
     assert torch.equal(_C.linear_grad_weight(dy, x, scale, True)[0], dw)  # a fixed order of the sums
-    if m > 32 and n % 4 == 0:
+    set_option("STREAM_MAX_ROWS", "1")  # (the kernel that splits in registers at any number of rows)
+    if m > 1 and n % 4 == 0:
         y = _C.ternary_linear_packed_forward(x, packed, scale, None, k)
         _close(y, x, tern.t(), _three_terms(k), scale.double()[None, :])
         _close(_C.ternary_linear_tiled_forward(x, _C.retile_weights(packed, k), scale, None, k, n), x, tern.t(),
@@ -223,3 +225,34 @@ def test_input_gradient_of_few_outputs(n):
     _close(got, gy, tern.float() * scale[:, None], _three_terms(n))
     if n < 8:
         assert torch.equal(got, gy @ _C.unpack_dequant(packed, 260, scale, torch.float32))
+
+
+@gpu
+@pytest.mark.parametrize("m,n,k", [(16384, 64, 100), (600, 1028, 260)])
+def test_fp32_forward_without_a_workspace(m, n, k):
+    """Through the C ABI with the scratch its query asks for, none: both weight layouts, on the kernel that splits in registers;
+    the SwiGLU output stage and the prologues still have what they need."""
+    from bittorch_amd import _C, _lib
+    announce("fp32 forward, no workspace", m, n, k)
+    lib = _lib.load()
+    set_option("STREAM_MAX_ROWS", "1")
+    x, _, packed, scale, tern = _case(m, n, k)
+    assert lib.bt_packed_forward_workspace_bytes(m, n, k, 0) == 0
+    tiled, stream = _C.retile_weights(packed, k), torch.cuda.current_stream().cuda_stream
+    rows, tiles = (torch.full((m, n), float("nan"), device="cuda") for _ in range(2))
+    assert lib.bt_ternary_linear_packed_forward(x.data_ptr(), 0, packed.data_ptr(), scale.data_ptr(), 0, n, None, 0,
+                                                rows.data_ptr(), m, n, k, None, 0, stream) == 0
+    assert lib.bt_ternary_linear_tiled_forward(x.data_ptr(), k, 0, 0, None, 0, 0.0, tiled.data_ptr(), scale.data_ptr(), 0, n, None, 0,
+                                               None, 0, tiles.data_ptr(), m, n, k, None, 0, stream) == 0
+    for y in (rows, tiles):
+        _close(y, x, tern.t(), _three_terms(k), scale.double()[None, :])
+    assert torch.equal(rows, _C.ternary_linear_packed_forward(x, packed, scale, None, k))
+    if n % 32 == 0:
+        gu = _C.ternary_linear_packed_forward(x, packed, scale, None, k)
+        pairs = _C.retile_weights(packed, k, True)
+        h = _C.ternary_linear_tiled_forward(x, pairs, scale, None, k, n, swiglu_pairs=True)
+        want = torch.nn.functional.silu(gu[:, :n // 2]) * gu[:, n // 2:]
+        assert torch.allclose(h, want, rtol=1e-4, atol=1e-5)
+    norm = _C.ternary_linear_tiled_forward(x, tiled, scale, None, k, n, norm=(None, 1e-5))
+    xn = torch.nn.functional.rms_norm(x, (k,), None, 1e-5)
+    assert torch.allclose(norm, (xn.double() @ (tern.double() * scale.double()[:, None]).t()).float(), rtol=1e-4, atol=1e-5)
