@@ -36,7 +36,7 @@ static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 enum Option {
     OPT_STREAM_MAX_ROWS,     // n: batches of up to n rows take the streaming kernel, larger ones the tiled GEMM
     OPT_GEMM_LONG_EPILOGUE,  // 1: the tiled int8 GEMM never takes its short epilogue
-    OPT_GEMM_TAIL_SPLIT,     // 0: the remainder of a tiled GEMM launch is not cut into finer tiles
+    OPT_GEMM_TAIL_SPLIT,     // 0: the tiled 16-bit and int8 GEMMs take tiles of 128 rows throughout
     OPT_GROUP_WALK,          // grouped GEMV: 1 / chunk / 0 force a kernel
     OPT_GROUP_NACC,          // grouped GEMV: 16-column blocks per wave of the slab kernel
     OPT_GROUP_UNITS,         // grouped GEMV: 1 forces the one-matrix kernel over (unit, tile) workgroups, 0 forbids it

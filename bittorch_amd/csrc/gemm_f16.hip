@@ -390,13 +390,15 @@ bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, co
 static int gemm_f16_plan(int64_t M, int64_t N, int64_t K, double* us) {
     const int64_t C = gemm_compute_units(), tn = ceil_div(N, F_BN);
     const int64_t t4 = ceil_div(M, 128) * tn, t2 = ceil_div(M, 64) * tn, t1 = ceil_div(M, 32) * tn;
-    if (t1 <= C) { *us = 4.0 + 0.0062 * (double)K; return 1; }
-    if (t2 <= C) { *us = 5.0 + 0.007 * (double)K; return 2; }
+    const bool whole = gemm_whole_tiles();
+    if (t1 <= C && !whole) { *us = 4.0 + 0.0062 * (double)K; return 1; }
+    if (t2 <= C && !whole) { *us = 5.0 + 0.007 * (double)K; return 2; }
     const int parts = gemm_dma_parts(t4);
     const double n4 = parts == 1 ? (double)ceil_div(t4, C) : (double)(2 * (t4 / (2 * C))) + (parts == 2 ? 1.2 : 0.6);
     const double p4 = n4 * (2.0 + 0.0113 * (double)K), p2 = (double)ceil_div(t2, C) * (1.3 + 0.0062 * (double)K);
-    *us = 4.0 + (p2 < p4 ? p2 : p4);
-    return p2 < p4 ? 2 : 4;
+    const bool half = p2 < p4 && !whole;
+    *us = 4.0 + (half ? p2 : p4);
+    return half ? 2 : 4;
 }
 double gemm_f16_cost(int64_t M, int64_t N, int64_t K) {
     double us;

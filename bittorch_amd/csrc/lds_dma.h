@@ -27,12 +27,18 @@ static inline int w_source(bool tiled, bool fields, const void* W, int64_t N) {
     return N % 16 == 0 && ((uintptr_t)W) % 16 == 0 ? W_ROWS16 : W_ROWS;
 }
 
+// Option GEMM_TAIL_SPLIT = 0 (tests, A/B runs): every tile of every launch has 128 rows.
+static inline bool gemm_whole_tiles() {
+    const char* env = option(OPT_GEMM_TAIL_SPLIT);
+    return env && env[0] == '0';
+}
 // Into how many finer ones the last, incomplete round of an XCD's 128-row tiles is cut (two workgroups per compute unit).
 // Two workgroups that end together free their compute unit for the next two, so a remainder of whole tiles runs in pairs on a
 // part of the chip.  Measured (int8, row-major weights, us, whole / halves / quarters; remainder of 64): 2048 x 11008 x 4096
 // (22) 104 / 97 / 111; 2900 x 6400 x 6400 (8) 136 / 120 / 122, tiled 120 / 112 / 106; 4096 x 4100 x 4096 (4) 98 / 88 / 86;
 // 2304 x 4096 x 4096 (36) 56 / 63 / 80.
 static inline int gemm_dma_parts(int64_t tiles) {
+    if (gemm_whole_tiles()) return 1;
     const int64_t slots = 2 * gemm_compute_units() / 8, rem = ceil_div(tiles, 8) % slots;
     return rem == 0 || 2 * rem > slots ? 1 : 5 * rem > slots ? 2 : 4;
 }

@@ -1,6 +1,7 @@
 """GPU: the tiled 16-bit GEMM (``csrc/gemm_f16.hip``) against float64 at the edges of its tiles and stages.
 
-Rows 128 / 64 / 32 a tile and 256 columns, the last round of a launch in finer tiles; stages of 64 k with a remainder of any
+Rows 128 / 64 / 32 a tile and 256 columns, the last round of a launch in halves or quarters of tiles (bit for bit the sums of
+tiles of 128 rows); stages of 64 k with a remainder of any
 multiple of 8, fewer stages than are in flight; row-major weights with N a multiple of 16 and of 4 only, and the tiled copy.
 The products are exact and summed in fp32: the error before the output's rounding is at most (K + 8) 2^-24 of the sum of the
 products' magnitudes, the scale and the output round once each.
@@ -14,7 +15,7 @@ from _util import random_ternary, set_option
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(33, 260, 64), (40, 1000, 8), (70, 1028, 200), (129, 4096, 336), (999, 2564, 1032), (2000, 1296, 120),
-          (1025, 16388, 72), (4111, 4356, 264), (8200, 2304, 328)]
+          (1025, 16388, 72), (4111, 4356, 264), (8200, 2304, 328), (4100, 5380, 136)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -35,9 +36,12 @@ def test_tiled_float_gemm_against_float64(m, n, k, dtype):
     mags = (x.double().abs() @ w.t().abs()) * scale.double()
     unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
     for r in (None, res):
+        set_option("GEMM_TAIL_SPLIT", None)
         y = _C.ternary_linear_packed_forward(x, wt, scale, None, k, residual=r)
         yt = _C.ternary_linear_tiled_forward(x, tiled, scale, None, k, n, residual=r)
         assert torch.equal(y, yt)
+        set_option("GEMM_TAIL_SPLIT", "0")
+        assert torch.equal(_C.ternary_linear_packed_forward(x, wt, scale, None, k, residual=r), y)
         want = ref if r is None else ref + r.double()
         bound = (k + 8) * 2.0 ** -24 * mags + unit * (want.abs() + (0 if r is None else ref.abs())) + 2e-7
         assert bool(((y.double() - want).abs() <= bound).all())

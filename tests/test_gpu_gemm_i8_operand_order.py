@@ -1,7 +1,7 @@
 """GPU: the tiled int8 GEMM on operand-order activations (``csrc/gemm_i8_dma.hip``), bit for bit against the kernel that reads
 row-major activations and against exact integer sums, at the edges of its tiles and stages.
 
-Rows 128 / 64 / 32 a tile and 256 columns; stages of 64 k (a remainder of 16, 32 or 48 in the last one), fewer stages than the
+Rows 128 / 64 / 32 a tile and 256 columns, the last round of a launch in halves or quarters of tiles or whole; stages of 64 k (a remainder of 16, 32 or 48 in the last one), fewer stages than the
 five in flight; a last row block that is partly or wholly past M; row-major, tiled and field-layout weights.
 """
 import pytest
@@ -13,7 +13,7 @@ from _util import random_ternary, set_option
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(33, 260, 64), (40, 1000, 48), (70, 1028, 208), (129, 4096, 336), (999, 2564, 1040), (2000, 1300, 112),
-          (1025, 16388, 192), (4111, 4356, 320), (8200, 2304, 704)]
+          (1025, 16388, 192), (4111, 4356, 320), (8200, 2304, 704), (4100, 5380, 256), (4111, 4356, 384)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
@@ -32,7 +32,8 @@ def test_operand_order_equals_row_major_activations(m, n, k, dtype):
     bias = torch.randn(n, generator=g, device="cuda").to(dtype)
     res = torch.randn(m, n, generator=g, device="cuda").to(dtype)
     q, s = _C.act_quant_int8(x, False)
-    qo, so = _C.act_quant_int8(x, True)
+    qo, so, rowsum = _C.act_quant_int8(x, True, return_rowsum=True)
+    fields = _C.retile_fields(tiled, k, n) if k % 128 == 0 else None
     s[m // 3] = so[m // 3] = 2.0 ** -125  # below the range of the two-operation division
     exact = (127 * (q.double() @ w.double().t())).int()
     for residual in (None, res):
@@ -42,3 +43,10 @@ def test_operand_order_equals_row_major_activations(m, n, k, dtype):
         yt, at = _C.ternary_gemm_int8_tiled(qo, so, tiled, scale, bias, k, n, q_operand_order=True, **kw)
         assert torch.equal(acc, exact) and torch.equal(ar, exact) and torch.equal(at, exact)
         assert torch.equal(yr, y) and torch.equal(yt, y)
+        if fields is not None:
+            yf, af = _C.ternary_gemm_int8_fields(qo, so, rowsum, fields, scale, bias, k, n, q_operand_order=True, **kw)
+            assert torch.equal(af, exact) and torch.equal(yf, y)
+        set_option("GEMM_TAIL_SPLIT", "0")
+        yw, aw = _C.ternary_gemm_int8(qo, so, wt, scale, bias, k, q_operand_order=True, **kw)
+        set_option("GEMM_TAIL_SPLIT", None)
+        assert torch.equal(aw, exact) and torch.equal(yw, y)

@@ -275,9 +275,10 @@ def test_field_layout_gemm_argument_errors(oracle):
         _C.ternary_gemm_int8_fields(q, sx, rs.float(), fields, torch.ones(64, device="cuda"), None, 192, 64)
 
 
-# (M, N, K) whose 128 x 256 tiles leave most of a 256-unit chip idle in their last round, so that the launch cuts
-# the remainder finer: 320 tiles (256 whole + 64 as 256 tiles of 32 rows), 128 tiles (as 256 of 64 rows), 64 tiles (as
-# 256 of 32 rows); the same with ragged last row tiles, ragged columns and several stages of K
+# (M, N, K) whose 128 x 256 tiles leave most of a 256-unit chip idle in their last round, so that a launch cuts the
+# remainder finer (int8, row-major activations: 320 tiles = 256 whole + 64 as 256 tiles of 32 rows) or takes tiles of 64 or
+# 32 rows throughout (128 tiles as 256 of 64 rows, 64 as 256 of 32); the same with ragged last row tiles, ragged columns and
+# several stages of K
 REMAINDER_SHAPES = [(4096, 2560, 256), (1024, 4096, 128), (512, 4096, 384), (1000, 4096, 256), (500, 4096, 128),
                     (512, 4000, 128), (4090, 2560, 128)]
 
@@ -285,8 +286,8 @@ REMAINDER_SHAPES = [(4096, 2560, 256), (1024, 4096, 128), (512, 4096, 384), (100
 # ... and config 5's two projections of 1.25 rounds at their full size
 @pytest.mark.parametrize("m,n,k", REMAINDER_SHAPES + [(4096, 2560, 2560), (4096, 2560, 6912)])
 def test_tiled_int8_remainder_in_finer_tiles(oracle, m, n, k, monkeypatch):
-    """The prefill GEMM computes the column tiles of a mostly empty last round in tiles of 64 or 32 rows
-    (a second launch behind the whole tiles).  Same bits as one launch of whole tiles -- outputs and int32
+    """The prefill GEMM computes the column tiles of a mostly empty last round in tiles of 64 or 32 rows (a second launch
+    behind the whole tiles) or the whole matrix in such tiles.  Same bits as one launch of tiles of 128 rows -- outputs and int32
     accumulators, both activation layouts, bias, residual, 16-bit and fp32 outputs -- and equal to the oracle on
     row slices at the start, across tile borders and at the ragged end."""
     from bittorch_amd import _C
@@ -323,8 +324,8 @@ def test_tiled_int8_remainder_in_finer_tiles(oracle, m, n, k, monkeypatch):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("m,n,k", REMAINDER_SHAPES)
 def test_tiled_forward_remainder_in_finer_tiles(oracle, dtype, m, n, k, monkeypatch):
-    """The same for the 16-bit matrix-core GEMM (fp32 rows: three bf16 planes): finer tiles for the remainder give the
-    bits of one launch of whole tiles, with bias and with a residual, and agree with the oracle's float64-free
+    """The same for the 16-bit matrix-core GEMM: tiles of 64 and 32 rows give the bits of tiles of 128, with bias and with a
+    residual, and agree (fp32 rows, whose GEMM has one size of tile for a shape, the same whatever the option says) with the oracle's float64-free
     restatement of the reference's loop within the rounding of 16-bit products summed in fp32."""
     from bittorch_amd import _C
     set_option("STREAM_MAX_ROWS", "32")
