@@ -351,9 +351,11 @@ def test_tiled_forward_remainder_in_finer_tiles(oracle, dtype, m, n, k, monkeypa
         assert rel_err(y[r0:r1], ref) <= (1e-3 if dtype == torch.float32 else 1e-2)  # output rounding of the 16-bit dtypes
 
 
-def test_remainder_tiles_replay_in_a_graph(oracle, monkeypatch):
-    """The two launches of a call with finer remainder tiles are captured like any other: every replay of the graph,
-    with eager work and synchronizations between the replays, gives the eager result."""
+@pytest.mark.parametrize("oo", [False, True])
+def test_remainder_tiles_replay_in_a_graph(oracle, oo):
+    """A call with finer tiles (row-major activations: two launches, the remainder's behind the whole tiles'; operand order:
+    one) is captured like any other: every replay of the graph, with eager work and synchronizations between the replays,
+    gives the eager result."""
     from bittorch_amd import _C
     set_option("STREAM_MAX_ROWS", "32")
     m, n, k = 4096, 2560, 256
@@ -362,23 +364,23 @@ def test_remainder_tiles_replay_in_a_graph(oracle, monkeypatch):
     scale = (torch.rand(n) * 0.05 + 0.01).cuda()
     xs = [seeded_acts(m, k, seed=s_, dtype=torch.bfloat16, outliers=True).cuda() for s_ in (1, 2, 3)]
     x = xs[0].clone()
-    q, s = _C.act_quant_int8(x, True)
+    q, s = _C.act_quant_int8(x, oo)
     eager = []
     for xi in xs:
-        qi, si = _C.act_quant_int8(xi, True)
-        eager.append(_C.ternary_gemm_int8_tiled(qi, si, tiled, scale, None, k, n, torch.bfloat16, False, None, True))
+        qi, si = _C.act_quant_int8(xi, oo)
+        eager.append(_C.ternary_gemm_int8_tiled(qi, si, tiled, scale, None, k, n, torch.bfloat16, False, None, oo))
     torch.cuda.synchronize()
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
-        _C.ternary_gemm_int8_tiled(q, s, tiled, scale, None, k, n, torch.bfloat16, False, None, True)
+        _C.ternary_gemm_int8_tiled(q, s, tiled, scale, None, k, n, torch.bfloat16, False, None, oo)
     torch.cuda.current_stream().wait_stream(side)
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        y = _C.ternary_gemm_int8_tiled(q, s, tiled, scale, None, k, n, torch.bfloat16, False, None, True)
+        y = _C.ternary_gemm_int8_tiled(q, s, tiled, scale, None, k, n, torch.bfloat16, False, None, oo)
     for xi, want in zip(xs, eager):
-        qi, si = _C.act_quant_int8(xi, True)  # eager work between the replays
+        qi, si = _C.act_quant_int8(xi, oo)  # eager work between the replays
         q.copy_(qi)
         s.copy_(si)
         graph.replay()
