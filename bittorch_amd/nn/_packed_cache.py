@@ -9,8 +9,8 @@ its storage address, dtype and device, and the quantizer's two settings.  Such a
 reads K*N/4 bytes of packed weights instead of 4*K*N bytes of masters -- and reads them from a decode-tiled copy
 built next to the packed bytes (``_C.retile_weights``; whole-cache-line loads: what ``TernaryLinearInference`` runs
 on), which such a module then holds as well, another K*N/4 bytes.  Up to 32 rows the output is the training forward's
-bit for bit; a larger batch may be routed to another kernel on the tiled copy than on the row-major bytes, and the two
-sum in fp32 in different orders (a difference in the last bits of the sums).
+bit for bit; a larger batch on the streaming kernel may split K differently on the tiled copy and on the row-major bytes,
+and then sums in fp32 in another order (a difference in the last bits of the sums).
 
 A training forward (gradient mode on and ``weight.requires_grad``) never uses the cache and
 quantizes every time, exactly as the reference does: training code is where weights get written

@@ -108,7 +108,7 @@ int bt_ternary_linear_forward(const void* X, int x_dtype, const int8_t* W_tern, 
  *   X [B,K] x_dtype; W_T [ceil(K/4),N] uint8; Y [B,N] x_dtype.
  *   A cost model fitted to measurements picks the kernel: the streaming kernel (weights read once
  *   per 16 rows, all 16-row blocks of the call in one launch) while B*N*K is small, the tiled 16-bit
- *   matrix-core GEMM beyond (crossover near 1.5-2 M outputs for K = 2560..4096;
+ *   matrix-core GEMM beyond (crossover near 1 M outputs for K = 2560..4096;
  *   the option STREAM_MAX_ROWS = n replaces the rule by "B <= n").  A single fp16 row (K % 16 == 0,
  *   K <= 16384, N % 4 == 0) runs the exact GEMV on the int8 matrix cores: the dot products are summed
  *   without rounding and rounded to fp32 once.  fp32 activations (any K) are split into three bf16
@@ -258,10 +258,9 @@ int bt_ternary_linear_packed_forward_fused(const void* X, int64_t ld_x, int x_dt
  *     pro_op = BT_PRO_NONE allowed (then ld_x must equal K); the weights are streamed once per 16
  *     rows of X, so it is meant for decode shapes.  workspace: without a prologue and with epi_op
  *     BT_EPI_NONE or BT_EPI_NATURAL_FROM_PAIRS, bt_packed_forward_workspace_bytes(...) bytes do.
- *     Results equal those of the row-major entry points bit for bit wherever both layouts take the same kernel
- *     (always up to 32 rows); a larger batch near the crossover between the streaming kernel and the tiled GEMM
- *     may be routed differently on the tiled copy (its remainder tiles are cheaper), and the two kernels add the
- *     fp32 partial sums in different orders.
+ *     Results equal those of the row-major entry points bit for bit up to 32 rows and in the tiled GEMMs; a larger
+ *     batch on the streaming kernel may split K among its waves differently on the two layouts, and then adds the
+ *     fp32 partial sums in another order.
  *     epi_op = BT_EPI_SWIGLU_PAIRS (pair-ordered copy, no residual, no SwiGLU prologue): Y is [B, N/2],
  *     Y[b, h] = what bt_swiglu makes of the stored projections, rd(rd(silu(g)) * u) with g = rd(linear
  *     column h), u = rd(linear column N/2 + h): the SwiGLU MLP's hidden vector leaves the gate|up kernel
@@ -271,9 +270,9 @@ int bt_ternary_linear_packed_forward_fused(const void* X, int64_t ld_x, int x_dt
  *     to the same call on a natural-order copy.  With the two, one pair-ordered copy serves every call of a fused
  *     [gate | up] layer in 16-bit and fp32 activations (the int8 entry point reads natural-order copies only).
  *   bt_ternary_gemm_i8_tiled: bt_ternary_gemm_i8_res on the tiled copy (same remark).
- *   A tall batch on the tiled copy may take two kernel launches on the stream instead of one (the column tiles of
- *   a mostly empty last round of 128 x 256 tiles run as tiles of 64 or 32 rows behind the whole tiles): same
- *   results, nothing for the caller to do; both launches are captured by a HIP graph like any other.
+ *   A tall int8 batch on the tiled copy may take two kernel launches on the stream instead of one (row-major
+ *   activations: the column tiles of a mostly empty last round of 128 x 256 tiles run as tiles of 64 or 32 rows
+ *   behind the whole tiles): same results, nothing for the caller to do; both are captured by a HIP graph like any other.
  */
 enum { BT_TILES_NATURAL = 0, BT_TILES_GATE_UP_PAIRS = 1 };
 enum { BT_EPI_NONE = 0, BT_EPI_SWIGLU_PAIRS = 1, BT_EPI_NATURAL_FROM_PAIRS = 2 };
