@@ -29,6 +29,9 @@ from torch import Tensor
 _MAX_K = 16384     # the grouped kernel keeps a row's digit planes in LDS
 _PLANS: "OrderedDict[tuple, _Plan]" = OrderedDict()
 _MAX_PLANS = 16
+# Tables that captured graphs read (a few kilobytes each): a graph's launches hold their addresses alone, and how long it lives
+# is not known here.  One entry for each set of layers and buffers that has been captured.
+_CAPTURED: dict = {}
 
 
 class _Plan:
@@ -45,6 +48,10 @@ class _Plan:
         self.w_tab = _C.pointer_table(self.tiled)
         self.s_tab = _C.pointer_table(self.scales)
         self.b_tab = None if self.biases is None else _C.pointer_table(self.biases)
+        self.own = [t for t in (self.w_tab, self.s_tab, self.b_tab) if t is not None]
+        self.own += [v for v, L in zip(self.scales, layers) if v is not L.scale]
+        self.own += [v for v, L in zip(self.biases or (), layers) if v is not L.bias]
+        self.streams = {torch.cuda.current_stream(self.w_tab.device).cuda_stream}
         self.io_tabs: "OrderedDict[tuple, tuple]" = OrderedDict()
         self.i8_tabs: "OrderedDict[tuple, tuple]" = OrderedDict()
 
@@ -57,20 +64,39 @@ class _Plan:
         """Tables of the G units' addresses inside q [G, M, K], s_x [G, M] and y [G, M, N]."""
         return self._tables(self.i8_tabs, q.shape[0], q.device, tuple((t.data_ptr(), _unit_bytes(t)) for t in (q, s_x, y)))
 
-    @staticmethod
-    def _tables(held, g: int, device, key):
+    def _tables(self, held, g: int, device, key):
         """One table of G addresses for each (first address, bytes from one unit to the next) of ``key``; kept by the whole
         key (the same buffers may hold units of another size on the next call), so a decode loop whose buffers repeat (and
         a captured graph, whose buffers are fixed) builds them once."""
-        hit = held.get(key)
-        if hit is not None:
-            held.move_to_end(key)
-            return hit
-        tabs = tuple(torch.tensor([base + u * step for u in range(g)], dtype=torch.int64, device=device) for base, step in key)
-        held[key] = tabs
-        if len(held) > 8:
-            held.popitem(last=False)
-        return tabs
+        entry = held.get(key)
+        if entry is None:
+            tabs = tuple(torch.tensor([base + u * step for u in range(g)], dtype=torch.int64, device=device) for base, step in key)
+            entry = held[key] = (tabs, set())
+            if len(held) > 8:
+                held.popitem(last=False)
+        else:
+            try:
+                held.move_to_end(key)
+            except KeyError:  # (another host thread has just dropped it)
+                pass
+        if device.type == "cuda":
+            stream = torch.cuda.current_stream(device)
+            self._read_on(stream, entry[0], entry[1])
+            self._read_on(stream, self.own, self.streams)
+            if torch.cuda.is_current_stream_capturing():
+                self._keep_for_graph(key, entry[0])
+        return entry[0]
+
+    @staticmethod
+    def _read_on(stream, tables, streams) -> None:
+        """Once for each stream: memory that this object drops is handed out again behind what that stream reads of it."""
+        if stream.cuda_stream not in streams:
+            streams.add(stream.cuda_stream)
+            for t in tables:
+                t.record_stream(stream)
+
+    def _keep_for_graph(self, key, tabs) -> None:
+        _CAPTURED[(self.w_tab.data_ptr(), key)] = (tabs, self.own)
 
 
 def _unit_bytes(t: Tensor) -> int:

@@ -122,3 +122,62 @@ def test_packed_weights_written_in_place_or_replaced(int8):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.allclose(got.float(), want.float(), rtol=2e-3, atol=1e-4)  # (fp16 of fp32 sums in another order)
+
+
+@pytest.mark.parametrize("int8", [False, True])
+def test_a_graph_keeps_its_tables(int8):
+    """Calls on other buffers and other layers after a capture, more than a plan and the plans hold."""
+    from bittorch_amd import _C, ops
+    announce("grouped plans, graph", int8)
+    n, k, g = 64, 128, 5
+    layers = _layers(n, k, g)
+    layers[1].scale = torch.rand(2 * n, device="cuda")[::2]  # (a plan reads a contiguous copy of it)
+    rows = torch.randn(g * 3, k, device="cuda").half()
+    q, s = (t.view(g, 3, *t.shape[1:]) for t in _C.act_quant_int8(rows))
+    x, out = rows[:g].clone(), torch.empty((g, 3, n) if int8 else (g, n), device="cuda", dtype=torch.float16)
+    if int8:
+        call = lambda ls, y: ops.ternary_linear_int8_grouped(ls, q=q, s_x=s, out_dtype=torch.float16, out=y)
+    else:
+        call = lambda ls, y: ops.ternary_linear_grouped(ls, x, out=y)
+    want = call(layers, out).clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(layers, out)
+    others = [_layers(n, k, g) for _ in range(18)]
+    outs = [torch.empty_like(out) for _ in range(12)]
+    for y in outs:
+        assert torch.equal(call(layers, y), want)
+    for ls in others:
+        call(ls, outs[0])
+    fill = [torch.full((4096,), -1, dtype=torch.int64, device="cuda") for _ in range(64)]
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert torch.equal(call(layers, outs[1]), want)
+    del fill
+
+
+def test_calls_from_several_streams_and_threads():
+    """One set of layers, each host thread on a stream and buffers of its own, more buffers than a plan keeps tables for."""
+    import threading
+    from bittorch_amd import ops
+    announce("grouped plans, streams")
+    layers, bad = _layers(), []
+    x = torch.randn(5, 128, device="cuda").half()
+    want = ops.ternary_linear_grouped(layers, x)
+    torch.cuda.synchronize()
+
+    def loop(stream):
+        with torch.cuda.stream(stream):
+            for i in range(60):
+                outs = [torch.empty_like(want) for _ in range(3)]
+                bad.extend(1 for y in outs if not torch.equal(ops.ternary_linear_grouped(layers, x, out=y), want))
+
+    threads = [threading.Thread(target=loop, args=(torch.cuda.Stream(),)) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad

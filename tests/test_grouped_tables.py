@@ -38,6 +38,28 @@ def test_float_tables_of_other_strides_at_the_same_addresses():
     assert plan.io_tab(row, ys[0], True)[0].tolist() == [x.data_ptr()] * g
 
 
+def test_tables_of_a_captured_call_outlive_the_plan():
+    """A graph's launches hold the tables' addresses alone: other buffers' tables and other plans must not free them."""
+    import gc
+    import weakref
+    plan, g = _plan(), 3
+    grouped = pytest.importorskip("bittorch_amd.ops.grouped")
+    plan.w_tab = torch.zeros(g, dtype=torch.int64)
+    plan.own = [plan.w_tab, torch.zeros(g)]
+    buffers = torch.zeros(100, g, 8)
+    tabs = plan.io_tab(buffers[0], buffers[1], False)
+    plan._keep_for_graph(((buffers[0].data_ptr(), 32), (buffers[1].data_ptr(), 32)), tabs)
+    alive = [weakref.ref(t) for t in (*tabs, *plan.own)]
+    for i in range(2, 50):
+        plan.io_tab(buffers[i], buffers[i + 1], False)
+    del tabs, plan
+    gc.collect()
+    assert all(r() is not None for r in alive)
+    grouped._CAPTURED.clear()
+    gc.collect()
+    assert all(r() is None for r in alive)
+
+
 def test_fingerprint_of_a_layer_whose_scale_and_bias_are_parameters():
     grouped = pytest.importorskip("bittorch_amd.ops.grouped")
     from bittorch_amd import nn
