@@ -287,6 +287,24 @@ __device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel)
     return __builtin_amdgcn_perm(hi, lo, sel);
 }
 
+// vectors that start on any dword, half or byte
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x4_a1 __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+
+// v without its first `bytes` bytes (0 or more), zeros behind: a group loaded that far ahead of its place
+__device__ __forceinline__ uint4 shift_group(uint4 v, int bytes) {
+    const int d = bytes >> 2;
+    const bool one = d & 1, two = d & 2, none = d >= 4;
+    v.x = one ? v.y : v.x; v.y = one ? v.z : v.y; v.z = one ? v.w : v.z; v.w = one ? 0u : v.w;
+    v.x = two ? v.z : v.x; v.y = two ? v.w : v.y; v.z = two ? 0u : v.z; v.w = two ? 0u : v.w;
+    const uint32_t r = (uint32_t)bytes & 3u;
+    const uint4 o = make_uint4(__builtin_amdgcn_alignbyte(v.y, v.x, r), __builtin_amdgcn_alignbyte(v.z, v.y, r),
+                               __builtin_amdgcn_alignbyte(v.w, v.z, r), __builtin_amdgcn_alignbyte(0u, v.w, r));
+    return make_uint4(none ? 0u : o.x, none ? 0u : o.y, none ? 0u : o.z, none ? 0u : o.w);
+}
+
 // g[i] = { r0.byte[i], r1.byte[i], r2.byte[i], r3.byte[i] }  (byte 0 first)
 __device__ __forceinline__ void transpose4x4_bytes(uint32_t r0, uint32_t r1, uint32_t r2,
                                                    uint32_t r3, uint32_t (&g)[4]) {

@@ -7,11 +7,11 @@
 // byte[kb, n] = c0 | c1<<2 | c2<<4 | c3<<6 for k = 4kb..4kb+3.
 //
 // Two kernels share that arithmetic:
-//   * quantize_pack_fast_kernel: K a multiple of 256, N a multiple of the row tile,
-//     aligned pointers.  A wave keeps one whole row in registers (K/64 values per
+//   * quantize_pack_fast_kernel: rows of 4 to 16384 values.  A wave keeps one whole row in registers (K/64 values per
 //     lane), reduces its absmax across the 64 lanes, encodes, and hands the row's
 //     bytes to LDS; a workgroup owns R = WAVES*RPW consecutive rows, so the
-//     transposed store writes R contiguous bytes per packed_T row.  One read of W.
+//     transposed store writes R contiguous bytes per packed_T row.  One read of W.  RAG: any K and N, rows that
+//     start on any element; without it K a multiple of 256, N of the row tile, aligned pointers.
 //   * quantize_pack_generic_kernel: any shape, alignment and dtype, optional dense
 //     ternary output; reads every row twice (absmax pass, encode pass) and walks K
 //     in segments so that the LDS tile is bounded.
@@ -62,7 +62,11 @@ constexpr int arith_dtype(int dt) { return dt == BT_F32_AS_F16 ? BT_F16 : dt; }
 // with nothing to overlap it (4096 x 11008 fp32: 45.4 us, of which 9.4 us encode; split over four waves: see below).
 // LDS tile: byte (kb, row) at kb*PITCHB + row, PITCHB = R + 4: the odd dword pitch keeps the
 // column writes (lanes = consecutive kb) and the row reads free of bank conflicts.
-template <int DT, int ITERS, int WAVES, int RPW, int SPLIT = 1>
+// RAG: a row's groups of four are loaded as they lie (4- or 2-byte aligned vector loads; the last one from K - 4 on and
+// shifted into place, so that no load leaves the row), and the 16-byte pieces of packed_T are stored as they lie too.
+// Bound by memory like the aligned form.  14656 x 8642 fp16 86 us = 3.3 TB/s (64 with
+// rows of 8704 in the aligned form, 313 in the generic kernel), 11007 x 4095 fp32 42.6 us (138.5).
+template <int DT, int ITERS, int WAVES, int RPW, int SPLIT = 1, bool RAG = false>
 __global__ __launch_bounds__(WAVES * 64) void quantize_pack_fast_kernel(
     const void* __restrict__ W, int N, int K, float tf, float clamp_min, int per_channel,
     uint8_t* __restrict__ packed_T, float* __restrict__ scale, int tiles, int per_xcd) {
@@ -77,8 +81,9 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_pack_fast_kernel(
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = wave / SPLIT, part = wave % SPLIT;
     const int n0 = tile * R;
-    const int nfull = (K >> 8) - part * ITERS;  // complete 256-element chunks of this wave's share (uniform)
-    const int Kb = K >> 2;
+    // 256-element chunks of this wave's share (uniform); RAG: the row's last one may be incomplete
+    const int nfull = (RAG ? (K + 255) >> 8 : K >> 8) - part * ITERS;
+    const int Kb = RAG ? (K + 3) >> 2 : K >> 2;
     const float tensor_scale = per_channel ? 0.0f : fmaxf(scale[0], clamp_min);
     // The tensor scale arrives unfloored; one thread stores the floored value.  Workgroups that read it afterwards
     // floor it again, which changes nothing.
@@ -98,7 +103,7 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_pack_fast_kernel(
                 for (int q = 0; q < SPLIT; q++) amax = fmaxf(amax, part_max[r][slot * SPLIT + q]);
             }
             s = fmaxf(amax, clamp_min);
-            if (lane == 0 && part == 0) scale[n] = s;
+            if (lane == 0 && part == 0 && (!RAG || n < N)) scale[n] = s;
         } else {
             s = tensor_scale;
         }
@@ -108,7 +113,52 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_pack_fast_kernel(
     for (int r = 0; r < RPW; r++) {
         const int n = n0 + RPW * slot + r;
         float4 v[ITERS];
-        if constexpr (f32_storage(DT)) {
+        if constexpr (RAG) {
+            const int nrow = n < N ? nfull : 0;  // (uniform)
+            const int64_t row0 = (int64_t)n * K;
+            int end = K;
+            asm volatile("" : "+s"(end));  // (or the masks of every chunk are computed once and kept through the loop)
+            uint32_t w[ITERS][f32_storage(DT) ? 4 : 2];
+#pragma unroll
+            for (int j = 0; j < ITERS; j++) {
+                if (j < nrow) {
+                    const int kc = min(256 * (part * ITERS + j) + 4 * lane, end - 4);
+                    if constexpr (f32_storage(DT)) {
+                        const u32x4_a4 t = *(const u32x4_a4*)((const float*)W + row0 + kc);
+                        w[j][0] = t.x; w[j][1] = t.y; w[j][2] = t.z; w[j][3] = t.w;
+                    } else {
+                        const u32x2_a2 t = *(const u32x2_a2*)((const uint16_t*)W + row0 + kc);
+                        w[j][0] = t.x; w[j][1] = t.y;
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < (f32_storage(DT) ? 4 : 2); e++) w[j][e] = 0u;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < ITERS; j++) {
+                float f[4];
+                if constexpr (f32_storage(DT)) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) f[e] = as_read<DT>(__builtin_bit_cast(float, w[j][e]));
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const uint16_t h = (uint16_t)(w[j][e >> 1] >> (16 * (e & 1)));
+                        f[e] = DT == BT_F16 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
+                    }
+                }
+                if (256 * (part * ITERS + j + 1) > end) {  // (uniform) the chunk that holds the row's end: shift, zeros behind it
+                    const int sh = max(256 * (part * ITERS + j) + 4 * lane + 4 - end, 0);  // elements of the group past the end
+                    const bool one = sh & 1, two = sh & 2;
+                    f[0] = one ? f[1] : f[0]; f[1] = one ? f[2] : f[1]; f[2] = one ? f[3] : f[2];
+                    f[0] = two ? f[2] : f[0]; f[1] = two ? f[3] : f[1];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) f[e] = e + sh < 4 ? f[e] : 0.0f;
+                }
+                v[j] = make_float4(f[0], f[1], f[2], f[3]);
+            }
+        } else if constexpr (f32_storage(DT)) {
             const float4* rowp = (const float4*)((const float*)W + (int64_t)n * K) + part * ITERS * 64 + lane;
 #pragma unroll
             for (int j = 0; j < ITERS; j++) {
@@ -152,7 +202,7 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_pack_fast_kernel(
     }
 #pragma unroll
     for (int j = 0; j < ITERS; j++) {
-        if (j < nfull) {
+        if (j < nfull && (!RAG || (part * ITERS + j) * 64 + lane < Kb)) {
             uint8_t* dst = lds_b + ((part * ITERS + j) * 64 + lane) * PITCHB + slot * RPW;
             if constexpr (RPW == 4) *(uint32_t*)dst = pk[j];
             else if constexpr (RPW == 2) *(uint16_t*)dst = (uint16_t)pk[j];
@@ -164,18 +214,28 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_pack_fast_kernel(
     for (int idx = threadIdx.x; idx < Kb * Q; idx += WAVES * 64) {
         const int kb = idx / Q, q = idx % Q;
         const uint32_t* src = (const uint32_t*)(lds_b + kb * PITCHB + 16 * q);
-        *(uint4*)(packed_T + (int64_t)kb * N + n0 + 16 * q) = make_uint4(src[0], src[1], src[2], src[3]);
+        uint8_t* dst = packed_T + (int64_t)kb * N + n0 + 16 * q;
+        if constexpr (RAG) {
+            if (n0 + 16 * q + 16 <= N) {
+                *(u32x4_a1*)dst = u32x4_a1{src[0], src[1], src[2], src[3]};
+            } else {
+                for (int i = 0; i < 16; i++)
+                    if (n0 + 16 * q + i < N) dst[i] = lds_b[kb * PITCHB + 16 * q + i];
+            }
+        } else {
+            *(uint4*)dst = make_uint4(src[0], src[1], src[2], src[3]);
+        }
     }
 }
 
-template <int DT, int ITERS, int WAVES, int RPW, int SPLIT = 1>
+template <int DT, int ITERS, int WAVES, int RPW, int SPLIT = 1, bool RAG = false>
 static int launch_fast_cfg(const void* W, int64_t N, int64_t K, float tf, float clamp_min, int per_channel,
                            uint8_t* packed_T, float* scale, hipStream_t st) {
     constexpr int R = (WAVES / SPLIT) * RPW;
-    const int tiles = (int)(N / R);
+    const int tiles = (int)ceil_div(N, R);
     const int per_xcd = (int)ceil_div(tiles, 8);
-    const size_t lds = (size_t)(K / 4) * (R + 4);
-    auto kern = quantize_pack_fast_kernel<DT, ITERS, WAVES, RPW, SPLIT>;
+    const size_t lds = (size_t)ceil_div(K, 4) * (R + 4);
+    auto kern = quantize_pack_fast_kernel<DT, ITERS, WAVES, RPW, SPLIT, RAG>;
     if (lds > 64 * 1024 &&
         hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
         set_error("bt_quantize_pack: cannot reserve %zu bytes of LDS", lds);
@@ -188,7 +248,7 @@ static int launch_fast_cfg(const void* W, int64_t N, int64_t K, float tf, float 
 
 // Row tile for the fast kernel: as many rows per wave (bytes per packed_T segment) as still
 // leave more than one tile per CU; at least 16 rows per workgroup (one 16-byte piece).
-template <int DT, int ITERS, int WAVES>
+template <int DT, int ITERS, int WAVES, bool RAG>
 static int launch_fast_rows(const void* W, int64_t N, int64_t K, float tf, float clamp_min, int per_channel,
                             uint8_t* packed_T, float* scale, hipStream_t st, int* rc) {
     constexpr int MIN_RPW = (WAVES >= 16) ? 1 : (WAVES >= 8) ? 2 : 4;
@@ -198,18 +258,18 @@ static int launch_fast_rows(const void* W, int64_t N, int64_t K, float tf, float
         // (workgroups of 8 waves run two to a compute unit: at least 640 of them, so that both places stay filled)
         const int64_t min_tiles = (WAVES == 8 && ITERS <= 16) ? 640 : 320;
         rpw = 4;
-        while (rpw > MIN_RPW && (N % (WAVES * rpw) != 0 || N / (WAVES * rpw) < min_tiles)) rpw >>= 1;
+        while (rpw > MIN_RPW && ((!RAG && N % (WAVES * rpw) != 0) || N / (WAVES * rpw) < min_tiles)) rpw >>= 1;
     }
     if (rpw < MIN_RPW) rpw = MIN_RPW;
-    if (N % (WAVES * rpw) != 0 || (size_t)(K / 4) * (WAVES * rpw + 4) > 150 * 1024) return 0;
+    if ((!RAG && N % (WAVES * rpw) != 0) || (size_t)ceil_div(K, 4) * (WAVES * rpw + 4) > 150 * 1024) return 0;
     if (rpw == 4) {
-        *rc = launch_fast_cfg<DT, ITERS, WAVES, 4>(W, N, K, tf, clamp_min, per_channel, packed_T, scale, st);
+        *rc = launch_fast_cfg<DT, ITERS, WAVES, 4, 1, RAG>(W, N, K, tf, clamp_min, per_channel, packed_T, scale, st);
     } else if (rpw == 2) {
         if constexpr (MIN_RPW <= 2)
-            *rc = launch_fast_cfg<DT, ITERS, WAVES, 2>(W, N, K, tf, clamp_min, per_channel, packed_T, scale, st);
+            *rc = launch_fast_cfg<DT, ITERS, WAVES, 2, 1, RAG>(W, N, K, tf, clamp_min, per_channel, packed_T, scale, st);
     } else {
         if constexpr (MIN_RPW <= 1)
-            *rc = launch_fast_cfg<DT, ITERS, WAVES, 1>(W, N, K, tf, clamp_min, per_channel, packed_T, scale, st);
+            *rc = launch_fast_cfg<DT, ITERS, WAVES, 1, 1, RAG>(W, N, K, tf, clamp_min, per_channel, packed_T, scale, st);
     }
     return 1;
 }
@@ -217,40 +277,55 @@ static int launch_fast_rows(const void* W, int64_t N, int64_t K, float tf, float
 // returns 1 if the fast kernel took the call (rc holds its status), 0 if the shape does not
 // qualify.  Register budget: a row of K elements costs K/64 data registers per lane, so 16 waves
 // per workgroup fit K <= 4096 with a row per wave, K <= 8192 with a row over two waves and K <= 16384 over four.
-template <int DT>
-static int try_launch_fast(const void* W, int64_t N, int64_t K, float tf, float clamp_min, int per_channel,
-                           uint8_t* packed_T, float* scale, int8_t* w_tern, hipStream_t st, int* rc) {
-    if (!packed_T || w_tern || K % 256 != 0 || ((uintptr_t)W) % 16 != 0 || ((uintptr_t)packed_T) % 16 != 0 ||
-        N * K >= (1ll << 31) || tuning_env("BITTORCH_QP_GENERIC"))
-        return 0;
-    const int chunks = (int)(K / 256);
+template <int DT, bool RAG>
+static int launch_fast(const void* W, int64_t N, int64_t K, float tf, float clamp_min, int per_channel,
+                       uint8_t* packed_T, float* scale, hipStream_t st, int* rc) {
+    const int chunks = (int)ceil_div(K, 256);
 #define BT_QF(IT, WV) \
-    if (chunks <= IT) return launch_fast_rows<DT, IT, WV>(W, N, K, tf, clamp_min, per_channel, packed_T, scale, st, rc)
+    if (chunks <= IT) return launch_fast_rows<DT, IT, WV, RAG>(W, N, K, tf, clamp_min, per_channel, packed_T, scale, st, rc)
     BT_QF(4, 16);
     BT_QF(8, 16);
     // 2048 < K <= 4096 and many rows: workgroups of 8 waves (16 rows), two per compute unit, so that one loads while the
     // other encodes and stores, and the last round is cut finer (11008 x 4096: 34.9 against 40.0 us; 4096 x 4096, one
     // workgroup per compute unit either way, stays on 16 waves: 15.4 against 16.4 us)
-    if (chunks > 8 && chunks <= 16 && N >= 6144 && N % 16 == 0)
-        return launch_fast_rows<DT, 16, 8>(W, N, K, tf, clamp_min, per_channel, packed_T, scale, st, rc);
+    if (chunks > 8 && chunks <= 16 && N >= 6144 && (RAG || N % 16 == 0))
+        return launch_fast_rows<DT, 16, 8, RAG>(W, N, K, tf, clamp_min, per_channel, packed_T, scale, st, rc);
     BT_QF(16, 16);
 #undef BT_QF
     // Longer rows are split over two or four waves of a 16-wave workgroup (16 rows per tile either way)
-    if (N % 16 != 0 || (size_t)(K / 4) * 20 > 150 * 1024) return 0;
+    if ((!RAG && N % 16 != 0) || (size_t)ceil_div(K, 4) * 20 > 150 * 1024) return 0;
     const bool two = chunks <= 32 && !tuning_env("BITTORCH_QP_SPLIT4");
     const int per_wave = (int)ceil_div(chunks, two ? 2 : 4);
 #define BT_QS(IT, SP, RP) \
     if (per_wave <= IT) { \
-        *rc = launch_fast_cfg<DT, IT, 16, RP, SP>(W, N, K, tf, clamp_min, per_channel, packed_T, scale, st); \
+        *rc = launch_fast_cfg<DT, IT, 16, RP, SP, RAG>(W, N, K, tf, clamp_min, per_channel, packed_T, scale, st); \
         return 1; \
     }
-    if (two) {
+    if constexpr (RAG) {  // (fewer variants: chunks that a row does not have cost registers and some encoding, no traffic)
+        if (two) {
+            BT_QS(12, 2, 2) BT_QS(16, 2, 2)
+        } else {
+            BT_QS(10, 4, 4) BT_QS(12, 4, 4) BT_QS(16, 4, 4)
+        }
+    } else if (two) {
         BT_QS(10, 2, 2) BT_QS(12, 2, 2) BT_QS(14, 2, 2) BT_QS(16, 2, 2)
     } else {
         BT_QS(6, 4, 4) BT_QS(8, 4, 4) BT_QS(10, 4, 4) BT_QS(11, 4, 4) BT_QS(12, 4, 4) BT_QS(14, 4, 4) BT_QS(16, 4, 4)
     }
 #undef BT_QS
     return 0;
+}
+
+template <int DT>
+static int try_launch_fast(const void* W, int64_t N, int64_t K, float tf, float clamp_min, int per_channel,
+                           uint8_t* packed_T, float* scale, int8_t* w_tern, hipStream_t st, int* rc) {
+    if (!packed_T || w_tern || N * K >= (1ll << 31) || tuning_env("BITTORCH_QP_GENERIC")) return 0;
+    if (K % 256 == 0 && ((uintptr_t)W) % 16 == 0 && ((uintptr_t)packed_T) % 16 == 0 &&
+        launch_fast<DT, false>(W, N, K, tf, clamp_min, per_channel, packed_T, scale, st, rc))
+        return 1;
+    // Everything else that fits in registers: rows of at least one group of four, on whole elements
+    if (K < 4 || ((uintptr_t)W) % (f32_storage(DT) ? 4 : 2) != 0) return 0;
+    return launch_fast<DT, true>(W, N, K, tf, clamp_min, per_channel, packed_T, scale, st, rc);
 }
 
 // ---- generic kernel --------------------------------------------------------------------

@@ -61,6 +61,34 @@ def test_quantize_pack_one_read_kernel_matches_oracle(oracle, n, k):
         _run(oracle, w, 0.05, False, want_tern=False)
 
 
+# The same kernel on rows that are no multiple of 256 values or start anywhere: a last group of one to four values, a last
+# chunk that is nearly empty or nearly full, row tiles with one row or one short, every split of a row, and past the longest.
+RAGGED_SHAPES = [(1, 4), (3, 5), (17, 255), (16, 257), (33, 1023), (63, 1025), (5, 2047), (40, 2050), (7, 4095), (6159, 2051),
+                 (9, 4097), (31, 6147), (17, 8190), (15, 8642), (3, 10243), (2, 12289), (5, 16381), (18, 16384), (3, 16385)]
+
+
+@pytest.mark.parametrize("n,k", RAGGED_SHAPES)
+def test_quantize_pack_ragged_rows_match_oracle_and_stay_inside(oracle, n, k):
+    from bittorch_amd import _C
+    announce("quantize_pack ragged", n, k)
+    for dtype, seed in ((torch.float32, 1), (torch.bfloat16, 2), (torch.float16, 3)):
+        w = seeded_weights(n, k, seed=seed * 1000 + n + k, dtype=dtype)
+        w[n // 2, k - 1] = w.abs().max() * 2   # the row's maximum at its very end
+        _run(oracle, w, 0.05, True, want_tern=False)
+        _run(oracle, w, 0.05, False, want_tern=False)
+        # weights that end where their buffer ends and start off a 16-byte boundary; guard bytes around packed and scale
+        kb = (k + 3) // 4
+        src = torch.empty(n * k + 1, dtype=dtype, device="cuda")
+        src[1:] = w.cuda().reshape(-1)
+        packed = torch.full((kb * n + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+        scale = torch.full((n + 8,), -7.0, device="cuda")
+        assert _C._L.bt_quantize_pack(src[1:].data_ptr(), BT_DT[dtype], n, k, 0.05, 1, packed[32:].data_ptr(), scale[4:].data_ptr(),
+                                      None, torch.cuda.current_stream().cuda_stream) == 0
+        want, s, _ = _C.ternary_quantize_pack(w.cuda(), 0.05, True)
+        assert torch.equal(packed[32:-32], want.reshape(-1)) and torch.equal(scale[4:-4], s.float())
+        assert (packed[:32] == 0xA5).all() and (packed[-32:] == 0xA5).all() and (scale[:4] == -7).all() and (scale[-4:] == -7).all()
+
+
 @pytest.mark.parametrize("tf", [0.0, 0.01, 0.1, 0.5, 1.0])
 def test_quantize_pack_threshold_factors(oracle, tf):
     announce("quantize_pack tf", tf)
