@@ -323,7 +323,7 @@ def ternary_linear_tiled_forward(X: Tensor, W_tiled: Tensor, scale: Tensor, bias
     y = torch.empty((B, Ny), dtype=X.dtype, device=X.device)
     res = None if residual is None else _residual_2d(residual, X, X.shape[:-1], N)
     with torch.cuda.device(X.device):
-        query = _L.bt_packed_forward_workspace_bytes if op == 0 and not swiglu_pairs else _L.bt_packed_forward_fused_workspace_bytes
+        query = _L.bt_tiled_forward_workspace_bytes if op == 0 and not swiglu_pairs else _L.bt_packed_forward_fused_workspace_bytes
         ws = _workspace(query(B, N, K, xdt), X.device)
         _status(_L.bt_ternary_linear_tiled_forward(
             x2.data_ptr(), x2.stride(0), xdt, op, _ptr(pb), ldb, float(eps), W_tiled.data_ptr(), scale.data_ptr(),

@@ -31,6 +31,7 @@ SIGNATURES = {
     "bt_ternary_linear_forward": (_int, [_vp, _int, _vp, _vp, _int, _i64, _vp, _int, _vp, _i64, _i64,
                                          _i64, _vp]),
     "bt_packed_forward_workspace_bytes": (_sz, [_i64, _i64, _i64, _int]),
+    "bt_tiled_forward_workspace_bytes": (_sz, [_i64, _i64, _i64, _int]),
     "bt_ternary_linear_packed_forward": (_int, [_vp, _int, _vp, _vp, _int, _i64, _vp, _int, _vp, _i64,
                                                 _i64, _i64, _vp, _sz, _vp]),
     "bt_act_quant_i8": (_int, [_vp, _int, _i64, _i64, _vp, _vp, _vp]),

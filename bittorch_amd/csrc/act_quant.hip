@@ -87,38 +87,72 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const void* __restrict__
     }
 }
 
+// Eight values of the row at `base` from k on, by clamped, unconditional loads: a group past the end repeats the row's last
+// one and is masked by the caller.  RAG: rows of any length that start on any element (4- or 2-byte aligned vector loads); the
+// group that crosses the row's end is shifted into place and filled with zeros, and groups past it are zero.
+// (Branches between the groups cost three times the kernel's time: 3847 x 8238 bf16 23 us as it is, 74 with them.)
+typedef uint32_t u32x4_a16 __attribute__((ext_vector_type(4), aligned(16)));
+template <int DT>
+struct Group8 { uint32_t d[DT == BT_F32 ? 8 : 4]; };
+template <int DT, bool RAG>
+__device__ __forceinline__ void load_group8(const void* X, int64_t base, int k, int K, Group8<DT>& u) {
+    typedef typename std::conditional<!RAG, u32x4_a16, typename std::conditional<DT == BT_F32, u32x4_a4, u32x4_a2>::type>::type vec;
+    const uint8_t* src = (const uint8_t*)X + (base + min(k, K - 8)) * (DT == BT_F32 ? 4 : 2);
+#pragma unroll
+    for (int h = 0; h < (DT == BT_F32 ? 2 : 1); h++) {
+        const vec v = *(const vec*)(src + 16 * h);
+#pragma unroll
+        for (int e = 0; e < 4; e++) u.d[4 * h + e] = v[e];
+    }
+}
+template <int DT, bool RAG>
+__device__ __forceinline__ void group8_values(Group8<DT> u, int k, int K, float (&v)[8]) {
+    if constexpr (RAG) {
+        const int sh = max(k + 8 - K, 0);  // values of the group past the row's end
+        if constexpr (DT == BT_F32) {
+            const bool one = sh & 1, two = sh & 2, four = sh & 4;
+#pragma unroll
+            for (int e = 0; e < 7; e++) u.d[e] = one ? u.d[e + 1] : u.d[e];
+#pragma unroll
+            for (int e = 0; e < 6; e++) u.d[e] = two ? u.d[e + 2] : u.d[e];
+#pragma unroll
+            for (int e = 0; e < 4; e++) u.d[e] = four ? u.d[e + 4] : u.d[e];
+#pragma unroll
+            for (int e = 0; e < 8; e++) u.d[e] = e + sh < 8 ? u.d[e] : 0u;
+        } else {
+            const uint4 s4 = shift_group(make_uint4(u.d[0], u.d[1], u.d[2], u.d[3]), 2 * sh);
+            u.d[0] = s4.x; u.d[1] = s4.y; u.d[2] = s4.z; u.d[3] = s4.w;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        if constexpr (DT == BT_F32) {
+            v[e] = __builtin_bit_cast(float, u.d[e]);
+        } else {
+            const uint16_t h = (uint16_t)(u.d[e >> 1] >> (16 * (e & 1)));
+            v[e] = (DT == BT_F16) ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
+        }
+    }
+}
+
 // One workgroup per row, the row held in registers between the absmax pass and the
 // quantization: X is read once and the row's latency chain is load -> reduce -> store.
-// Needs K % 8 == 0, K <= 2048*ITERS and aligned pointers (16 bytes X, 8 bytes Q).
-template <int DT, int ITERS>
-__global__ __launch_bounds__(256) void act_quant_row_kernel(const void* __restrict__ X, int K,
+// Needs K % 8 == 0, K <= 2048*ITERS and aligned pointers (16 bytes X, 8 bytes Q).  RAG: any K from 8 on and any X; Q's rows
+// have Kq >= K bytes (a multiple of 16, at most 2048*ITERS), those past K zero: what the tiled GEMM reads of such rows.
+template <int DT, int ITERS, bool RAG>
+__global__ __launch_bounds__(256) void act_quant_row_kernel(const void* __restrict__ X, int K, int Kq,
                                                             int8_t* __restrict__ Q, float* __restrict__ s_x,
                                                             int q_layout, int32_t* __restrict__ rowsum) {
     __shared__ float part[4];
     __shared__ int part_sum[4];
     const int tid = threadIdx.x;
-    const int64_t base = (int64_t)blockIdx.x * K;
+    const int64_t base = (int64_t)blockIdx.x * K, qbase = (int64_t)blockIdx.x * Kq;
+    Group8<DT> u[ITERS];
     float v[ITERS][8];
 #pragma unroll
-    for (int i = 0; i < ITERS; i++) {
-        const int k = (i * 256 + tid) * 8;
-        const int kc = min(k, K - 8);  // clamped, unconditional loads; zeroed below
-        if constexpr (DT == BT_F32) {
-            const uint4 a = *(const uint4*)((const float*)X + base + kc);
-            const uint4 b = *(const uint4*)((const float*)X + base + kc + 4);
-            const uint32_t da[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    for (int i = 0; i < ITERS; i++) load_group8<DT, RAG>(X, base, (i * 256 + tid) * 8, K, u[i]);
 #pragma unroll
-            for (int e = 0; e < 8; e++) v[i][e] = __builtin_bit_cast(float, da[e]);
-        } else {
-            const uint4 u = *(const uint4*)((const uint16_t*)X + base + kc);
-            const uint32_t d[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const uint16_t h = (uint16_t)(d[e >> 1] >> (16 * (e & 1)));
-                v[i][e] = (DT == BT_F16) ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
-            }
-        }
-    }
+    for (int i = 0; i < ITERS; i++) group8_values<DT, RAG>(u[i], (i * 256 + tid) * 8, K, v[i]);
     float amax = 0.0f;
 #pragma unroll
     for (int i = 0; i < ITERS; i++) {
@@ -148,7 +182,7 @@ __global__ __launch_bounds__(256) void act_quant_row_kernel(const void* __restri
             else hi |= byte << (8 * (e - 4));
         }
         const uint2 o = q_layout == Q_OPERAND_ORDER ? q_to_operand_order(lo, hi, tid & 1) : make_uint2(lo, hi);
-        if (k < K) st2_nt(Q + base + k, o.x, o.y);  // K % 16 == 0 in operand order: both lanes of a pair store
+        if (k < Kq) st2_nt(Q + qbase + k, o.x, o.y);  // Kq % 16 == 0 in operand order: both lanes of a pair store
     }
     if (rowsum) {  // (uniform)
         qsum = wave_sum_i32(qsum);
@@ -161,34 +195,20 @@ __global__ __launch_bounds__(256) void act_quant_row_kernel(const void* __restri
 // Many short rows: one wave per row (four rows per workgroup), lane l holding the 8-element chunks i * 64 + l -- all
 // 64 lanes busy where the workgroup kernel above leaves lanes idle, the absmax a shuffle tree, no LDS and no barrier.
 // The same bits.
-template <int DT, int ITERS>
-__global__ __launch_bounds__(256) void act_quant_wave_kernel(const void* __restrict__ X, int64_t B, int K,
+template <int DT, int ITERS, bool RAG>
+__global__ __launch_bounds__(256) void act_quant_wave_kernel(const void* __restrict__ X, int64_t B, int K, int Kq,
                                                              int8_t* __restrict__ Q, float* __restrict__ s_x,
                                                              int q_layout, int32_t* __restrict__ rowsum) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= B) return;  // (whole waves; the kernel has no barrier)
-    const int64_t base = row * K;
+    const int64_t base = row * K, qbase = row * Kq;
+    Group8<DT> u[ITERS];
     float v[ITERS][8];
 #pragma unroll
-    for (int i = 0; i < ITERS; i++) {
-        const int kc = min((i * 64 + lane) * 8, K - 8);  // clamped, unconditional loads; masked below
-        if constexpr (DT == BT_F32) {
-            const uint4 a = *(const uint4*)((const float*)X + base + kc);
-            const uint4 b = *(const uint4*)((const float*)X + base + kc + 4);
-            const uint32_t da[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    for (int i = 0; i < ITERS; i++) load_group8<DT, RAG>(X, base, (i * 64 + lane) * 8, K, u[i]);
 #pragma unroll
-            for (int e = 0; e < 8; e++) v[i][e] = __builtin_bit_cast(float, da[e]);
-        } else {
-            const uint4 u = *(const uint4*)((const uint16_t*)X + base + kc);
-            const uint32_t d[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const uint16_t h = (uint16_t)(d[e >> 1] >> (16 * (e & 1)));
-                v[i][e] = (DT == BT_F16) ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
-            }
-        }
-    }
+    for (int i = 0; i < ITERS; i++) group8_values<DT, RAG>(u[i], (i * 64 + lane) * 8, K, v[i]);
     float amax = 0.0f;
 #pragma unroll
     for (int i = 0; i < ITERS; i++) {
@@ -215,7 +235,7 @@ __global__ __launch_bounds__(256) void act_quant_wave_kernel(const void* __restr
             else hi |= byte << (8 * (e - 4));
         }
         const uint2 o = q_layout == Q_OPERAND_ORDER ? q_to_operand_order(lo, hi, lane & 1) : make_uint2(lo, hi);
-        if (k < K) st2_nt(Q + base + k, o.x, o.y);
+        if (k < Kq) st2_nt(Q + qbase + k, o.x, o.y);
     }
     if (rowsum) {  // (uniform)
         qsum = wave_sum_i32(qsum);
@@ -223,32 +243,31 @@ __global__ __launch_bounds__(256) void act_quant_wave_kernel(const void* __restr
     }
 }
 
-template <int DT>
-static bool launch_act_quant_rows(const void* X, int64_t B, int64_t K, int8_t* Q, float* s_x, int ql, int32_t* rs,
+template <int DT, bool RAG>
+static bool launch_act_quant_rows(const void* X, int64_t B, int64_t K, int64_t Kq, int8_t* Q, float* s_x, int ql, int32_t* rs,
                                   hipStream_t st) {
-    if (K % 8 != 0 || K > 16384 || ((uintptr_t)X) % 16 != 0 || ((uintptr_t)Q) % 8 != 0 || B > 0x7fffffff ||
-        tuning_env("BITTORCH_ACTQ_GENERIC"))
-        return false;
+    if (Kq > 16384 || ((uintptr_t)Q) % 8 != 0 || B > 0x7fffffff || tuning_env("BITTORCH_ACTQ_GENERIC")) return false;
+    if (!RAG && (K % 8 != 0 || ((uintptr_t)X) % 16 != 0)) return false;
     const dim3 grid((unsigned)B), block(256);
-    const int k = (int)K;
+    const int k = (int)K, kq = (int)Kq;
     if (B >= 2048 && K <= 3072) {  // many short rows: a wave per row (4096 x 2560 bf16 9.4 -> 7.6 us, 4096 x 1024 6.9 -> 4.5,
                                    // 4096 x 2048 7.3 -> 6.6; from K = 3584 on the workgroup kernel is as fast or faster)
         const dim3 wgrid((unsigned)((B + 3) / 4));
-        switch ((k + 511) / 512) {
-            case 1: hipLaunchKernelGGL((act_quant_wave_kernel<DT, 1>), wgrid, block, 0, st, X, B, k, Q, s_x, ql, rs); break;
-            case 2: hipLaunchKernelGGL((act_quant_wave_kernel<DT, 2>), wgrid, block, 0, st, X, B, k, Q, s_x, ql, rs); break;
-            case 3: hipLaunchKernelGGL((act_quant_wave_kernel<DT, 3>), wgrid, block, 0, st, X, B, k, Q, s_x, ql, rs); break;
-            case 4: hipLaunchKernelGGL((act_quant_wave_kernel<DT, 4>), wgrid, block, 0, st, X, B, k, Q, s_x, ql, rs); break;
-            case 5: hipLaunchKernelGGL((act_quant_wave_kernel<DT, 5>), wgrid, block, 0, st, X, B, k, Q, s_x, ql, rs); break;
-            default: hipLaunchKernelGGL((act_quant_wave_kernel<DT, 6>), wgrid, block, 0, st, X, B, k, Q, s_x, ql, rs); break;
+        switch ((kq + 511) / 512) {
+            case 1: hipLaunchKernelGGL((act_quant_wave_kernel<DT, 1, RAG>), wgrid, block, 0, st, X, B, k, kq, Q, s_x, ql, rs); break;
+            case 2: hipLaunchKernelGGL((act_quant_wave_kernel<DT, 2, RAG>), wgrid, block, 0, st, X, B, k, kq, Q, s_x, ql, rs); break;
+            case 3: hipLaunchKernelGGL((act_quant_wave_kernel<DT, 3, RAG>), wgrid, block, 0, st, X, B, k, kq, Q, s_x, ql, rs); break;
+            case 4: hipLaunchKernelGGL((act_quant_wave_kernel<DT, 4, RAG>), wgrid, block, 0, st, X, B, k, kq, Q, s_x, ql, rs); break;
+            case 5: hipLaunchKernelGGL((act_quant_wave_kernel<DT, 5, RAG>), wgrid, block, 0, st, X, B, k, kq, Q, s_x, ql, rs); break;
+            default: hipLaunchKernelGGL((act_quant_wave_kernel<DT, 6, RAG>), wgrid, block, 0, st, X, B, k, kq, Q, s_x, ql, rs); break;
         }
         return true;
     }
-    if (K <= 2048) hipLaunchKernelGGL((act_quant_row_kernel<DT, 1>), grid, block, 0, st, X, k, Q, s_x, ql, rs);
-    else if (K <= 4096) hipLaunchKernelGGL((act_quant_row_kernel<DT, 2>), grid, block, 0, st, X, k, Q, s_x, ql, rs);
-    else if (K <= 8192) hipLaunchKernelGGL((act_quant_row_kernel<DT, 4>), grid, block, 0, st, X, k, Q, s_x, ql, rs);
-    else if (K <= 12288) hipLaunchKernelGGL((act_quant_row_kernel<DT, 6>), grid, block, 0, st, X, k, Q, s_x, ql, rs);
-    else hipLaunchKernelGGL((act_quant_row_kernel<DT, 8>), grid, block, 0, st, X, k, Q, s_x, ql, rs);
+    if (Kq <= 2048) hipLaunchKernelGGL((act_quant_row_kernel<DT, 1, RAG>), grid, block, 0, st, X, k, kq, Q, s_x, ql, rs);
+    else if (Kq <= 4096) hipLaunchKernelGGL((act_quant_row_kernel<DT, 2, RAG>), grid, block, 0, st, X, k, kq, Q, s_x, ql, rs);
+    else if (Kq <= 8192) hipLaunchKernelGGL((act_quant_row_kernel<DT, 4, RAG>), grid, block, 0, st, X, k, kq, Q, s_x, ql, rs);
+    else if (Kq <= 12288) hipLaunchKernelGGL((act_quant_row_kernel<DT, 6, RAG>), grid, block, 0, st, X, k, kq, Q, s_x, ql, rs);
+    else hipLaunchKernelGGL((act_quant_row_kernel<DT, 8, RAG>), grid, block, 0, st, X, k, kq, Q, s_x, ql, rs);
     return true;
 }
 
@@ -263,15 +282,60 @@ int launch_act_quant(const void* X, int x_dtype, int64_t B, int64_t K, int8_t* Q
         return BT_ERR_INVALID;
     }
     int32_t* rs = rowsum;
-    const bool done = (x_dtype == BT_F32)   ? launch_act_quant_rows<BT_F32>(X, B, K, Q, s_x, ql, rs, st)
-                      : (x_dtype == BT_F16) ? launch_act_quant_rows<BT_F16>(X, B, K, Q, s_x, ql, rs, st)
-                                            : launch_act_quant_rows<BT_BF16>(X, B, K, Q, s_x, ql, rs, st);
+    const bool done = (x_dtype == BT_F32)   ? launch_act_quant_rows<BT_F32, false>(X, B, K, K, Q, s_x, ql, rs, st)
+                      : (x_dtype == BT_F16) ? launch_act_quant_rows<BT_F16, false>(X, B, K, K, Q, s_x, ql, rs, st)
+                                            : launch_act_quant_rows<BT_BF16, false>(X, B, K, K, Q, s_x, ql, rs, st);
     if (done) return check_launch("bt_act_quant_i8");
     const dim3 grid((unsigned)ceil_div(B, 4)), block(256);
     if (x_dtype == BT_F32) hipLaunchKernelGGL(act_quant_kernel<BT_F32>, grid, block, 0, st, X, B, K, Q, s_x, ql, rs);
     else if (x_dtype == BT_F16) hipLaunchKernelGGL(act_quant_kernel<BT_F16>, grid, block, 0, st, X, B, K, Q, s_x, ql, rs);
     else hipLaunchKernelGGL(act_quant_kernel<BT_BF16>, grid, block, 0, st, X, B, K, Q, s_x, ql, rs);
     return check_launch("bt_act_quant_i8");
+}
+
+// Rows of any length and start into operand order with rows of Kq = K rounded up to 16 (zeros behind K): the same bytes and
+// scales as launch_act_quant's for the K values.
+bool act_quant_padded_ok(const void* X, int x_dtype, int64_t B, int64_t K) {
+    return K >= 8 && K <= 16384 && B <= 0x7fffffff && ((uintptr_t)X) % (uintptr_t)dtype_size(x_dtype) == 0;
+}
+int launch_act_quant_padded(const void* X, int x_dtype, int64_t B, int64_t K, int64_t Kq, int8_t* Q, float* s_x, hipStream_t st) {
+    const int ql = Q_OPERAND_ORDER;
+    const bool done = (x_dtype == BT_F32)   ? launch_act_quant_rows<BT_F32, true>(X, B, K, Kq, Q, s_x, ql, nullptr, st)
+                      : (x_dtype == BT_F16) ? launch_act_quant_rows<BT_F16, true>(X, B, K, Kq, Q, s_x, ql, nullptr, st)
+                                            : launch_act_quant_rows<BT_BF16, true>(X, B, K, Kq, Q, s_x, ql, nullptr, st);
+    if (!done) {
+        set_error("bt_act_quant_i8: rows of %lld values cannot be padded", (long long)K);
+        return BT_ERR_INVALID;
+    }
+    return check_launch("bt_act_quant_i8");
+}
+
+// 16-bit rows of any length as rows of Kp = K rounded up to 8, zeros behind K: what the tiled 16-bit GEMM's 16-byte loads
+// need.  Bound by its bytes; a thread copies one group of eight, the one that crosses the row's end element by element.
+__global__ __launch_bounds__(256) void pad_rows_kernel(const uint16_t* __restrict__ X, int64_t groups, uint32_t row_groups, int K,
+                                                       uint4* __restrict__ P) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < groups; i += (int64_t)gridDim.x * 256) {
+        const int64_t row = i / row_groups;
+        const int k = 8 * (int)(i - row * row_groups);
+        const uint16_t* src = X + row * K + k;
+        uint32_t d[4] = {0u, 0u, 0u, 0u};
+        if (k + 8 <= K) {
+            const u32x4_a2 v = *(const u32x4_a2*)src;
+#pragma unroll
+            for (int e = 0; e < 4; e++) d[e] = v[e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (k + e < K) d[e >> 1] |= (uint32_t)src[e] << (16 * (e & 1));
+        }
+        P[i] = make_uint4(d[0], d[1], d[2], d[3]);
+    }
+}
+int launch_pad_rows(const void* X, int64_t B, int64_t K, void* P, hipStream_t st) {
+    const int64_t row_groups = ceil_div(K, 8), groups = B * row_groups;
+    const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(groups, 256), 1 << 20);
+    hipLaunchKernelGGL(pad_rows_kernel, dim3(blocks), dim3(256), 0, st, (const uint16_t*)X, groups, (uint32_t)row_groups, (int)K, (uint4*)P);
+    return check_launch("bt_ternary_linear_packed_forward(pad)");
 }
 
 // fp32 activations as three bf16 planes: x = hi + mid + lo exactly, each term the truncation to

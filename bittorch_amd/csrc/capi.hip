@@ -66,7 +66,7 @@ size_t tiled_bytes(int64_t N, int64_t K);
 int launch_stream(int mode, const void* X, int x_elem_size, const float* s_x, const uint8_t* W_T, int w_layout,
                   const Epilogue& epi, void* Y, int y_dtype, int32_t* acc_out, int64_t B, int64_t N,
                   int64_t K, int planes, int q_layout, int pro_op, const void* pro_b, float pro_eps, int epi_op,
-                  hipStream_t st);
+                  hipStream_t st, int64_t Kw = 0);
 bool stream_prologue_fusable(int mode, int64_t B, int64_t N, int64_t K, const void* X, const void* pro_b, int w_layout,
                              int epi_op);
 int launch_retile(const uint8_t* W_T, int64_t N, int64_t K, int pairs, void* T, bool inverse, uint8_t* W_out,
@@ -78,15 +78,18 @@ int launch_unpacked(const void* X, int x_dtype, const int8_t* W, const Epilogue&
                     int64_t N, int64_t K, hipStream_t st);
 int launch_act_quant(const void* X, int x_dtype, int64_t B, int64_t K, int8_t* Q, float* s_x, int q_layout,
                      int32_t* rowsum, hipStream_t st);
+bool act_quant_padded_ok(const void* X, int x_dtype, int64_t B, int64_t K);
+int launch_act_quant_padded(const void* X, int x_dtype, int64_t B, int64_t K, int64_t Kq, int8_t* Q, float* s_x, hipStream_t st);
 int launch_retile_fields(const uint8_t* W_tiled, int64_t N, int64_t K, uint8_t* W_fields, hipStream_t st);
 bool gemm_i8_supported(int64_t N, int64_t K, const void* Q, const void* W_T);
 int launch_row_op(int op, int dtype, const void* A, int64_t lda, const void* Bv, int64_t ldb, float eps, int64_t B,
                   int64_t K, void* H, int8_t* Q, float* s_x, int q_layout, int32_t* rowsum, hipStream_t st,
                   const char* who);
-bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, const void* Y);
+bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, const void* Y, bool tiled);
 double gemm_f16_cost(int64_t M, int64_t N, int64_t K);
 int launch_gemm_f16(int mode, const void* X, const uint8_t* W_T, int w_layout, const Epilogue& epi, void* Y, int64_t M,
-                    int64_t N, int64_t K, hipStream_t st);
+                    int64_t N, int64_t K, hipStream_t st, int64_t Kw = 0);
+int launch_pad_rows(const void* X, int64_t B, int64_t K, void* P, hipStream_t st);
 bool gemm_f32_shape_ok(int64_t N, int64_t K);
 bool gemm_f32_supported(int64_t N, int64_t K, const void* X, const void* Y);
 double gemm_f32_cost(int64_t M, int64_t N, int64_t K);
@@ -107,11 +110,11 @@ int launch_i8_group(const int8_t* const* Q_tab, int q_layout, const float* const
 bool planes_bf16_shape_ok(int64_t N, int64_t K);
 bool planes_bf16_wide(int64_t N, int64_t K);
 int launch_planes_bf16_wide(const void* X, const uint8_t* W, const Epilogue& epi, void* Y, int64_t N, int64_t K, hipStream_t st);
-bool gemm_i8_supported_tiled(int64_t N, int64_t K, const void* Q);
+bool gemm_i8_supported_tiled(int64_t N, int64_t K, const void* Q, bool operand_order);
 double gemm_i8_cost(int64_t M, int64_t N, int64_t K, bool tiled, bool operand_order);
 int launch_gemm_i8(const int8_t* Q, int q_layout, const float* s_x, const int32_t* q_rowsum, const uint8_t* W_T, int w_layout,
                    const Epilogue& epi, void* Y, int y_dtype, int32_t* acc_out, int64_t M, int64_t N, int64_t K,
-                   hipStream_t st);
+                   hipStream_t st, int64_t Kw = 0);
 
 static bool valid_dtype(int dt) { return dt == BT_F32 || dt == BT_F16 || dt == BT_BF16; }
 
@@ -270,10 +273,35 @@ static bool packed_uses_f32_planes(const void* W_T, const void* Y, int64_t N, in
     return stream_supported(N, 3 * plane_len(K), W_T) && fast_path_ok(Y, N, 3 * plane_len(K));
 }
 
-extern "C" size_t bt_packed_forward_workspace_bytes(int64_t B, int64_t N, int64_t K, int x_dtype) {
+// Scratch of a forward on the decode-tiled copy: fp32 rows' planes where the streaming kernel takes them, and more than 16
+// 16-bit rows of K % 8 != 0 padded to whole groups of 8 values: the tiled GEMM reads no other, and the streaming kernel reads
+// them again for every 64 columns (37 x 11152 x 10447 bf16 67 us as they lie, 43 with the 3 us of the copy; 16 rows and fewer
+// 1 x 704 x 10801 38 us by element, 18.5 as they lie).
+static bool pads_rows(int64_t B, int64_t K, int x_dtype) { return x_dtype != BT_F32 && K % 8 != 0 && B > 16; }
+static size_t pad_bytes(int64_t B, int64_t K) { return align256((size_t)B * ceil_div(K, 8) * 16); }
+extern "C" size_t bt_tiled_forward_workspace_bytes(int64_t B, int64_t N, int64_t K, int x_dtype) {
     if (B <= 0 || N <= 0 || K <= 0) return 0;
     if (x_dtype == BT_F32) return !prefers_stream_f32(B, N, K) && gemm_f32_shape_ok(N, K) ? 0 : f32_planes_bytes(B, K);
-    return stream_workspace_bytes(x_dtype == BT_F16 ? MODE_F16 : MODE_BF16, B, N, ceil_div(K, 4));
+    return pads_rows(B, K, x_dtype) ? pad_bytes(B, K) : 0;
+}
+
+// Packed rows of N % 4 != 0 start on any byte, which the kernels that stream them pay for byte by byte, once per 16 rows of
+// activations: from 2^24 weights times row blocks on they are re-tiled into the workspace first.  Measured (int8, us, byte by byte /
+// re-tiled with the 3 us of that launch): 16 rows, 2051 x 1040 5.4 / 7.2, 4099 x 2064 6.2 / 8.9; 29 rows, 6606 x 14272 38.2 / 29.2.
+// (The fp32 GEMM reads such rows as they are, the 16-bit and int8 ones only the copy.)
+static bool can_retile(int64_t N, int64_t K) {
+    return N % 4 != 0 && K < (1ll << 26) && N < (1ll << 30) && tiled_bytes(N, K) < (1ull << 32);
+}
+static bool retile_pays(int64_t B, int64_t N, int64_t K) { return can_retile(N, K) && ceil_div(B, 16) * N * K >= (1ll << 24); }
+static bool packed_retiles(int64_t B, int64_t N, int64_t K, int x_dtype) {
+    if (x_dtype == BT_F32) return retile_pays(B, N, K) && (prefers_stream_f32(B, N, K) || !gemm_f32_shape_ok(N, K));
+    return can_retile(N, K) && (retile_pays(B, N, K) || !prefers_stream(B, N, K, false));  // (the tiled GEMM takes no other)
+}
+extern "C" size_t bt_packed_forward_workspace_bytes(int64_t B, int64_t N, int64_t K, int x_dtype) {
+    if (B <= 0 || N <= 0 || K <= 0) return 0;
+    // (fp32 rows of N % 4 != 0 are asked the planes for at any size: what this query has always said of them)
+    const size_t own = x_dtype == BT_F32 && N % 4 != 0 ? f32_planes_bytes(B, K) : bt_tiled_forward_workspace_bytes(B, N, K, x_dtype);
+    return align256(own) + (packed_retiles(B, N, K, x_dtype) ? tiled_bytes(N, K) : 0);
 }
 
 // residual (optional): [B, N] in Y's dtype, 16-byte aligned; Y = round(round(linear) + residual)
@@ -284,6 +312,15 @@ static int set_residual(const char* who, const void* residual, Epilogue* e) {
     }
     e->residual = residual;
     return BT_OK;
+}
+
+// The rows a call's kernels read: X, or (pads_rows, and room for it) its padded copy.
+static int pad_rows_if(const void* X, int x_dtype, int64_t B, int64_t K, void* workspace, size_t workspace_bytes, hipStream_t st,
+                       const void** rows, int64_t* row_len) {
+    if (!pads_rows(B, K, x_dtype) || !workspace || workspace_bytes < pad_bytes(B, K) || ((uintptr_t)workspace) % 256 != 0) return BT_OK;
+    *rows = workspace;
+    *row_len = ceil_div(K, 8) * 8;
+    return launch_pad_rows(X, B, K, workspace, st);
 }
 
 static int packed_forward_impl(const char* who, const void* X, int x_dtype, const uint8_t* W_T, int w_layout, int epi_op,
@@ -323,10 +360,13 @@ static int packed_forward_impl(const char* who, const void* X, int x_dtype, cons
         if (x_dtype != BT_F32) {
             const int mode = (x_dtype == BT_F16) ? MODE_F16 : MODE_BF16;
             // tall batches: the tiled matrix-core GEMM reads the copy too (not with the SwiGLU output stage)
-            if (!prefers_stream(B, N, K, false, true) && epi_op == 0 && gemm_f16_supported(N, K, X, W_T, Y))
-                return launch_gemm_f16(mode, X, W_T, w_layout, epi, Y, B, N, K, st);
-            return launch_stream(mode, X, 2, nullptr, W_T, w_layout, epi, Y, x_dtype, nullptr, B, N, K, 1,
-                                 Q_ROW_MAJOR, 0, nullptr, 0.0f, epi_op, st);
+            const void* rows = X;
+            int64_t Kr = K;  // values of a row of them
+            if ((rc = pad_rows_if(X, x_dtype, B, K, workspace, workspace_bytes, st, &rows, &Kr))) return rc;
+            if (!prefers_stream(B, N, K, false, true) && epi_op == 0 && gemm_f16_supported(N, Kr, rows, W_T, Y, true))
+                return launch_gemm_f16(mode, rows, W_T, w_layout, epi, Y, B, N, Kr, st, K);
+            return launch_stream(mode, rows, 2, nullptr, W_T, w_layout, epi, Y, x_dtype, nullptr, B, N, Kr, 1,
+                                 Q_ROW_MAJOR, 0, nullptr, 0.0f, epi_op, st, K);
         }
         if (!prefers_stream_f32(B, N, K) && epi_op == 0 && gemm_f32_supported(N, K, X, Y))
             return launch_gemm_f32(X, W_T, w_layout, epi, Y, B, N, K, st);
@@ -340,14 +380,26 @@ static int packed_forward_impl(const char* who, const void* X, int x_dtype, cons
         return launch_stream(MODE_BF16, workspace, 2, nullptr, W_T, w_layout, epi, Y, BT_F32, nullptr, B, N, K, 3,
                              Q_ROW_MAJOR, 0, nullptr, 0.0f, epi_op, st);
     }
+    // rows of packed weights that start on any byte: through a tiled copy of them, if there is room for one
+    const size_t own = align256(bt_tiled_forward_workspace_bytes(B, N, K, x_dtype));
+    if (packed_retiles(B, N, K, x_dtype) && !generic_forced() && workspace && workspace_bytes >= own + tiled_bytes(N, K) &&
+        ((uintptr_t)workspace) % 256 == 0 && fast_path_ok(Y, N, 3 * K) && 3 * K < (1ll << 26)) {
+        uint8_t* tiled = (uint8_t*)workspace + own;
+        rc = launch_retile(W_T, N, K, 0, tiled, false, nullptr, st);
+        return rc ? rc : packed_forward_impl(who, X, x_dtype, tiled, W_LAYOUT_TILED, 0, scale, scale_dtype, scale_len, bias, bias_dtype,
+                                             residual, Y, B, N, K, workspace, own, stream);
+    }
     if (packed_uses_stream(x_dtype, W_T, Y, N, K)) {
         if (planes_supported(x_dtype, x_dtype, B, N, K, X, W_T, Y, W_LAYOUT_ROW_MAJOR))
             return launch_planes(X, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, N, K, 0, st);
         const int mode = (x_dtype == BT_F16) ? MODE_F16 : MODE_BF16;
         // tall batches go to the tiled matrix-core kernel, decode shapes stream the weights
-        if (!prefers_stream(B, N, K, false) && gemm_f16_supported(N, K, X, W_T, Y))
-            return launch_gemm_f16(mode, X, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, B, N, K, st);
-        return launch_stream(mode, X, 2, nullptr, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, x_dtype, nullptr, B, N, K, 1, Q_ROW_MAJOR, 0, nullptr, 0.0f, 0, st);
+        const void* rows = X;
+        int64_t Kr = K;
+        if ((rc = pad_rows_if(X, x_dtype, B, K, workspace, workspace_bytes, st, &rows, &Kr))) return rc;
+        if (!prefers_stream(B, N, K, false) && gemm_f16_supported(N, Kr, rows, W_T, Y, false))
+            return launch_gemm_f16(mode, rows, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, B, N, Kr, st, K);
+        return launch_stream(mode, rows, 2, nullptr, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, x_dtype, nullptr, B, N, Kr, 1, Q_ROW_MAJOR, 0, nullptr, 0.0f, 0, st, K);
     }
     if (x_dtype == BT_F32 && packed_uses_f32_planes(W_T, Y, N, K)) {
         if (!prefers_stream_f32(B, N, K) && gemm_f32_supported(N, K, X, Y))
@@ -436,7 +488,9 @@ extern "C" size_t bt_gemm_i8_workspace_bytes(int64_t B, int64_t N, int64_t K) {
 static int gemm_i8_impl(const char* who, const int8_t* Q, int q_layout, const float* s_x, const uint8_t* W_T, int w_layout,
                         const void* scale,
                         int scale_dtype, int64_t scale_len, const void* bias, int bias_dtype, const void* residual,
-                        void* Y, int y_dtype, int32_t* acc_out, int64_t B, int64_t N, int64_t K, void* stream) {
+                        void* Y, int y_dtype, int32_t* acc_out, int64_t B, int64_t N, int64_t Kw, void* stream, int64_t Kq = 0) {
+    // Kq: bytes of a row of Q where that is more than the weights' K (zeros behind it)
+    const int64_t K = Kq ? Kq : Kw;
     int rc = check_shape(who, Q, W_T, Y, y_dtype, B, N, K);
     if (rc) return rc;
     if (!s_x) {
@@ -445,8 +499,8 @@ static int gemm_i8_impl(const char* who, const int8_t* Q, int q_layout, const fl
     }
     rc = check_q_layout(who, q_layout, K, Q, nullptr);
     if (rc) return rc;
-    if (K > kMaxKInt8) {
-        set_error("%s: K=%lld could overflow the int32 accumulators (limit %lld)", who, (long long)K,
+    if (Kw > kMaxKInt8) {
+        set_error("%s: K=%lld could overflow the int32 accumulators (limit %lld)", who, (long long)Kw,
                   (long long)kMaxKInt8);
         return BT_ERR_INVALID;
     }
@@ -465,10 +519,11 @@ static int gemm_i8_impl(const char* who, const int8_t* Q, int q_layout, const fl
             set_error("%s: tiled weights must be 256-byte aligned and below 4 GiB", who);
             return BT_ERR_INVALID;
         }
-        if (!prefers_stream(B, N, K, true, true, q_layout == Q_OPERAND_ORDER) && gemm_i8_supported_tiled(N, K, Q))
-            return launch_gemm_i8(Q, q_layout, s_x, nullptr, W_T, w_layout, epi, Y, y_dtype, acc_out, B, N, K, st);
+        const bool oo = q_layout == Q_OPERAND_ORDER;
+        if (!prefers_stream(B, N, K, true, true, oo) && gemm_i8_supported_tiled(N, K, Q, oo))
+            return launch_gemm_i8(Q, q_layout, s_x, nullptr, W_T, w_layout, epi, Y, y_dtype, acc_out, B, N, K, st, Kw);
         return launch_stream(MODE_I8, Q, 1, s_x, W_T, w_layout, epi, Y, y_dtype, acc_out, B, N, K, 1, q_layout, 0, nullptr,
-                             0.0f, 0, st);
+                             0.0f, 0, st, Kw);
     }
     // decode-shape batches, and any batch whose N the tiled kernel's 4-column
     // vector accesses cannot take, stream the weights once per 16 rows
@@ -478,9 +533,9 @@ static int gemm_i8_impl(const char* who, const int8_t* Q, int q_layout, const fl
                       (long long)ceil_div(K, 4), (long long)N);
             return BT_ERR_INVALID;
         }
-        return launch_stream(MODE_I8, Q, 1, s_x, W_T, w_layout, epi, Y, y_dtype, acc_out, B, N, K, 1, q_layout, 0, nullptr, 0.0f, 0, st);
+        return launch_stream(MODE_I8, Q, 1, s_x, W_T, w_layout, epi, Y, y_dtype, acc_out, B, N, K, 1, q_layout, 0, nullptr, 0.0f, 0, st, Kw);
     }
-    return launch_gemm_i8(Q, q_layout, s_x, nullptr, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, y_dtype, acc_out, B, N, K, st);
+    return launch_gemm_i8(Q, q_layout, s_x, nullptr, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, y_dtype, acc_out, B, N, K, st, Kw);
 }
 
 extern "C" int bt_ternary_gemm_i8(const int8_t* Q, const float* s_x, const uint8_t* W_T, const void* scale,
@@ -500,10 +555,45 @@ extern "C" int bt_ternary_gemm_i8_res(const int8_t* Q, int q_layout, const float
                         Y, y_dtype, acc_out, B, N, K, stream);
 }
 
+// What the matrix-core forward keeps in its workspace: [Q int8, B rows][s_x fp32 B][the weights, decode-tiled].
+// Rows of Q have K bytes rounded up to 16, so that they are written in operand order and the tiled GEMM takes any K.
+static int64_t q_row_bytes(int64_t K) { return ceil_div(K, 16) * 16; }
+static bool tensor_core_retiles(int64_t B, int64_t N, int64_t K) {
+    return can_retile(N, K) && K >= 8 && K <= 16384 && (retile_pays(B, N, K) || !prefers_stream(B, N, K, true, true, true));
+}
+static size_t tensor_core_plain_bytes(int64_t B, int64_t K) { return align256((size_t)B * K) + align256((size_t)B * 4); }
+
 extern "C" size_t bt_tensor_core_workspace_bytes(int64_t B, int64_t N, int64_t K) {
     if (B <= 0 || N <= 0 || K <= 0) return 0;
-    // [GEMM scratch (none at present)] [Q int8 B*K] [s_x fp32 B]
-    return align256(bt_gemm_i8_workspace_bytes(B, N, K)) + align256((size_t)B * K) + align256((size_t)B * 4);
+    return tensor_core_plain_bytes(B, q_row_bytes(K)) + (tensor_core_retiles(B, N, K) ? tiled_bytes(N, K) : 0);
+}
+
+// The activations quantized into Q (rows padded where K % 16 != 0 or X starts on an odd place, if there is room for them),
+// then the GEMM on the row-major weights, or on tiled, the room for a copy of them.
+static int tensor_core_run(const char* who, const void* X, int x_dtype, const uint8_t* W_T, const void* scale, int scale_dtype,
+                           int64_t scale_len, const void* bias, int bias_dtype, void* Y, int64_t B, int64_t N, int64_t K,
+                           int8_t* Q, float* s_x, bool room_for_padding, uint8_t* tiled, void* stream) {
+    // Q is private to this call: written in operand order whenever the layout applies, so that
+    // neither GEMM kernel has to permute activations
+    // (BITTORCH_Q_LAYOUT=rowmajor keeps the row-major layout, for A/B runs)
+    const char* lay = tuning_env("BITTORCH_Q_LAYOUT");
+    const bool row_major = lay && !strcmp(lay, "rowmajor");
+    const bool in_order = K % 16 == 0 && ((uintptr_t)X) % 16 == 0 && !row_major;
+    const bool padded = !in_order && !row_major && room_for_padding && act_quant_padded_ok(X, x_dtype, B, K);
+    const int64_t Kq = padded ? q_row_bytes(K) : K;
+    const int q_layout = in_order || padded ? Q_OPERAND_ORDER : Q_ROW_MAJOR;
+    hipStream_t st = (hipStream_t)stream;
+    int rc = padded ? launch_act_quant_padded(X, x_dtype, B, K, Kq, Q, s_x, st)
+                    : launch_act_quant(X, x_dtype, B, K, Q, s_x, q_layout, nullptr, st);
+    if (rc) return rc;
+    if (tiled && q_layout == Q_OPERAND_ORDER) {
+        rc = launch_retile(W_T, N, K, 0, tiled, false, nullptr, st);
+        if (rc) return rc;
+        return gemm_i8_impl(who, Q, q_layout, s_x, tiled, W_LAYOUT_TILED, scale, scale_dtype, scale_len, bias, bias_dtype, nullptr,
+                            Y, x_dtype, nullptr, B, N, K, stream, Kq);
+    }
+    return gemm_i8_impl(who, Q, q_layout, s_x, W_T, W_LAYOUT_ROW_MAJOR, scale, scale_dtype, scale_len, bias, bias_dtype, nullptr,
+                        Y, x_dtype, nullptr, B, N, K, stream, Kq);
 }
 
 extern "C" int bt_ternary_linear_tensor_core_forward(const void* X, int x_dtype, const uint8_t* W_T,
@@ -514,25 +604,17 @@ extern "C" int bt_ternary_linear_tensor_core_forward(const void* X, int x_dtype,
     const char* who = "bt_ternary_linear_tensor_core_forward";
     int rc = check_shape(who, X, W_T, Y, x_dtype, B, N, K);
     if (rc) return rc;
-    const size_t need = bt_tensor_core_workspace_bytes(B, N, K);
-    if (!workspace || workspace_bytes < need || ((uintptr_t)workspace) % 256 != 0) {
+    const size_t need = bt_tensor_core_workspace_bytes(B, N, K), least = tensor_core_plain_bytes(B, K);
+    if (!workspace || workspace_bytes < least || ((uintptr_t)workspace) % 256 != 0) {
         set_error("%s: workspace of %zu bytes (256-byte aligned) needed, %zu given", who, need, workspace_bytes);
         return BT_ERR_WORKSPACE;
     }
-    const size_t gemm_bytes = align256(bt_gemm_i8_workspace_bytes(B, N, K));
-    int8_t* Q = (int8_t*)((uint8_t*)workspace + gemm_bytes);
-    float* s_x = (float*)((uint8_t*)Q + align256((size_t)B * K));
-    // Q is private to this call: written in operand order whenever the layout applies, so that
-    // neither GEMM kernel has to permute activations
-    // (BITTORCH_Q_LAYOUT=rowmajor keeps the row-major layout, for A/B runs)
-    const char* lay = tuning_env("BITTORCH_Q_LAYOUT");
-    const int q_layout = (K % 16 == 0 && ((uintptr_t)X) % 16 == 0 && !(lay && !strcmp(lay, "rowmajor")))
-                             ? Q_OPERAND_ORDER : Q_ROW_MAJOR;
-    rc = launch_act_quant(X, x_dtype, B, K, Q, s_x, q_layout, nullptr, (hipStream_t)stream);
-    if (rc) return rc;
-    (void)gemm_bytes;
-    return gemm_i8_impl(who, Q, q_layout, s_x, W_T, W_LAYOUT_ROW_MAJOR, scale, scale_dtype, scale_len, bias, bias_dtype, nullptr,
-                        Y, x_dtype, nullptr, B, N, K, stream);
+    const bool room = workspace_bytes >= need;
+    int8_t* Q = (int8_t*)workspace;
+    float* s_x = (float*)(Q + align256((size_t)B * (room ? q_row_bytes(K) : K)));
+    uint8_t* tiled = room && tensor_core_retiles(B, N, K) ? (uint8_t*)workspace + tensor_core_plain_bytes(B, q_row_bytes(K)) : nullptr;
+    return tensor_core_run(who, X, x_dtype, W_T, scale, scale_dtype, scale_len, bias, bias_dtype, Y, B, N, K, Q, s_x, room, tiled,
+                           stream);
 }
 
 // ---- the matrix-core forward for callers that cannot allocate ----------------------------------
@@ -591,11 +673,9 @@ extern "C" int bt_ternary_linear_tensor_core_forward_static(const void* X, int x
     int8_t* Q = (int8_t*)base;
     float* s_x = (float*)(base + kStaticQBytes);
     // both are written in full by the quantizer before the GEMM reads them: nothing has to start at zero
-    const int q_layout = (K % 16 == 0 && ((uintptr_t)X) % 16 == 0) ? Q_OPERAND_ORDER : Q_ROW_MAJOR;
-    rc = launch_act_quant(X, x_dtype, B, K, Q, s_x, q_layout, nullptr, (hipStream_t)stream);
-    if (rc) return rc;
-    return gemm_i8_impl(who, Q, q_layout, s_x, W_T, W_LAYOUT_ROW_MAJOR, scale, scale_dtype, scale_len, bias, bias_dtype,
-                        nullptr, Y, x_dtype, nullptr, B, N, K, stream);
+    const bool room = (uint64_t)B * (uint64_t)q_row_bytes(K) <= kStaticQBytes;
+    return tensor_core_run(who, X, x_dtype, W_T, scale, scale_dtype, scale_len, bias, bias_dtype, Y, B, N, K, Q, s_x, room, nullptr,
+                           stream);
 }
 
 // ---- G decode GEMVs in one launch ---------------------------------------------------------------
@@ -939,7 +1019,7 @@ extern "C" int bt_ternary_gemm_i8_fields(const int8_t* Q, int q_layout, const fl
         return BT_ERR_INVALID;
     }
     if (!fast_path_ok(Y, N, K) || (acc_out && ((uintptr_t)acc_out) % 16 != 0) || !stream_supported_tiled(N, K, W_fields) ||
-        !gemm_i8_supported_tiled(N, K, Q)) {
+        !gemm_i8_supported_tiled(N, K, Q, false)) {
         set_error("%s: N %% 4 == 0, 16-byte aligned Q, Y and acc_out and a 256-byte aligned copy below 4 GiB are needed", who);
         return BT_ERR_INVALID;
     }

@@ -51,7 +51,8 @@ constexpr int fd_stages(int NB) { return NB == 4 ? 3 : NB == 2 ? 4 : 5; }  // in
 constexpr int fd_lds_bytes(int NB) { return fd_stages(NB) * (NB * 4096 + 4096); }
 
 // y = sum * scale + bias, row block by row block (the empty asm keeps a row's address from being computed ahead of its turn)
-template <int MODE, bool RES, int NB>
+// RN: rows of any length, so that a lane's four columns start on any element and the last ones may be fewer.
+template <int MODE, bool RES, int NB, bool RN>
 __device__ __forceinline__ void fd_epilogue(const GemmFParams& p, const v4f (&acc)[2 * NB][4], int64_t m0, int g, int64_t ncol,
                                             int rows_left, const float (&ws)[4], const float (&bs)[4]) {
     constexpr int YDT = MODE == MODE_F16 ? BT_F16 : BT_BF16;
@@ -68,7 +69,15 @@ __device__ __forceinline__ void fd_epilogue(const GemmFParams& p, const v4f (&ac
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 asm volatile("" : "+s"(res));
-                rv[r] = *(const uint2*)(res + (16 * mb + 4 * g + r < rows_left ? lane_off : 0u));
+                const char* src = res + (16 * mb + 4 * g + r < rows_left ? lane_off : 0u);
+                if constexpr (RN) {
+                    uint32_t d[4];
+#pragma unroll
+                    for (int t = 0; t < 4; t++) d[t] = ((const uint16_t*)src)[ncol + t < p.N ? t : 0];
+                    rv[r] = make_uint2(d[0] | d[1] << 16, d[2] | d[3] << 16);
+                } else {
+                    rv[r] = *(const uint2*)src;
+                }
                 res += (16 * mb + r + 1 < rows_left) ? row_bytes : 0;
             }
         }
@@ -88,7 +97,14 @@ __device__ __forceinline__ void fd_epilogue(const GemmFParams& p, const v4f (&ac
                     }
                     h[t] = YDT == BT_F16 ? f32_to_f16_bits(y) : f32_to_bf16_bits(y);
                 }
-                st2_nt(row + lane_off, (uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+                if (RN && ncol + 4 > p.N) {
+                    for (int t = 0; t < 3; t++)
+                        if (ncol + t < p.N) ((uint16_t*)(row + lane_off))[t] = h[t];
+                } else if constexpr (RN) {
+                    *(u32x2_a2*)(row + lane_off) = u32x2_a2{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
+                } else {
+                    st2_nt(row + lane_off, (uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+                }
             }
             row += row_bytes;
         }
@@ -100,7 +116,7 @@ __device__ __forceinline__ void fd_epilogue(const GemmFParams& p, const v4f (&ac
 
 // One tile of 32 NB rows.  TAIL: K is not a multiple of 64 (of 8 it is): the lanes whose k lies past
 // the end load something of their own row or column instead and their activations are zeroed on the way to the MFMAs.
-template <int MODE, int SRC, int NB, bool TAIL>
+template <int MODE, int SRC, int NB, bool TAIL, bool RN>
 __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_t m0, const int tile_n, uint8_t* lds) {
     constexpr int BM = 32 * NB, A_BYTES = NB * 4096, STAGE = A_BYTES + 4096, NST = fd_stages(NB);
     constexpr int A_LOADS = NB, W_LOADS = SRC == W_ROWS ? 4 : 1, LOADS = A_LOADS + W_LOADS;
@@ -330,7 +346,7 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
     uint32_t ws_bits[4], bs_bits[4];
 #pragma unroll
     for (int t = 0; t < 4; t++) {
-        const int64_t n = col_ok ? ncol + t : 0;
+        const int64_t n = !col_ok ? 0 : RN ? min(ncol + t, p.N - 1) : ncol + t;
         ws_bits[t] = load_bits_rt(p.epi.scale, p.epi.scale_dtype, p.epi.scale_bcast ? 0 : n);
         bs_bits[t] = p.epi.bias ? load_bits_rt(p.epi.bias, p.epi.bias_dtype, n) : 0u;
     }
@@ -340,12 +356,12 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
         bs[t] = p.epi.bias ? bits_to_f32_rt(bs_bits[t], p.epi.bias_dtype) : 0.0f;
     }
     if (!col_ok) return;
-    if (p.epi.residual) fd_epilogue<MODE, true, NB>(p, acc, m0, g, ncol, (int)rows_left, ws, bs);
-    else fd_epilogue<MODE, false, NB>(p, acc, m0, g, ncol, (int)rows_left, ws, bs);
+    if (p.epi.residual) fd_epilogue<MODE, true, NB, RN>(p, acc, m0, g, ncol, (int)rows_left, ws, bs);
+    else fd_epilogue<MODE, false, NB, RN>(p, acc, m0, g, ncol, (int)rows_left, ws, bs);
 }
 
 // NB: tiles of 32 NB rows.  NF > 0: an XCD's tiles from p.fine_from on are computed in tiles of 32 NF rows.
-template <int MODE, int SRC, int NB, int NF, bool TAIL>
+template <int MODE, int SRC, int NB, int NF, bool TAIL, bool RN>
 __global__ __launch_bounds__(256, NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_f16_kernel(GemmFParams p) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[fd_lds_bytes(NB)];
     // XCD-aware tile order: the 8 XCDs each take a contiguous run of tiles, walked in groups of four row tiles, so that one
@@ -367,18 +383,18 @@ __global__ __launch_bounds__(256, NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_f16_k
     if constexpr (NF > 0) {
         if (fine) {
             const int64_t mf = m0 + (int64_t)(f % parts) * (32 * NF);
-            if (mf < p.M) gemm_f16_tile<MODE, SRC, NF, TAIL>(p, mf, (int)tn, lds);
+            if (mf < p.M) gemm_f16_tile<MODE, SRC, NF, TAIL, RN>(p, mf, (int)tn, lds);
             return;
         }
     }
-    gemm_f16_tile<MODE, SRC, NB, TAIL>(p, m0, (int)tn, lds);
+    gemm_f16_tile<MODE, SRC, NB, TAIL, RN>(p, m0, (int)tn, lds);
 }
 
 // X and Y are read and written in 16- and 8-byte pieces; 32-bit byte offsets span a tile's rows of X, 16 rows of Y and, for
-// row-major weights, 16 rows of W_T.  W_T 4-byte aligned, or the decode-tiled copy (256-byte aligned, below 4 GiB: checked by
-// the caller).
-bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, const void* Y) {
-    return N % 4 == 0 && N < (1ll << 27) && K % 8 == 0 && K >= 8 && K < (1ll << 23) && ((uintptr_t)W_T) % 4 == 0 &&
+// row-major weights, 16 rows of W_T.  W_T 4-byte aligned and N % 4 == 0, or the decode-tiled copy (256-byte aligned, below
+// 4 GiB: checked by the caller), with which Y's rows have any length.
+bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, const void* Y, bool tiled) {
+    return (tiled || N % 4 == 0) && N < (1ll << 27) && K % 8 == 0 && K >= 8 && K < (1ll << 23) && ((uintptr_t)W_T) % 4 == 0 &&
            ((uintptr_t)X) % 16 == 0 && ((uintptr_t)Y) % 16 == 0;
 }
 
@@ -406,7 +422,7 @@ double gemm_f16_cost(int64_t M, int64_t N, int64_t K) {
     return us;
 }
 
-template <int MODE, int SRC, int NB, bool TAIL>
+template <int MODE, int SRC, int NB, bool TAIL, bool RN = false>
 static int launch_gemm_f16_cfg(GemmFParams p, hipStream_t st) {
     const char* who = SRC == W_TILES ? "bt_ternary_linear_tiled_forward" : "bt_ternary_linear_packed_forward";
     p.tiles_n = (int)ceil_div(p.N, F_BN);
@@ -425,16 +441,19 @@ static int launch_gemm_f16_cfg(GemmFParams p, hipStream_t st) {
             const int rem = p.per_xcd % (int)(2 * gemm_compute_units() / 8);
             p.fine_from = p.per_xcd - rem;
             const dim3 grid((unsigned)(8 * (p.fine_from + parts * rem)));
-            if (parts == 2) hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 4, 2, TAIL>), grid, block, 0, st, p);
-            else hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 4, 1, TAIL>), grid, block, 0, st, p);
+            if (parts == 2) hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 4, 2, TAIL, RN>), grid, block, 0, st, p);
+            else hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 4, 1, TAIL, RN>), grid, block, 0, st, p);
             return check_launch(who);
         }
     }
-    hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, NB, 0, TAIL>), dim3((unsigned)(8 * p.per_xcd)), block, 0, st, p);
+    hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, NB, 0, TAIL, RN>), dim3((unsigned)(8 * p.per_xcd)), block, 0, st, p);
     return check_launch(who);
 }
 template <int MODE, int SRC, int NB>
 static int launch_gemm_f16_src(const GemmFParams& p, hipStream_t st) {
+    if constexpr (SRC == W_TILES) {  // (rows of any length come with K of any length: one instance)
+        if (p.N % 4 != 0) return launch_gemm_f16_cfg<MODE, SRC, NB, true, true>(p, st);
+    }
     return p.K % F_BK != 0 ? launch_gemm_f16_cfg<MODE, SRC, NB, true>(p, st) : launch_gemm_f16_cfg<MODE, SRC, NB, false>(p, st);
 }
 template <int MODE, int NB>
@@ -447,11 +466,12 @@ static int launch_gemm_f16_rows(const GemmFParams& p, int rows, int src, hipStre
     return rows == 4 ? launch_gemm_f16_mode<MODE, 4>(p, src, st)
          : rows == 2 ? launch_gemm_f16_mode<MODE, 2>(p, src, st) : launch_gemm_f16_mode<MODE, 1>(p, src, st);
 }
+// Kw: the weights' K where the rows of X are longer (zeros behind it; 0: K)
 int launch_gemm_f16(int mode, const void* X, const uint8_t* W_T, int w_layout, const Epilogue& epi, void* Y, int64_t M,
-                    int64_t N, int64_t K, hipStream_t st) {
+                    int64_t N, int64_t K, hipStream_t st, int64_t Kw) {
     GemmFParams p = {};
     p.X = (const uint16_t*)X; p.W_T = W_T; p.Y = Y; p.epi = epi;
-    p.M = M; p.N = N; p.K = K; p.Kb = ceil_div(K, 4);
+    p.M = M; p.N = N; p.K = K; p.Kb = ceil_div(Kw ? Kw : K, 4);
     p.wstages = (int)ceil_div(K, F_BK);
     p.tiles16 = tiles16_arg(N, w_layout);
     double us;

@@ -118,11 +118,13 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
         a_off[b] = (r * (uint32_t)p.C + 8u * g) * 4u;
     }
     uint32_t b_off[NG];
+    uint32_t b_shift = 0;  // row-major rows of N % 4 != 0: bits by which the last columns, loaded as the last four, stand too high
 #pragma unroll
     for (int q = 0; q < NG; q++) {
         const int64_t col = c0 + 64 * q + 4 * i;
         if constexpr (SRC == B_ROW_MAJOR) {
-            b_off[q] = 2u * g * (uint32_t)p.ldw + (uint32_t)(col < p.NC ? col : p.NC - 4);
+            b_off[q] = 2u * g * (uint32_t)p.ldw + (uint32_t)(col < p.NC - 4 ? col : p.NC - 4);
+            if (col < p.NC && col > p.NC - 4) b_shift = 8u * (uint32_t)(col - (p.NC - 4));  // (one q at most)
         } else if constexpr (SRC == B_TILED) {
             const int tt = stored_tile16((int)(col >> 4), p.tiles16);
             b_off[q] = ((uint32_t)tt * (uint32_t)p.wsteps * 64u + 16u * (g >> 1) + 4u * (i & 3)) * 4u;
@@ -228,6 +230,15 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
 
     auto step = [&](int nx, bool more, auto any) __attribute__((always_inline)) {  // nx: the step whose operands are requested behind this one's use (uniform)
         u32x4 w[4 * NG];
+        if constexpr (SRC == B_ROW_MAJOR) {
+            if (p.NC % 4 != 0) {  // (uniform)
+#pragma unroll
+                for (int q = 0; q < NG; q++)
+#pragma unroll
+                    for (int r = 0; r < 2; r++)
+                        if (c0 + 64 * q + 4 * i > p.NC - 4) braw[q][r] >>= b_shift;
+            }
+        }
 #pragma unroll
         for (int q = 0; q < NG; q++)
 #pragma unroll
@@ -326,8 +337,9 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
         if constexpr (SRC != B_TRANSPOSED) {
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                ws[t] = epi_scale(p.epi, col + t);
-                bs[t] = epi_bias(p.epi, col + t);
+                const int64_t n = col + t < p.NC ? col + t : p.NC - 1;
+                ws[t] = epi_scale(p.epi, n);
+                bs[t] = epi_bias(p.epi, n);
             }
         }
 #pragma unroll
@@ -353,6 +365,15 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
                 } else {
 #pragma unroll
                     for (int t = 0; t < 4; t++) y[t] = epi_float(y[t], ws[t], bs[t]);
+                    if (p.NC % 4 != 0) {  // rows of any length: element by element
+#pragma unroll
+                        for (int t = 0; t < 4; t++) {
+                            if (col + t >= p.NC) continue;
+                            if (p.epi.residual) y[t] = add_residual(y[t], p.epi.residual, BT_F32, m * p.NC + col + t);
+                            p.Y[m * p.NC + col + t] = y[t];
+                        }
+                        continue;
+                    }
                     if (p.epi.residual) add_residual4(y, p.epi.residual, BT_F32, m * p.NC + col);
                 }
                 st4_nt(p.Y + m * p.NC + col, f2u(y[0]), f2u(y[1]), f2u(y[2]), f2u(y[3]));
@@ -410,7 +431,7 @@ static int launch_gemm_f32_src(const GemmF32Params& p, const char* who, hipStrea
 
 // the kernel's 32-bit offsets span 64 rows of X and the whole of W
 bool gemm_f32_shape_ok(int64_t N, int64_t K) {
-    return N % 4 == 0 && K < (1ll << 23) && N < (1ll << 30) && ceil_div(K, 4) * N < (1ll << 32);
+    return N >= 4 && K < (1ll << 23) && N < (1ll << 30) && ceil_div(K, 4) * N < (1ll << 32);
 }
 // X 4-byte, Y (and the residual) 16-byte aligned
 bool gemm_f32_supported(int64_t N, int64_t K, const void* X, const void* Y) {

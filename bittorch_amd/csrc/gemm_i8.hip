@@ -486,9 +486,10 @@ __global__ __launch_bounds__(512) void gemm_i8_kernel(GemmParams p) {
 
 
 // the same kernel on the decode-tiled weight copy (256-byte aligned, below 4 GiB: checked by the caller)
-bool gemm_i8_supported_tiled(int64_t N, int64_t K, const void* Q) {
+// operand_order: gemm_i8_dma_kernel also stores rows of any length
+bool gemm_i8_supported_tiled(int64_t N, int64_t K, const void* Q, bool operand_order) {
     // (N: 32-bit byte offsets within 16 rows of a 32-bit output)
-    return N % 4 == 0 && N < (1ll << 26) && K % 16 == 0 && ((uintptr_t)Q) % 16 == 0 && (G_BM + 1) * K < (1ll << 32);
+    return (N % 4 == 0 || operand_order) && N < (1ll << 26) && K % 16 == 0 && ((uintptr_t)Q) % 16 == 0 && (G_BM + 1) * K < (1ll << 32);
 }
 
 // the tiled kernel reads Q with 16-byte loads and W_T / Y with 4-column vectors
@@ -536,12 +537,13 @@ static int launch_gemm_i8_part(GemmParams p, int tile_n0, int tiles_n, bool qoo,
 }
 
 // q_rowsum: the rows' sums of Q, needed (and only read) with a field-layout copy
+// Kw: the weights' K where Q's rows, in operand order, are longer (zeros behind it; 0: K)
 int launch_gemm_i8(const int8_t* Q, int q_layout, const float* s_x, const int32_t* q_rowsum, const uint8_t* W_T, int w_layout,
                    const Epilogue& epi, void* Y, int y_dtype, int32_t* acc_out, int64_t M, int64_t N, int64_t K,
-                   hipStream_t st) {
+                   hipStream_t st, int64_t Kw) {
     GemmParams p = {};
     p.Q = Q; p.s_x = s_x; p.W_T = W_T; p.Y = Y; p.acc_out = acc_out; p.epi = epi; p.q_rowsum = q_rowsum;
-    p.M = M; p.N = N; p.K = K; p.Kb = ceil_div(K, 4);
+    p.M = M; p.N = N; p.K = K; p.Kb = ceil_div(Kw ? Kw : K, 4);
     p.y_dtype = y_dtype;
     p.long_epilogue = option(OPT_GEMM_LONG_EPILOGUE) != nullptr;
     p.wsteps = (int)ceil_div(p.Kb, 16);

@@ -35,6 +35,33 @@ struct GemmParams {
 };
 static_assert(offsetof(GemmParams, s_x) == 64, "first argument line as laid out above");
 
+// up to four consecutive outputs (left: how many the row still has) that start on any element
+template <int DT>
+__device__ __forceinline__ void store4_any(void* Y, const float (&v)[4], int left) {
+    if constexpr (DT == BT_F32) {
+        if (left >= 4) {
+            u32x4_a4 o;
+#pragma unroll
+            for (int t = 0; t < 4; t++) o[t] = __builtin_bit_cast(uint32_t, v[t]);
+            *(u32x4_a4*)Y = o;
+            return;
+        }
+#pragma unroll
+        for (int t = 0; t < 3; t++)
+            if (t < left) ((float*)Y)[t] = v[t];
+    } else {
+        uint16_t h[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) h[t] = DT == BT_F16 ? f32_to_f16_bits(v[t]) : f32_to_bf16_bits(v[t]);
+        if (left >= 4) {
+            *(u32x2_a2*)Y = u32x2_a2{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
+            return;
+        }
+#pragma unroll
+        for (int t = 0; t < 3; t++)
+            if (t < left) ((uint16_t*)Y)[t] = h[t];
+    }
+}
 __device__ __forceinline__ void store4(void* Y, int dt, int64_t idx, const float (&v)[4]) {
     if (dt == BT_F32) {
         st4_nt((float*)Y + idx, __builtin_bit_cast(uint32_t, v[0]), __builtin_bit_cast(uint32_t, v[1]),

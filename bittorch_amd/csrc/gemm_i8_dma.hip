@@ -24,7 +24,8 @@ constexpr int D_NST = 5;   // stages in LDS (60 KiB: what M0's 16-bit byte offse
 // Output stage: row block by row block, addresses as a uniform row base plus a lane offset fixed for the whole tile.  The
 // empty asm statements keep a row's address from being computed ahead of its turn (left alone, the compiler holds all 32
 // row addresses and residual values at once and spills).
-template <int NB, bool FL>
+// RN: rows of any length, so that a lane's four columns start on any element and the last ones may be fewer.
+template <int NB, bool FL, bool RN>
 __device__ __forceinline__ void dma_store_acc(const GemmParams& p, const v4i (&acc)[2 * NB][4], int64_t m0, int g, int64_t ncol,
                                               int rows_left) {
     const uint32_t lane_off = (uint32_t)(4 * g) * (uint32_t)p.N * 4u + (uint32_t)(ncol & (G_BN - 1)) * 4u;
@@ -39,7 +40,12 @@ __device__ __forceinline__ void dma_store_acc(const GemmParams& p, const v4i (&a
                 uint32_t a[4];
 #pragma unroll
                 for (int t = 0; t < 4; t++) a[t] = (uint32_t)times127(acc[mb][t][r] >> field_shift<FL>(t));
-                st4_nt(row + lane_off, a[0], a[1], a[2], a[3]);
+                if constexpr (RN) {
+                    for (int t = 0; t < 4; t++)
+                        if (ncol + t < p.N) ((uint32_t*)(row + lane_off))[t] = a[t];
+                } else {
+                    st4_nt(row + lane_off, a[0], a[1], a[2], a[3]);
+                }
             }
             row += p.N * 4;
         }
@@ -47,7 +53,7 @@ __device__ __forceinline__ void dma_store_acc(const GemmParams& p, const v4i (&a
         __builtin_amdgcn_sched_barrier(0);
     }
 }
-template <int YDT, bool RES, int NB, bool FL>
+template <int YDT, bool RES, int NB, bool FL, bool RN>
 __device__ __forceinline__ void dma_epilogue(const GemmParams& p, const v4i (&acc)[2 * NB][4], int64_t m0, int g, int64_t ncol,
                                              int rows_left, const float* sx_lds, const float (&ws)[4], const float (&bs)[4]) {
     constexpr int ES = (YDT == BT_F32) ? 4 : 2;
@@ -67,7 +73,12 @@ __device__ __forceinline__ void dma_epilogue(const GemmParams& p, const v4i (&ac
             for (int r = 0; r < 4; r++) {
                 asm volatile("" : "+s"(res));
                 const char* src = res + (16 * mb + 4 * g + r < rows_left ? lane_off : 0u);
-                if constexpr (YDT == BT_F32) rv[r] = *(const uint4*)src;
+                if constexpr (RN) {
+                    uint32_t d[4];
+#pragma unroll
+                    for (int t = 0; t < 4; t++) d[t] = load_bits_rt(src, YDT, ncol + t < p.N ? t : 0);
+                    rv[r] = YDT == BT_F32 ? make_uint4(d[0], d[1], d[2], d[3]) : make_uint4(d[0] | d[1] << 16, d[2] | d[3] << 16, 0u, 0u);
+                } else if constexpr (YDT == BT_F32) rv[r] = *(const uint4*)src;
                 else { const uint2 v = *(const uint2*)src; rv[r] = make_uint4(v.x, v.y, 0u, 0u); }
                 res += (16 * mb + r + 1 < rows_left) ? row_bytes : 0;
             }
@@ -87,7 +98,8 @@ __device__ __forceinline__ void dma_epilogue(const GemmParams& p, const v4i (&ac
                         y[t] = sum_in_dtype(round_to_dtype(y[t], YDT), bits_to_f32_rt(bits, YDT), YDT);
                     }
                 }
-                store4(row + lane_off, YDT, 0, y);
+                if constexpr (RN) store4_any<YDT>(row + lane_off, y, (int)(p.N - ncol));
+                else store4(row + lane_off, YDT, 0, y);
             }
             row += row_bytes;
         }
@@ -100,8 +112,9 @@ __device__ __forceinline__ void dma_epilogue(const GemmParams& p, const v4i (&ac
 constexpr int dma_lds_bytes(int NB) { return D_NST * (2 * NB * 1024 + 4096); }
 
 // One tile of 32 NB rows.  TAIL: K is not a multiple of the stage.  The activations past the end of K are some of the same
-// row's and meet weights of zero: the tiled copy is padded with them, raw row-major dwords are masked.
-template <int SRC, int NB, bool TAIL>
+// row's and meet weights of zero: the tiled copy is padded with them, raw row-major dwords are masked.  (Where the activation
+// rows are longer than the weights' K, zeros meet a repetition of the last packed row.)
+template <int SRC, int NB, bool TAIL, bool RN>
 __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int64_t m0, const int tile_n, uint8_t* lds) {
     constexpr int BM = 32 * NB;
     constexpr int A_BYTES = 2 * NB * 1024, STAGE = A_BYTES + 4096;
@@ -132,12 +145,12 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
 #pragma unroll
         for (int r = 0; r < W_LOADS; r++) {
             w_off[r] = (uint32_t)(col_ok ? ncol : 0) + (uint32_t)(4 * g + r) * (uint32_t)p.N;
-            w_tail[r] = (uint32_t)(col_ok ? ncol : 0) + (w_in ? (uint32_t)(4 * g + r) * (uint32_t)p.N : 0u);
+            w_tail[r] = (uint32_t)(col_ok ? ncol : 0) + (uint32_t)min((int64_t)(4 * g + r), p.Kb - 1 - (k_last >> 2)) * (uint32_t)p.N;
         }
     } else if constexpr (SRC == W_ROWS16) {
         const int64_t col = (int64_t)tile_n * G_BN + 64 * wave + 16 * (lane & 3);
         w_off[0] = (uint32_t)(col < p.N ? col : 0) + (uint32_t)(lane >> 2) * (uint32_t)p.N;
-        w_tail[0] = k_last + 4 * (lane >> 2) < p.K ? w_off[0] : (uint32_t)(col < p.N ? col : 0);
+        w_tail[0] = (uint32_t)(col < p.N ? col : 0) + (uint32_t)min((int64_t)(lane >> 2), p.Kb - 1 - (k_last >> 2)) * (uint32_t)p.N;
     } else {
         const int tt = stored_tile16((int)(ncol >> 4), p.tiles16);
         w_off[0] = ((uint32_t)tt * (uint32_t)p.wsteps * 64u + (uint32_t)(16 * g + 4 * (j & 3))) * 4u;
@@ -328,7 +341,7 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
     }
 #pragma unroll
     for (int t = 0; t < 4; t++) {
-        const int64_t n = col_ok ? ncol + t : 0;
+        const int64_t n = !col_ok ? 0 : RN ? min(ncol + t, p.N - 1) : ncol + t;
         ws_bits[t] = load_bits_rt(p.epi.scale, p.epi.scale_dtype, p.epi.scale_bcast ? 0 : n);
         bs_bits[t] = p.epi.bias ? load_bits_rt(p.epi.bias, p.epi.bias_dtype, n) : 0u;
     }
@@ -339,21 +352,21 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
         bs[t] = p.epi.bias ? bits_to_f32_rt(bs_bits[t], p.epi.bias_dtype) : 0.0f;
     }
     if (!col_ok) return;
-    if (p.acc_out) dma_store_acc<NB, SRC == W_FIELDS>(p, acc, m0, g, ncol, (int)rows_left);
+    if (p.acc_out) dma_store_acc<NB, SRC == W_FIELDS, RN>(p, acc, m0, g, ncol, (int)rows_left);
     if (p.y_dtype == BT_BF16) {
-        if (p.epi.residual) dma_epilogue<BT_BF16, true, NB, SRC == W_FIELDS>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
-        else dma_epilogue<BT_BF16, false, NB, SRC == W_FIELDS>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
+        if (p.epi.residual) dma_epilogue<BT_BF16, true, NB, SRC == W_FIELDS, RN>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
+        else dma_epilogue<BT_BF16, false, NB, SRC == W_FIELDS, RN>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
     } else if (p.y_dtype == BT_F16) {
-        if (p.epi.residual) dma_epilogue<BT_F16, true, NB, SRC == W_FIELDS>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
-        else dma_epilogue<BT_F16, false, NB, SRC == W_FIELDS>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
+        if (p.epi.residual) dma_epilogue<BT_F16, true, NB, SRC == W_FIELDS, RN>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
+        else dma_epilogue<BT_F16, false, NB, SRC == W_FIELDS, RN>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
     } else {
-        if (p.epi.residual) dma_epilogue<BT_F32, true, NB, SRC == W_FIELDS>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
-        else dma_epilogue<BT_F32, false, NB, SRC == W_FIELDS>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
+        if (p.epi.residual) dma_epilogue<BT_F32, true, NB, SRC == W_FIELDS, RN>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
+        else dma_epilogue<BT_F32, false, NB, SRC == W_FIELDS, RN>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
     }
 }
 
 // NB: tiles of 32 NB rows.  NF > 0: the last p.fine_from .. of an XCD's tiles are computed in tiles of 32 NF rows.
-template <int SRC, int NB, int NF, bool TAIL>
+template <int SRC, int NB, int NF, bool TAIL, bool RN>
 __global__ __launch_bounds__(256, NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_i8_dma_kernel(GemmParams p) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[dma_lds_bytes(NB)];
     // XCD-aware tile order, as in gemm_i8_kernel
@@ -374,11 +387,11 @@ __global__ __launch_bounds__(256, NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_i8_dm
     if constexpr (NF > 0) {
         if (fine) {
             const int64_t mf = m0 + (int64_t)(f % parts) * (32 * NF);
-            if (mf < p.M) gemm_i8_dma_tile<SRC, NF, TAIL>(p, mf, (int)tn, lds);
+            if (mf < p.M) gemm_i8_dma_tile<SRC, NF, TAIL, RN>(p, mf, (int)tn, lds);
             return;
         }
     }
-    gemm_i8_dma_tile<SRC, NB, TAIL>(p, m0, (int)tn, lds);
+    gemm_i8_dma_tile<SRC, NB, TAIL, RN>(p, m0, (int)tn, lds);
 }
 
 // Rows of the tiles in units of 32 (4, 2 or 1), or 0 where gemm_i8_kernel is the better one: tiled weights in whole stages
@@ -392,7 +405,7 @@ __global__ __launch_bounds__(256, NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_i8_dm
 static int gemm_i8_dma_plan(int64_t M, int64_t N, int64_t K, bool tiled, double* us) {
     const int64_t C = gemm_compute_units(), tn = ceil_div(N, G_BN);
     const int64_t t4 = ceil_div(M, 128) * tn, t2 = ceil_div(M, 64) * tn, t1 = ceil_div(M, 32) * tn;
-    if (tiled && K % 128 == 0 && t4 <= C) return 0;
+    if (tiled && K % 128 == 0 && N % 4 == 0 && t4 <= C) return 0;
     const bool whole = gemm_whole_tiles();
     if (t1 <= C && !whole) { *us = 5.2 + 0.0035 * (double)K; return 1; }
     if (t2 <= C && !whole) { *us = 5.2 + 0.0045 * (double)K; return 2; }
@@ -414,7 +427,7 @@ double gemm_i8_cost(int64_t M, int64_t N, int64_t K, bool tiled, bool operand_or
     return gemm_split(M, N, tiled && K % 128 == 0).rounds * (8.6 + 0.0044 * (double)K);
 }
 
-template <int SRC, int NB, bool TAIL>
+template <int SRC, int NB, bool TAIL, bool RN = false>
 static int launch_gemm_i8_dma_src(GemmParams p, hipStream_t st) {
     p.tile_n0 = 0;
     p.tiles_n = (int)ceil_div(p.N, G_BN);
@@ -433,17 +446,18 @@ static int launch_gemm_i8_dma_src(GemmParams p, hipStream_t st) {
             const int rem = p.per_xcd % (int)(2 * gemm_compute_units() / 8);
             p.fine_from = p.per_xcd - rem;
             const dim3 grid((unsigned)(8 * (p.fine_from + parts * rem)));
-            if (parts == 2) hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, 4, 2, TAIL>), grid, block, 0, st, p);
-            else hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, 4, 1, TAIL>), grid, block, 0, st, p);
+            if (parts == 2) hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, 4, 2, TAIL, RN>), grid, block, 0, st, p);
+            else hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, 4, 1, TAIL, RN>), grid, block, 0, st, p);
             return check_launch("bt_ternary_gemm_i8");
         }
     }
-    hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, NB, 0, TAIL>), dim3((unsigned)(8 * p.per_xcd)), block, 0, st, p);
+    hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, NB, 0, TAIL, RN>), dim3((unsigned)(8 * p.per_xcd)), block, 0, st, p);
     return check_launch("bt_ternary_gemm_i8");
 }
 template <int NB>
 static int launch_gemm_i8_dma_rows(const GemmParams& p, int src, hipStream_t st) {
     const bool tail = p.K % D_BK != 0;
+    if (src == W_TILES && p.N % 4 != 0) return launch_gemm_i8_dma_src<W_TILES, NB, true, true>(p, st);
     if (src == W_FIELDS) return launch_gemm_i8_dma_src<W_FIELDS, NB, false>(p, st);
     if (src == W_TILES) return tail ? launch_gemm_i8_dma_src<W_TILES, NB, true>(p, st) : launch_gemm_i8_dma_src<W_TILES, NB, false>(p, st);
     if (src == W_ROWS16) return tail ? launch_gemm_i8_dma_src<W_ROWS16, NB, true>(p, st) : launch_gemm_i8_dma_src<W_ROWS16, NB, false>(p, st);

@@ -194,28 +194,46 @@ __global__ __launch_bounds__(256) void unpack_dequant_kernel(const uint8_t* __re
 }
 
 // ---- decode-tiled copy of the packed weights (W_LAYOUT_TILED) -----------------------------------
-// One thread per dword of the tiled copy: lane = 16 g + j of step s of tile t collects the bytes of
-// rows 16 s + 4 g .. + 3 of column 16 t + j.  The sixteen threads of a g read 16 contiguous bytes per row.
+// Dword 16 g + j of step s of tile t holds the bytes of rows 16 s + 4 g .. + 3 of column 16 t + j.
 // pairs (N % 32 == 0): tile 2P of the copy is tile P of the matrix, tile 2P + 1 is tile N/32 + P, so that
 // column h of the first half (gate) and column h of the second half (up) land in one workgroup.
-__device__ __forceinline__ int64_t source_tile(int64_t t, int64_t tiles, int pairs) {
-    return pairs ? ((t & 1) ? (tiles >> 1) + (t >> 1) : (t >> 1)) : t;
-}
-
-__global__ __launch_bounds__(256) void retile_kernel(const uint8_t* __restrict__ W_T, uint32_t* __restrict__ T,
-                                                     int64_t N, int64_t Kb, int64_t S, int64_t total, int pairs) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= total) return;
-    const int lane = (int)(i & 63);
-    const int64_t s = (i >> 6) % S, t = source_tile((i >> 6) / S, total / (64 * S), pairs);
-    const int64_t n = 16 * t + (lane & 15), kb0 = 16 * s + 4 * (lane >> 4);
-    uint32_t d = 0;
-    if (n < N) {
+// A workgroup re-tiles 16 packed rows (a step) of 256 columns: a thread reads 16 bytes of one row, wherever they start, the
+// block passes through LDS, and a thread writes four dwords (columns j .. j + 3 of one row group).  Bound by its bytes, read and
+// written once; a thread per dword with four byte loads of its own took 24 us for 14272 x 6606, this 14 (3.3 TB/s).
+__global__ __launch_bounds__(256) void retile_kernel(const uint8_t* __restrict__ W_T, uint4* __restrict__ T, int64_t N, int64_t Kb,
+                                                     int64_t S, int64_t tiles, int pairs, uint32_t steps) {
+    constexpr int PITCH = 256 + 16;  // (rows 4 g + r of a read lie in different banks)
+    __shared__ __attribute__((aligned(16))) uint8_t block[16 * PITCH];
+    const int64_t s = blockIdx.x % steps;
+    const int64_t n0 = (int64_t)(blockIdx.x / steps) * 256;
+    {
+        const int r = threadIdx.x >> 4, c = 16 * (threadIdx.x & 15);
+        const int64_t kb = 16 * s + r, n = n0 + c;
+        uint32_t d[4] = {0u, 0u, 0u, 0u};
+        if (kb < Kb && n < N) {
+            const uint8_t* src = W_T + kb * N + n;
+            if (n + 16 <= N) {
+                const u32x4_a1 v = *(const u32x4_a1*)src;
 #pragma unroll
-        for (int r = 0; r < 4; r++)
-            if (kb0 + r < Kb) d |= (uint32_t)W_T[(kb0 + r) * N + n] << (8 * r);
+                for (int e = 0; e < 4; e++) d[e] = v[e];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 16; e++)
+                    if (n + e < N) d[e >> 2] |= (uint32_t)src[e] << (8 * (e & 3));
+            }
+        }
+        *(uint4*)(block + r * PITCH + c) = make_uint4(d[0], d[1], d[2], d[3]);
     }
-    T[i] = d;
+    __syncthreads();
+    const int tile = threadIdx.x >> 4, g = (threadIdx.x >> 2) & 3, j = 4 * (threadIdx.x & 3);
+    const int64_t t = (n0 >> 4) + tile;
+    if (t >= tiles) return;
+    uint32_t row[4], out[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) row[r] = *(const uint32_t*)(block + (4 * g + r) * PITCH + 16 * tile + j);
+    transpose4x4_bytes(row[0], row[1], row[2], row[3], out);
+    const int64_t half = tiles >> 1, to = !pairs ? t : t < half ? 2 * t : 2 * (t - half) + 1;
+    T[(to * S + s) * 16 + 4 * g + (j >> 2)] = make_uint4(out[0], out[1], out[2], out[3]);
 }
 
 // the inverse: one thread per byte of W_T
@@ -271,9 +289,8 @@ int launch_retile_fields(const uint8_t* W_tiled, int64_t N, int64_t K, uint8_t* 
 int launch_retile(const uint8_t* W_T, int64_t N, int64_t K, int pairs, void* T, bool inverse, uint8_t* W_out, hipStream_t st) {
     const int64_t Kb = ceil_div(K, 4), S = ceil_div(Kb, 16);
     if (!inverse) {
-        const int64_t total = ceil_div(N, 16) * S * 64;
-        hipLaunchKernelGGL(retile_kernel, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, st, W_T, (uint32_t*)T, N, Kb, S,
-                           total, pairs);
+        hipLaunchKernelGGL(retile_kernel, dim3((unsigned)(S * ceil_div(N, 256))), dim3(256), 0, st, W_T, (uint4*)T, N, Kb, S,
+                           ceil_div(N, 16), pairs, (uint32_t)S);
     } else {
         hipLaunchKernelGGL(untile_kernel, dim3((unsigned)ceil_div(N * Kb, 256)), dim3(256), 0, st, (const uint32_t*)T, W_out,
                            N, Kb, S, pairs);
@@ -289,7 +306,6 @@ namespace bt {
 // its bytes (2 read and 4 written per entry); the scale and the widening as torch operations read and write the 16-bit
 // gradient once more each.  11008 x 4096 fp16: 43 us = 6.3 TB/s, the two operations 80.  Four neighbouring entries a lane, so that a wave's stores are whole
 // lines, and two such runs per thread; rows begin at any entry of any length, hence the small alignments.
-typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
 typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 template <int DT>
 __global__ __launch_bounds__(256) void scale_widen_kernel(const uint16_t* __restrict__ G, const float* __restrict__ scale,

@@ -56,7 +56,8 @@ struct StreamParams {
     int per_xcd;          // tiles per XCD (grid = 8 * per_xcd)
     int tiles16;          // LD_T*: 16-column tiles of the decode-tiled weights (< 0: stored_tile16)
     int M;                // 1..16: rows of a 16-row block (of the last one when the launch covers several)
-    int x_vec_ok;         // activation rows may be read with 16-byte loads
+    int x_vec_ok;         // activation rows are read with 16-byte loads: they hold at least one group of 16 bytes
+    int x_ragged;         // rows are no whole number of such groups: the last one is shifted into place (shift_group)
     int64_t B;            // rows of the whole call: grid.y = ceil(B / 16) blocks of 16 rows, all in one launch
     const float* s_x;     // MODE_I8: per-row activation scales [M]
     void* Y;              // [M, N] of y_dtype
@@ -115,18 +116,24 @@ __device__ __forceinline__ uint32_t add_bits(uint32_t a, uint32_t b) {
 }
 
 // 16 bytes of activations of row i starting at element k, in natural k order.
-// XV: rows are 16-byte aligned and K is a multiple of the 16-byte group, so a group that
-// starts below K lies wholly inside its row; the load is unconditional on a clamped address
-// (xrow = element offset of row min(i, M-1)) and the caller zeroes groups at k >= K when it
-// consumes them: a load under a per-lane predicate becomes a branch with a wait behind it,
-// which serialises the stream.  !XV: element-wise gather (unaligned or ragged rows), zero filled.
+// XV: the row holds at least one group of 16 bytes.  The load is unconditional, on an address clamped to the row's last
+// group, and wherever a row starts (xrow = element offset of row min(i, M-1)); the caller zeroes groups at k >= K, and shifts
+// the one that crosses the row's end into place, when it consumes them: a load under a per-lane predicate becomes a branch
+// with a wait behind it, which serialises the stream (a gather by element took 152 us for 37 rows of 10447 bf16 values times
+// 11152 columns, 67 this way).  !XV: element-wise gather of shorter rows, zero filled.
+template <int MODE>
+__device__ __forceinline__ uint4 load_x16_any(const void* src) {
+    typedef typename std::conditional<MODE == MODE_I8, u32x4_a1, u32x4_a2>::type vec;
+    const vec v = *(const vec*)src;
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
 template <int MODE, bool XV>
 __device__ __forceinline__ uint4 load_x16(const StreamParams& p, uint32_t xrow, int i, int k) {
     constexpr int GE = (MODE == MODE_I8) ? 16 : 8;
     constexpr int ES = (MODE == MODE_I8) ? 1 : 2;
     if constexpr (XV) {
         const uint32_t kc = (uint32_t)min(k, (int)p.K - GE);
-        return *(const uint4*)((const uint8_t*)p.X + (xrow + kc) * ES);
+        return load_x16_any<MODE>((const uint8_t*)p.X + (xrow + kc) * ES);
     } else {
         uint32_t d[4] = {0u, 0u, 0u, 0u};
         if (i < p.M && k < p.K) {
@@ -143,7 +150,6 @@ __device__ __forceinline__ uint4 load_x16(const StreamParams& p, uint32_t xrow, 
         return make_uint4(d[0], d[1], d[2], d[3]);
     }
 }
-
 __device__ __forceinline__ uint4 zero_unless(uint4 v, bool ok) {
     v.x = ok ? v.x : 0u; v.y = ok ? v.y : 0u; v.z = ok ? v.z : 0u; v.w = ok ? v.w : 0u;
     return v;
@@ -267,7 +273,7 @@ __global__ __launch_bounds__(WAVES * 64) void stream_kernel(StreamParams p_in) {
         for (int u = 0; u < XC_MAX; u++) {
             if (u * 64 < nchunks) {  // uniform
                 const int k = s_begin * 64 + (lane + 64 * u) * EPC;
-                xr[u] = *(const uint4*)((const uint8_t*)p.X + (uint32_t)min(k, (int)p.K - EPC) * ES);
+                xr[u] = load_x16_any<MODE>((const uint8_t*)p.X + (uint32_t)min(k, (int)p.K - EPC) * ES);
                 if constexpr (PRO != 0) {  // second operand; RMSNorm without a weight reads X again (unused)
                     const uint8_t* bsrc = p.pro_b ? (const uint8_t*)p.pro_b : (const uint8_t*)p.X;
                     xb[u] = *(const uint4*)(bsrc + (uint32_t)min(k, (int)p.K - EPC) * ES);
@@ -378,6 +384,7 @@ __global__ __launch_bounds__(WAVES * 64) void stream_kernel(StreamParams p_in) {
                 // parked in the order the MFMA wants (each 16-byte chunk is one operand
                 // fragment), so that the steps below read their A operand ready-made
                 uint4 v = zero_unless(xr[u], k < (int)p.K);
+                if (p.x_ragged) v = shift_group(xr[u], max(k + EPC - (int)p.K, 0) * ES);  // (uniform)
                 if constexpr (MODE != MODE_I8 && PRO != 0) {
                     {
                         constexpr int DT = (MODE == MODE_F16) ? BT_F16 : BT_BF16;
@@ -446,6 +453,13 @@ __global__ __launch_bounds__(WAVES * 64) void stream_kernel(StreamParams p_in) {
                 for (int f = 0; f < PF; f++)
 #pragma unroll
                     for (int h = 0; h < XN; h++) xa[f][h] = load_x16<MODE, true>(p, xrow, j, k0 + f * 64 + 8 * h);
+                if (p.x_ragged && base + PF >= nsteps) {  // (uniform: the batch with the row's end)
+#pragma unroll
+                    for (int f = 0; f < PF; f++)
+#pragma unroll
+                        for (int h = 0; h < XN; h++)
+                            xa[f][h] = shift_group(xa[f][h], max(k0 + f * 64 + 8 * h + 16 / ES - (int)p.K, 0) * ES);
+                }
             } else {
 #pragma unroll
                 for (int f = 0; f < PF; f++)
@@ -714,7 +728,7 @@ static void launch_stream_w(const StreamParams& p, int waves, bool xlds, dim3 gr
     launch_stream_k<MODE, LD, 4>(p, xlds, grid, lds, st);
 }
 
-// x slice in LDS (the M = 1 variant): one row, aligned, at most XC_MAX 16-byte chunks per lane and
+// x slice in LDS (the M = 1 variant): one row, at most XC_MAX 16-byte chunks per lane and
 // wave, and within the default 64 KiB of dynamic LDS
 static bool xlds_ok(int es, int M, bool x_vec_ok, const StreamPlan& pl, int64_t K) {
     const int64_t tile_n = ld_columns(pl.ld);
@@ -788,10 +802,12 @@ static int launch_stream_mode(StreamParams p, const StreamPlan& pl, hipStream_t 
 // q_layout: MODE_I8 only (Q_OPERAND_ORDER needs K % 16 == 0 and 16-byte aligned rows)
 // pro_op / pro_b / pro_eps: activation prologue (PRO_*), only where stream_prologue_fusable() said yes
 // epi_op: EPI_SWIGLU_PAIRS makes Y [B, N/2] (tiled weights in gate/up pair order, 16-bit modes)
+// Kw: the weights' K where the activation rows are longer (zeros behind it; 0: K)
 int launch_stream(int mode, const void* X, int x_elem_size, const float* s_x, const uint8_t* W_T, int w_layout,
                   const Epilogue& epi, void* Y, int y_dtype, int32_t* acc_out, int64_t B, int64_t N,
-                  int64_t K, int planes, int q_layout, int pro_op, const void* pro_b, float pro_eps, int epi_op, hipStream_t st) {
-    const int64_t Kb = ceil_div(K, 4);
+                  int64_t K, int planes, int q_layout, int pro_op, const void* pro_b, float pro_eps, int epi_op, hipStream_t st,
+                  int64_t Kw) {
+    const int64_t Kb = ceil_div(Kw ? Kw : K, 4);
     const int64_t Kx = (planes == 3) ? 3 * ceil_div(K, 64) * 64 : K;
     const StreamPlan pl = stream_plan(mode, B, N, Kb, w_layout, epi_op == EPI_SWIGLU_PAIRS ? 2 : 1);
     const int64_t Ny = (epi_op == EPI_SWIGLU_PAIRS) ? N / 2 : N;  // columns of Y
@@ -805,7 +821,7 @@ int launch_stream(int mode, const void* X, int x_elem_size, const float* s_x, co
             const int rc = launch_stream(mode, (const uint8_t*)X + r0 * Kx * x_elem_size, x_elem_size, s_x ? s_x + r0 : nullptr, W_T,
                                          w_layout, e, (uint8_t*)Y + r0 * Ny * y_size, y_dtype, acc_out ? acc_out + r0 * N : nullptr,
                                          (B - r0 < max_rows) ? B - r0 : max_rows, N, K, planes, q_layout, pro_op, pro_b, pro_eps,
-                                         epi_op, st);
+                                         epi_op, st, Kw);
             if (rc) return rc;
         }
         return BT_OK;
@@ -826,8 +842,8 @@ int launch_stream(int mode, const void* X, int x_elem_size, const float* s_x, co
     p.B = B;
     p.M = (int)((B < 16) ? B : 16);
     p.y_dtype = y_dtype;
-    // (a row is a multiple of 16 bytes, so every 16-row block starts as aligned as the first)
-    p.x_vec_ok = (((uintptr_t)p.X) % 16 == 0) && ((Kx * x_elem_size) % 16 == 0);
+    p.x_vec_ok = Kx * x_elem_size >= 16;
+    p.x_ragged = p.x_vec_ok && (Kx * x_elem_size) % 16 != 0;
     if (mode == MODE_I8) return launch_stream_mode<MODE_I8>(p, pl, st);
     if (mode == MODE_F16) return launch_stream_mode<MODE_F16>(p, pl, st);
     return launch_stream_mode<MODE_BF16>(p, pl, st);

@@ -117,8 +117,10 @@ int bt_ternary_linear_forward(const void* X, int x_dtype, const int8_t* W_tern, 
  *   products beyond), into planes in the workspace, each zero-padded to a multiple of 64 values.
  *   Unaligned operands, a workspace missing where the planes need one and BITTORCH_KERNEL=generic run
  *   a generic kernel that accumulates in the reference's k order.
- *   workspace: at least bt_packed_forward_workspace_bytes(B,N,K,x_dtype) bytes (6*B*Kp rounded up to
- *   256, Kp = K rounded up to 64, for fp32 on the streaming kernel; 0 otherwise: may be NULL).
+ *   workspace: at least bt_packed_forward_workspace_bytes(B,N,K,x_dtype) bytes (0: may be NULL).  It holds the
+ *   planes (6*B*Kp, Kp = K rounded up to 64), more than 16 rows of 16-bit activations padded to whole groups of 8
+ *   values (K % 8 != 0), and a decode-tiled copy of packed rows that start on any byte (N % 4 != 0; for the
+ *   tiled GEMM, and for the streaming kernel where that pays).  Without it the call still succeeds, on slower kernels.
  */
 size_t bt_packed_forward_workspace_bytes(int64_t B, int64_t N, int64_t K, int x_dtype);
 int bt_ternary_linear_packed_forward(const void* X, int x_dtype, const uint8_t* W_T,
@@ -257,7 +259,7 @@ int bt_ternary_linear_packed_forward_fused(const void* X, int64_t ld_x, int x_dt
  *   bt_ternary_linear_tiled_forward: bt_ternary_linear_packed_forward_fused on the tiled copy, with
  *     pro_op = BT_PRO_NONE allowed (then ld_x must equal K); the weights are streamed once per 16
  *     rows of X, so it is meant for decode shapes.  workspace: without a prologue and with epi_op
- *     BT_EPI_NONE or BT_EPI_NATURAL_FROM_PAIRS, bt_packed_forward_workspace_bytes(...) bytes do.
+ *     BT_EPI_NONE or BT_EPI_NATURAL_FROM_PAIRS, bt_tiled_forward_workspace_bytes(...) bytes do.
  *     Results equal those of the row-major entry points bit for bit up to 32 rows and in the tiled GEMMs; a larger
  *     batch on the streaming kernel may split K among its waves differently on the two layouts, and then adds the
  *     fp32 partial sums in another order.
@@ -279,6 +281,7 @@ enum { BT_EPI_NONE = 0, BT_EPI_SWIGLU_PAIRS = 1, BT_EPI_NATURAL_FROM_PAIRS = 2 }
 size_t bt_tiled_weights_bytes(int64_t N, int64_t K);
 int bt_retile_weights(const uint8_t* W_T, int64_t N, int64_t K, int order, uint8_t* W_tiled, void* stream);
 int bt_untile_weights(const uint8_t* W_tiled, int64_t N, int64_t K, int order, uint8_t* W_T, void* stream);
+size_t bt_tiled_forward_workspace_bytes(int64_t B, int64_t N, int64_t K, int x_dtype);
 int bt_ternary_linear_tiled_forward(const void* X, int64_t ld_x, int x_dtype, int pro_op, const void* pro_b,
                                     int64_t ld_b, float eps, const uint8_t* W_tiled, const void* scale,
                                     int scale_dtype, int64_t scale_len, const void* bias, int bias_dtype,
@@ -368,7 +371,9 @@ int bt_ternary_gemm_i8_grouped(const int8_t* const* Q_tab, int q_layout, const f
  * (bittorch_bindings.cpp:65-87, ternary_gemm_tensor_core.cu:663-727) for
  * version == 2; version == 1 (the reference's float-compute validation kernel,
  * :120-271) is served by bt_ternary_linear_packed_forward.
- *   workspace: at least bt_tensor_core_workspace_bytes(B,N,K) bytes; holds Q and s_x.
+ *   workspace: at least bt_tensor_core_workspace_bytes(B,N,K) bytes; holds Q (rows of K rounded up to 16 bytes), s_x and,
+ *   where that pays, a decode-tiled copy of packed rows that start on any byte (N % 4 != 0).  B*K bytes and 4*B
+ *   bytes, each rounded up to 256, are enough for the same results at a lower speed.
  */
 size_t bt_tensor_core_workspace_bytes(int64_t B, int64_t N, int64_t K);
 int bt_ternary_linear_tensor_core_forward(const void* X, int x_dtype, const uint8_t* W_T,
