@@ -751,6 +751,26 @@ def linear_grad_weight(dY: Tensor, X: Tensor, scale: Tensor, want_bias: bool = F
     return dW, dB
 
 
+def linear_grad_weight_16(dY: Tensor, X: Tensor, scale: Tensor, out_dtype: torch.dtype) -> Tensor:
+    """Weight gradient of a 16-bit layer, ``scale[:, None] * (dY.T @ X)`` ``[N, K]`` in their dtype or fp32, with the roundings
+    of the unfused operations (``dY`` ``[M, N]``, ``X`` ``[M, K]``, N and K multiples of 8)."""
+    _check(dY.dim() == 2 and X.dim() == 2 and dY.shape[0] == X.shape[0] and dY.numel() > 0 and X.numel() > 0,
+           "dY [M, N] and X [M, K] must be 2D with the same rows")
+    _check(dY.dtype == X.dtype and dY.dtype in (torch.float16, torch.bfloat16), "dY and X must be fp16 or bf16")
+    _check(out_dtype in (dY.dtype, torch.float32), "the gradient is of the operands' dtype or fp32")
+    _check(scale.dtype in _DT and scale.numel() in (dY.shape[1], 1), "scale must be fp32 or 16-bit, [N] or one entry")
+    _check(_all_cuda(dY, X, scale), "All tensors must be CUDA")
+    dY, X, scale = dY.contiguous(), X.contiguous(), scale.reshape(-1).contiguous()
+    (M, N), K = dY.shape, X.shape[1]
+    out = torch.empty((N, K), dtype=out_dtype, device=dY.device)
+    with torch.cuda.device(dY.device):
+        ws = _workspace(_L.bt_linear_grad_weight_16_workspace_bytes(M, N, K), dY.device)
+        _status(_L.bt_linear_grad_weight_16(dY.data_ptr(), X.data_ptr(), _DT[dY.dtype], scale.data_ptr(), _DT[scale.dtype],
+                                            scale.numel(), out.data_ptr(), _DT[out_dtype], M, N, K, _ptr(ws), 0 if ws is None else ws.numel(),
+                                            _stream(dY)))
+    return out
+
+
 def scale_grad_weight(G: Tensor, scale: Tensor) -> Tensor:
     """``(G * scale[:, None].to(G.dtype)).float()`` in one pass (``G`` ``[N, K]`` fp16 or bf16, ``scale`` ``[N]`` or one entry)."""
     _check(G.dim() == 2 and G.dtype in (torch.float16, torch.bfloat16) and G.numel() > 0, "G must be 2D fp16 or bf16")

@@ -50,6 +50,8 @@ SIGNATURES = {
     "bt_ternary_linear_grad_input": (_int, [_vp, _vp, _vp, _i64, _vp, _i64, _i64, _i64, _vp]),
     "bt_linear_grad_weight_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "bt_linear_grad_weight": (_int, [_vp, _vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _vp, _sz, _vp]),
+    "bt_linear_grad_weight_16_workspace_bytes": (_sz, [_i64, _i64, _i64]),
+    "bt_linear_grad_weight_16": (_int, [_vp, _vp, _int, _vp, _int, _i64, _vp, _int, _i64, _i64, _i64, _vp, _sz, _vp]),
     "bt_scale_grad_weight": (_int, [_vp, _int, _vp, _i64, _vp, _i64, _i64, _vp]),
     "bt_pack_ternary_i8": (_int, [_vp, _i64, _i64, _vp, _vp]),
     "bt_ternary_linear_packed_forward_res": (_int, [_vp, _int, _vp, _vp, _int, _i64, _vp, _int, _vp, _vp,

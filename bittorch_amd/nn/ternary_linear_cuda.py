@@ -4,9 +4,9 @@ API mirror of ``bittorch/nn/ternary_linear_cuda.py:23-228``.  Forward: one fused
 HIP kernel quantizes and packs the master weights, a second one multiplies the
 activations with the packed weights (fp32 accumulation).  Backward is the
 straight-through estimator, as in the reference (``:73-111``): fp32 layers run on
-the library's gradient kernels, which read the packed bytes; the other dtypes use torch
-matmuls on dense effective weights rebuilt from the packed bytes instead of being
-kept alive from the forward.
+the library's gradient kernels, which read the packed bytes; the 16-bit dtypes have a kernel
+for the weight gradient and use a torch matmul for the input's, on dense effective weights
+rebuilt from the packed bytes instead of being kept alive from the forward.
 """
 
 from __future__ import annotations
@@ -59,6 +59,20 @@ def _scale_to_master(g: Tensor, scale: Tensor, master_dtype: torch.dtype) -> Ten
         from .. import _C
         return _C.scale_grad_weight(g, scale)
     return g * scale.reshape(-1, 1).to(g.dtype)
+
+
+def _w16_kernel_serves(g2: Tensor, x2: Tensor, scale: Tensor) -> bool:
+    """Whether the weight gradient is the library's 16-bit kernel: 16-byte rows of both operands as they lie, no graph of the
+    backward itself and no batched gradient wanted.  Of fewer than 2^16 weights the product takes no longer than its launch
+    (256 x 256: 15 us a call against 35 for the two torch operations; the torch product serves other strides too)."""
+    if torch.is_grad_enabled() or _batched(g2) or _batched(x2) or _generic_forced() or g2.numel() == 0:
+        return False
+    if not (g2.is_cuda and g2.dtype == x2.dtype and g2.dtype in (torch.float16, torch.bfloat16)
+            and scale.dtype in (torch.float32, torch.float16, torch.bfloat16)):
+        return False
+    n, k = g2.shape[1], x2.shape[1]
+    return (n % 8 == 0 and k % 8 == 0 and 2 ** 16 <= n * k < 2 ** 40 and n < 2 ** 24 and k < 2 ** 24 and g2.shape[0] < 2 ** 40 // max(n, k)
+            and g2.is_contiguous() and x2.is_contiguous() and g2.data_ptr() % 16 == 0 and x2.data_ptr() % 16 == 0)
 
 
 class TernaryLinearCUDAFunction(torch.autograd.Function):
@@ -141,7 +155,10 @@ class TernaryLinearCUDAFunction(torch.autograd.Function):
             grad_x = (g2 @ w_eff.to(g2.dtype)).reshape(x.shape)
         if ctx.needs_input_grad[1]:
             # d(w_eff)/d(weight) = scale under the straight-through estimator
-            grad_w = _scale_to_master(g2.t() @ x2, scale, ctx.master_dtype)
+            if _w16_kernel_serves(g2, x2, scale):
+                grad_w = _C.linear_grad_weight_16(g2, x2, scale, torch.float32 if ctx.master_dtype == torch.float32 else g2.dtype)
+            else:
+                grad_w = _scale_to_master(g2.t() @ x2, scale, ctx.master_dtype)
         if want_bias:
             grad_b = g2.sum(dim=0)
         return grad_x, grad_w, grad_b, None, None, None

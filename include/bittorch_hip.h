@@ -49,8 +49,8 @@ typedef enum {
  * At present bt_ternary_linear_tensor_core_forward uses one (the int8 activations
  * and their row scales), bt_ternary_linear_packed_forward uses one for small
  * batches of fp32 activations (three bf16 planes), its fused and tiled forms also
- * one for a prologue that runs as its own kernel, and bt_linear_grad_weight one for
- * partial sums; bt_ternary_gemm_i8 keeps the argument so that a kernel that needs
+ * one for a prologue that runs as its own kernel, and bt_linear_grad_weight and
+ * bt_linear_grad_weight_16 one for partial sums; bt_ternary_gemm_i8 keeps the argument so that a kernel that needs
  * scratch can be introduced without an ABI change.
  */
 /* ABI version of the loaded library (BT_ABI_VERSION at build time). */
@@ -429,6 +429,13 @@ int bt_ternary_linear_grad_input(const float* dY, const uint8_t* W_T, const floa
 size_t bt_linear_grad_weight_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int bt_linear_grad_weight(const float* dY, const float* X, const float* scale, int64_t scale_len, float* dW, float* dBias,
                           int64_t M, int64_t N, int64_t K, void* workspace, size_t workspace_bytes, void* stream);
+
+/* The weight gradient of a 16-bit layer, dW [N,K] = scale[n] * sum_m dY[m,n] X[m,k]: dY and X of one 16-bit dtype, dW of that
+ * dtype or fp32; N and K multiples of 8, dY, X and dW 16-byte aligned; workspace as described above.  Sums are fp32; each is rounded to the 16-bit dtype,
+ * multiplied by the scale rounded to it (scale_len: N, or 1) and rounded again. */
+size_t bt_linear_grad_weight_16_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int bt_linear_grad_weight_16(const void* dY, const void* X, int dtype, const void* scale, int scale_dtype, int64_t scale_len,
+                             void* dW, int out_dtype, int64_t M, int64_t N, int64_t K, void* workspace, size_t workspace_bytes, void* stream);
 
 /* The weight gradient of a 16-bit product (dY^T X, [N,K] fp16 or bf16) as fp32 masters receive it: each entry times its
  * row's scale (rounded to the dtype; scale_len: N, or 1), rounded to the dtype, then widened. */
