@@ -12,6 +12,7 @@ Importing this module raises ``ImportError`` when the library is not built.
 
 from __future__ import annotations
 
+import contextlib
 import os
 
 from typing import Optional, Tuple
@@ -38,8 +39,18 @@ def _status(rc: int) -> None:
         raise RuntimeError(_lib.last_error() or f"libbittorch_hip call failed ({rc})")
 
 
+# A call's host time is most of a small launch's (one fp16 row through 4096 x 4096: 4.6 us on the GPU, 14 us a call).  The public
+# forms of the next two build a stream object and enter a context, 3 us a call: the handle and the device are asked for instead.
+_HERE = contextlib.nullcontext()
+
+
 def _stream(t: Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+def _on(t: Tensor):
+    """Context in which ``t``'s device is the current one."""
+    return _HERE if torch._C._cuda_getDevice() == t.get_device() else torch.cuda.device(t.device)
 
 
 def _ptr(t: Optional[Tensor]) -> Optional[int]:
@@ -61,7 +72,19 @@ def _workspace(nbytes: int, device) -> Optional[Tensor]:
 
 
 def _all_cuda(*ts: Optional[Tensor]) -> bool:
-    return all(t is None or t.is_cuda for t in ts)
+    for t in ts:
+        if t is not None and not t.is_cuda:
+            return False
+    return True
+
+
+def _flat_rows(X: Tensor, K: int) -> Tensor:
+    """``X`` as contiguous ``[rows, K]``; most calls' already are."""
+    return X if X.dim() == 2 and X.stride(0) == K and X.is_contiguous() else X.contiguous().reshape(-1, K)
+
+
+def _unflat(y: Tensor, X: Tensor, N: int) -> Tensor:
+    return y if X.dim() == 2 else y.reshape(*X.shape[:-1], N)
 
 
 def _prep_vec(v: Tensor, x: Tensor) -> Tensor:
@@ -90,7 +113,7 @@ def pack_ternary_int8(W_tern: Tensor) -> Tensor:
     W_tern = W_tern.contiguous()
     N, K = W_tern.shape
     packed = torch.empty(((K + 3) // 4, N), dtype=torch.uint8, device=W_tern.device)
-    with torch.cuda.device(W_tern.device):
+    with _on(W_tern):
         _status(_L.bt_pack_ternary_i8(W_tern.data_ptr(), N, K, packed.data_ptr(), _stream(W_tern)))
     return packed
 
@@ -121,17 +144,17 @@ def ternary_linear_forward(X: Tensor, W_tern: Tensor, scale: Tensor,
         # the weights are packed on the device (one read of N*K bytes) and the call joins the
         # packed matrix-core path; entries are taken as ternary (sign of anything non-zero)
         return ternary_linear_packed_forward(X, pack_ternary_int8(W_tern), scale, bias, K)
-    x2 = X.contiguous().reshape(-1, K)
+    x2 = _flat_rows(X, K)
     scale = _prep_vec(scale, x2)
     bias = None if bias is None else _prep_vec(bias, x2)
     B = x2.shape[0]
     y = torch.empty((B, N), dtype=X.dtype, device=X.device)
-    with torch.cuda.device(X.device):
+    with _on(X):
         _status(_L.bt_ternary_linear_forward(
             x2.data_ptr(), _dt(x2, "X"), W_tern.data_ptr(), scale.data_ptr(), _dt(scale, "scale"),
             scale.numel(), _ptr(bias), 0 if bias is None else _dt(bias, "bias"), y.data_ptr(),
             B, N, K, _stream(X)))
-    return y.reshape(*X.shape[:-1], N)
+    return _unflat(y, X, N)
 
 
 def _packed_checks(X, W_T, scale, bias, in_features, flatten: bool = True):
@@ -177,14 +200,14 @@ def ternary_linear_packed_forward(X: Tensor, W_T: Tensor, scale: Tensor,
     if X.dtype == torch.float64:
         y = _float64_packed(X, W_T, scale, bias, in_features)
         return y if residual is None else y + residual
-    x2 = X.contiguous().reshape(-1, K)
+    x2 = _flat_rows(X, K)
     W_T = W_T.contiguous()
     scale = _prep_vec(scale, x2)
     bias = None if bias is None else _prep_vec(bias, x2)
     B = x2.shape[0]
     xdt = _dt(x2, "X")
     y = torch.empty((B, N), dtype=X.dtype, device=X.device)
-    with torch.cuda.device(X.device):
+    with _on(X):
         ws_bytes = _L.bt_packed_forward_workspace_bytes(B, N, K, xdt)
         ws = _workspace(ws_bytes, X.device)
         if residual is None:
@@ -198,7 +221,7 @@ def ternary_linear_packed_forward(X: Tensor, W_T: Tensor, scale: Tensor,
                 x2.data_ptr(), xdt, W_T.data_ptr(), scale.data_ptr(), _dt(scale, "scale"), scale.numel(),
                 _ptr(bias), 0 if bias is None else _dt(bias, "bias"), res.data_ptr(), y.data_ptr(), B, N, K,
                 _ptr(ws), 0 if ws is None else ws.numel(), _stream(X)))
-    return y.reshape(*X.shape[:-1], N)
+    return _unflat(y, X, N)
 
 
 def ternary_linear_packed_forward_fused(X: Tensor, W_T: Tensor, scale: Tensor, bias: Optional[Tensor] = None,
@@ -232,13 +255,13 @@ def ternary_linear_packed_forward_fused(X: Tensor, W_T: Tensor, scale: Tensor, b
     xdt = _dt(x2, "X")
     y = torch.empty((B, N), dtype=X.dtype, device=X.device)
     res = None if residual is None else _residual_2d(residual, X, X.shape[:-1], N)
-    with torch.cuda.device(X.device):
+    with _on(X):
         ws = _workspace(_L.bt_packed_forward_fused_workspace_bytes(B, N, K, xdt), X.device)
         _status(_L.bt_ternary_linear_packed_forward_fused(
             x2.data_ptr(), x2.stride(0), xdt, op, _ptr(pb), ldb, float(eps), W_T.data_ptr(), scale.data_ptr(),
             _dt(scale, "scale"), scale.numel(), _ptr(bias), 0 if bias is None else _dt(bias, "bias"), _ptr(res),
             y.data_ptr(), B, N, K, _ptr(ws), 0 if ws is None else ws.numel(), _stream(X)))
-    return y.reshape(*X.shape[:-1], N)
+    return _unflat(y, X, N)
 
 
 def retile_weights(W_T: Tensor, in_features: int, gate_up_pairs: bool = False) -> Tensor:
@@ -252,7 +275,7 @@ def retile_weights(W_T: Tensor, in_features: int, gate_up_pairs: bool = False) -
     _check(_all_cuda(W_T), "All tensors must be CUDA")
     W_T = W_T.contiguous()
     N = W_T.shape[1]
-    with torch.cuda.device(W_T.device):
+    with _on(W_T):
         out = torch.empty((_L.bt_tiled_weights_bytes(N, in_features),), dtype=torch.uint8, device=W_T.device)
         _status(_L.bt_retile_weights(W_T.data_ptr(), N, in_features, 1 if gate_up_pairs else 0, out.data_ptr(),
                                      _stream(W_T)))
@@ -270,7 +293,7 @@ def untile_weights(W_tiled: Tensor, out_features: int, in_features: int, gate_up
     """``W_T [ceil(K/4), N]`` back from its decode-tiled copy (exact inverse of :func:`retile_weights`)."""
     _tiled_checks(W_tiled, out_features, in_features)
     _check(_all_cuda(W_tiled), "All tensors must be CUDA")
-    with torch.cuda.device(W_tiled.device):
+    with _on(W_tiled):
         out = torch.empty(((in_features + 3) // 4, out_features), dtype=torch.uint8, device=W_tiled.device)
         _status(_L.bt_untile_weights(W_tiled.data_ptr(), out_features, in_features, 1 if gate_up_pairs else 0,
                                      out.data_ptr(), _stream(W_tiled)))
@@ -302,7 +325,7 @@ def ternary_linear_tiled_forward(X: Tensor, W_tiled: Tensor, scale: Tensor, bias
     _check(bias is None or (bias.dim() == 1 and bias.shape[0] == N), "bias shape mismatch")
     _check(_all_cuda(X, W_tiled, scale, bias), "All tensors must be CUDA")
     _check(X.dtype in _DT, "X must be float32, float16 or bfloat16")
-    x2 = _rows_2d(X, K) if (norm is not None or swiglu_up is not None) else X.contiguous().reshape(-1, K)
+    x2 = _rows_2d(X, K) if (norm is not None or swiglu_up is not None) else _flat_rows(X, K)
     scale = _prep_vec(scale, x2)
     bias = None if bias is None else _prep_vec(bias, x2)
     B = x2.shape[0]
@@ -322,14 +345,14 @@ def ternary_linear_tiled_forward(X: Tensor, W_tiled: Tensor, scale: Tensor, bias
     Ny = N // 2 if swiglu_pairs else N
     y = torch.empty((B, Ny), dtype=X.dtype, device=X.device)
     res = None if residual is None else _residual_2d(residual, X, X.shape[:-1], N)
-    with torch.cuda.device(X.device):
+    with _on(X):
         query = _L.bt_tiled_forward_workspace_bytes if op == 0 and not swiglu_pairs else _L.bt_packed_forward_fused_workspace_bytes
         ws = _workspace(query(B, N, K, xdt), X.device)
         _status(_L.bt_ternary_linear_tiled_forward(
             x2.data_ptr(), x2.stride(0), xdt, op, _ptr(pb), ldb, float(eps), W_tiled.data_ptr(), scale.data_ptr(),
             _dt(scale, "scale"), scale.numel(), _ptr(bias), 0 if bias is None else _dt(bias, "bias"), _ptr(res),
             1 if swiglu_pairs else 2 if natural_from_pairs else 0, y.data_ptr(), B, N, K, _ptr(ws), 0 if ws is None else ws.numel(), _stream(X)))
-    return y.reshape(*X.shape[:-1], Ny)
+    return _unflat(y, X, Ny)
 
 
 def pointer_table(tensors) -> Tensor:
@@ -358,7 +381,7 @@ def ternary_gemv_grouped(x_tab: Tensor, w_tiled_tab: Tensor, scale_tab: Tensor, 
     _check(_all_cuda(*tabs), "All tensors must be CUDA")
     _check(scale_dtype in _DT and bias_dtype in _DT, "scale / bias dtype must be float32, float16 or bfloat16")
     _check(x_dtype in (torch.float16, torch.bfloat16), "x_dtype must be float16 or bfloat16")
-    with torch.cuda.device(x_tab.device):
+    with _on(x_tab):
         _status(_L.bt_ternary_gemv_grouped(
             x_tab.data_ptr(), _DT[x_dtype], w_tiled_tab.data_ptr(), scale_tab.data_ptr(), _DT[scale_dtype],
             out_features if scale_len < 0 else scale_len, _ptr(bias_tab), _DT[bias_dtype], y_tab.data_ptr(), G,
@@ -383,7 +406,7 @@ def ternary_gemm_int8_grouped(q_tab: Tensor, sx_tab: Tensor, w_tiled_tab: Tensor
     _check(_all_cuda(*tabs), "All tensors must be CUDA")
     _check(scale_dtype in _DT and bias_dtype in _DT and out_dtype in _DT,
            "scale / bias / output dtype must be float32, float16 or bfloat16")
-    with torch.cuda.device(q_tab.device):
+    with _on(q_tab):
         _status(_L.bt_ternary_gemm_i8_grouped(
             q_tab.data_ptr(), 1 if q_operand_order else 0, sx_tab.data_ptr(), w_tiled_tab.data_ptr(), scale_tab.data_ptr(),
             _DT[scale_dtype], out_features if scale_len < 0 else scale_len, _ptr(bias_tab), _DT[bias_dtype],
@@ -395,7 +418,7 @@ def retile_fields(W_tiled: Tensor, in_features: int, out_features: int) -> Tenso
     their order): what :func:`ternary_gemm_int8_fields` reads."""
     _tiled_checks(W_tiled, out_features, in_features)
     _check(W_tiled.is_cuda, "All tensors must be CUDA")
-    with torch.cuda.device(W_tiled.device):
+    with _on(W_tiled):
         out = torch.empty_like(W_tiled)
         _status(_L.bt_retile_fields(W_tiled.data_ptr(), out_features, in_features, out.data_ptr(), _stream(W_tiled)))
     return out
@@ -428,7 +451,7 @@ def ternary_gemm_int8_fields(Q: Tensor, s_x: Tensor, q_rowsum: Tensor, W_fields:
     y = torch.empty((B, N), dtype=out_dtype, device=q.device)
     acc = torch.empty((B, N), dtype=torch.int32, device=q.device) if return_acc else None
     res = None if residual is None else _residual_2d(residual, y, (B,), N)
-    with torch.cuda.device(q.device):
+    with _on(q):
         _status(_L.bt_ternary_gemm_i8_fields(
             q.data_ptr(), 1 if q_operand_order else 0, s_x.data_ptr(), q_rowsum.data_ptr(), W_fields.data_ptr(),
             1 if natural_from_pairs else 0, scale.data_ptr(), _dt(scale, "scale"), scale.numel(), _ptr(bias),
@@ -459,7 +482,7 @@ def ternary_gemm_int8_tiled(Q: Tensor, s_x: Tensor, W_tiled: Tensor, scale: Tens
     y = torch.empty((B, N), dtype=out_dtype, device=q.device)
     acc = torch.empty((B, N), dtype=torch.int32, device=q.device) if return_acc else None
     res = None if residual is None else _residual_2d(residual, y, (B,), N)
-    with torch.cuda.device(q.device):
+    with _on(q):
         _status(_L.bt_ternary_gemm_i8_tiled(
             q.data_ptr(), 1 if q_operand_order else 0, s_x.data_ptr(), W_tiled.data_ptr(), scale.data_ptr(),
             _dt(scale, "scale"), scale.numel(), _ptr(bias), 0 if bias is None else _dt(bias, "bias"), _ptr(res),
@@ -491,7 +514,7 @@ def ternary_linear_tensor_core_forward(X: Tensor, W_T: Tensor, scale: Tensor,
     bias = None if bias is None else _prep_vec(bias, x2)
     B = x2.shape[0]
     y = torch.empty((B, N), dtype=X.dtype, device=X.device)
-    with torch.cuda.device(X.device):
+    with _on(X):
         ws_bytes = _L.bt_tensor_core_workspace_bytes(B, N, K)
         ws = _workspace(ws_bytes, X.device)
         _status(_L.bt_ternary_linear_tensor_core_forward(
@@ -548,7 +571,7 @@ def act_quant_int8(X: Tensor, operand_order: bool = False, return_rowsum: bool =
     B, K = x.shape
     q = torch.empty((B, K), dtype=torch.int8, device=x.device)
     s = torch.empty((B,), dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x):
         if return_rowsum:
             rs = torch.empty((B,), dtype=torch.int32, device=x.device)
             _status(_L.bt_act_quant_i8_rowsum(x.data_ptr(), _dt(x, "X"), B, K, q.data_ptr(), s.data_ptr(), rs.data_ptr(),
@@ -581,7 +604,7 @@ def ternary_gemm_int8(Q: Tensor, s_x: Tensor, W_T: Tensor, scale: Tensor,
     B = q.shape[0]
     y = torch.empty((B, N), dtype=out_dtype, device=q.device)
     acc = torch.empty((B, N), dtype=torch.int32, device=q.device) if return_acc else None
-    with torch.cuda.device(q.device):
+    with _on(q):
         ws_bytes = _L.bt_gemm_i8_workspace_bytes(B, N, K)
         ws = _workspace(ws_bytes, q.device)
         if residual is None and not q_operand_order:
@@ -641,7 +664,7 @@ def swiglu(gate: Tensor, up: Tensor, store: bool = True, quantize: bool = False,
     g2, u2 = _rows_2d(gate, K), _rows_2d(up, K)
     h, q, s = _row_op_outputs(g2, store, quantize)
     rs = None
-    with torch.cuda.device(gate.device):
+    with _on(gate):
         if return_rowsum:
             _check(q is not None, "return_rowsum needs quantize=True")
             rs = torch.empty((g2.shape[0],), dtype=torch.int32, device=gate.device)
@@ -673,7 +696,7 @@ def rmsnorm(x: Tensor, weight: Optional[Tensor] = None, eps: float = 1e-6, store
     x2 = _rows_2d(x, K)
     h, q, s = _row_op_outputs(x2, store, quantize)
     rs = None
-    with torch.cuda.device(x.device):
+    with _on(x):
         if return_rowsum:
             _check(q is not None, "return_rowsum needs quantize=True")
             rs = torch.empty((x2.shape[0],), dtype=torch.int32, device=x.device)
@@ -708,7 +731,7 @@ def unpack_dequant(W_T: Tensor, in_features: int, scale: Optional[Tensor] = None
         if scale_f is not None:
             _check(scale_f.numel() in (N, 1), "scale size doesn't match N")
     out = torch.empty((N, in_features), dtype=out_dtype, device=W_T.device)
-    with torch.cuda.device(W_T.device):
+    with _on(W_T):
         _status(_L.bt_unpack_dequant(W_T.data_ptr(), _ptr(scale_f),
                                      0 if scale_f is None else scale_f.numel(), out.data_ptr(), odt,
                                      N, in_features, _stream(W_T)))
@@ -726,7 +749,7 @@ def linear_grad_input(dY: Tensor, W_T: Tensor, scale: Tensor, in_features: int) 
     dY, W_T, scale = dY.contiguous(), W_T.contiguous(), scale.contiguous()
     M, N = dY.shape
     out = torch.empty((M, in_features), dtype=torch.float32, device=dY.device)
-    with torch.cuda.device(dY.device):
+    with _on(dY):
         _status(_L.bt_ternary_linear_grad_input(dY.data_ptr(), W_T.data_ptr(), scale.data_ptr(), scale.numel(),
                                                 out.data_ptr(), M, N, in_features, _stream(dY)))
     return out
@@ -744,7 +767,7 @@ def linear_grad_weight(dY: Tensor, X: Tensor, scale: Tensor, want_bias: bool = F
     (M, N), K = dY.shape, X.shape[1]
     dW = torch.empty((N, K), dtype=torch.float32, device=dY.device)
     dB = torch.empty((N,), dtype=torch.float32, device=dY.device) if want_bias else None
-    with torch.cuda.device(dY.device):
+    with _on(dY):
         ws = _workspace(_L.bt_linear_grad_weight_workspace_bytes(M, N, K), dY.device)
         _status(_L.bt_linear_grad_weight(dY.data_ptr(), X.data_ptr(), scale.data_ptr(), scale.numel(), dW.data_ptr(), _ptr(dB),
                                          M, N, K, _ptr(ws), 0 if ws is None else ws.numel(), _stream(dY)))
@@ -763,7 +786,7 @@ def linear_grad_weight_16(dY: Tensor, X: Tensor, scale: Tensor, out_dtype: torch
     dY, X, scale = dY.contiguous(), X.contiguous(), scale.reshape(-1).contiguous()
     (M, N), K = dY.shape, X.shape[1]
     out = torch.empty((N, K), dtype=out_dtype, device=dY.device)
-    with torch.cuda.device(dY.device):
+    with _on(dY):
         ws = _workspace(_L.bt_linear_grad_weight_16_workspace_bytes(M, N, K), dY.device)
         _status(_L.bt_linear_grad_weight_16(dY.data_ptr(), X.data_ptr(), _DT[dY.dtype], scale.data_ptr(), _DT[scale.dtype],
                                             scale.numel(), out.data_ptr(), _DT[out_dtype], M, N, K, _ptr(ws), 0 if ws is None else ws.numel(),
@@ -778,7 +801,7 @@ def scale_grad_weight(G: Tensor, scale: Tensor) -> Tensor:
     _check(_all_cuda(G, scale), "All tensors must be CUDA")
     G, scale = G.contiguous(), scale.reshape(-1).to(torch.float32).contiguous()
     out = torch.empty(G.shape, dtype=torch.float32, device=G.device)
-    with torch.cuda.device(G.device):
+    with _on(G):
         _status(_L.bt_scale_grad_weight(G.data_ptr(), _DT[G.dtype], scale.data_ptr(), scale.numel(), out.data_ptr(),
                                         G.shape[0], G.shape[1], _stream(G)))
     return out

@@ -63,6 +63,11 @@ class TernaryLinearInference(nn.Module):
         self._fields: Optional[Tensor] = None
         self._fields_src: Optional[Tensor] = None
 
+    def _scale_bias(self):
+        """``scale`` and ``bias``, as the buffers they normally are without two walks through ``__getattr__`` (2 us a call)."""
+        b = self.__dict__["_buffers"]
+        return (b["scale"], b["bias"]) if "scale" in b and "bias" in b else (self.scale, self.bias)
+
     # ---- which copies of the weights the layer holds ----------------------------------------
     def _has_row_major(self) -> bool:
         return "weight_packed" in self.__dict__["_buffers"]
@@ -272,7 +277,8 @@ class TernaryLinearInference(nn.Module):
             tiled = self._tiled_for(x, x.numel() // max(x.shape[-1], 1))
             if tiled is not None:
                 from .. import _C
-                return _C.ternary_linear_tiled_forward(x, tiled, self.scale, self.bias, self.in_features,
+                scale, bias = self._scale_bias()
+                return _C.ternary_linear_tiled_forward(x, tiled, scale, bias, self.in_features,
                                                        self.out_features, residual, norm, swiglu_up, False,
                                                        self._natural_from_pairs)
         if x.is_cuda and (norm is not None or swiglu_up is not None):
@@ -301,7 +307,8 @@ class TernaryLinearInference(nn.Module):
             tiled = self._tiled_for(x, x.numel() // max(x.shape[-1], 1), "gate_up_pairs")
             if tiled is not None and x.dtype in (torch.float16, torch.bfloat16):
                 from .. import _C
-                return _C.ternary_linear_tiled_forward(x, tiled, self.scale, self.bias, self.in_features,
+                scale, bias = self._scale_bias()
+                return _C.ternary_linear_tiled_forward(x, tiled, scale, bias, self.in_features,
                                                        self.out_features, None, norm, None, True)
         gu = self.forward(x, None, norm)
         half = self.out_features // 2
