@@ -128,16 +128,18 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
     const int nst = (int)((p.K + F_BK - 1) / F_BK);
     const int64_t k_last = (int64_t)(nst - 1) * F_BK;
 
-    // slot (sub, block, lane (i, g)) of a stage: 16 bytes of row i of the block at k = 16 g + 8 sub; wave w loads slots
-    // NB w .. +NB-1.  Rows past M repeat the last one, columns past N column 0 or the copy's last tile (never stored).
+    // A stage's row is 128 bytes of LDS, eight pieces of 16; piece q of row r lies at place q ^ (r / 2 % 8), so that the 16 rows
+    // of a fragment read meet every bank once.  A wave loads whole rows, eight lanes each: lanes of a load that each have a
+    // row of their own take the cache four times as long.  Wave w loads rows 8 NB w .. +8 NB-1, eight at a time.  Rows past M
+    // repeat the last one, columns past N column 0 or the copy's last tile (never stored).
     const int64_t rows_left = (p.M - m0 < BM) ? p.M - m0 : BM;
     uint32_t a_off[A_LOADS], a_tail[A_LOADS];
 #pragma unroll
     for (int b = 0; b < A_LOADS; b++) {
-        const int slot = NB * wave + b, sub = slot / (2 * NB), row = 16 * (slot % (2 * NB)) + j;
+        const int row = 8 * (NB * wave + b) + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
         const uint32_t r = (uint32_t)(row < rows_left ? row : rows_left - 1);
-        a_off[b] = (r * (uint32_t)p.K + 16u * g + 8u * sub) * 2u;
-        a_tail[b] = k_last + 16 * g + 8 * sub < p.K ? a_off[b] : r * (uint32_t)p.K * 2u;
+        a_off[b] = (r * (uint32_t)p.K + 8u * piece) * 2u;
+        a_tail[b] = k_last + 8 * piece < p.K ? a_off[b] : r * (uint32_t)p.K * 2u;
     }
     uint32_t w_off[W_LOADS], w_tail[W_LOADS];
     if constexpr (SRC == W_ROWS16) {
@@ -198,9 +200,9 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
     constexpr int RB = NB == 4 ? 4 : 2 * NB;
     u32x4 a_x[RB], a_y[RB], b0[4], b1[4];
     uint32_t raw[4];
-    auto frag = [&](uint32_t buf, int sub, int mb) {
-        return *(const u32x4*)(lds + buf + 16 * lane + (sub * 2 * NB + mb) * 1024);
-    };
+    // lane (j, g): k = 16 g + 8 sub .. +7 of row 16 mb + j
+    const uint32_t frag_at[2] = {128u * j + 16u * ((2u * g) ^ (j >> 1)), 128u * j + 16u * ((2u * g + 1) ^ (j >> 1))};
+    auto frag = [&](uint32_t buf, int sub, int mb) { return *(const u32x4*)(lds + (buf + frag_at[sub]) + 2048 * mb); };
     auto read_raw = [&](uint32_t buf) {
         const uint8_t* src = lds + buf + A_BYTES + wave * 1024;
         if constexpr (SRC == W_TILES) {
