@@ -127,17 +127,18 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
     const int nst = (int)((p.K + D_BK - 1) / D_BK);
     const int64_t k_last = (int64_t)(nst - 1) * D_BK;
 
-    // Lane (i, c = lane / 16) loads 16 bytes of row i of its row block at k = 16 c: LDS then holds slot (block, lane) as
-    // the MFMA lane reads it.  Rows past M repeat the last one (their outputs are never stored); columns past N read
-    // column 0 of row-major weights and the last tile of the copy.
+    // A stage's row is 64 bytes of LDS, four pieces of 16; piece q of row r lies at place q ^ (r / 4 % 4), so that the 16 rows of
+    // a fragment read meet every bank once.  Four lanes load a row: lanes of a load that each have a row of their own take the
+    // cache four times as long.  Rows past M repeat the last one (their outputs are never stored); columns past N read column 0
+    // of row-major weights and the last tile of the copy.
     const int64_t rows_left = (p.M - m0 < BM) ? p.M - m0 : BM;
     uint32_t a_off[A_LOADS], a_tail[A_LOADS];
 #pragma unroll
     for (int b = 0; b < A_LOADS; b++) {
-        const int row = 16 * ((A_LOADS * wave + b) % (2 * NB)) + j;
+        const int row = 16 * ((A_LOADS * wave + b) % (2 * NB)) + (lane >> 2), piece = (lane & 3) ^ (lane >> 4);
         const uint32_t r = (uint32_t)(row < rows_left ? row : rows_left - 1);
-        a_off[b] = r * (uint32_t)p.K + 16u * g;
-        a_tail[b] = r * (uint32_t)p.K + (k_last + 16 * g < p.K ? 16u * g : 0u);
+        a_off[b] = r * (uint32_t)p.K + 16u * piece;
+        a_tail[b] = r * (uint32_t)p.K + (k_last + 16 * piece < p.K ? 16u * piece : 0u);
     }
     uint32_t w_off[W_LOADS], w_tail[W_LOADS];
     const bool w_in = !TAIL || SRC > W_ROWS16 || k_last + 16 * g < p.K;  // this lane's rows of the last stage exist
@@ -156,6 +157,7 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
         w_off[0] = ((uint32_t)tt * (uint32_t)p.wsteps * 64u + (uint32_t)(16 * g + 4 * (j & 3))) * 4u;
     }
     const int8_t* const a_base = p.Q + m0 * p.K;  // uniform
+    const uint32_t frag_at = 64u * j + 16u * (g ^ (j >> 2));  // lane (j, g): k = 16 g .. +15 of row j of a block
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
 
     // the next stage to load: its global addresses, and the byte offset of its buffer
@@ -219,7 +221,7 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
         }
     };
     auto read_a = [&](uint32_t buf, int mb0, uint4 (&dst)[NB]) {
-        const uint8_t* src = lds + buf + 16 * lane;
+        const uint8_t* src = lds + (buf + frag_at);
 #pragma unroll
         for (int i = 0; i < NB; i++) {
             dst[i] = *(const uint4*)(src + (mb0 + i) * 1024);
@@ -296,7 +298,7 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
                 const v4i a = {(int)a_lo[i].x, (int)a_lo[i].y, (int)a_lo[i].z, (int)a_lo[i].w};
                 acc[i][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b_cur[t], acc[i][t], 0, 0, 0);
             }
-            if (c < NB) a_hi[c] = *(const uint4*)(lds + buf + 16 * lane + (NB + c) * 1024);
+            if (c < NB) a_hi[c] = *(const uint4*)(lds + (buf + frag_at) + (NB + c) * 1024);
             decode_slice(c, b_nxt);
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -310,7 +312,7 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
                 const v4i a = {(int)a_hi[i].x, (int)a_hi[i].y, (int)a_hi[i].z, (int)a_hi[i].w};
                 acc[NB + i][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b_cur[t], acc[NB + i][t], 0, 0, 0);
             }
-            if (c < NB) a_lo[c] = *(const uint4*)(lds + nxt + 16 * lane + c * 1024);
+            if (c < NB) a_lo[c] = *(const uint4*)(lds + (nxt + frag_at) + c * 1024);
             if (c == 4) read_raw(s + 2, nxt2);
             // stage s + 5 over stage s
             if (c >= 6 && c < 6 + A_LOADS) issue_a(c - 6);
