@@ -47,13 +47,21 @@ struct GemmFParams {
 };
 static_assert(offsetof(GemmFParams, Y) == 64, "first argument line as laid out above");
 
-constexpr int fd_stages(int NB) { return NB == 4 ? 3 : NB == 2 ? 4 : 5; }  // in LDS: 60, 48, 40 KiB
-constexpr int fd_lds_bytes(int NB) { return fd_stages(NB) * (NB * 4096 + 4096); }
+// Stages of activations in LDS; of weights one fewer, since a wave has its own in registers half a stage before it needs them.
+// One group of four waves: 56, 44, 36 KiB; two groups: 64 (NB = 2), 56 (NB = 1).
+constexpr int fd_stages(int NB, int KG) { return NB == 4 || (NB == 2 && KG == 2) ? 3 : NB == 2 || KG == 2 ? 4 : 5; }
+constexpr int fd_group_bytes(int NB, int KG) { return fd_stages(NB, KG) * NB * 4096 + (fd_stages(NB, KG) - 1) * 4096; }
+
+// Piece q of row r of a stage lies at place q ^ fd_place(r / 2).  A 16-byte read from LDS takes its lanes in groups that hold
+// rows 0 .. 3 and 12 .. 15 of one pair of pieces with rows 4 .. 11 of the next pair: those must differ.  (With r / 2 itself every
+// fragment read met half of the banks twice: 2.2 M of the 4.9 M
+// LDS cycles of 1000 x 2560 x 6912 were conflicts, now none of 2.7 M; 49.6 -> 44.1 us there with the decode below.)
+__device__ __forceinline__ uint32_t fd_place(uint32_t half_row) { return (half_row & 1u) | ((half_row >> 2) & 1u) * 6u; }
 
 // y = sum * scale + bias, row block by row block (the empty asm keeps a row's address from being computed ahead of its turn)
 // RN: rows of any length, so that a lane's four columns start on any element and the last ones may be fewer.
-template <int MODE, bool RES, int NB, bool RN>
-__device__ __forceinline__ void fd_epilogue(const GemmFParams& p, const v4f (&acc)[2 * NB][4], int64_t m0, int g, int64_t ncol,
+template <int MODE, bool RES, bool RN, int MB>
+__device__ __forceinline__ void fd_epilogue(const GemmFParams& p, const v4f (&acc)[MB][4], int64_t m0, int g, int64_t ncol,
                                             int rows_left, const float (&ws)[4], const float (&bs)[4]) {
     constexpr int YDT = MODE == MODE_F16 ? BT_F16 : BT_BF16;
     const uint32_t lane_off = ((uint32_t)(4 * g) * (uint32_t)p.N + (uint32_t)(ncol & (F_BN - 1))) * 2u;
@@ -62,7 +70,7 @@ __device__ __forceinline__ void fd_epilogue(const GemmFParams& p, const v4f (&ac
     char* row = (char*)p.Y + first;
     const char* res = (const char*)p.epi.residual + first;
 #pragma unroll
-    for (int mb = 0; mb < 2 * NB; mb++) {
+    for (int mb = 0; mb < MB; mb++) {
         if (16 * mb >= rows_left) return;  // (uniform)
         uint2 rv[4];
         if constexpr (RES) {  // the block's four rows at once; lanes past the last row read a row that exists
@@ -116,27 +124,31 @@ __device__ __forceinline__ void fd_epilogue(const GemmFParams& p, const v4f (&ac
 
 // One tile of 32 NB rows.  TAIL: K is not a multiple of 64 (of 8 it is): the lanes whose k lies past
 // the end load something of their own row or column instead and their activations are zeroed on the way to the MFMAs.
-template <int MODE, int SRC, int NB, bool TAIL, bool RN>
-__device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_t m0, const int tile_n, uint8_t* lds) {
-    constexpr int BM = 32 * NB, A_BYTES = NB * 4096, STAGE = A_BYTES + 4096, NST = fd_stages(NB);
+// KG = 2: two groups of four waves, each on its run of the stages; they add their sums through LDS and store half the rows each.
+template <int MODE, int SRC, int NB, int KG, bool TAIL, bool RN>
+__device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_t m0, const int tile_n, uint8_t* lds_all) {
+    constexpr int BM = 32 * NB, A_BYTES = NB * 4096, NST = fd_stages(NB, KG), W_AT = NST * A_BYTES;
     constexpr int A_LOADS = NB, W_LOADS = SRC == W_ROWS ? 4 : 1, LOADS = A_LOADS + W_LOADS;
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = wave_all & 3, group = KG == 1 ? 0 : wave_all >> 2;
+    uint8_t* const lds = lds_all + group * fd_group_bytes(NB, KG);
     const int j = lane & 15, g = lane >> 4;
     const int64_t ncol = (int64_t)tile_n * F_BN + 64 * wave + 4 * j;
     const bool col_ok = ncol < p.N;
     const int nst = (int)((p.K + F_BK - 1) / F_BK);
     const int64_t k_last = (int64_t)(nst - 1) * F_BK;
+    // this group's stages: st0 .. st0 + mine - 1 (every group meets `rounds` barriers in the loop; mine >= 1)
+    const int rounds = KG == 1 ? nst : (nst + 1) / 2, st0 = group * rounds, mine = KG == 1 ? nst : min(rounds, nst - st0);
+    const int st_tail = group == KG - 1 ? mine - 1 : rounds;  // TAIL: the partial stage, if it is this group's
 
-    // A stage's row is 128 bytes of LDS, eight pieces of 16; piece q of row r lies at place q ^ (r / 2 % 8), so that the 16 rows
-    // of a fragment read meet every bank once.  A wave loads whole rows, eight lanes each: lanes of a load that each have a
+    // A stage's row is 128 bytes of LDS, eight pieces of 16; at the places fd_place gives them.  A wave loads whole rows, eight lanes each: lanes of a load that each have a
     // row of their own take the cache four times as long.  Wave w loads rows 8 NB w .. +8 NB-1, eight at a time.  Rows past M
     // repeat the last one, columns past N column 0 or the copy's last tile (never stored).
     const int64_t rows_left = (p.M - m0 < BM) ? p.M - m0 : BM;
     uint32_t a_off[A_LOADS], a_tail[A_LOADS];
 #pragma unroll
     for (int b = 0; b < A_LOADS; b++) {
-        const int row = 8 * (NB * wave + b) + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+        const int row = 8 * (NB * wave + b) + (lane >> 3), piece = (lane & 7) ^ fd_place(row >> 1);
         const uint32_t r = (uint32_t)(row < rows_left ? row : rows_left - 1);
         a_off[b] = (r * (uint32_t)p.K + 8u * piece) * 2u;
         a_tail[b] = k_last + 8 * piece < p.K ? a_off[b] : r * (uint32_t)p.K * 2u;
@@ -166,28 +178,30 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
     }
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
 
-    const uint8_t* a_next = (const uint8_t*)(p.X + m0 * p.K);
-    const uint8_t* w_next = p.W_T;
-    uint32_t into = 0;
-    int st_next = 0;
     const int64_t w_step = SRC == W_TILES ? 256 : 16 * p.N;
+    const uint8_t* a_next = (const uint8_t*)(p.X + m0 * p.K + (int64_t)st0 * F_BK);
+    const uint8_t* w_next = p.W_T + st0 * w_step;
+    uint32_t into = 0, w_into = W_AT;
+    int st_next = 0;
     auto issue_a = [&](int b) {
-        const bool last = TAIL && st_next >= nst - 1;
+        const bool last = TAIL && st_next >= st_tail;
         dma16(lds0 + into + (uint32_t)(NB * wave + b) * 1024u, last ? a_tail[b] : a_off[b], a_next);
     };
     auto issue_w = [&](int r) {
-        const bool last = TAIL && st_next >= nst - 1;
-        const uint32_t wd = lds0 + into + A_BYTES + (uint32_t)wave * 1024u;
+        const bool last = TAIL && st_next >= st_tail;
+        const uint32_t wd = lds0 + w_into + (uint32_t)wave * 1024u;
         if constexpr (SRC == W_TILES) dma16(wd, w_off[0], w_next);
         else if constexpr (SRC == W_ROWS16) dma16(wd, last ? w_tail[0] : w_off[0], w_next);
         else dma4(wd + 256u * r, last ? w_tail[r] : w_off[r], w_next);
     };
-    auto next_buf = [](uint32_t b) { return b + STAGE == NST * STAGE ? 0u : b + STAGE; };
+    auto next_buf = [](uint32_t b) { return b + A_BYTES == W_AT ? 0u : b + A_BYTES; };
+    auto next_wbuf = [](uint32_t b) { return b + 4096 == fd_group_bytes(NB, KG) ? (uint32_t)W_AT : b + 4096; };
     auto advance = [&]() {  // past the end: the last stage again, never read
         st_next++;
-        a_next += st_next < nst ? 2 * F_BK : 0;
-        w_next += st_next < nst ? w_step : 0;
+        a_next += st_next < mine ? 2 * F_BK : 0;
+        w_next += st_next < mine ? w_step : 0;
         into = next_buf(into);
+        w_into = next_wbuf(w_into);
     };
 
     v4f acc[2 * NB][4];
@@ -201,10 +215,10 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
     u32x4 a_x[RB], a_y[RB], b0[4], b1[4];
     uint32_t raw[4];
     // lane (j, g): k = 16 g + 8 sub .. +7 of row 16 mb + j
-    const uint32_t frag_at[2] = {128u * j + 16u * ((2u * g) ^ (j >> 1)), 128u * j + 16u * ((2u * g + 1) ^ (j >> 1))};
+    const uint32_t at_j = fd_place(j >> 1), frag_at[2] = {128u * j + 16u * ((2u * g) ^ at_j), 128u * j + 16u * ((2u * g + 1) ^ at_j)};
     auto frag = [&](uint32_t buf, int sub, int mb) { return *(const u32x4*)(lds + (buf + frag_at[sub]) + 2048 * mb); };
-    auto read_raw = [&](uint32_t buf) {
-        const uint8_t* src = lds + buf + A_BYTES + wave * 1024;
+    auto read_raw = [&](uint32_t wbuf) {
+        const uint8_t* src = lds + wbuf + wave * 1024;
         if constexpr (SRC == W_TILES) {
             const u32x4 v = *(const u32x4*)(src + 16 * lane);
 #pragma unroll
@@ -214,21 +228,21 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
             for (int r = 0; r < 4; r++) raw[r] = *(const uint32_t*)(src + (SRC == W_ROWS16 ? 64 * (4 * g + r) + 4 * j : 256 * r + 4 * lane));
         }
     };
-    // operand dword e = 4 t + d of column t.  The byte of a row with codes c0 .. c3 times 2^8 + 2^22 has c0 at bit 8 and c1 at
-    // bit 24, c2 and c3 four bits above: the selectors of two table lookups (dwords d and d + 1, decoded in this order).
+    // Decode of a raw dword's 16 codes: code c of its four bytes becomes the high bytes of four operand values by one table
+    // lookup (the low bytes of +-1 in fp16 and of +-2 in bf16 are zero), and an operand dword is the high bytes of codes 2 h and
+    // 2 h + 1 of one byte: 19 operations for eight dwords.  Byte by byte it took 28.
+    // Column t's codes of its byte r (k = 4 r .. +3) are in byte r of raw[t] (the copy) or byte t of raw[r] (rows); sub-step s
+    // takes bytes 2 s and 2 s + 1.
     constexpr uint32_t LUT = (MODE == MODE_F16) ? LUT_F16_ONE : LUT_BF16_TWO;
-    uint32_t spread = 0;
-    auto decode = [&](int e, int sub, u32x4 (&out)[4]) {
-        const int t = e >> 2, d = e & 3;
-        if ((d & 1) == 0) {
-            const int r = 2 * sub + (d >> 1);
-            const uint32_t byte = SRC == W_TILES ? (raw[t] >> (8 * r)) & 0xffu : (raw[r] >> (8 * t)) & 0xffu;
-            spread = __umul24(byte, 0x400100u);
-            out[t][d] = perm(0u, LUT, spread & 0x03000300u);
-        } else {
-            out[t][d] = perm(0u, LUT, (spread >> 4) & 0x03000300u);
-        }
+    uint32_t hi[4][4];
+    auto table = [&](int e) { hi[e >> 2][e & 3] = perm(0u, LUT, (raw[e >> 2] >> (2 * (e & 3))) & 0x03030303u); };
+    auto emit = [&](int e, int sub, u32x4 (&out)[4]) {  // dword e % 4 of column e / 4
+        const int t = e >> 2, d = e & 3, r = 2 * sub + (d >> 1), h = d & 1;
+        const int q = SRC == W_TILES ? t : r, byte = SRC == W_TILES ? r : t;
+        out[t][d] = perm(hi[q][2 * h + 1], hi[q][2 * h], ((uint32_t)(4 + byte) << 24) | (0x0Cu << 16) | ((uint32_t)byte << 8) | 0x0Cu);
     };
+    // The first sub-step's tables are all of them (the copy) or those of raw[0] and raw[1] (rows).
+    constexpr int T0 = SRC == W_TILES ? 16 : 8;
     auto mfma = [&](const u32x4& a, const u32x4& b, v4f& c) {
         if constexpr (MODE == MODE_F16)
             c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), c, 0, 0, 0);
@@ -236,26 +250,33 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
             c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
     };
 
-    uint32_t buf = 0;
+    uint32_t buf = 0, wbuf = W_AT;
 #pragma unroll
     for (int s = 0; s < NST; s++) {
 #pragma unroll
         for (int b = 0; b < A_LOADS; b++) issue_a(b);
+        if (s == NST - 1) break;
 #pragma unroll
         for (int r = 0; r < W_LOADS; r++) issue_w(r);
         advance();
     }
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NST - 1) * LOADS) : "memory");  // stage 0
-    read_raw(0);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NST - 1) * LOADS - W_LOADS) : "memory");  // stage 0
+    read_raw(wbuf);
 #pragma unroll
     for (int i = 0; i < RB; i++) a_x[i] = frag(0, 0, i);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the first weights' place is free again
 #pragma unroll
-    for (int e = 0; e < 16; e++) decode(e, 0, b0);
+    for (int r = 0; r < W_LOADS; r++) issue_w(r);
+    advance();
+#pragma unroll
+    for (int e = 0; e < T0; e++) table(e);
+#pragma unroll
+    for (int e = 0; e < 16; e++) emit(e, 0, b0);
 
     // Everything but the MFMAs is dealt out between them (16 slots a run), two or three instructions behind each:
     // instructions in a row of their own would leave the matrix pipe idle.
     constexpr int SL = NB == 1 ? 2 : 1;  // slots per MFMA
-    for (int s = 0; s < nst; s++) {
+    for (int s = 0; s < mine; s++) {
         const uint32_t nxt = next_buf(buf);
         auto run_mfma = [&](int c, const u32x4 (&a)[RB], const u32x4 (&b)[4], int mb0) {
             if (c % SL != 0) return;
@@ -264,7 +285,7 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
         };
         auto mask = [&](u32x4 (&a)[RB], int sub) {
             if constexpr (TAIL) {
-                if (s == nst - 1) {  // (uniform)
+                if (s == st_tail) {  // (uniform)
 #pragma unroll
                     for (int i = 0; i < RB; i++) a[i] &= keep[sub];
                 }
@@ -281,7 +302,10 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
             for (int c = 0; c < 16; c++) {
                 run_mfma(c, a_x, b0, 0);
                 if (c < 4) a_y[c] = frag(buf, 0, 4 + c);
-                if (c % 2 == 0) decode(c / 2, 1, b1);
+                if (c % 2 == 0) {
+                    if (SRC == W_TILES) emit(c / 2, 1, b1);
+                    else table(8 + c / 2);
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
             mask(a_y, 0);
@@ -289,7 +313,8 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
             for (int c = 0; c < 16; c++) {
                 run_mfma(c, a_y, b0, 4);
                 if (c < 4) a_x[c] = frag(buf, 1, c);
-                if (c % 2 == 0) decode(8 + c / 2, 1, b1);
+                if (SRC != W_TILES) emit(c, 1, b1);
+                else if (c % 2 == 0) emit(8 + c / 2, 1, b1);
                 __builtin_amdgcn_sched_barrier(0);
             }
             mask(a_x, 1);
@@ -297,9 +322,12 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
 #pragma unroll
             for (int c = 0; c < 16; c++) {
                 run_mfma(c, a_x, b1, 0);
-                if (c == 0) read_raw(nxt);
+                if (c == 0) read_raw(next_wbuf(wbuf));
                 if (c < 4) a_y[c] = frag(buf, 1, 4 + c);
-                if (c >= 8) decode(c - 8, 0, b0);  // (the weights have arrived)
+                if (c >= 8) {  // (the weights have arrived)
+                    table(c - 8);
+                    if (T0 == 16) table(c);
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
             mask(a_y, 1);
@@ -308,7 +336,7 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
             for (int c = 0; c < 16; c++) {
                 run_mfma(c, a_y, b1, 4);
                 if (c < 4) a_x[c] = frag(nxt, 0, c);
-                if (c % 2 == 0) decode(8 + c / 2, 0, b0);
+                emit(c, 0, b0);
                 load_next(c);
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -318,11 +346,16 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
             for (int c = 0; c < 16; c++) {
                 run_mfma(c, a_x, b0, 0);
                 if (c < RB) a_y[c] = frag(buf, 1, c);
-                if (c < 12) decode(c, 1, b1);
-                else if (c < 14) { decode(2 * c - 12, 1, b1); decode(2 * c - 11, 1, b1); }
+                if (SRC == W_TILES) {
+                    if (c < 12) emit(c, 1, b1);
+                    else if (c < 14) { emit(2 * c - 12, 1, b1); emit(2 * c - 11, 1, b1); }
+                } else {
+                    if (c < 4) { table(8 + 2 * c); table(9 + 2 * c); }
+                    else if (c < 12) { emit(2 * (c - 4), 1, b1); emit(2 * (c - 4) + 1, 1, b1); }
+                }
                 if (c == 15) {
                     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 2) * LOADS) : "memory");  // stage s + 1
-                    read_raw(nxt);
+                    read_raw(next_wbuf(wbuf));
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -332,16 +365,26 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
             for (int c = 0; c < 16; c++) {
                 run_mfma(c, a_y, b1, 0);
                 if (c < RB) a_x[c] = frag(nxt, 0, c);
-                if (c >= 4 && c < 8) { decode(2 * (c - 4), 0, b0); decode(2 * (c - 4) + 1, 0, b0); }
-                else if (c >= 8) decode(c, 0, b0);
+                if (T0 == 16) {
+                    if (c >= 4 && c < 12) { table(2 * (c - 4)); table(2 * (c - 4) + 1); }
+                    else if (c >= 12) {
+#pragma unroll
+                        for (int e = 0; e < 4; e++) emit(4 * (c - 12) + e, 0, b0);
+                    }
+                } else {
+                    if (c >= 4 && c < 8) { table(2 * (c - 4)); table(2 * (c - 4) + 1); }
+                    else if (c >= 8) { emit(2 * (c - 8), 0, b0); emit(2 * (c - 8) + 1, 0, b0); }
+                }
                 load_next(c);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
         buf = nxt;
+        wbuf = next_wbuf(wbuf);
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the fragments arrived under these MFMAs
         __builtin_amdgcn_sched_barrier(0);
     }
+    if (KG > 1 && mine < rounds) asm volatile("s_barrier" ::: "memory");  // (uniform; the other group has one stage more)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (no load may reach LDS that another workgroup owns by then)
 
     float ws[4], bs[4];
@@ -357,15 +400,39 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
         ws[t] = bits_to_f32_rt(ws_bits[t], p.epi.scale_dtype);
         bs[t] = p.epi.bias ? bits_to_f32_rt(bs_bits[t], p.epi.bias_dtype) : 0.0f;
     }
-    if (!col_ok) return;
-    if (p.epi.residual) fd_epilogue<MODE, true, NB, RN>(p, acc, m0, g, ncol, (int)rows_left, ws, bs);
-    else fd_epilogue<MODE, false, NB, RN>(p, acc, m0, g, ncol, (int)rows_left, ws, bs);
+    auto store = [&](const auto& sums, int64_t row0, int left) {
+        if (p.epi.residual) fd_epilogue<MODE, true, RN>(p, sums, row0, g, ncol, left, ws, bs);
+        else fd_epilogue<MODE, false, RN>(p, sums, row0, g, ncol, left, ws, bs);
+    };
+    if constexpr (KG == 1) {
+        if (col_ok) store(acc, m0, (int)rows_left);
+    } else {
+        // group 0 takes the first NB row blocks, group 1 the others: each hands over the sums that it does not store
+        v4f* const mine_at = (v4f*)lds_all + wave_all * (256 * NB) + lane;
+        const v4f* const theirs_at = (const v4f*)lds_all + (wave_all ^ 4) * (256 * NB) + lane;
+        v4f sums[NB][4];
+        __syncthreads();  // (both groups have read their last stages)
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                mine_at[64 * (4 * i + t)] = group ? acc[i][t] : acc[NB + i][t];
+                sums[i][t] = group ? acc[NB + i][t] : acc[i][t];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) sums[i][t] += theirs_at[64 * (4 * i + t)];
+        const int left = (int)rows_left - 16 * NB * group;
+        if (col_ok && left > 0) store(sums, m0 + 16 * NB * group, left);
+    }
 }
 
 // NB: tiles of 32 NB rows.  NF > 0: an XCD's tiles from p.fine_from on are computed in tiles of 32 NF rows.
-template <int MODE, int SRC, int NB, int NF, bool TAIL, bool RN>
-__global__ __launch_bounds__(256, NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_f16_kernel(GemmFParams p) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[fd_lds_bytes(NB)];
+template <int MODE, int SRC, int NB, int NF, int KG, bool TAIL, bool RN>
+__global__ __launch_bounds__(256 * KG, KG == 2 || NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_f16_kernel(GemmFParams p) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds[KG * fd_group_bytes(NB, KG)];
     // XCD-aware tile order: the 8 XCDs each take a contiguous run of tiles, walked in groups of four row tiles, so that one
     // XCD's L2 holds a compact block of rows and columns
     const uint32_t idx = blockIdx.x >> 3;
@@ -385,11 +452,11 @@ __global__ __launch_bounds__(256, NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_f16_k
     if constexpr (NF > 0) {
         if (fine) {
             const int64_t mf = m0 + (int64_t)(f % parts) * (32 * NF);
-            if (mf < p.M) gemm_f16_tile<MODE, SRC, NF, TAIL, RN>(p, mf, (int)tn, lds);
+            if (mf < p.M) gemm_f16_tile<MODE, SRC, NF, 1, TAIL, RN>(p, mf, (int)tn, lds);
             return;
         }
     }
-    gemm_f16_tile<MODE, SRC, NB, TAIL, RN>(p, m0, (int)tn, lds);
+    gemm_f16_tile<MODE, SRC, NB, KG, TAIL, RN>(p, m0, (int)tn, lds);
 }
 
 // X and Y are read and written in 16- and 8-byte pieces; 32-bit byte offsets span a tile's rows of X, 16 rows of Y and, for
@@ -400,6 +467,14 @@ bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, co
            ((uintptr_t)X) % 16 == 0 && ((uintptr_t)Y) % 16 == 0;
 }
 
+// A launch of one tile of 64 or 32 rows for each compute unit at most: two groups of waves, half of the stages each.  With one
+// group a SIMD has a single wave, whose chain of LDS reads, decode and MFMAs leaves it idle half of the time.  One / two groups,
+// us, decode-tiled bf16: tiles of 32 rows, 512 x 2560 x 6912 43.2 / 34.1, 128 x 4096 x 11008 62.3 / 49.2, 256 x 7680 x 2560
+// 19.3 / 17.1, 128 x 6000 x 1536 13.0 / 12.0; of 64 rows, 1000 x 2560 x 6912 49.6 / 44.1, 256 x 11008 x 4096 32.7 / 29.7,
+// 512 x 6000 x 1536 15.8 / 15.7.  Fewer stages than 24 would not pay for the exchange of the sums; deeper launches have
+// the other tiles' waves for company (1000 x 13824 x 2560 66.9 / 81.2).
+static bool f16_splits_k(int64_t stages) { return stages >= 24; }
+
 // Rows of the tiles in units of 32, and what the launch takes in microseconds.  Up to one tile of 32, then of 64 rows for each
 // compute unit the launch is one tile deep; beyond that a compute unit's run of tiles is priced.  Measured (tiles of 128 / 64 /
 // 32 rows, us, row-major weights): M = 512, 1024, 1536, 2048, 3072, 4096 with N = K = 4096 48 / 34 / 31, 49 / 35 / 43,
@@ -408,9 +483,9 @@ bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, co
 static int gemm_f16_plan(int64_t M, int64_t N, int64_t K, double* us) {
     const int64_t C = gemm_compute_units(), tn = ceil_div(N, F_BN);
     const int64_t t4 = ceil_div(M, 128) * tn, t2 = ceil_div(M, 64) * tn, t1 = ceil_div(M, 32) * tn;
-    const bool whole = gemm_whole_tiles();
-    if (t1 <= C && !whole) { *us = 4.0 + 0.0062 * (double)K; return 1; }
-    if (t2 <= C && !whole) { *us = 5.0 + 0.007 * (double)K; return 2; }
+    const bool whole = gemm_whole_tiles(), split = f16_splits_k(ceil_div(K, F_BK));
+    if (t1 <= C && !whole) { *us = split ? 5.7 + 0.0042 * (double)K : 4.0 + 0.0055 * (double)K; return 1; }
+    if (t2 <= C && !whole) { *us = split ? 6.0 + 0.0056 * (double)K : 5.0 + 0.0065 * (double)K; return 2; }
     const int parts = gemm_dma_parts(t4);
     const double n4 = parts == 1 ? (double)ceil_div(t4, C) : (double)(2 * (t4 / (2 * C))) + (parts == 2 ? 1.2 : 0.6);
     const double p4 = n4 * (2.0 + 0.0113 * (double)K), p2 = (double)ceil_div(t2, C) * (1.3 + 0.0062 * (double)K);
@@ -443,12 +518,18 @@ static int launch_gemm_f16_cfg(GemmFParams p, hipStream_t st) {
             const int rem = p.per_xcd % (int)(2 * gemm_compute_units() / 8);
             p.fine_from = p.per_xcd - rem;
             const dim3 grid((unsigned)(8 * (p.fine_from + parts * rem)));
-            if (parts == 2) hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 4, 2, TAIL, RN>), grid, block, 0, st, p);
-            else hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 4, 1, TAIL, RN>), grid, block, 0, st, p);
+            if (parts == 2) hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 4, 2, 1, TAIL, RN>), grid, block, 0, st, p);
+            else hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 4, 1, 1, TAIL, RN>), grid, block, 0, st, p);
             return check_launch(who);
         }
     }
-    hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, NB, 0, TAIL, RN>), dim3((unsigned)(8 * p.per_xcd)), block, 0, st, p);
+    if constexpr (NB != 4) {
+        if (total <= gemm_compute_units() && f16_splits_k(p.wstages)) {
+            hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, NB, 0, 2, TAIL, RN>), dim3((unsigned)(8 * p.per_xcd)), dim3(512), 0, st, p);
+            return check_launch(who);
+        }
+    }
+    hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, NB, 0, 1, TAIL, RN>), dim3((unsigned)(8 * p.per_xcd)), block, 0, st, p);
     return check_launch(who);
 }
 template <int MODE, int SRC, int NB>

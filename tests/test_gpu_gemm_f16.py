@@ -64,3 +64,31 @@ def test_infinities_past_the_end_of_a_row_stay_in_their_row():
         rest = torch.ones(m, dtype=torch.bool)
         rest[[7, 9, 150]] = False
         assert bool((y[rest.cuda()] == k).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(33, 260, 1536), (97, 1004, 1544), (250, 516, 1480), (640, 5000, 1608), (129, 1024, 2112), (70, 1030, 1800)])
+def test_stages_in_two_groups(m, n, k, dtype):
+    """Launches of at most one tile a compute unit, 24 stages and more: an even and an odd number of stages, a remainder of K in the
+    second group, rows that end in either group's half of a tile, tiles of 32 and 64 rows, N % 4 != 0.  Bound as above."""
+    from bittorch_amd import _C
+    announce("gemm_f16 two groups", m, n, k, dtype)
+    set_option("STREAM_MAX_ROWS", "1")
+    g = torch.Generator("cuda").manual_seed(m + n + k)
+    w = random_ternary(n, k, seed=m).cuda()
+    wt = _C.ternary_quantize_pack(w.float(), 0.05, True)[0]
+    tiled = _C.retile_weights(wt, k)
+    x = torch.randn(m, k, generator=g, device="cuda").to(dtype)
+    scale = torch.rand(n, generator=g, device="cuda") + 0.5
+    res = torch.randn(m, n, generator=g, device="cuda").to(dtype)
+    w = w.double()
+    ref = (x.double() @ w.t()) * scale.double()
+    mags = (x.double().abs() @ w.t().abs()) * scale.double()
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for r in (None, res):
+        want = ref if r is None else ref + r.double()
+        bound = (k + 8) * 2.0 ** -24 * mags + unit * (want.abs() + (0 if r is None else ref.abs())) + 2e-7
+        y = _C.ternary_linear_packed_forward(x, wt, scale, None, k, residual=r)
+        yt = _C.ternary_linear_tiled_forward(x, tiled, scale, None, k, n, residual=r)
+        assert torch.equal(y, yt)
+        assert bool(((y.double() - want).abs() <= bound).all())
