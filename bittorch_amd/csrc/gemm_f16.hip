@@ -156,8 +156,8 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
     uint32_t w_off[W_LOADS], w_tail[W_LOADS];
     if constexpr (SRC == W_ROWS16) {
         const int64_t col = (int64_t)tile_n * F_BN + 64 * wave + 16 * (lane & 3);
-        w_off[0] = (uint32_t)(col < p.N ? col : 0) + (uint32_t)(lane >> 2) * (uint32_t)p.N;
-        w_tail[0] = (k_last >> 2) + (lane >> 2) < p.Kb ? w_off[0] : (uint32_t)(col < p.N ? col : 0);
+        w_off[0] = (uint32_t)(col < p.N ? col : 0) + (uint32_t)rows16_row(lane) * (uint32_t)p.N;
+        w_tail[0] = (k_last >> 2) + rows16_row(lane) < p.Kb ? w_off[0] : (uint32_t)(col < p.N ? col : 0);
     } else if constexpr (SRC == W_TILES) {
         const int tt = stored_tile16((int)(ncol >> 4), p.tiles16);
         w_off[0] = ((uint32_t)tt * (uint32_t)p.wstages * 64u + (uint32_t)(16 * g + 4 * (j & 3))) * 4u;
@@ -225,7 +225,7 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
             for (int t = 0; t < 4; t++) raw[t] = v[t];
         } else {
 #pragma unroll
-            for (int r = 0; r < 4; r++) raw[r] = *(const uint32_t*)(src + (SRC == W_ROWS16 ? 64 * (4 * g + r) + 4 * j : 256 * r + 4 * lane));
+            for (int r = 0; r < 4; r++) raw[r] = *(const uint32_t*)(src + 256 * r + 4 * lane);
         }
     };
     // Decode of a raw dword's 16 codes: code c of its four bytes becomes the high bytes of four operand values by one table

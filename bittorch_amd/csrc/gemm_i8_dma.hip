@@ -127,15 +127,18 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
     const int nst = (int)((p.K + D_BK - 1) / D_BK);
     const int64_t k_last = (int64_t)(nst - 1) * D_BK;
 
-    // A stage's row is 64 bytes of LDS, four pieces of 16; piece q of row r lies at place q ^ (r / 4 % 4), so that the 16 rows of
-    // a fragment read meet every bank once.  Four lanes load a row: lanes of a load that each have a row of their own take the
-    // cache four times as long.  Rows past M repeat the last one (their outputs are never stored); columns past N read column 0
-    // of row-major weights and the last tile of the copy.
+    // A stage's row is 64 bytes of LDS, four pieces of 16; piece q of row r lies at place q ^ (r / 4 & 2).  A 16-byte read from
+    // LDS takes its lanes in groups that hold rows 0 .. 3 and 12 .. 15 of one piece with rows 4 .. 11 of the next, so it meets
+    // every bank once.  (With q ^ (r / 4 % 4), and row-major weights as [row][64 columns], 7.5 M of the 15.5 M LDS cycles of
+    // 2048 x 11008 x 4096 were conflicts, now none of 8.0 M; us a call, 4096 x 11008 x 4096 180.4 -> 176.4, 4096 x 13824 x 2560
+    // 143.7 -> 140.9, 4096 x 2560 x 6912 91.6 -> 89.2.)  Four lanes load a row: lanes of a load that each have a row of their
+    // own take the cache four times as long.  Rows past M repeat the last one (their outputs are never stored); columns past N
+    // read column 0 of row-major weights and the last tile of the copy.
     const int64_t rows_left = (p.M - m0 < BM) ? p.M - m0 : BM;
     uint32_t a_off[A_LOADS], a_tail[A_LOADS];
 #pragma unroll
     for (int b = 0; b < A_LOADS; b++) {
-        const int row = 16 * ((A_LOADS * wave + b) % (2 * NB)) + (lane >> 2), piece = (lane & 3) ^ (lane >> 4);
+        const int row = 16 * ((A_LOADS * wave + b) % (2 * NB)) + (lane >> 2), piece = (lane & 3) ^ ((lane >> 4) & 2);
         const uint32_t r = (uint32_t)(row < rows_left ? row : rows_left - 1);
         a_off[b] = r * (uint32_t)p.K + 16u * piece;
         a_tail[b] = r * (uint32_t)p.K + (k_last + 16 * piece < p.K ? 16u * piece : 0u);
@@ -150,14 +153,14 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
         }
     } else if constexpr (SRC == W_ROWS16) {
         const int64_t col = (int64_t)tile_n * G_BN + 64 * wave + 16 * (lane & 3);
-        w_off[0] = (uint32_t)(col < p.N ? col : 0) + (uint32_t)(lane >> 2) * (uint32_t)p.N;
-        w_tail[0] = (uint32_t)(col < p.N ? col : 0) + (uint32_t)min((int64_t)(lane >> 2), p.Kb - 1 - (k_last >> 2)) * (uint32_t)p.N;
+        w_off[0] = (uint32_t)(col < p.N ? col : 0) + (uint32_t)rows16_row(lane) * (uint32_t)p.N;
+        w_tail[0] = (uint32_t)(col < p.N ? col : 0) + (uint32_t)min((int64_t)rows16_row(lane), p.Kb - 1 - (k_last >> 2)) * (uint32_t)p.N;
     } else {
         const int tt = stored_tile16((int)(ncol >> 4), p.tiles16);
         w_off[0] = ((uint32_t)tt * (uint32_t)p.wsteps * 64u + (uint32_t)(16 * g + 4 * (j & 3))) * 4u;
     }
     const int8_t* const a_base = p.Q + m0 * p.K;  // uniform
-    const uint32_t frag_at = 64u * j + 16u * (g ^ (j >> 2));  // lane (j, g): k = 16 g .. +15 of row j of a block
+    const uint32_t frag_at = 64u * j + 16u * (g ^ ((j >> 2) & 2));  // lane (j, g): k = 16 g .. +15 of row j of a block
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
 
     // the next stage to load: its global addresses, and the byte offset of its buffer
@@ -210,7 +213,7 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
         const uint8_t* src = lds + buf + A_BYTES + wave * 1024;
         if constexpr (SRC <= W_ROWS16) {
 #pragma unroll
-            for (int r = 0; r < 4; r++) raw[r] = *(const uint32_t*)(src + (SRC == W_ROWS16 ? 64 * (4 * g + r) + 4 * j : 256 * r + 4 * lane));
+            for (int r = 0; r < 4; r++) raw[r] = *(const uint32_t*)(src + 256 * r + 4 * lane);
             if (TAIL && s >= nst - 1) {
 #pragma unroll
                 for (int r = 0; r < 4; r++) raw[r] = w_in ? raw[r] : 0u;

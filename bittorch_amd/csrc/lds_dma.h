@@ -18,10 +18,11 @@ __device__ __forceinline__ void dma4(uint32_t lds_off, uint32_t voff, const void
 // Where a wave's packed weights come from, per stage of 64 k: 16 rows of 64 columns of row-major W_T, lane (j, g) decoding the
 // four bytes of its columns 4 j .. +3 in its rows 4 g .. +3.
 //   W_ROWS    four 4-byte loads a lane, a row each; LDS holds [r][lane]
-//   W_ROWS16  N % 16 == 0 and W_T 16-byte aligned: one 16-byte load a lane (row lane / 4, columns 16 (lane % 4) .. +15); LDS
-//             holds [row][64 columns].  A quarter of the requests: 2048 x 4096 x 4096 bf16 59 -> 54 us
+//   W_ROWS16  N % 16 == 0 and W_T 16-byte aligned: one 16-byte load a lane (row rows16_row(lane), columns 16 (lane % 4) .. +15),
+//             so that LDS holds the same [r][lane].  A quarter of the requests: 2048 x 4096 x 4096 bf16 59 -> 54 us
 //   W_TILES   the decode-tiled copy, W_FIELDS its field layout: one 16-byte load a lane, its four columns
 enum { W_ROWS = 0, W_ROWS16 = 1, W_TILES = 2, W_FIELDS = 3 };
+__device__ __forceinline__ int rows16_row(int lane) { return 4 * ((lane >> 2) & 3) + (lane >> 4); }  // lane (j, g) / 4 of LDS row r
 static inline int w_source(bool tiled, bool fields, const void* W, int64_t N) {
     if (tiled) return fields ? W_FIELDS : W_TILES;
     return N % 16 == 0 && ((uintptr_t)W) % 16 == 0 ? W_ROWS16 : W_ROWS;
