@@ -19,19 +19,20 @@
 namespace bt {
 
 constexpr int D_BK = 64;   // k per stage
-constexpr int D_NST = 5;   // stages in LDS (60 KiB: what M0's 16-bit byte offset reaches)
+// stages in LDS: 30 to 60 KiB, two groups of waves 60 (NB = 1) and 64 KiB (what M0's 16-bit byte offset reaches)
+constexpr int d_stages(int NB, int KG) { return KG == 2 && NB == 2 ? 4 : 5; }
 
 // Output stage: row block by row block, addresses as a uniform row base plus a lane offset fixed for the whole tile.  The
 // empty asm statements keep a row's address from being computed ahead of its turn (left alone, the compiler holds all 32
 // row addresses and residual values at once and spills).
 // RN: rows of any length, so that a lane's four columns start on any element and the last ones may be fewer.
-template <int NB, bool FL, bool RN>
-__device__ __forceinline__ void dma_store_acc(const GemmParams& p, const v4i (&acc)[2 * NB][4], int64_t m0, int g, int64_t ncol,
+template <bool FL, bool RN, int MB>
+__device__ __forceinline__ void dma_store_acc(const GemmParams& p, const v4i (&acc)[MB][4], int64_t m0, int g, int64_t ncol,
                                               int rows_left) {
     const uint32_t lane_off = (uint32_t)(4 * g) * (uint32_t)p.N * 4u + (uint32_t)(ncol & (G_BN - 1)) * 4u;
     char* row = (char*)p.acc_out + (m0 * p.N + (int64_t)__builtin_amdgcn_readfirstlane((int)(ncol / G_BN)) * G_BN) * 4;
 #pragma unroll
-    for (int mb = 0; mb < 2 * NB; mb++) {
+    for (int mb = 0; mb < MB; mb++) {
         if (16 * mb >= rows_left) return;  // (uniform)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
@@ -53,8 +54,8 @@ __device__ __forceinline__ void dma_store_acc(const GemmParams& p, const v4i (&a
         __builtin_amdgcn_sched_barrier(0);
     }
 }
-template <int YDT, bool RES, int NB, bool FL, bool RN>
-__device__ __forceinline__ void dma_epilogue(const GemmParams& p, const v4i (&acc)[2 * NB][4], int64_t m0, int g, int64_t ncol,
+template <int YDT, bool RES, bool FL, bool RN, int MB>
+__device__ __forceinline__ void dma_epilogue(const GemmParams& p, const v4i (&acc)[MB][4], int64_t m0, int g, int64_t ncol,
                                              int rows_left, const float* sx_lds, const float (&ws)[4], const float (&bs)[4]) {
     constexpr int ES = (YDT == BT_F32) ? 4 : 2;
     const uint32_t lane_off = ((uint32_t)(4 * g) * (uint32_t)p.N + (uint32_t)(ncol & (G_BN - 1))) * ES;
@@ -63,7 +64,7 @@ __device__ __forceinline__ void dma_epilogue(const GemmParams& p, const v4i (&ac
     char* row = (char*)p.Y + first;
     const char* res = (const char*)p.epi.residual + first;
 #pragma unroll
-    for (int mb = 0; mb < 2 * NB; mb++) {
+    for (int mb = 0; mb < MB; mb++) {
         if (16 * mb >= rows_left) return;  // (uniform)
         const float4 s4 = *(const float4*)(sx_lds + 16 * mb + 4 * g);
         const float sx[4] = {s4.x, s4.y, s4.z, s4.w};
@@ -109,23 +110,28 @@ __device__ __forceinline__ void dma_epilogue(const GemmParams& p, const v4i (&ac
     }
 }
 
-constexpr int dma_lds_bytes(int NB) { return D_NST * (2 * NB * 1024 + 4096); }
+constexpr int dma_group_bytes(int NB, int KG) { return d_stages(NB, KG) * (2 * NB * 1024 + 4096); }
 
 // One tile of 32 NB rows.  TAIL: K is not a multiple of the stage.  The activations past the end of K are some of the same
 // row's and meet weights of zero: the tiled copy is padded with them, raw row-major dwords are masked.  (Where the activation
 // rows are longer than the weights' K, zeros meet a repetition of the last packed row.)
-template <int SRC, int NB, bool TAIL, bool RN>
-__device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int64_t m0, const int tile_n, uint8_t* lds) {
-    constexpr int BM = 32 * NB;
+// KG = 2: two groups of four waves, each on its run of the stages; they add their sums through LDS and store half the rows each.
+template <int SRC, int NB, int KG, bool TAIL, bool RN>
+__device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int64_t m0, const int tile_n, uint8_t* lds_all) {
+    constexpr int BM = 32 * NB, D_NST = d_stages(NB, KG);
     constexpr int A_BYTES = 2 * NB * 1024, STAGE = A_BYTES + 4096;
     constexpr int A_LOADS = NB == 4 ? 2 : 1, W_LOADS = SRC == W_ROWS ? 4 : 1, LOADS = A_LOADS + W_LOADS;
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = wave_all & 3, group = KG == 1 ? 0 : wave_all >> 2;
+    uint8_t* const lds = lds_all + group * dma_group_bytes(NB, KG);
     const int j = lane & 15, g = lane >> 4;
     const int64_t ncol = (int64_t)tile_n * G_BN + 64 * wave + 4 * j;
     const bool col_ok = ncol < p.N;
     const int nst = (int)((p.K + D_BK - 1) / D_BK);
     const int64_t k_last = (int64_t)(nst - 1) * D_BK;
+    // this group's stages: st0 .. st0 + mine - 1 (every group meets `rounds` barriers in the loop; mine >= 1)
+    const int rounds = KG == 1 ? nst : (nst + 1) / 2, st0 = group * rounds, mine = KG == 1 ? nst : min(rounds, nst - st0);
+    const int st_tail = group == KG - 1 ? mine - 1 : nst;  // TAIL: the partial stage, if it is this group's
 
     // A stage's row is 64 bytes of LDS, four pieces of 16; piece q of row r lies at place q ^ (r / 4 & 2).  A 16-byte read from
     // LDS takes its lanes in groups that hold rows 0 .. 3 and 12 .. 15 of one piece with rows 4 .. 11 of the next, so it meets
@@ -164,17 +170,17 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
 
     // the next stage to load: its global addresses, and the byte offset of its buffer
-    const int8_t* a_next = a_base;
-    const uint8_t* w_next = p.W_T;
+    const int64_t w_step = SRC <= W_ROWS16 ? 16 * p.N : 256;
+    const int8_t* a_next = a_base + (int64_t)st0 * D_BK;
+    const uint8_t* w_next = p.W_T + st0 * w_step;
     uint32_t into = 0;
     int st_next = 0;
-    const int64_t w_step = SRC <= W_ROWS16 ? 16 * p.N : 256;
     auto issue_a = [&](int b) {
-        const bool last = TAIL && st_next >= nst - 1;
+        const bool last = TAIL && st_next >= st_tail;
         dma16(lds0 + into + (uint32_t)((A_LOADS * wave + b) % (2 * NB)) * 1024u, last ? a_tail[b] : a_off[b], a_next);
     };
     auto issue_w = [&](int r) {
-        const bool last = TAIL && st_next >= nst - 1;
+        const bool last = TAIL && st_next >= st_tail;
         const uint32_t wd = lds0 + into + A_BYTES + (uint32_t)wave * 1024u;
         if constexpr (SRC == W_ROWS) dma4(wd + 256u * r, last ? w_tail[r] : w_off[r], w_next);
         else dma16(wd, SRC == W_ROWS16 && last ? w_tail[0] : w_off[0], w_next);
@@ -182,8 +188,8 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
     auto next_buf = [](uint32_t b) { return b + STAGE == D_NST * STAGE ? 0u : b + STAGE; };
     auto advance = [&]() {  // past the end: the last stage again, never read
         st_next++;
-        a_next += st_next < nst ? D_BK : 0;
-        w_next += st_next < nst ? w_step : 0;
+        a_next += st_next < mine ? D_BK : 0;
+        w_next += st_next < mine ? w_step : 0;
         into = next_buf(into);
     };
 
@@ -214,7 +220,7 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
         if constexpr (SRC <= W_ROWS16) {
 #pragma unroll
             for (int r = 0; r < 4; r++) raw[r] = *(const uint32_t*)(src + 256 * r + 4 * lane);
-            if (TAIL && s >= nst - 1) {
+            if (TAIL && s >= st_tail) {
 #pragma unroll
                 for (int r = 0; r < 4; r++) raw[r] = w_in ? raw[r] : 0u;
             }
@@ -328,12 +334,34 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
         __builtin_amdgcn_sched_barrier(0);
     };
     int s = 0;
-    for (; s + 1 < nst; s += 2) {
+    for (; s + 1 < mine; s += 2) {
         stage(s, b_dec[0], b_dec[1]);
         stage(s + 1, b_dec[1], b_dec[0]);
     }
-    if (s < nst) stage(s, b_dec[0], b_dec[1]);
+    if (s < mine) stage(s, b_dec[0], b_dec[1]);
+    if (KG > 1 && mine < rounds) asm volatile("s_barrier" ::: "memory");  // (uniform; the other group has one stage more)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (no load may reach LDS that another workgroup owns by then)
+
+    v4i sums[KG == 1 ? 1 : NB][4];
+    if constexpr (KG > 1) {
+        // group 0 takes the first NB row blocks, group 1 the others: each hands over the sums that it does not store
+        v4i* const given = (v4i*)lds_all + wave_all * (256 * NB) + lane;
+        const v4i* const taken = (const v4i*)lds_all + (wave_all ^ 4) * (256 * NB) + lane;
+        __syncthreads();  // (both groups have read their last stages)
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                given[64 * (4 * i + t)] = group ? acc[i][t] : acc[NB + i][t];
+                sums[i][t] = group ? acc[NB + i][t] : acc[i][t];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) sums[i][t] += taken[64 * (4 * i + t)];
+        __syncthreads();  // (the row scales come over them)
+    }
 
     // ---- output.  The row scales of the tile pass through the wave's own weight area in LDS (nobody else's loads reach it),
     // so that a row block's four come with one read. ----
@@ -357,23 +385,32 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
         bs[t] = p.epi.bias ? bits_to_f32_rt(bs_bits[t], p.epi.bias_dtype) : 0.0f;
     }
     if (!col_ok) return;
-    if (p.acc_out) dma_store_acc<NB, SRC == W_FIELDS, RN>(p, acc, m0, g, ncol, (int)rows_left);
-    if (p.y_dtype == BT_BF16) {
-        if (p.epi.residual) dma_epilogue<BT_BF16, true, NB, SRC == W_FIELDS, RN>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
-        else dma_epilogue<BT_BF16, false, NB, SRC == W_FIELDS, RN>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
-    } else if (p.y_dtype == BT_F16) {
-        if (p.epi.residual) dma_epilogue<BT_F16, true, NB, SRC == W_FIELDS, RN>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
-        else dma_epilogue<BT_F16, false, NB, SRC == W_FIELDS, RN>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
+    constexpr bool FL = SRC == W_FIELDS;
+    auto store = [&](const auto& v, int64_t row0, int left, const float* sx) {
+        if (p.acc_out) dma_store_acc<FL, RN>(p, v, row0, g, ncol, left);
+        if (p.y_dtype == BT_BF16) {
+            if (p.epi.residual) dma_epilogue<BT_BF16, true, FL, RN>(p, v, row0, g, ncol, left, sx, ws, bs);
+            else dma_epilogue<BT_BF16, false, FL, RN>(p, v, row0, g, ncol, left, sx, ws, bs);
+        } else if (p.y_dtype == BT_F16) {
+            if (p.epi.residual) dma_epilogue<BT_F16, true, FL, RN>(p, v, row0, g, ncol, left, sx, ws, bs);
+            else dma_epilogue<BT_F16, false, FL, RN>(p, v, row0, g, ncol, left, sx, ws, bs);
+        } else {
+            if (p.epi.residual) dma_epilogue<BT_F32, true, FL, RN>(p, v, row0, g, ncol, left, sx, ws, bs);
+            else dma_epilogue<BT_F32, false, FL, RN>(p, v, row0, g, ncol, left, sx, ws, bs);
+        }
+    };
+    if constexpr (KG == 1) {
+        store(acc, m0, (int)rows_left, sx_lds);
     } else {
-        if (p.epi.residual) dma_epilogue<BT_F32, true, NB, SRC == W_FIELDS, RN>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
-        else dma_epilogue<BT_F32, false, NB, SRC == W_FIELDS, RN>(p, acc, m0, g, ncol, (int)rows_left, sx_lds, ws, bs);
+        const int first = 16 * NB * group;
+        if (rows_left > first) store(sums, m0 + first, (int)rows_left - first, sx_lds + first);
     }
 }
 
 // NB: tiles of 32 NB rows.  NF > 0: the last p.fine_from .. of an XCD's tiles are computed in tiles of 32 NF rows.
-template <int SRC, int NB, int NF, bool TAIL, bool RN>
-__global__ __launch_bounds__(256, NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_i8_dma_kernel(GemmParams p) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[dma_lds_bytes(NB)];
+template <int SRC, int NB, int NF, int KG, bool TAIL, bool RN>
+__global__ __launch_bounds__(256 * KG, KG == 2 || NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_i8_dma_kernel(GemmParams p) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds[KG * dma_group_bytes(NB, KG)];
     // XCD-aware tile order, as in gemm_i8_kernel
     const uint32_t idx = blockIdx.x >> 3;
     const bool fine = NF > 0 && idx >= (uint32_t)p.fine_from;  // (uniform)
@@ -392,12 +429,20 @@ __global__ __launch_bounds__(256, NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_i8_dm
     if constexpr (NF > 0) {
         if (fine) {
             const int64_t mf = m0 + (int64_t)(f % parts) * (32 * NF);
-            if (mf < p.M) gemm_i8_dma_tile<SRC, NF, TAIL, RN>(p, mf, (int)tn, lds);
+            if (mf < p.M) gemm_i8_dma_tile<SRC, NF, 1, TAIL, RN>(p, mf, (int)tn, lds);
             return;
         }
     }
-    gemm_i8_dma_tile<SRC, NB, TAIL, RN>(p, m0, (int)tn, lds);
+    gemm_i8_dma_tile<SRC, NB, KG, TAIL, RN>(p, m0, (int)tn, lds);
 }
+
+// A launch of one tile of 64 or 32 rows for each compute unit at most: two groups of waves, half of the stages each, so that a
+// SIMD has two waves where one's chain of LDS reads, decode and MFMAs left it idle half of the time.  One / two groups, us a
+// call with the quantizer, row-major weights: tiles of 32 rows, 256 x 7680 x 2560 18.7 / 17.1, 512 x 4096 x 11008 50.0 / 42.2;
+// of 64 rows, 256 x 11008 x 4096 28.2 / 24.0, 1000 x 2560 x 6912 42.5 / 34.9, 1000 x 4096 x 11008 62.8 / 51.8.  The gain grows
+// with K; below 24 stages it is lost in the exchange of the sums.  The field layout keeps one group (its sums start at minus
+// the row sums).
+static bool i8_splits_k(int64_t stages) { return stages >= 24; }
 
 // Rows of the tiles in units of 32 (4, 2 or 1), or 0 where gemm_i8_kernel is the better one: tiled weights in whole stages
 // with at most one tile of 128 x 256 for each compute unit.  There a second workgroup has nothing to do, and splitting K
@@ -412,8 +457,9 @@ static int gemm_i8_dma_plan(int64_t M, int64_t N, int64_t K, bool tiled, double*
     const int64_t t4 = ceil_div(M, 128) * tn, t2 = ceil_div(M, 64) * tn, t1 = ceil_div(M, 32) * tn;
     if (tiled && K % 128 == 0 && N % 4 == 0 && t4 <= C) return 0;
     const bool whole = gemm_whole_tiles();
-    if (t1 <= C && !whole) { *us = 5.2 + 0.0035 * (double)K; return 1; }
-    if (t2 <= C && !whole) { *us = 5.2 + 0.0045 * (double)K; return 2; }
+    const bool split = i8_splits_k(ceil_div(K, D_BK));
+    if (t1 <= C && !whole) { *us = split ? 5.7 + 0.0027 * (double)K : 5.2 + 0.0035 * (double)K; return 1; }
+    if (t2 <= C && !whole) { *us = split ? 5.5 + 0.0034 * (double)K : 5.2 + 0.0045 * (double)K; return 2; }
     const int parts = gemm_dma_parts(t4);
     const double n4 = parts == 1 ? (double)ceil_div(t4, C) : (double)(2 * (t4 / (2 * C))) + (parts == 2 ? 1.2 : 0.6);
     const double p4 = n4 * (3.5 + 0.0055 * (double)K), p2 = (double)ceil_div(t2, C) * (2.2 + 0.0029 * (double)K);
@@ -451,12 +497,18 @@ static int launch_gemm_i8_dma_src(GemmParams p, hipStream_t st) {
             const int rem = p.per_xcd % (int)(2 * gemm_compute_units() / 8);
             p.fine_from = p.per_xcd - rem;
             const dim3 grid((unsigned)(8 * (p.fine_from + parts * rem)));
-            if (parts == 2) hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, 4, 2, TAIL, RN>), grid, block, 0, st, p);
-            else hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, 4, 1, TAIL, RN>), grid, block, 0, st, p);
+            if (parts == 2) hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, 4, 2, 1, TAIL, RN>), grid, block, 0, st, p);
+            else hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, 4, 1, 1, TAIL, RN>), grid, block, 0, st, p);
             return check_launch("bt_ternary_gemm_i8");
         }
     }
-    hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, NB, 0, TAIL, RN>), dim3((unsigned)(8 * p.per_xcd)), block, 0, st, p);
+    if constexpr (NB != 4 && SRC != W_FIELDS) {
+        if (total <= gemm_compute_units() && i8_splits_k(ceil_div(p.K, D_BK))) {
+            hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, NB, 0, 2, TAIL, RN>), dim3((unsigned)(8 * p.per_xcd)), dim3(512), 0, st, p);
+            return check_launch("bt_ternary_gemm_i8");
+        }
+    }
+    hipLaunchKernelGGL((gemm_i8_dma_kernel<SRC, NB, 0, 1, TAIL, RN>), dim3((unsigned)(8 * p.per_xcd)), block, 0, st, p);
     return check_launch("bt_ternary_gemm_i8");
 }
 template <int NB>

@@ -50,3 +50,11 @@ def test_operand_order_equals_row_major_activations(m, n, k, dtype):
         yw, aw = _C.ternary_gemm_int8(qo, so, wt, scale, bias, k, q_operand_order=True, **kw)
         set_option("GEMM_TAIL_SPLIT", None)
         assert torch.equal(aw, exact) and torch.equal(yw, y)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(33, 260, 1536), (97, 1004, 1552), (250, 516, 1584), (640, 5000, 1616), (129, 1024, 2112)])
+def test_stages_in_two_groups(m, n, k, dtype):
+    """Launches of at most one tile a compute unit, 24 stages and more: even and odd numbers of stages, a remainder of K in the
+    second group, rows that end in either group's half of a tile, tiles of 32 and 64 rows."""
+    test_operand_order_equals_row_major_activations(m, n, k, dtype)
