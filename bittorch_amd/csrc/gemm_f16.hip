@@ -11,7 +11,8 @@
 // workgroups share a compute unit, so that one's MFMAs run while the other waits, starts, drains or stores (a 512-thread
 // workgroup that split K over the two waves of a SIMD: 6.9 us a round of tiles with nothing beside it, fp16 / bf16 row-major
 // weights, 4096 x 11008 x 4096 338 -> 260 us, tiled 300 -> 257; 16384 x 768 x 768 30 -> 21.5; 512 x 4096 x 4096 49 -> 31).
-// Bound by the issue of a stage, 64 MFMAs (1024 cycles) and some 150 other instructions: 1.43 PFLOP/s at that size.
+// Bound by the issue of a stage, 64 MFMAs (1024 cycles) and some 150 other
+// instructions, 80 of them vector ones: 1.46 PFLOP/s at that size (252 us).
 // Activations and packed weights go to LDS by global_load_lds, three stages of 64 k.  The order of k inside an MFMA is free:
 // lane (j, g) of the stage's first sub-step takes k = 16 g .. +7 and of the second 16 g + 8 .. +15, so the 16 weight bytes a
 // lane loads are all its own, and the weights are decoded in natural order, so the activations are fed as they lie in memory.
