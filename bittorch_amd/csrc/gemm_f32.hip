@@ -88,7 +88,9 @@ constexpr uint32_t LUT_BF16_HALF = 0x00BF3F00u;
 // KS > 1: all KS waves of a workgroup work on one tile, each on its run of the contraction, and add their sums through LDS
 // (pairwise, always in the same order): for outputs with too few tiles to occupy the chip.
 // SC: X's columns are scaled (input gradient with one scale per row of W).
-template <int SRC, int NG, int KS, bool SC>
+// RN: forward outputs of N % 4 != 0, an instance of its own: asked at run time, every other output paid half a microsecond for
+// the clamped columns and the second way to store (us, fp32, 300 x 4096 x 512 17.9 / 17.0, 4096 x 768 x 768 28.2 / 27.5).
+template <int SRC, int NG, int KS, bool SC, bool RN>
 __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(GemmF32Params p) {
     constexpr int TM = (KS == 1) ? 128 : 64, TN = (KS == 1) ? 128 * NG : 64 * NG;  // a workgroup's tile
     // the 8 XCDs each take a contiguous run of tiles, walked in groups of four row tiles (as in gemm_f16.hip)
@@ -118,13 +120,13 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
         a_off[b] = (r * (uint32_t)p.C + 8u * g) * 4u;
     }
     uint32_t b_off[NG];
-    uint32_t b_shift = 0;  // row-major rows of N % 4 != 0: bits by which the last columns, loaded as the last four, stand too high
+    uint32_t b_shift = 0;  // RN: bits by which the last columns, loaded as the last four, stand too high
 #pragma unroll
     for (int q = 0; q < NG; q++) {
         const int64_t col = c0 + 64 * q + 4 * i;
         if constexpr (SRC == B_ROW_MAJOR) {
-            b_off[q] = 2u * g * (uint32_t)p.ldw + (uint32_t)(col < p.NC - 4 ? col : p.NC - 4);
-            if (col < p.NC && col > p.NC - 4) b_shift = 8u * (uint32_t)(col - (p.NC - 4));  // (one q at most)
+            b_off[q] = 2u * g * (uint32_t)p.ldw + (uint32_t)(col < (RN ? p.NC - 4 : p.NC) ? col : p.NC - 4);
+            if (RN && col < p.NC && col > p.NC - 4) b_shift = 8u * (uint32_t)(col - (p.NC - 4));  // (one q at most)
         } else if constexpr (SRC == B_TILED) {
             const int tt = stored_tile16((int)(col >> 4), p.tiles16);
             b_off[q] = ((uint32_t)tt * (uint32_t)p.wsteps * 64u + 16u * (g >> 1) + 4u * (i & 3)) * 4u;
@@ -230,14 +232,12 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
 
     auto step = [&](int nx, bool more, auto any) __attribute__((always_inline)) {  // nx: the step whose operands are requested behind this one's use (uniform)
         u32x4 w[4 * NG];
-        if constexpr (SRC == B_ROW_MAJOR) {
-            if (p.NC % 4 != 0) {  // (uniform)
+        if constexpr (RN && SRC == B_ROW_MAJOR) {
 #pragma unroll
-                for (int q = 0; q < NG; q++)
+            for (int q = 0; q < NG; q++)
 #pragma unroll
-                    for (int r = 0; r < 2; r++)
-                        if (c0 + 64 * q + 4 * i > p.NC - 4) braw[q][r] >>= b_shift;
-            }
+                for (int r = 0; r < 2; r++)
+                    if (c0 + 64 * q + 4 * i > p.NC - 4) braw[q][r] >>= b_shift;
         }
 #pragma unroll
         for (int q = 0; q < NG; q++)
@@ -337,7 +337,7 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
         if constexpr (SRC != B_TRANSPOSED) {
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                const int64_t n = col + t < p.NC ? col + t : p.NC - 1;
+                const int64_t n = !RN || col + t < p.NC ? col + t : p.NC - 1;
                 ws[t] = epi_scale(p.epi, n);
                 bs[t] = epi_bias(p.epi, n);
             }
@@ -365,7 +365,7 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
                 } else {
 #pragma unroll
                     for (int t = 0; t < 4; t++) y[t] = epi_float(y[t], ws[t], bs[t]);
-                    if (p.NC % 4 != 0) {  // rows of any length: element by element
+                    if constexpr (RN) {  // element by element
 #pragma unroll
                         for (int t = 0; t < 4; t++) {
                             if (col + t >= p.NC) continue;
@@ -382,7 +382,7 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
     }
 }
 
-template <int SRC, int NG, int KS, bool SC>
+template <int SRC, int NG, int KS, bool SC, bool RN>
 static int launch_gemm_f32_cfg(GemmF32Params p, const char* who, hipStream_t st) {
     p.tiles_m = (int)ceil_div(p.M, KS == 1 ? 128 : 64);
     p.tiles_n = (int)ceil_div(p.NC, KS == 1 ? 128 * NG : 64 * NG);
@@ -392,7 +392,7 @@ static int launch_gemm_f32_cfg(GemmF32Params p, const char* who, hipStream_t st)
         return BT_ERR_INVALID;
     }
     p.per_xcd = (int)ceil_div(total, 8);
-    hipLaunchKernelGGL((gemm_f32_kernel<SRC, NG, KS, SC>), dim3((unsigned)(p.per_xcd * 8)), dim3(KS == 1 ? 256 : 64 * KS), 0, st, p);
+    hipLaunchKernelGGL((gemm_f32_kernel<SRC, NG, KS, SC, RN>), dim3((unsigned)(p.per_xcd * 8)), dim3(KS == 1 ? 256 : 64 * KS), 0, st, p);
     return check_launch(who);
 }
 // Which split of the work?  0: tiles of 64 x 128 per wave, 1: the same with the contraction over the four waves of a
@@ -420,13 +420,17 @@ static int gemm_f32_config(int64_t M, int64_t NC, int64_t C) {
 // microseconds of launch_gemm_f32, for the rule that chooses between it and the streaming kernel
 double gemm_f32_cost(int64_t M, int64_t N, int64_t K) { return gemm_f32_price(M, N, K, gemm_f32_config(M, N, K)); }
 
-template <int SRC, bool SC>
+template <int SRC, bool SC, bool RN = false>
 static int launch_gemm_f32_src(const GemmF32Params& p, const char* who, hipStream_t st) {
     switch (gemm_f32_config(p.M, p.NC, p.C)) {
-        case 0: return launch_gemm_f32_cfg<SRC, 2, 1, SC>(p, who, st);
-        case 1: return launch_gemm_f32_cfg<SRC, 2, 4, SC>(p, who, st);
-        default: return launch_gemm_f32_cfg<SRC, 1, 8, SC>(p, who, st);
+        case 0: return launch_gemm_f32_cfg<SRC, 2, 1, SC, RN>(p, who, st);
+        case 1: return launch_gemm_f32_cfg<SRC, 2, 4, SC, RN>(p, who, st);
+        default: return launch_gemm_f32_cfg<SRC, 1, 8, SC, RN>(p, who, st);
     }
+}
+template <int SRC>
+static int launch_gemm_f32_forward(const GemmF32Params& p, const char* who, hipStream_t st) {
+    return p.NC % 4 != 0 ? launch_gemm_f32_src<SRC, false, true>(p, who, st) : launch_gemm_f32_src<SRC, false>(p, who, st);
 }
 
 // the kernel's 32-bit offsets span 64 rows of X and the whole of W
@@ -446,8 +450,8 @@ int launch_gemm_f32(const void* X, const uint8_t* W, int w_layout, const Epilogu
     p.tiles16 = tiles16_arg(N, w_layout);
     p.ldw = (int)N;
     p.kb = (int)ceil_div(K, 4);
-    return layout_tiled(w_layout) ? launch_gemm_f32_src<B_TILED, false>(p, "bt_ternary_linear_tiled_forward", st)
-                                  : launch_gemm_f32_src<B_ROW_MAJOR, false>(p, "bt_ternary_linear_packed_forward", st);
+    return layout_tiled(w_layout) ? launch_gemm_f32_forward<B_TILED>(p, "bt_ternary_linear_tiled_forward", st)
+                                  : launch_gemm_f32_forward<B_ROW_MAJOR>(p, "bt_ternary_linear_packed_forward", st);
 }
 
 // ---- weight gradient ---------------------------------------------------------------------------------------------------
