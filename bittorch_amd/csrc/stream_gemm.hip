@@ -56,8 +56,8 @@ struct StreamParams {
     int per_xcd;          // tiles per XCD (grid = 8 * per_xcd)
     int tiles16;          // LD_T*: 16-column tiles of the decode-tiled weights (< 0: stored_tile16)
     int M;                // 1..16: rows of a 16-row block (of the last one when the launch covers several)
-    int x_vec_ok;         // activation rows are read with 16-byte loads: they hold at least one group of 16 bytes
-    int x_ragged;         // rows are no whole number of such groups: the last one is shifted into place (shift_group)
+    int x_vec_ok;         // activation rows are aligned and whole groups of 16 bytes
+    int x_ragged;         // they are not, but hold at least one group: the last one is shifted into place (shift_group)
     int64_t B;            // rows of the whole call: grid.y = ceil(B / 16) blocks of 16 rows, all in one launch
     const float* s_x;     // MODE_I8: per-row activation scales [M]
     void* Y;              // [M, N] of y_dtype
@@ -116,23 +116,26 @@ __device__ __forceinline__ uint32_t add_bits(uint32_t a, uint32_t b) {
 }
 
 // 16 bytes of activations of row i starting at element k, in natural k order.
-// XV: the row holds at least one group of 16 bytes.  The load is unconditional, on an address clamped to the row's last
-// group, and wherever a row starts (xrow = element offset of row min(i, M-1)); the caller zeroes groups at k >= K, and shifts
-// the one that crosses the row's end into place, when it consumes them: a load under a per-lane predicate becomes a branch
-// with a wait behind it, which serialises the stream (a gather by element took 152 us for 37 rows of 10447 bf16 values times
-// 11152 columns, 67 this way).  !XV: element-wise gather of shorter rows, zero filled.
+// X_GROUPS: rows are aligned and whole groups of 16 bytes; X_RAGGED: they start anywhere and hold at least one group.  The load
+// is unconditional, on an address clamped to the row's last group (xrow = element offset of row min(i, M-1)); the caller zeroes
+// groups at k >= K, and shifts the one that crosses the end of a ragged row into place, when it consumes them: a load under a
+// per-lane predicate becomes a branch with a wait behind it, which serialises the stream (a gather by element took 152 us for
+// 37 rows of 10447 bf16 values times 11152 columns, 67 this way).  X_SHORT: element-wise gather of shorter rows, zero filled.
+// The kernel has a branch for each: with the first two in one, 256 x 2560 x 6912 bf16 took 43.2 us, 41.5 this way.
+enum { X_GROUPS = 0, X_RAGGED = 1, X_SHORT = 2 };
 template <int MODE>
 __device__ __forceinline__ uint4 load_x16_any(const void* src) {
     typedef typename std::conditional<MODE == MODE_I8, u32x4_a1, u32x4_a2>::type vec;
     const vec v = *(const vec*)src;
     return make_uint4(v[0], v[1], v[2], v[3]);
 }
-template <int MODE, bool XV>
+template <int MODE, int XS>
 __device__ __forceinline__ uint4 load_x16(const StreamParams& p, uint32_t xrow, int i, int k) {
     constexpr int GE = (MODE == MODE_I8) ? 16 : 8;
     constexpr int ES = (MODE == MODE_I8) ? 1 : 2;
-    if constexpr (XV) {
+    if constexpr (XS != X_SHORT) {
         const uint32_t kc = (uint32_t)min(k, (int)p.K - GE);
+        if constexpr (XS == X_GROUPS) return *(const uint4*)((const uint8_t*)p.X + (xrow + kc) * ES);
         return load_x16_any<MODE>((const uint8_t*)p.X + (xrow + kc) * ES);
     } else {
         uint32_t d[4] = {0u, 0u, 0u, 0u};
@@ -452,8 +455,13 @@ __global__ __launch_bounds__(WAVES * 64) void stream_kernel(StreamParams p_in) {
 #pragma unroll
                 for (int f = 0; f < PF; f++)
 #pragma unroll
-                    for (int h = 0; h < XN; h++) xa[f][h] = load_x16<MODE, true>(p, xrow, j, k0 + f * 64 + 8 * h);
-                if (p.x_ragged && base + PF >= nsteps) {  // (uniform: the batch with the row's end)
+                    for (int h = 0; h < XN; h++) xa[f][h] = load_x16<MODE, X_GROUPS>(p, xrow, j, k0 + f * 64 + 8 * h);
+            } else if (p.x_ragged) {
+#pragma unroll
+                for (int f = 0; f < PF; f++)
+#pragma unroll
+                    for (int h = 0; h < XN; h++) xa[f][h] = load_x16<MODE, X_RAGGED>(p, xrow, j, k0 + f * 64 + 8 * h);
+                if (base + PF >= nsteps) {  // (uniform: the batch with the row's end)
 #pragma unroll
                     for (int f = 0; f < PF; f++)
 #pragma unroll
@@ -464,7 +472,7 @@ __global__ __launch_bounds__(WAVES * 64) void stream_kernel(StreamParams p_in) {
 #pragma unroll
                 for (int f = 0; f < PF; f++)
 #pragma unroll
-                    for (int h = 0; h < XN; h++) xa[f][h] = load_x16<MODE, false>(p, xrow, j, k0 + f * 64 + 8 * h);
+                    for (int h = 0; h < XN; h++) xa[f][h] = load_x16<MODE, X_SHORT>(p, xrow, j, k0 + f * 64 + 8 * h);
             }
         } else {
             if constexpr (!PRELOAD) {
@@ -764,7 +772,7 @@ static int launch_stream_mode(StreamParams p, const StreamPlan& pl, hipStream_t 
     const int es = (MODE == MODE_I8) ? 1 : 2;
     const size_t red_bytes = (size_t)waves * p.M * tile_n * 4;
     const size_t xs_bytes = (size_t)waves * XC_MAX * 64 * 16;
-    const bool xlds = xlds_ok(es, p.M, p.x_vec_ok != 0, pl, p.K);
+    const bool xlds = xlds_ok(es, p.M, p.x_vec_ok || p.x_ragged, pl, p.K);
     const size_t lds = red_bytes + (xlds ? xs_bytes : 0);
     if (p.epi_op == EPI_SWIGLU_PAIRS && (MODE == MODE_I8 || (pl.ld != LD_T2 && pl.ld != LD_T4) || p.N % 32 != 0 ||
                                          p.pro_op == PRO_SWIGLU || p.epi.residual)) {
@@ -842,8 +850,9 @@ int launch_stream(int mode, const void* X, int x_elem_size, const float* s_x, co
     p.B = B;
     p.M = (int)((B < 16) ? B : 16);
     p.y_dtype = y_dtype;
-    p.x_vec_ok = Kx * x_elem_size >= 16;
-    p.x_ragged = p.x_vec_ok && (Kx * x_elem_size) % 16 != 0;
+    // (a row of whole groups: every 16-row block starts as aligned as the first)
+    p.x_vec_ok = ((uintptr_t)p.X) % 16 == 0 && (Kx * x_elem_size) % 16 == 0;
+    p.x_ragged = !p.x_vec_ok && Kx * x_elem_size >= 16;
     if (mode == MODE_I8) return launch_stream_mode<MODE_I8>(p, pl, st);
     if (mode == MODE_F16) return launch_stream_mode<MODE_F16>(p, pl, st);
     return launch_stream_mode<MODE_BF16>(p, pl, st);
