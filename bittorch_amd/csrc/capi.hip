@@ -286,16 +286,34 @@ extern "C" size_t bt_tiled_forward_workspace_bytes(int64_t B, int64_t N, int64_t
 }
 
 // Packed rows of N % 4 != 0 start on any byte, which the kernels that stream them pay for byte by byte, once per 16 rows of
-// activations: from 2^24 weights times row blocks on they are re-tiled into the workspace first.  Measured (int8, us, byte by byte /
-// re-tiled with the 3 us of that launch): 16 rows, 2051 x 1040 5.4 / 7.2, 4099 x 2064 6.2 / 8.9; 29 rows, 6606 x 14272 38.2 / 29.2.
-// (The fp32 GEMM reads such rows as they are, the 16-bit and int8 ones only the copy.)
+// activations; a copy in tiles costs a launch, and the weights written and read once more.  (The fp32 GEMM reads such rows as they
+// are, the 16-bit and int8 ones only the copy.)  Measured, byte by byte / re-tiled, us of the whole call:
+//   fp32   the copy is read three times, once a plane, and a single row of up to 5461 values (three planes in LDS) goes fast byte by
+//          byte.  1 row: 11007 x 4096 20.9 / 26.1, 8193 x 5120 21.9 / 27.4, 8193 x 6144 40.6 / 36.1; 2 rows: 4097 x 5120 25.1 / 23.3
+//   16-bit 1 row: 4097 x 4096 6.5 / 9.2, 16383 x 16384 29.7 / 46.3, 32769 x 512 11.5 / 9.7.  Up to 16 rows the copy pays for much
+//          work, or for many columns of few values: 8 rows, 8193 x 4096 13.8 / 16.0, 8191 x 8192 20.0 / 20.5, 16383 x 8192 34.9 /
+//          31.1; 2 rows, 16383 x 4096 17.0 / 23.0, 16383 x 16384 52.3 / 50.0, 16385 x 1024 13.6 / 10.3; not for a narrow matrix,
+//          16 rows, 4095 x 16384 25.5 / 30.0.  17 rows: 2049 x 8192 14.3 / 18.8, 4097 x 4096 14.6 / 14.6, 8193 x 4096 22.9 / 19.6,
+//          1025 x 16384 25.5 / 22.5
+//   int8   bytes cost less here.  16 rows: 16383 x 8192 29.8 / 31.3, 16383 x 16384 52.1 / 47.6, 32769 x 1024 26.0 / 22.2; 24 rows:
+//          4097 x 8192 19.6 / 21.5, 11007 x 4096 21.6 / 22.1, 8191 x 8192 29.2 / 24.2; 17 rows, 8191 x 2048 16.1 / 14.0
+// and below 2^24 weights times row blocks it does not: 16 rows, int8, 2051 x 1040 5.4 / 7.2, 4099 x 2064 6.2 / 8.9.
+enum { RETILE_F32, RETILE_16BIT, RETILE_INT8 };
 static bool can_retile(int64_t N, int64_t K) {
     return N % 4 != 0 && K < (1ll << 26) && N < (1ll << 30) && tiled_bytes(N, K) < (1ull << 32);
 }
-static bool retile_pays(int64_t B, int64_t N, int64_t K) { return can_retile(N, K) && ceil_div(B, 16) * N * K >= (1ll << 24); }
+static bool retile_pays(int64_t B, int64_t N, int64_t K, int kind) {
+    if (!can_retile(N, K) || ceil_div(B, 16) * N * K < (1ll << 24)) return false;
+    if (kind == RETILE_F32) return B > 1 || 3 * K > 16384;
+    if (B > 32) return true;
+    const double work = (double)(B * N * K);
+    if (B > 16) return kind == RETILE_16BIT ? N >= 4000 || K >= 15 * N : N >= 4000 && (work >= 1.0e9 || 2 * N >= 7 * K);
+    if (kind == RETILE_16BIT) return B == 1 ? N >= 60 * K : N >= 6000 && (work >= 5.5e8 || N >= 6 * K);
+    return B >= 4 && (work >= 4.0e9 || N >= 15 * K);
+}
 static bool packed_retiles(int64_t B, int64_t N, int64_t K, int x_dtype) {
-    if (x_dtype == BT_F32) return retile_pays(B, N, K) && (prefers_stream_f32(B, N, K) || !gemm_f32_shape_ok(N, K));
-    return can_retile(N, K) && (retile_pays(B, N, K) || !prefers_stream(B, N, K, false));  // (the tiled GEMM takes no other)
+    if (x_dtype == BT_F32) return retile_pays(B, N, K, RETILE_F32) && (prefers_stream_f32(B, N, K) || !gemm_f32_shape_ok(N, K));
+    return can_retile(N, K) && (retile_pays(B, N, K, RETILE_16BIT) || !prefers_stream(B, N, K, false));  // (the tiled GEMM takes no other)
 }
 extern "C" size_t bt_packed_forward_workspace_bytes(int64_t B, int64_t N, int64_t K, int x_dtype) {
     if (B <= 0 || N <= 0 || K <= 0) return 0;
@@ -559,7 +577,7 @@ extern "C" int bt_ternary_gemm_i8_res(const int8_t* Q, int q_layout, const float
 // Rows of Q have K bytes rounded up to 16, so that they are written in operand order and the tiled GEMM takes any K.
 static int64_t q_row_bytes(int64_t K) { return ceil_div(K, 16) * 16; }
 static bool tensor_core_retiles(int64_t B, int64_t N, int64_t K) {
-    return can_retile(N, K) && K >= 8 && K <= 16384 && (retile_pays(B, N, K) || !prefers_stream(B, N, K, true, true, true));
+    return can_retile(N, K) && K >= 8 && K <= 16384 && (retile_pays(B, N, K, RETILE_INT8) || !prefers_stream(B, N, K, true, true, true));
 }
 static size_t tensor_core_plain_bytes(int64_t B, int64_t K) { return align256((size_t)B * K) + align256((size_t)B * 4); }
 

@@ -1,0 +1,41 @@
+"""Host-side: which calls ask for scratch memory, and so take the route that needs it (no kernel is launched)."""
+import pytest
+
+F32, F16, BF16 = 0, 1, 2
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from bittorch_amd import _lib
+    return _lib.load()
+
+
+def _tensor_core_plain(b, k):
+    def up(v):
+        return -(-v // 256) * 256
+    return up(b * (-(-k // 16) * 16)) + up(4 * b)
+
+
+@pytest.mark.parametrize("n,k", [(4097, 4096), (11007, 4096), (4095, 11008), (16383, 16384), (8193, 3072)])
+def test_single_rows_read_odd_packed_rows_as_they_are(lib, n, k):
+    """A copy of the weights in tiles costs one row more than the bytes it would read one by one: 11007 x 4096 9.3 us against 17."""
+    for dt in (F16, BF16):
+        assert lib.bt_packed_forward_workspace_bytes(1, n, k, dt) == 0
+    assert lib.bt_tensor_core_workspace_bytes(1, n, k) == _tensor_core_plain(1, k)
+
+
+@pytest.mark.parametrize("b,n,k,float16,int8", [
+    (2, 16383, 4096, False, False), (16, 4095, 16384, False, False), (8, 8193, 4096, False, False), (17, 2049, 8192, False, False),
+    (24, 4097, 8192, True, False), (16, 16383, 8192, True, False), (3, 16383, 16384, True, False), (17, 1025, 16384, True, False), (1, 65537, 256, True, False), (2, 16385, 1024, True, False),
+    (4, 32769, 1024, True, True), (16, 16383, 16384, True, True), (17, 8191, 2048, True, True), (24, 8191, 8192, True, True),
+    (40, 4097, 4096, True, True), (16, 2051, 1040, False, False), (40, 4096, 4096, False, False)])
+def test_odd_packed_rows_are_copied_where_that_pays(lib, b, n, k, float16, int8):
+    tiles = lib.bt_tiled_weights_bytes(n, k)
+    assert lib.bt_packed_forward_workspace_bytes(b, n, k, BF16) == (tiles if float16 else 0)
+    assert lib.bt_tensor_core_workspace_bytes(b, n, k) == _tensor_core_plain(b, k) + (tiles if int8 else 0)
+
+
+def test_fp32_rows_copy_odd_packed_rows_for_two_rows_or_long_ones(lib):
+    for b, n, k, copies in ((1, 11007, 4096, False), (1, 8193, 5120, False), (1, 8193, 6144, True), (2, 11007, 4096, True)):
+        planes = -(-b * 3 * (-(-k // 64) * 64) * 2 // 256) * 256
+        assert lib.bt_packed_forward_workspace_bytes(b, n, k, F32) == planes + (lib.bt_tiled_weights_bytes(n, k) if copies else 0)
