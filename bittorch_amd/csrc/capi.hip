@@ -273,11 +273,13 @@ static bool packed_uses_f32_planes(const void* W_T, const void* Y, int64_t N, in
     return stream_supported(N, 3 * plane_len(K), W_T) && fast_path_ok(Y, N, 3 * plane_len(K));
 }
 
-// Scratch of a forward on the decode-tiled copy: fp32 rows' planes where the streaming kernel takes them, and more than 16
-// 16-bit rows of K % 8 != 0 padded to whole groups of 8 values: the tiled GEMM reads no other, and the streaming kernel reads
-// them again for every 64 columns (37 x 11152 x 10447 bf16 67 us as they lie, 43 with the 3 us of the copy; 16 rows and fewer
-// 1 x 704 x 10801 38 us by element, 18.5 as they lie).
-static bool pads_rows(int64_t B, int64_t K, int x_dtype) { return x_dtype != BT_F32 && K % 8 != 0 && B > 16; }
+// Scratch of a forward on the decode-tiled copy: fp32 rows' planes where the streaming kernel takes them, and 16-bit rows of
+// K % 8 != 0 padded to whole groups of 8 values.  More than 16 rows: the tiled GEMM reads no other, and the streaming kernel reads
+// them again for every 64 columns (37 x 11152 x 10447 bf16 67 us as they lie, 43 with the 3 us of the copy).  Fewer rows are read
+// as they lie (1 x 704 x 10801 10.7 us padded, 8.6 as they lie; 16 x 4096 x 4090 10.7 / 8.2), but rows of odd length start on odd
+// halves, for which a 16-byte load takes the cache several times as long: from 4 rows on they are padded too (16 x 256 x 257 6.6 us
+// padded, 11.1 as they lie, 9.2 gathered by element; 4 x 512 x 385 6.5 / 7.5; 2 x 256 x 257 6.1 / 5.8).
+static bool pads_rows(int64_t B, int64_t K, int x_dtype) { return x_dtype != BT_F32 && K % 8 != 0 && B > (K % 2 != 0 ? 3 : 16); }
 static size_t pad_bytes(int64_t B, int64_t K) { return align256((size_t)B * ceil_div(K, 8) * 16); }
 extern "C" size_t bt_tiled_forward_workspace_bytes(int64_t B, int64_t N, int64_t K, int x_dtype) {
     if (B <= 0 || N <= 0 || K <= 0) return 0;

@@ -118,8 +118,8 @@ int bt_ternary_linear_forward(const void* X, int x_dtype, const int8_t* W_tern, 
  *   Unaligned operands, a workspace missing where the planes need one and BITTORCH_KERNEL=generic run
  *   a generic kernel that accumulates in the reference's k order.
  *   workspace: at least bt_packed_forward_workspace_bytes(B,N,K,x_dtype) bytes (0: may be NULL).  It holds the
- *   planes (6*B*Kp, Kp = K rounded up to 64), more than 16 rows of 16-bit activations padded to whole groups of 8
- *   values (K % 8 != 0), and a decode-tiled copy of packed rows that start on any byte (N % 4 != 0; for the
+ *   planes (6*B*Kp, Kp = K rounded up to 64), 16-bit activations padded to whole groups of 8 values (K % 8 != 0:
+ *   more than 16 rows, or more than 3 of odd K), and a decode-tiled copy of packed rows that start on any byte (N % 4 != 0; for the
  *   tiled GEMM, and for the streaming kernel where that pays).  Without it the call still succeeds, on slower kernels.
  */
 size_t bt_packed_forward_workspace_bytes(int64_t B, int64_t N, int64_t K, int x_dtype);

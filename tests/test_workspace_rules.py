@@ -39,3 +39,13 @@ def test_fp32_rows_copy_odd_packed_rows_for_two_rows_or_long_ones(lib):
     for b, n, k, copies in ((1, 11007, 4096, False), (1, 8193, 5120, False), (1, 8193, 6144, True), (2, 11007, 4096, True)):
         planes = -(-b * 3 * (-(-k // 64) * 64) * 2 // 256) * 256
         assert lib.bt_packed_forward_workspace_bytes(b, n, k, F32) == planes + (lib.bt_tiled_weights_bytes(n, k) if copies else 0)
+
+
+@pytest.mark.parametrize("b,k,padded", [(1, 257, False), (3, 257, False), (4, 257, True), (16, 385, True), (16, 258, False), (16, 4092, False),
+                                        (17, 258, True), (17, 256, False)])
+def test_16_bit_rows_of_odd_length_are_padded_from_four_on(lib, b, k, padded):
+    """Their 16-byte loads start on odd halves: 16 rows of 257 bf16 values 11.1 us as they lie, 6.6 through a copy."""
+    want = -(-b * (-(-k // 8)) * 16 // 256) * 256 if padded else 0
+    for dt in (F16, BF16):
+        assert lib.bt_tiled_forward_workspace_bytes(b, 256, k, dt) == want
+        assert lib.bt_packed_forward_workspace_bytes(b, 256, k, dt) == want
