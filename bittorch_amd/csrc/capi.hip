@@ -593,6 +593,10 @@ extern "C" size_t bt_tensor_core_workspace_bytes(int64_t B, int64_t N, int64_t K
 static int tensor_core_run(const char* who, const void* X, int x_dtype, const uint8_t* W_T, const void* scale, int scale_dtype,
                            int64_t scale_len, const void* bias, int bias_dtype, void* Y, int64_t B, int64_t N, int64_t K,
                            int8_t* Q, float* s_x, bool room_for_padding, uint8_t* tiled, void* stream) {
+    if (((uintptr_t)W_T) % 16 != 0) {  // (also where the kernels would read a copy: whether a call is taken does not depend on its size)
+        set_error("%s: W_T, Y and acc_out must be 16-byte aligned", who);
+        return BT_ERR_INVALID;
+    }
     // Q is private to this call: written in operand order whenever the layout applies, so that
     // neither GEMM kernel has to permute activations
     // (BITTORCH_Q_LAYOUT=rowmajor keeps the row-major layout, for A/B runs)

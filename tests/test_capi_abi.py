@@ -71,6 +71,19 @@ def test_validation_errors_do_not_need_a_gpu():
     assert lib.bt_packed_forward_fused_workspace_bytes(16384, 768, 768, 0) == 16384 * (6 + 4) * 768
 
 
+@pytest.mark.parametrize("n,k", [(1024, 1024), (1026, 1024), (4097, 8192)])
+def test_tensor_core_forward_refuses_misaligned_weights_of_any_size(n, k):
+    """The largest of these reads a copy of the weights, which is aligned; the weights have to be all the same."""
+    from bittorch_amd import _lib
+    lib = _lib.load()
+    b = 64
+    nbytes = lib.bt_tensor_core_workspace_bytes(b, n, k)
+    assert (nbytes > b * k + lib.bt_tiled_weights_bytes(n, k)) == (n == 4097)
+    addr = 1 << 20  # (never read: the call ends before any launch)
+    assert lib.bt_ternary_linear_tensor_core_forward(addr, 2, addr + 4, addr, 0, 1, None, 0, addr, b, n, k, addr, nbytes, None) == -1
+    assert "16-byte aligned" in _lib.last_error()
+
+
 def test_extension_probes_are_truthful():
     import bittorch_amd as bt
     from bittorch_amd.nn.ternary_linear import _cuda_kernel_available
