@@ -319,9 +319,7 @@ static bool packed_retiles(int64_t B, int64_t N, int64_t K, int x_dtype) {
 }
 extern "C" size_t bt_packed_forward_workspace_bytes(int64_t B, int64_t N, int64_t K, int x_dtype) {
     if (B <= 0 || N <= 0 || K <= 0) return 0;
-    // (fp32 rows of N % 4 != 0 are asked the planes for at any size: what this query has always said of them)
-    const size_t own = x_dtype == BT_F32 && N % 4 != 0 ? f32_planes_bytes(B, K) : bt_tiled_forward_workspace_bytes(B, N, K, x_dtype);
-    return align256(own) + (packed_retiles(B, N, K, x_dtype) ? tiled_bytes(N, K) : 0);
+    return align256(bt_tiled_forward_workspace_bytes(B, N, K, x_dtype)) + (packed_retiles(B, N, K, x_dtype) ? tiled_bytes(N, K) : 0);
 }
 
 // residual (optional): [B, N] in Y's dtype, 16-byte aligned; Y = round(round(linear) + residual)

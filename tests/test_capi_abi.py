@@ -64,10 +64,11 @@ def test_validation_errors_do_not_need_a_gpu():
     # workspace sizes are plain arithmetic
     assert lib.bt_tensor_core_workspace_bytes(16, 4096, 4096) >= 16 * 4096 + 16 * 4
     assert lib.bt_tensor_core_workspace_bytes(0, 1, 1) == 0
-    # fp32 rows: planes for the streaming kernel, none for the GEMM that splits in registers (N % 4 == 0)
+    # fp32 rows: planes for the streaming kernel, none for the GEMM that splits in registers (any N from 4 on)
     assert lib.bt_packed_forward_workspace_bytes(20, 768, 700, 0) == 20 * 6 * 704
     assert lib.bt_packed_forward_workspace_bytes(16384, 768, 768, 0) == 0
-    assert lib.bt_packed_forward_workspace_bytes(16384, 770, 768, 0) == 16384 * 6 * 768
+    assert lib.bt_packed_forward_workspace_bytes(16384, 770, 768, 0) == 0
+    assert lib.bt_packed_forward_workspace_bytes(16384, 3, 768, 0) == 16384 * 6 * 768
     assert lib.bt_packed_forward_fused_workspace_bytes(16384, 768, 768, 0) == 16384 * (6 + 4) * 768
 
 
