@@ -27,7 +27,8 @@ struct GradW16Params {
     int tail_from;        // tiles from this one on are summed in parts of the rows,
     int splits;           // so many (1: there are none),
     int per_xcd_tail;     // so many (tile, part) per XCD (grid = 8 * (whole + per_xcd_tail)),
-    int64_t part_rows;    // of so many rows, a multiple of 128,
+    int64_t part_rows;    // of so many rows, a multiple of 128 (the last part: what is left),
+    int long_first;       // 1: two parts of unequal length, an XCD's long ones in front of its short ones,
     float* part;          // into [part][tile][accumulator][thread]
     int scale_bcast, scale_dtype;
     const void* scale;    // [N] or one entry
@@ -81,9 +82,17 @@ __global__ __launch_bounds__(256, 1) void grad_w16_kernel(GradW16Params p) {
     uint32_t lin, item = 0, part = 0;
     if (tail) {
         const uint32_t tiles = tiles_n * tiles_k - (uint32_t)p.tail_from;
-        item = (blockIdx.x & 7u) * (uint32_t)p.per_xcd_tail + (idx - (uint32_t)p.whole);
-        if (item >= tiles * (uint32_t)p.splits) return;
-        part = item / tiles;
+        const uint32_t j = idx - (uint32_t)p.whole, per_xcd = (uint32_t)p.per_xcd_tail;
+        if (p.long_first) {  // (uniform)
+            const uint32_t half = per_xcd / 2, tile = (blockIdx.x & 7u) * half + (j < half ? j : j - half);
+            if (tile >= tiles) return;
+            part = j < half ? 0u : 1u;
+            item = part * tiles + tile;
+        } else {
+            item = (blockIdx.x & 7u) * per_xcd + j;
+            if (item >= tiles * (uint32_t)p.splits) return;
+            part = item / tiles;
+        }
         lin = (uint32_t)p.tail_from + (item - part * tiles);
     } else {
         lin = (blockIdx.x & 7u) * (uint32_t)p.whole + idx;
@@ -313,31 +322,52 @@ __global__ __launch_bounds__(256) void grad_w16_reduce_kernel(GradW16Params p) {
     }
 }
 
-// Tiles of 256 or of 128 (T = 8, 4): whole rounds of a tile for each compute unit, and what remains in parts of the rows where
-// that takes less.  Priced in microseconds: a round by its rows and its stores (a share of which goes with the share of the
-// compute units it fills: one wave a SIMD leaves the clock to the others), a part of a tile by writing its sums and reading them
-// again.  Measured (bf16 to fp32, 256 / 128 / the vendor's product with scale_widen_kernel behind it): 4096 x 4096 x 4096
-// 113 / 154 / 132; 16384 x 4096 x 4096 417 / 593 / 468; 2048 x 2048 x 2048 43 / 27 / 34; 4096 x 2048 x 2048 56 / 44 / 50;
-// 4096 x 1024 x 1024 34 / 23 / 33; 16384 x 768 x 768 41 / 35 / 94; 4096 x 2560 x 2560 71 / 79 / 72; 300 x 4096 x 4096 27 / 43 / 42.
-// Slower than the vendor's: one long round over little more than half of the chip, 16384 x 3072 x 3072 350 / 328 / 302.
-struct GradW16Plan { int T; int64_t tiles, tail, splits, part_rows; double us; };
+// Tiles of 256 or of 128 (T = 8, 4): whole rounds of a tile for each compute unit, and what remains as one round more, or in
+// parts of the rows where that takes less.  Parts of equal length fill what would be idle when at most half of the compute units
+// have a tile.  With some more tiles than that, each is cut in two parts of unequal length: an XCD starts its long parts, the
+// compute units left over take its short ones, two in turn at most, and the lengths are chosen for both to end together (three
+// and more in turn are no better: their rows are no longer those that the long parts read, 16384 x 3584 x 3584 390 / 435 us).  Priced in microseconds, f
+// the share of compute units that a round fills (one wave a SIMD leaves clock and memory to the others), by the measurements of
+// 112 sizes, most of them within 5 %:
+//   a round   5.4 + 10 f + (0.0183 + 0.0055 f) rows for tiles of 256, 1.2 + 4.5 f + (0.0073 + 0.0018 f) rows for tiles of 128
+//   parts     5 + 0.11 or 2.5 + 0.04 a part in place of the constant: writing the sums and adding them up
+// Measured, bf16 to fp32, tiles of 256 whole / in parts / tiles of 128 / the vendor's product with scale_widen_kernel behind it
+// (the vendor's takes up to 1.6 times as long at neighbouring sizes): 300 x 768 x 768 17.9 / 16.4 / 10.3 / 13.1; 2048 x 2048 x 2048
+// 53.2 / 45.6 / 29.3 / 37.0; 4096 x 2560 x 2560 96.8 / 78.5 / 83.2 / 81.8; 4096 x 3584 x 3584 111 / - / 143 / 141;
+// 4096 x 2048 x 4096 97.2 / 89.2 / 88.4 / 84.0; in two unequal parts, 8192 x 3072 x 3072 188 / 162 / 191 / 176 and
+// 16384 x 3072 x 3072 348 / 291 / 373 / 327.
+struct GradW16Plan { int T; int64_t tiles, tail, splits, part_rows; bool long_first; double us; };
 static GradW16Plan grad_w16_plan(int64_t M, int64_t N, int64_t K) {
     GradW16Plan best = {};
     const int64_t C = gemm_compute_units();
     for (int T = 8; T >= 4; T -= 4) {
         const int64_t side = 32 * T, unit = T == 8 ? 128 : 256;  // rows of four stages
-        auto round_us = [&](int64_t wgs, int64_t rows, bool stores) {
-            const double fill = (double)wgs / (double)C, r = (double)(ceil_div(rows, unit) * unit);
-            return T == 8 ? (stores ? 13.0 * fill : 0.0) + (0.016 + 0.0105 * fill) * r : (stores ? 4.0 : 0.0) + 0.009 * r;
+        auto rows_us = [&](int64_t wgs, int64_t rows) {
+            const double fill = (double)wgs / (double)C;
+            return (T == 8 ? 0.0183 + 0.0055 * fill : 0.0073 + 0.0018 * fill) * (double)(ceil_div(rows, unit) * unit);
         };
-        GradW16Plan r = {T, ceil_div(N, side) * ceil_div(K, side), 0, 1, M, 0.0};
+        auto round_us = [&](int64_t wgs) {
+            const double fill = (double)wgs / (double)C;
+            return (T == 8 ? 5.4 + 10.0 * fill : 1.2 + 4.5 * fill) + rows_us(wgs, M);
+        };
+        auto parts_us = [&](int64_t parts) { return T == 8 ? 5.0 + 0.11 * (double)parts : 2.5 + 0.04 * (double)parts; };
+        GradW16Plan r = {T, ceil_div(N, side) * ceil_div(K, side), 0, 1, M, false, 0.0};
         const int64_t rounds = r.tiles / C, rem = r.tiles % C;
-        const double whole = 5.0 + (double)rounds * round_us(C, M, true);
-        r.us = whole + (rem ? round_us(rem, M, true) : 0.0);
+        const double whole = 5.0 + (double)rounds * round_us(C);
+        r.us = whole + (rem ? round_us(rem) : 0.0);
+        auto consider = [&](int64_t rows, bool long_first, double us) {
+            const int64_t splits = ceil_div(M, rows);
+            if (splits > 1 && us < r.us) { r.us = us; r.tail = rem; r.splits = splits; r.part_rows = rows; r.long_first = long_first; }
+        };
         for (int64_t want = 2; rem && want <= std::min<int64_t>(C / rem, ceil_div(M, unit)); want++) {
-            const int64_t rows = ceil_div(ceil_div(M, want), unit) * unit, splits = ceil_div(M, rows);
-            const double us = whole + round_us(rem * splits, rows, false) + 4.0 + (T == 8 ? 0.1 : 0.025) * (double)(rem * splits);
-            if (splits > 1 && us < r.us) { r.us = us; r.tail = rem; r.splits = splits; r.part_rows = rows; }
+            const int64_t rows = ceil_div(ceil_div(M, want), unit) * unit, parts = rem * ceil_div(M, rows);
+            consider(rows, false, whole + parts_us(parts) + rows_us(parts, rows));
+        }
+        // an XCD's C / 8 compute units: `held` with a long part, `left` for as many short ones, `turns` each at most
+        const int64_t held = ceil_div(rem, 8), left = C / 8 - held;
+        if (T == 8 && 2 * rem > C && 2 * left >= held) {
+            const int64_t turns = ceil_div(held, left), rows = ceil_div(ceil_div(M * turns, turns + 1), unit) * unit;
+            consider(rows, true, whole + parts_us(2 * rem) + rows_us(C, rows));
         }
         if (!best.T || r.us < best.us) best = r;
     }
@@ -400,7 +430,8 @@ extern "C" int bt_linear_grad_weight_16(const void* dY, const void* X, int dtype
     p.whole = (int)ceil_div(plan.tiles - plan.tail, 8);
     p.tail_from = (int)(plan.tiles - plan.tail);
     p.splits = (int)plan.splits; p.part_rows = plan.part_rows; p.part = (float*)workspace;
-    p.per_xcd_tail = (int)ceil_div(plan.tail * plan.splits, 8);
+    p.long_first = plan.long_first ? 1 : 0;
+    p.per_xcd_tail = (int)(plan.long_first ? 2 * ceil_div(plan.tail, 8) : ceil_div(plan.tail * plan.splits, 8));
     hipStream_t st = (hipStream_t)stream;
     if (dtype == BT_F16) {
         if (out_dtype == BT_F32) launch_grad_w16<MODE_F16, true>(p, plan, st);

@@ -32,6 +32,30 @@ def test_weight_gradient(m, n, k, dtype, out):
         assert bool(((got.float() - sums * s).abs() <= bound).all())
 
 
+# What each kind of launch stores, with the scratch that shows which it is: parts x bytes of one (256 KiB for tiles of 256, 64 KiB
+# for tiles of 128).  Tiles of 128 whole and in parts, tiles of 256 whole, a round and the rest in equal parts, in two unequal ones
+# (an XCD's share of the tiles full and one short, columns and rows that end inside a tile)
+BIG, SMALL = 256 << 10, 64 << 10
+LAUNCHES = [((257, 2040, 2048), 0), ((600, 2048, 2048), 0), ((1025, 256, 264), 6 * 5 * SMALL), ((9001, 264, 520), 15 * 12 * SMALL),
+            ((70, 2560, 6920), 0), ((300, 4104, 3840), 0), ((2305, 11008, 2048), 88 * 2 * BIG), ((2048, 2560, 6912), 14 * 4 * BIG),
+            ((8192, 3072, 3072), 144 * 2 * BIG), ((6200, 3080, 3000), 156 * 2 * BIG), ((6000, 2056, 4200), 153 * 2 * BIG)]
+
+
+@pytest.mark.parametrize("dtype,out", [(torch.float16, torch.float32), (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("shape,scratch", LAUNCHES)
+def test_every_launch_is_exact_on_small_integers(shape, scratch, dtype, out):
+    """Sums of small whole numbers have one value in any order and any parts; it is rounded to the operands' dtype once."""
+    from bittorch_amd import _C
+    m, n, k = shape
+    announce("exact sums", m, n, k, dtype)
+    assert _C._L.bt_linear_grad_weight_16_workspace_bytes(m, n, k) == scratch
+    gen = torch.Generator("cuda").manual_seed(m + n + k)
+    gy = torch.randint(-2, 3, (m, n), device="cuda", generator=gen).to(dtype)
+    x = torch.randint(-1, 2, (m, k), device="cuda", generator=gen).to(dtype)
+    got = _C.linear_grad_weight_16(gy, x, torch.ones(n, device="cuda"), out)
+    assert torch.equal(got, (gy.float().t() @ x.float()).to(dtype).to(out))
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_small_integers_are_exact(dtype):
     """Sums of small whole numbers have one value in any order: every output, by row and column, of both tile sizes."""

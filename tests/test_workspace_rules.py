@@ -49,3 +49,31 @@ def test_16_bit_rows_of_odd_length_are_padded_from_four_on(lib, b, k, padded):
     for dt in (F16, BF16):
         assert lib.bt_tiled_forward_workspace_bytes(b, 256, k, dt) == want
         assert lib.bt_packed_forward_workspace_bytes(b, 256, k, dt) == want
+
+
+@pytest.mark.parametrize("m,n,k,scratch", [
+    (300, 768, 768, 0), (64, 1024, 1024, 0),                                    # tiles of 128, one of them at most a compute unit
+    (16384, 3072, 3072, 144 * 2 * (256 << 10)), (8192, 3072, 3072, 144 * 2 * (256 << 10)),  # 144 tiles of 256: two parts each
+    (16384, 3584, 3584, 0), (4096, 4096, 4096, 0)])                             # 196 and 256 tiles: whole
+def test_16_bit_weight_gradient_cuts_long_rounds(lib, m, n, k, scratch):
+    """One long round over little more than half of the chip, 16384 x 3072 x 3072: 348 us whole, 291 in two parts a tile."""
+    assert lib.bt_linear_grad_weight_16_workspace_bytes(m, n, k) == scratch
+
+
+def test_16_bit_weight_gradient_refuses_what_the_kernel_cannot_take(lib):
+    """(every call ends before a launch; the addresses are never read)"""
+    from bittorch_amd import _lib
+    a = 1 << 20
+
+    def call(dy=a, x=a, dtype=BF16, scale=a, scale_dtype=F32, scale_len=256, dw=a, out=F32, m=64, n=256, k=512, ws=None, nbytes=0):
+        return lib.bt_linear_grad_weight_16(dy, x, dtype, scale, scale_dtype, scale_len, dw, out, m, n, k, ws, nbytes, None)
+
+    for bad in (dict(dy=None), dict(m=0), dict(scale_len=255), dict(dtype=F32), dict(out=F16), dict(scale_dtype=9), dict(n=252, scale_len=1),
+                dict(k=508), dict(dy=a + 8), dict(x=a + 2), dict(dw=a + 4), dict(scale=a + 2), dict(n=1 << 24, scale_len=1)):
+        assert call(**bad) == -1, bad
+        assert "bt_linear_grad_weight_16" in _lib.last_error()
+    need = lib.bt_linear_grad_weight_16_workspace_bytes(8192, 3072, 3072)
+    big = dict(m=8192, n=3072, k=3072, scale_len=1)
+    for ws, nbytes in ((None, 0), (a, need - 1), (a + 64, need)):
+        assert call(ws=ws, nbytes=nbytes, **big) == -2
+        assert "workspace" in _lib.last_error()
