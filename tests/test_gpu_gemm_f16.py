@@ -67,10 +67,12 @@ def test_infinities_past_the_end_of_a_row_stay_in_their_row():
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("m,n,k", [(33, 260, 1536), (97, 1004, 1544), (250, 516, 1480), (640, 5000, 1608), (129, 1024, 2112), (70, 1030, 1800)])
+@pytest.mark.parametrize("m,n,k", [(33, 260, 1536), (97, 1004, 1544), (250, 516, 1480), (640, 5000, 1608), (129, 1024, 2112), (70, 1030, 1800),
+                                   (129, 1024, 1608), (300, 4096, 1576)])
 def test_stages_in_two_groups(m, n, k, dtype):
     """Launches of at most one tile a compute unit, 24 stages and more: an even and an odd number of stages, a remainder of K in the
-    second group, rows that end in either group's half of a tile, tiles of 32 and 64 rows, N % 4 != 0.  Bound as above."""
+    second group, rows that end in either group's half of a tile, tiles of 32 and 64 rows, N % 4 != 0; N % 16 == 0 (row-major weights
+    16 bytes a lane) with a remainder of K.  Bound as above."""
     from bittorch_amd import _C
     announce("gemm_f16 two groups", m, n, k, dtype)
     set_option("STREAM_MAX_ROWS", "1")

@@ -57,6 +57,31 @@ def test_static_scratch_entry_point_matches_workspace_entry_point(dtype):
         assert torch.equal(y_st, y_ws), (dtype, b, n, k)
 
 
+@pytest.mark.parametrize("b,n,k,room", [(33, 258, 1047, True), (33, 256, 1047, True), (300, 514, 2051, True), (64, 36, 8200, True),
+                                        (16140, 20, 1039, False), (4097, 20, 4095, False)])
+def test_static_scratch_entry_point_on_rows_of_any_length(b, n, k, room):
+    """Rows of K % 16 != 0 are quantized into rows rounded up to 16 bytes where the array holds those (``room``), as they are
+    where it holds only them (the last two: 16 MiB lie between the two lengths); activations that start off 16 bytes too."""
+    from bittorch_amd import _lib
+    from bittorch_amd.quant import pack_ternary_transposed
+    lib = _lib.load()
+    assert b * k <= 16 << 20 and (b * (-(-k // 16) * 16) <= 16 << 20) == room
+    g = torch.Generator().manual_seed(b)
+    packed = pack_ternary_transposed(random_ternary(n, k, seed=b))[0].cuda()
+    scale = (torch.rand(n, generator=g) * 0.05 + 0.01).cuda()
+    bias = (torch.randn(n, generator=g) * 0.01).cuda()
+    for dtype in (torch.bfloat16, torch.float32):
+        announce("static scratch, ragged", dtype, b, n, k)
+        x = seeded_acts(b, k, seed=b + 1, dtype=dtype, outliers=True).cuda()
+        off = torch.empty(b * k + 1, dtype=dtype, device="cuda")[1:].view(b, k).copy_(x)
+        want = None
+        for xi in (x, off):
+            y_st, y_ws = _both(lib, xi, packed, scale, bias, n, k, warmed=_WARM["done"])
+            _WARM["done"] = True
+            want = y_ws if want is None else want
+            assert torch.equal(y_st, y_ws) and torch.equal(y_ws, want)
+
+
 def test_static_scratch_entry_point_inside_a_graph_capture():
     """The use the entry point is for: after one call outside a capture (which looks the array's address up), the
     call is recorded into a HIP graph and replayed, with eager work between the replays; every replay equals the
