@@ -500,7 +500,7 @@ bool gemm_i8_supported(int64_t N, int64_t K, const void* Q, const void* W_T) {
 }
 
 // gemm_i8_dma.hip
-int gemm_i8_dma_rows(int64_t M, int64_t N, int64_t K, bool tiled);
+int gemm_i8_dma_rows(int64_t M, int64_t N, int64_t K, bool tiled, bool fields);
 int launch_gemm_i8_dma(const GemmParams& p, int rows, bool tiled, bool fields, hipStream_t st);
 
 // One launch over column tiles [tile_n0, tile_n0 + tiles_n) in tiles of 32 * NB rows.
@@ -550,7 +550,7 @@ int launch_gemm_i8(const int8_t* Q, int q_layout, const float* s_x, const int32_
     p.tiles16 = tiles16_arg(N, w_layout);
     const bool qoo = q_layout == Q_OPERAND_ORDER, tiled = layout_tiled(w_layout), fields = layout_fields(w_layout);
     const int64_t tiles_n = ceil_div(N, G_BN);
-    const int dma_nb = qoo ? gemm_i8_dma_rows(M, N, K, tiled) : 0;  // (gemm_i8_dma.hip)
+    const int dma_nb = qoo ? gemm_i8_dma_rows(M, N, K, tiled, fields) : 0;  // (gemm_i8_dma.hip)
     if (dma_nb) return launch_gemm_i8_dma(p, dma_nb, tiled, fields, st);
     // the column tiles of a mostly empty last round in finer tiles, a launch of their own behind the whole tiles
     // (gemm_split; same sums, same bits)

@@ -444,20 +444,22 @@ __global__ __launch_bounds__(256 * KG, KG == 2 || NB == 4 ? 2 : NB == 2 ? 3 : 4)
 // the row sums).
 static bool i8_splits_k(int64_t stages) { return stages >= 24; }
 
-// Rows of the tiles in units of 32 (4, 2 or 1), or 0 where gemm_i8_kernel is the better one: tiled weights in whole stages
-// with at most one tile of 128 x 256 for each compute unit.  There a second workgroup has nothing to do, and splitting K
-// over the two waves of a SIMD halves the one tile's chain (K = N = 4096: M = 2048 28.3 us against 30.5 here, M = 512 in its
-// tiles of 32 rows 15.9 against 18.5).  With more tiles (tiled / row-major weights, us, that kernel first): 4096 x 13824 x
-// 2560 133 -> 122 / 148 -> 134; 2048 x 11008 x 4096 93 -> 82 / 104 -> 88; 4096 x 2560 x 6912 (64-row tiles) 67 -> 65 / 85 ->
-// 73; 4096 x 8192 x 8192 207 -> 192 / 250 -> 208; 3000 x 1008 x 1040, K not in whole stages, 38 -> 13 / 16 -> 14.
-// Row-major weights of few tiles: M = 1024, 512 (N = K = 4096) 27.3 -> 25.2, 22.9.
+// Rows of the tiles in units of 32 (4, 2 or 1), or 0 where gemm_i8_kernel is the better one: tiled weights in whole stages with
+// at most one tile of 128 x 256 for each compute unit, but not with two groups of waves on finer tiles.  Measured, decode-tiled
+// weights, gemm_i8_kernel / tiles of 32 / 64 / 128 rows here, us: one tile of 32 rows for each compute unit at most, 256 x 4096 x
+// 4096 16.2 / 14.6 / 17.2 / 18.1, 512 x 2560 x 6912 24.3 / 21.8 / 25.2 / 27.1; of 64 rows, 256 x 11008 x 4096 20.5 / 21.9 / 18.6 /
+// 21.9, 1000 x 2560 x 6912 30.1 / 32.7 / 25.9 / 31.5; of 128 rows, 512 x 11008 x 4096 26.4 / 30.9 / 29.1 / 29.4, 2048 x 4096 x 4096
+// 30.1 / 40.2 / 32.7 / 32.8, 2048 x 4096 x 11008 67.6 / 105 / 78.0 / 77.1; 16 stages (one group), 128 x 16384 x 1024 8.3 / 8.5 /
+// 10.1 / 8.6.  The field layout has one group here, so it stays there.  With more tiles (tiled / row-major weights, us, that kernel
+// first): 4096 x 13824 x 2560 133 -> 122 / 148 -> 134; 2048 x 11008 x 4096 93 -> 82 / 104 -> 88; 4096 x 2560 x 6912 (64-row tiles)
+// 67 -> 65 / 85 -> 73; 4096 x 8192 x 8192 207 -> 192 / 250 -> 208; 3000 x 1008 x 1040, K not in whole stages, 38 -> 13 / 16 -> 14.
 // The prices are microseconds of a compute unit's run of tiles, fitted to the same runs.
-static int gemm_i8_dma_plan(int64_t M, int64_t N, int64_t K, bool tiled, double* us) {
+static int gemm_i8_dma_plan(int64_t M, int64_t N, int64_t K, bool tiled, bool fields, double* us) {
     const int64_t C = gemm_compute_units(), tn = ceil_div(N, G_BN);
     const int64_t t4 = ceil_div(M, 128) * tn, t2 = ceil_div(M, 64) * tn, t1 = ceil_div(M, 32) * tn;
-    if (tiled && K % 128 == 0 && N % 4 == 0 && t4 <= C) return 0;
     const bool whole = gemm_whole_tiles();
-    const bool split = i8_splits_k(ceil_div(K, D_BK));
+    const bool split = i8_splits_k(ceil_div(K, D_BK)) && !fields;
+    if (tiled && K % 128 == 0 && N % 4 == 0 && t4 <= C && (t2 > C || !split || whole)) return 0;
     if (t1 <= C && !whole) { *us = split ? 5.7 + 0.0027 * (double)K : 5.2 + 0.0035 * (double)K; return 1; }
     if (t2 <= C && !whole) { *us = split ? 5.5 + 0.0034 * (double)K : 5.2 + 0.0045 * (double)K; return 2; }
     const int parts = gemm_dma_parts(t4);
@@ -467,14 +469,14 @@ static int gemm_i8_dma_plan(int64_t M, int64_t N, int64_t K, bool tiled, double*
     *us = 2.0 + (half ? p2 : p4);
     return half ? 2 : 4;
 }
-int gemm_i8_dma_rows(int64_t M, int64_t N, int64_t K, bool tiled) {
+int gemm_i8_dma_rows(int64_t M, int64_t N, int64_t K, bool tiled, bool fields) {
     double us;
-    return gemm_i8_dma_plan(M, N, K, tiled, &us);
+    return gemm_i8_dma_plan(M, N, K, tiled, fields, &us);
 }
 // microseconds of launch_gemm_i8: this file's plan, or gemm_i8_kernel's rounds of whole tiles (of finer ones at their price)
 double gemm_i8_cost(int64_t M, int64_t N, int64_t K, bool tiled, bool operand_order) {
     double us;
-    if (operand_order && gemm_i8_dma_plan(M, N, K, tiled, &us)) return us;
+    if (operand_order && gemm_i8_dma_plan(M, N, K, tiled, false, &us)) return us;
     return gemm_split(M, N, tiled && K % 128 == 0).rounds * (8.6 + 0.0044 * (double)K);
 }
 

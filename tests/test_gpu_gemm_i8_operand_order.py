@@ -54,8 +54,9 @@ def test_operand_order_equals_row_major_activations(m, n, k, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("m,n,k", [(33, 260, 1536), (97, 1004, 1552), (250, 516, 1584), (640, 5000, 1616), (129, 1024, 2112),
-                                   (129, 1024, 1616), (300, 4096, 1584)])
+                                   (129, 1024, 1616), (300, 4096, 1584), (250, 516, 1664), (640, 5000, 1536), (1000, 2560, 6912)])
 def test_stages_in_two_groups(m, n, k, dtype):
     """Launches of at most one tile a compute unit, 24 stages and more: even and odd numbers of stages, a remainder of K in the
-    second group, rows that end in either group's half of a tile, tiles of 32 and 64 rows; N % 16 == 0 with a remainder of K."""
+    second group, rows that end in either group's half of a tile, tiles of 32 and 64 rows; N % 16 == 0 with a remainder of K; whole stages of
+    128, where decode-tiled weights leave the other kernel for this one."""
     test_operand_order_equals_row_major_activations(m, n, k, dtype)
