@@ -3,16 +3,17 @@
 //
 // A 256-thread workgroup (4 waves) owns a tile of 32 NB x 256 outputs; wave w works on columns 64 w .. +63 over the whole of
 // K, so nothing has to be added up at the end, and two workgroups share a compute unit: while one waits, starts, drains or
-// stores, the other one's MFMAs run.  Bound by the issue of a stage: 32 MFMAs (512 cycles) and some 60 other instructions;
+// stores, the other one's MFMAs run.  Launches of at most one tile a compute unit have two such groups of waves in a workgroup
+// instead, half of the stages each, which add their sums through LDS at the end (i8_splits_k).  Bound by the issue of a stage: 32 MFMAs (512 cycles) and some 60 other instructions;
 // 2.2 to 2.9 POPS at K = 2560 .. 8192 (4096 x 8192 x 8192 192 us, 207 with the K halves of gemm_i8_kernel).
 //   * Everything that comes from memory goes to LDS without passing through registers (global_load_lds, 16 bytes a lane):
 //     the activations in the operand order the quantizer wrote them in, and each wave's packed weights (1 KiB a stage).  A
-//     stage is 64 k; five stages are in LDS, so a load has three stages (1500 to 4000 cycles) to arrive.
+//     stage is 64 k; n = d_stages of them are in LDS, five as a rule, so a load has n - 2 stages (1500 to 4000 cycles) to arrive.
 //   * A stage: 16 MFMAs of row blocks 0..3 with the decode of the next stage's weights behind them, the one barrier, 16
 //     MFMAs of row blocks 4..7 under which the fragments of the next stage's row blocks 0..3 arrive.
 // The loads are counted by hand (the compiler does not see them): `vmcnt` in front of the barrier of stage s leaves the
-// loads of stages s + 3 and s + 4 in flight, so stage s + 1 (fragments) and s + 2 (the weights decoded one stage ahead) are
-// complete; that barrier also stands between the last read of stage s's buffer and the loads of stage s + 5 into it.
+// loads of stages s + 3 .. s + n - 1 in flight, so stage s + 1 (fragments) and s + 2 (the weights decoded one stage ahead) are
+// complete; that barrier also stands between the last read of stage s's buffer and the loads of stage s + n into it.
 #include "gemm_i8_common.h"
 #include "lds_dma.h"
 
@@ -323,7 +324,7 @@ __device__ __forceinline__ void gemm_i8_dma_tile(const GemmParams& p, const int6
             }
             if (c < NB) a_lo[c] = *(const uint4*)(lds + (nxt + frag_at) + c * 1024);
             if (c == 4) read_raw(s + 2, nxt2);
-            // stage s + 5 over stage s
+            // stage s + D_NST over stage s
             if (c >= 6 && c < 6 + A_LOADS) issue_a(c - 6);
             if (c >= 8 && c < 8 + W_LOADS) issue_w(c - 8);
             if (c == 13) advance();

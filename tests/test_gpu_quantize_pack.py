@@ -64,7 +64,7 @@ def test_quantize_pack_one_read_kernel_matches_oracle(oracle, n, k):
 # The same kernel on rows that are no multiple of 256 values or start anywhere: a last group of one to four values, a last
 # chunk that is nearly empty or nearly full, row tiles with one row or one short, every split of a row, and past the longest.
 RAGGED_SHAPES = [(1, 4), (3, 5), (17, 255), (16, 257), (33, 1023), (63, 1025), (5, 2047), (40, 2050), (7, 4095), (6159, 2051),
-                 (9, 4097), (31, 6147), (17, 8190), (15, 8642), (3, 10243), (2, 12289), (5, 16381), (18, 16384), (3, 16385)]
+                 (9, 4097), (31, 6147), (17, 8190), (15, 8642), (3, 10243), (2, 12289), (5, 16381), (18, 16384), (3, 16385), (10240, 100), (10256, 252)]
 
 
 @pytest.mark.parametrize("n,k", RAGGED_SHAPES)
