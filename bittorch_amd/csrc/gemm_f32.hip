@@ -89,7 +89,9 @@ constexpr uint32_t LUT_BF16_HALF = 0x00BF3F00u;
 // (pairwise, always in the same order): for outputs with too few tiles to occupy the chip.
 // SC: X's columns are scaled (input gradient with one scale per row of W).
 // RN: forward outputs of N % 4 != 0, an instance of its own: asked at run time, every other output paid half a microsecond for
-// the clamped columns and the second way to store (us, fp32, 300 x 4096 x 512 17.9 / 17.0, 4096 x 768 x 768 28.2 / 27.5).
+// the clamped columns and the second way to store (us, fp32, 300 x 4096 x 512 17.9 / 17.0, 4096 x 768 x 768 28.2 / 27.5).  Only
+// the tile of one wave's 64 x 64 outputs gains from the question: with a branch between them the compiler sends each row's
+// stores off by themselves (512 x 2048 x 1032 17.0 without, 16.0 with it; 4096 x 128 x 2048 24.1 / 23.1).
 template <int SRC, int NG, int KS, bool SC, bool RN>
 __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(GemmF32Params p) {
     constexpr int TM = (KS == 1) ? 128 : 64, TN = (KS == 1) ? 128 * NG : 64 * NG;  // a workgroup's tile
@@ -365,7 +367,7 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
                 } else {
 #pragma unroll
                     for (int t = 0; t < 4; t++) y[t] = epi_float(y[t], ws[t], bs[t]);
-                    if constexpr (RN) {  // element by element
+                    if (KS == 8 ? p.NC % 4 != 0 : RN) {  // element by element
 #pragma unroll
                         for (int t = 0; t < 4; t++) {
                             if (col + t >= p.NC) continue;
