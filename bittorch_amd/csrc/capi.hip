@@ -362,7 +362,7 @@ static int packed_forward_impl(const char* who, const void* X, int x_dtype, cons
         return BT_ERR_INVALID;
     }
     if (layout_tiled(w_layout)) {
-        // the decode-tiled copy is read by the streaming kernel only, once per 16 rows
+        // the decode-tiled copy: read by the streaming kernel, once per 16 rows, and by the tiled GEMMs
         if (!stream_supported_tiled(N, K, W_T) || !fast_path_ok(Y, N, 3 * K) || 3 * K >= (1ll << 26)) {
             set_error("%s: tiled weights must be 256-byte aligned and below 4 GiB, Y 16-byte aligned", who);
             return BT_ERR_INVALID;

@@ -11,16 +11,18 @@
 // workgroups share a compute unit, so that one's MFMAs run while the other waits, starts, drains or stores (a 512-thread
 // workgroup that split K over the two waves of a SIMD: 6.9 us a round of tiles with nothing beside it, fp16 / bf16 row-major
 // weights, 4096 x 11008 x 4096 338 -> 260 us, tiled 300 -> 257; 16384 x 768 x 768 30 -> 21.5; 512 x 4096 x 4096 49 -> 31).
-// Bound by the issue of a stage, 64 MFMAs (1024 cycles) and some 150 other
+// A launch of at most one tile a compute unit has two such groups of waves in a workgroup, half of the stages each, which add
+// their sums through LDS at the end (f16_splits_k).  Bound by the issue of a stage, 64 MFMAs (1024 cycles) and some 150 other
 // instructions, 80 of them vector ones: 1.46 PFLOP/s at that size (252 us).
-// Activations and packed weights go to LDS by global_load_lds, three stages of 64 k.  The order of k inside an MFMA is free:
-// lane (j, g) of the stage's first sub-step takes k = 16 g .. +7 and of the second 16 g + 8 .. +15, so the 16 weight bytes a
-// lane loads are all its own, and the weights are decoded in natural order, so the activations are fed as they lie in memory.
+// Activations and packed weights go to LDS by global_load_lds, n = fd_stages of 64 k, three for tiles of 128 rows.  The order
+// of k inside an MFMA is free: lane (j, g) of the stage's first sub-step takes k = 16 g .. +7 and of the second 16 g + 8 .. +15,
+// so the 16 weight bytes a lane loads are all its own, and the weights are decoded in natural order, so the activations are fed
+// as they lie in memory.
 // A stage is four runs of 16 MFMAs (two halves of the rows for each sub-step).  The decode of the second sub-step's weights is
 // dealt out behind the MFMAs of the first, that of the next stage's first sub-step behind the second's.
-// Loads are counted by hand: in front of a stage's third run vmcnt leaves the loads of stage s + 2 in flight, so stage s + 1 is
-// complete (its weights are read there, its activations behind the barrier in front of the fourth run); the loads of stage
-// s + 3 go out behind that barrier, into the buffer whose last fragments were read before it.
+// Loads are counted by hand: in front of a stage's third run vmcnt leaves the loads of stages s + 2 .. s + n - 1 in flight, so
+// stage s + 1 is complete (its weights are read there, its activations behind the barrier in front of the fourth run); the loads
+// of stage s + n go out behind that barrier, into the buffer whose last fragments were read before it.
 #include <cstddef>
 
 #include "lds_dma.h"
@@ -55,8 +57,8 @@ constexpr int fd_group_bytes(int NB, int KG) { return fd_stages(NB, KG) * NB * 4
 
 // Piece q of row r of a stage lies at place q ^ fd_place(r / 2).  A 16-byte read from LDS takes its lanes in groups that hold
 // rows 0 .. 3 and 12 .. 15 of one pair of pieces with rows 4 .. 11 of the next pair: those must differ.  (With r / 2 itself every
-// fragment read met half of the banks twice: 2.2 M of the 4.9 M
-// LDS cycles of 1000 x 2560 x 6912 were conflicts, now none of 2.7 M; 49.6 -> 44.1 us there with the decode below.)
+// fragment read met half of the banks twice: 2.2 M of the 4.9 M LDS cycles of 1000 x 2560 x 6912 were conflicts, now none of
+// 2.7 M; 49.6 -> 44.1 us there with the decode below.)
 __device__ __forceinline__ uint32_t fd_place(uint32_t half_row) { return (half_row & 1u) | ((half_row >> 2) & 1u) * 6u; }
 
 // y = sum * scale + bias, row block by row block (the empty asm keeps a row's address from being computed ahead of its turn)
@@ -142,9 +144,10 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
     const int rounds = KG == 1 ? nst : (nst + 1) / 2, st0 = group * rounds, mine = KG == 1 ? nst : min(rounds, nst - st0);
     const int st_tail = group == KG - 1 ? mine - 1 : rounds;  // TAIL: the partial stage, if it is this group's
 
-    // A stage's row is 128 bytes of LDS, eight pieces of 16; at the places fd_place gives them.  A wave loads whole rows, eight lanes each: lanes of a load that each have a
-    // row of their own take the cache four times as long.  Wave w loads rows 8 NB w .. +8 NB-1, eight at a time.  Rows past M
-    // repeat the last one, columns past N column 0 or the copy's last tile (never stored).
+    // A stage's row is 128 bytes of LDS, eight pieces of 16 at the places fd_place gives them.  A wave loads whole rows, eight
+    // lanes each: lanes of a load that each have a row of their own take the cache four times as long.  Wave w loads rows
+    // 8 NB w .. +8 NB-1, eight at a time.  Rows past M repeat the last one, columns past N column 0 or the copy's last tile
+    // (never stored).
     const int64_t rows_left = (p.M - m0 < BM) ? p.M - m0 : BM;
     uint32_t a_off[A_LOADS], a_tail[A_LOADS];
 #pragma unroll
@@ -478,9 +481,9 @@ static bool f16_splits_k(int64_t stages) { return stages >= 24; }
 
 // Rows of the tiles in units of 32, and what the launch takes in microseconds.  Up to one tile of 32, then of 64 rows for each
 // compute unit the launch is one tile deep; beyond that a compute unit's run of tiles is priced.  Measured (tiles of 128 / 64 /
-// 32 rows, us, row-major weights): M = 512, 1024, 1536, 2048, 3072, 4096 with N = K = 4096 48 / 34 / 31, 49 / 35 / 43,
-// 50 / 53 / 59, 53 / 57 / 74, 89 / 82 / 107, 101 / 110 / 141; 1000 x 13824 x 2560 61 / 68 / 78; 1000 x 2560 x 6912 80 / 54 / 70;
-// 16384 x 768 x 768 23 / 21 / 26; 4096 x 11008 x 4096 (the last round in halves) 260 / 279 / 360.
+// 32 rows, us, row-major weights): M = 512, 1024, 1536, 2048, 3072, 4096 with N = K = 4096 30 / 30 / 25, 33 / 31 / 40,
+// 49 / 49 / 53, 52 / 54 / 75, 89 / 81 / 107, 95 / 106 / 139; 1000 x 13824 x 2560 60 / 66 / 81; 1000 x 2560 x 6912 66 / 45 / 62;
+// 16384 x 768 x 768 21 / 20 / 26; 4096 x 11008 x 4096 (the last round in halves) 251 / 264 / 333.
 static int gemm_f16_plan(int64_t M, int64_t N, int64_t K, double* us) {
     const int64_t C = gemm_compute_units(), tn = ceil_div(N, F_BN);
     const int64_t t4 = ceil_div(M, 128) * tn, t2 = ceil_div(M, 64) * tn, t1 = ceil_div(M, 32) * tn;
