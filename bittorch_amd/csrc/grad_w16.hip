@@ -10,10 +10,11 @@
 // A 256-thread workgroup owns 256 x 256 outputs, a wave 128 x 128 of them (256 accumulators a lane, one wave a SIMD): a stage
 // of 32 m is 64 MFMAs a wave (1024 cycles) for 64 KiB read from and 32 KiB written to LDS per workgroup, and an XCD's 32
 // workgroups read 12 strips of 256 columns.  The matrix cores are busy for 62 % of the time (69 % in
-// one long round), and the rest goes to the issue of a lone wave's other instructions.  4096 x 11008 x 4096 (rows, dY's columns, X's), fp16 to fp32, 345 us = 1.07 PFLOP/s, the last
-// of three rounds of tiles two thirds full; the vendor's product (393 us in a profile) and the pass that scaled and widened its
-// result 449.  The same stages make tiles of 128 x 128 for outputs that would leave compute units idle: a stage is
-// 64 m, half of them for each wave of an operand, and a wave 64 x 64 outputs (768 x 768 of 300 rows 10.2 us, 17.5 in tiles of 256).
+// one long round), and the rest goes to the issue of a lone wave's other instructions.  4096 x 11008 x 4096 (rows, dY's columns,
+// X's), fp16 to fp32, 345 us = 1.07 PFLOP/s, the last of three rounds of tiles two thirds full; the vendor's product (393 us in a
+// profile) and the pass that scaled and widened its result 449.  The same stages make tiles of 128 x 128 for outputs that would
+// leave compute units idle: a stage is 64 m, half of them for each wave of an operand, and a wave 64 x 64 outputs (768 x 768 of 300
+// rows 10.2 us, 17.5 in tiles of 256).
 #include "bt_common.h"
 
 namespace bt {
