@@ -88,7 +88,7 @@ int launch_row_op(int op, int dtype, const void* A, int64_t lda, const void* Bv,
 bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, const void* Y, bool tiled);
 double gemm_f16_cost(int64_t M, int64_t N, int64_t K);
 int launch_gemm_f16(int mode, const void* X, const uint8_t* W_T, int w_layout, const Epilogue& epi, void* Y, int64_t M,
-                    int64_t N, int64_t K, hipStream_t st, int64_t Kw = 0);
+                    int64_t N, int64_t K, hipStream_t st, int64_t Kw = 0, int epi_op = 0);
 int launch_pad_rows(const void* X, int64_t B, int64_t K, void* P, hipStream_t st);
 bool gemm_f32_shape_ok(int64_t N, int64_t K);
 bool gemm_f32_supported(int64_t N, int64_t K, const void* X, const void* Y);
@@ -377,12 +377,12 @@ static int packed_forward_impl(const char* who, const void* X, int x_dtype, cons
             return launch_planes_bf16_wide(X, W_T, epi, Y, N, K, st);
         if (x_dtype != BT_F32) {
             const int mode = (x_dtype == BT_F16) ? MODE_F16 : MODE_BF16;
-            // tall batches: the tiled matrix-core GEMM reads the copy too (not with the SwiGLU output stage)
+            // tall batches: the tiled matrix-core GEMM reads the copy too
             const void* rows = X;
             int64_t Kr = K;  // values of a row of them
             if ((rc = pad_rows_if(X, x_dtype, B, K, workspace, workspace_bytes, st, &rows, &Kr))) return rc;
-            if (!prefers_stream(B, N, K, false, true) && epi_op == 0 && gemm_f16_supported(N, Kr, rows, W_T, Y, true))
-                return launch_gemm_f16(mode, rows, W_T, w_layout, epi, Y, B, N, Kr, st, K);
+            if (!prefers_stream(B, N, K, false, true) && gemm_f16_supported(N, Kr, rows, W_T, Y, true))
+                return launch_gemm_f16(mode, rows, W_T, w_layout, epi, Y, B, N, Kr, st, K, epi_op);
             return launch_stream(mode, rows, 2, nullptr, W_T, w_layout, epi, Y, x_dtype, nullptr, B, N, Kr, 1,
                                  Q_ROW_MAJOR, 0, nullptr, 0.0f, epi_op, st, K);
         }

@@ -26,6 +26,7 @@
 #include <cstddef>
 
 #include "lds_dma.h"
+#include "row_math.h"
 
 namespace bt {
 
@@ -125,10 +126,66 @@ __device__ __forceinline__ void fd_epilogue(const GemmFParams& p, const v4f (&ac
     }
 }
 
+// The SwiGLU output stage (EPI_SWIGLU_PAIRS): a lane holds columns c, c + 1 of the gate in t = 0, 1 and the same of up in t = 2, 3,
+// and stores what the SwiGLU row kernel would make of the rounded outputs: the same element arithmetic, hence the same bits.  Bound by
+// that arithmetic, 64 values a lane behind the last stage of a tile (3 us where all tiles end together); it saves the projections'
+// way to memory and back and a launch.  GEMM and row kernel / this, us, bf16: 1000 x 13824 x 2560 73.4 / 65.4, 4096 x 13824 x 2560
+// 238 / 217, 300 x 8192 x 2048 23.8 / 19.5.  (4-byte stores of each row 67.2 and 222 on the first two.)
+template <int MODE, int MB>
+__device__ __forceinline__ void fd_epilogue_swiglu(const GemmFParams& p, const v4f (&acc)[MB][4], int64_t m0, int g, int64_t col,
+                                                   int rows_left, const float (&ws)[4], const float (&bs)[4]) {
+    constexpr int YDT = MODE == MODE_F16 ? BT_F16 : BT_BF16;
+    const int64_t row_bytes = p.N;  // (N / 2 outputs of two bytes)
+    char* row = (char*)p.Y + m0 * row_bytes;
+    const uint32_t lane_off = (uint32_t)(4 * g) * (uint32_t)row_bytes + (uint32_t)col * 2u;
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++) {
+        if (16 * mb >= rows_left) return;  // (uniform)
+        float y[4][4];
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                float a = acc[mb][t][r];
+                if constexpr (MODE == MODE_BF16) a *= 0.5f;  // weights were decoded as +-2.0
+                y[t][r] = round_to_dtype(epi_float(a, ws[t], bs[t]), YDT);
+            }
+        float gate[8], up[8];
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                gate[2 * r + t] = y[t][r];
+                up[2 * r + t] = y[2 + t][r];
+            }
+        swiglu8<YDT>(gate, up);
+        // lanes 2 i and 2 i + 1 hold neighbouring columns: the even one takes two of the rows, the odd one the other two
+        uint32_t d[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const uint16_t h0 = YDT == BT_F16 ? f32_to_f16_bits(gate[2 * r]) : f32_to_bf16_bits(gate[2 * r]);
+            const uint16_t h1 = YDT == BT_F16 ? f32_to_f16_bits(gate[2 * r + 1]) : f32_to_bf16_bits(gate[2 * r + 1]);
+            d[r] = (uint32_t)h0 | ((uint32_t)h1 << 16);
+        }
+        const bool odd = threadIdx.x & 1;
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const uint32_t keep = odd ? d[2 + r] : d[r], give = odd ? d[r] : d[2 + r];
+            const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give, 0xB1, 0xf, 0xf, true);
+            char* at = row + r * row_bytes + lane_off + (odd ? 2 * (uint32_t)row_bytes - 4u : 0u);
+            if (16 * mb + 4 * g + r + (odd ? 2 : 0) < rows_left) st2_nt(at, odd ? got : keep, odd ? keep : got);
+        }
+        row += 16 * row_bytes;
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 // One tile of 32 NB rows.  TAIL: K is not a multiple of 64 (of 8 it is): the lanes whose k lies past
 // the end load something of their own row or column instead and their activations are zeroed on the way to the MFMAs.
 // KG = 2: two groups of four waves, each on its run of the stages; they add their sums through LDS and store half the rows each.
-template <int MODE, int SRC, int NB, int KG, bool TAIL, bool RN>
+// SW: the SwiGLU output stage on a copy in gate/up pair order (stored tiles 2 i, 2 i + 1 are 16 columns of the gate and the same of up):
+// a lane takes two columns of either, so that no sum changes lanes.
+template <int MODE, int SRC, int NB, int KG, bool TAIL, bool RN, bool SW>
 __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_t m0, const int tile_n, uint8_t* lds_all) {
     constexpr int BM = 32 * NB, A_BYTES = NB * 4096, NST = fd_stages(NB, KG), W_AT = NST * A_BYTES;
     constexpr int A_LOADS = NB, W_LOADS = SRC == W_ROWS ? 4 : 1, LOADS = A_LOADS + W_LOADS;
@@ -224,9 +281,15 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
     auto read_raw = [&](uint32_t wbuf) {
         const uint8_t* src = lds + wbuf + wave * 1024;
         if constexpr (SRC == W_TILES) {
-            const u32x4 v = *(const u32x4*)(src + 16 * lane);
+            if constexpr (SW) {  // lane (j, g)'s 16 bytes are those of columns 4 (j % 4) .. +3 of stored tile j / 4
+                const uint8_t* at = src + 256 * g + 128 * (j >> 3) + 8 * (j & 7);
+                const u32x2 a = *(const u32x2*)at, b = *(const u32x2*)(at + 64);
+                raw[0] = a[0]; raw[1] = a[1]; raw[2] = b[0]; raw[3] = b[1];
+            } else {
+                const u32x4 v = *(const u32x4*)(src + 16 * lane);
 #pragma unroll
-            for (int t = 0; t < 4; t++) raw[t] = v[t];
+                for (int t = 0; t < 4; t++) raw[t] = v[t];
+            }
         } else {
 #pragma unroll
             for (int r = 0; r < 4; r++) raw[r] = *(const uint32_t*)(src + 256 * r + 4 * lane);
@@ -391,11 +454,12 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
     if (KG > 1 && mine < rounds) asm volatile("s_barrier" ::: "memory");  // (uniform; the other group has one stage more)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (no load may reach LDS that another workgroup owns by then)
 
+    const int64_t half_n = p.N / 2, scol = (int64_t)tile_n * (F_BN / 2) + 32 * wave + 2 * j;  // SW: the first of this lane's outputs
     float ws[4], bs[4];
     uint32_t ws_bits[4], bs_bits[4];
 #pragma unroll
     for (int t = 0; t < 4; t++) {
-        const int64_t n = !col_ok ? 0 : RN ? min(ncol + t, p.N - 1) : ncol + t;
+        const int64_t n = SW ? (scol < half_n ? scol + (t & 1) + (t >> 1) * half_n : 0) : !col_ok ? 0 : RN ? min(ncol + t, p.N - 1) : ncol + t;
         ws_bits[t] = load_bits_rt(p.epi.scale, p.epi.scale_dtype, p.epi.scale_bcast ? 0 : n);
         bs_bits[t] = p.epi.bias ? load_bits_rt(p.epi.bias, p.epi.bias_dtype, n) : 0u;
     }
@@ -404,12 +468,14 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
         ws[t] = bits_to_f32_rt(ws_bits[t], p.epi.scale_dtype);
         bs[t] = p.epi.bias ? bits_to_f32_rt(bs_bits[t], p.epi.bias_dtype) : 0.0f;
     }
+    const bool stores = SW ? scol < half_n : col_ok;
     auto store = [&](const auto& sums, int64_t row0, int left) {
-        if (p.epi.residual) fd_epilogue<MODE, true, RN>(p, sums, row0, g, ncol, left, ws, bs);
+        if constexpr (SW) fd_epilogue_swiglu<MODE>(p, sums, row0, g, scol, left, ws, bs);
+        else if (p.epi.residual) fd_epilogue<MODE, true, RN>(p, sums, row0, g, ncol, left, ws, bs);
         else fd_epilogue<MODE, false, RN>(p, sums, row0, g, ncol, left, ws, bs);
     };
     if constexpr (KG == 1) {
-        if (col_ok) store(acc, m0, (int)rows_left);
+        if (stores) store(acc, m0, (int)rows_left);
     } else {
         // group 0 takes the first NB row blocks, group 1 the others: each hands over the sums that it does not store
         v4f* const mine_at = (v4f*)lds_all + wave_all * (256 * NB) + lane;
@@ -429,12 +495,12 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
 #pragma unroll
             for (int t = 0; t < 4; t++) sums[i][t] += theirs_at[64 * (4 * i + t)];
         const int left = (int)rows_left - 16 * NB * group;
-        if (col_ok && left > 0) store(sums, m0 + 16 * NB * group, left);
+        if (stores && left > 0) store(sums, m0 + 16 * NB * group, left);
     }
 }
 
 // NB: tiles of 32 NB rows.  NF > 0: an XCD's tiles from p.fine_from on are computed in tiles of 32 NF rows.
-template <int MODE, int SRC, int NB, int NF, int KG, bool TAIL, bool RN>
+template <int MODE, int SRC, int NB, int NF, int KG, bool TAIL, bool RN, bool SW>
 __global__ __launch_bounds__(256 * KG, KG == 2 || NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_f16_kernel(GemmFParams p) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[KG * fd_group_bytes(NB, KG)];
     // XCD-aware tile order: the 8 XCDs each take a contiguous run of tiles, walked in groups of four row tiles, so that one
@@ -456,11 +522,11 @@ __global__ __launch_bounds__(256 * KG, KG == 2 || NB == 4 ? 2 : NB == 2 ? 3 : 4)
     if constexpr (NF > 0) {
         if (fine) {
             const int64_t mf = m0 + (int64_t)(f % parts) * (32 * NF);
-            if (mf < p.M) gemm_f16_tile<MODE, SRC, NF, 1, TAIL, RN>(p, mf, (int)tn, lds);
+            if (mf < p.M) gemm_f16_tile<MODE, SRC, NF, 1, TAIL, RN, SW>(p, mf, (int)tn, lds);
             return;
         }
     }
-    gemm_f16_tile<MODE, SRC, NB, KG, TAIL, RN>(p, m0, (int)tn, lds);
+    gemm_f16_tile<MODE, SRC, NB, KG, TAIL, RN, SW>(p, m0, (int)tn, lds);
 }
 
 // X and Y are read and written in 16- and 8-byte pieces; 32-bit byte offsets span a tile's rows of X, 16 rows of Y and, for
@@ -503,7 +569,7 @@ double gemm_f16_cost(int64_t M, int64_t N, int64_t K) {
     return us;
 }
 
-template <int MODE, int SRC, int NB, bool TAIL, bool RN = false>
+template <int MODE, int SRC, int NB, bool TAIL, bool RN = false, bool SW = false>
 static int launch_gemm_f16_cfg(GemmFParams p, hipStream_t st) {
     const char* who = SRC == W_TILES ? "bt_ternary_linear_tiled_forward" : "bt_ternary_linear_packed_forward";
     p.tiles_n = (int)ceil_div(p.N, F_BN);
@@ -522,40 +588,45 @@ static int launch_gemm_f16_cfg(GemmFParams p, hipStream_t st) {
             const int rem = p.per_xcd % (int)(2 * gemm_compute_units() / 8);
             p.fine_from = p.per_xcd - rem;
             const dim3 grid((unsigned)(8 * (p.fine_from + parts * rem)));
-            if (parts == 2) hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 4, 2, 1, TAIL, RN>), grid, block, 0, st, p);
-            else hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 4, 1, 1, TAIL, RN>), grid, block, 0, st, p);
+            if (parts == 2) hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 4, 2, 1, TAIL, RN, SW>), grid, block, 0, st, p);
+            else hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 4, 1, 1, TAIL, RN, SW>), grid, block, 0, st, p);
             return check_launch(who);
         }
     }
     if constexpr (NB != 4) {
         if (total <= gemm_compute_units() && f16_splits_k(p.wstages)) {
-            hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, NB, 0, 2, TAIL, RN>), dim3((unsigned)(8 * p.per_xcd)), dim3(512), 0, st, p);
+            hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, NB, 0, 2, TAIL, RN, SW>), dim3((unsigned)(8 * p.per_xcd)), dim3(512), 0, st, p);
             return check_launch(who);
         }
     }
-    hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, NB, 0, 1, TAIL, RN>), dim3((unsigned)(8 * p.per_xcd)), block, 0, st, p);
+    hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, NB, 0, 1, TAIL, RN, SW>), dim3((unsigned)(8 * p.per_xcd)), block, 0, st, p);
     return check_launch(who);
 }
 template <int MODE, int SRC, int NB>
-static int launch_gemm_f16_src(const GemmFParams& p, hipStream_t st) {
-    if constexpr (SRC == W_TILES) {  // (rows of any length come with K of any length: one instance)
+static int launch_gemm_f16_src(const GemmFParams& p, int epi_op, hipStream_t st) {
+    if constexpr (SRC == W_TILES) {
+        if (epi_op == EPI_SWIGLU_PAIRS)
+            return p.K % F_BK != 0 ? launch_gemm_f16_cfg<MODE, SRC, NB, true, false, true>(p, st)
+                                   : launch_gemm_f16_cfg<MODE, SRC, NB, false, false, true>(p, st);
+        // (rows of any length come with K of any length: one instance)
         if (p.N % 4 != 0) return launch_gemm_f16_cfg<MODE, SRC, NB, true, true>(p, st);
     }
     return p.K % F_BK != 0 ? launch_gemm_f16_cfg<MODE, SRC, NB, true>(p, st) : launch_gemm_f16_cfg<MODE, SRC, NB, false>(p, st);
 }
 template <int MODE, int NB>
-static int launch_gemm_f16_mode(const GemmFParams& p, int src, hipStream_t st) {
-    return src == W_TILES ? launch_gemm_f16_src<MODE, W_TILES, NB>(p, st)
-         : src == W_ROWS16 ? launch_gemm_f16_src<MODE, W_ROWS16, NB>(p, st) : launch_gemm_f16_src<MODE, W_ROWS, NB>(p, st);
+static int launch_gemm_f16_mode(const GemmFParams& p, int src, int epi_op, hipStream_t st) {
+    return src == W_TILES ? launch_gemm_f16_src<MODE, W_TILES, NB>(p, epi_op, st)
+         : src == W_ROWS16 ? launch_gemm_f16_src<MODE, W_ROWS16, NB>(p, 0, st) : launch_gemm_f16_src<MODE, W_ROWS, NB>(p, 0, st);
 }
 template <int MODE>
-static int launch_gemm_f16_rows(const GemmFParams& p, int rows, int src, hipStream_t st) {
-    return rows == 4 ? launch_gemm_f16_mode<MODE, 4>(p, src, st)
-         : rows == 2 ? launch_gemm_f16_mode<MODE, 2>(p, src, st) : launch_gemm_f16_mode<MODE, 1>(p, src, st);
+static int launch_gemm_f16_rows(const GemmFParams& p, int rows, int src, int epi_op, hipStream_t st) {
+    return rows == 4 ? launch_gemm_f16_mode<MODE, 4>(p, src, epi_op, st)
+         : rows == 2 ? launch_gemm_f16_mode<MODE, 2>(p, src, epi_op, st) : launch_gemm_f16_mode<MODE, 1>(p, src, epi_op, st);
 }
+// epi_op: 0, or EPI_SWIGLU_PAIRS (w_layout W_LAYOUT_TILED in pair order, N % 32 == 0, no residual; Y is [M, N / 2])
 // Kw: the weights' K where the rows of X are longer (zeros behind it; 0: K)
 int launch_gemm_f16(int mode, const void* X, const uint8_t* W_T, int w_layout, const Epilogue& epi, void* Y, int64_t M,
-                    int64_t N, int64_t K, hipStream_t st, int64_t Kw) {
+                    int64_t N, int64_t K, hipStream_t st, int64_t Kw, int epi_op) {
     GemmFParams p = {};
     p.X = (const uint16_t*)X; p.W_T = W_T; p.Y = Y; p.epi = epi;
     p.M = M; p.N = N; p.K = K; p.Kb = ceil_div(Kw ? Kw : K, 4);
@@ -563,7 +634,7 @@ int launch_gemm_f16(int mode, const void* X, const uint8_t* W_T, int w_layout, c
     p.tiles16 = tiles16_arg(N, w_layout);
     double us;
     const int rows = gemm_f16_plan(M, N, K, &us), src = w_source(layout_tiled(w_layout), false, W_T, N);
-    return mode == MODE_F16 ? launch_gemm_f16_rows<MODE_F16>(p, rows, src, st) : launch_gemm_f16_rows<MODE_BF16>(p, rows, src, st);
+    return mode == MODE_F16 ? launch_gemm_f16_rows<MODE_F16>(p, rows, src, epi_op, st) : launch_gemm_f16_rows<MODE_BF16>(p, rows, src, epi_op, st);
 }
 
 }  // namespace bt

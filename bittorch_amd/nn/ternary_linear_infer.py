@@ -32,8 +32,6 @@ from ..quant.ternary import ternary_quantize
 from ..quant.ternary_packed import pack_ternary_transposed, unpack_ternary_transposed
 
 
-# batches up to this many rows stream the tiled weights (once per 16 rows) instead of running the tiled GEMM
-DECODE_ROWS = 128
 # From this many rows an int8 call with row sums takes the prefill GEMM on the field-layout copy (prepare_prefill):
 # below it the routing between the streaming kernel and the tiled GEMM on the decode-tiled copy does as well or better.
 PREFILL_ROWS = 384
@@ -221,15 +219,15 @@ class TernaryLinearInference(nn.Module):
             return self._fields
         return None
 
-    def _tiled_for(self, x: Tensor, rows: int, order: str = "natural") -> Optional[Tensor]:
+    def _tiled_for(self, x: Tensor, order: str = "natural") -> Optional[Tensor]:
         """The tiled copy if this call can run on it, else None.  ``order`` is what the call wants: ``"natural"`` (a
         plain linear output; a copy in gate/up pair order serves it too, the kernels looking every column tile up
         where the pair order put it -- float activations only, see ``_natural_from_pairs``) or ``"gate_up_pairs"``
-        (the SwiGLU output stage: pair-ordered copy, decode shapes)."""
+        (the SwiGLU output stage: pair-ordered copy)."""
         if not (self.decode_tiled and x.is_cuda):
             return None
         if order == "gate_up_pairs":
-            if self._tile_order != order or rows > DECODE_ROWS:
+            if self._tile_order != order:
                 return None
         elif self._tile_order != "natural" and x.dtype == torch.int8:
             return None  # the int8 entry point reads natural-order copies only
@@ -274,7 +272,7 @@ class TernaryLinearInference(nn.Module):
         ``swiglu_up=u`` makes the input ``silu(x) * u`` (for a single decode token both run inside the
         GEMV kernel itself)."""
         if x.is_cuda:
-            tiled = self._tiled_for(x, x.numel() // max(x.shape[-1], 1))
+            tiled = self._tiled_for(x)
             if tiled is not None:
                 from .. import _C
                 scale, bias = self._scale_bias()
@@ -301,10 +299,10 @@ class TernaryLinearInference(nn.Module):
 
     def forward_swiglu(self, x: Tensor, norm=None) -> Tensor:
         """For a layer whose columns are ``[gate | up]``: ``swiglu(gate(h), up(h))`` ``(*, N/2)`` with ``h = x`` or
-        ``rmsnorm(x, *norm)``.  Decode-shape calls on a layer with ``tile_order == "gate_up_pairs"`` form the product
-        in the output stage of the GEMV kernel; everything else runs the projection and the SwiGLU kernel."""
+        ``rmsnorm(x, *norm)``.  16-bit calls on a layer with ``tile_order == "gate_up_pairs"`` form the product
+        in the output stage of the GEMV or GEMM kernel; everything else runs the projection and the SwiGLU kernel."""
         if x.is_cuda:
-            tiled = self._tiled_for(x, x.numel() // max(x.shape[-1], 1), "gate_up_pairs")
+            tiled = self._tiled_for(x, "gate_up_pairs")
             if tiled is not None and x.dtype in (torch.float16, torch.bfloat16):
                 from .. import _C
                 scale, bias = self._scale_bias()
@@ -334,7 +332,7 @@ class TernaryLinearInference(nn.Module):
                                             None if residual is None else residual.reshape(-1, residual.shape[-1]),
                                             q_operand_order, self._natural_from_pairs)
             return y.reshape(*q.shape[:-1], self.out_features)
-        tiled = self._tiled_for(q, rows)
+        tiled = self._tiled_for(q)
         if tiled is not None:
             from .. import _C
             lead = q.shape[:-1]

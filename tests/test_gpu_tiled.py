@@ -593,6 +593,33 @@ def test_swiglu_output_stage_equals_projection_then_swiglu(oracle, dtype, n, k):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,n,k", [(33, 96, 100), (200, 96, 64), (70, 64, 1536), (40, 8192, 4096), (300, 8192, 1600), (500, 320, 1030),
+                                   (1000, 13824, 512), (2048, 11008, 256), (1700, 10240, 136)])
+def test_swiglu_output_stage_of_the_tiled_gemm(oracle, dtype, b, n, k):
+    """Bit for bit what the SwiGLU kernel makes of the same GEMM's stored projections: tiles of 32, 64 and 128 rows and the finer ones
+    of a remainder, one and two groups of waves, a last wave of 16 of its 32 columns, K past whole stages, rows that are padded,
+    infinities and NaN."""
+    from bittorch_amd import _C
+    _, wt = _packed(oracle, n, k, seed=7)
+    pairs = _C.retile_weights(wt, k, True)
+    g = torch.Generator().manual_seed(n)
+    scale = (torch.rand(n, generator=g) + 0.5).cuda() * 0.05
+    bias = (torch.randn(n, generator=g) * 0.1).to(dtype).cuda()
+    x = seeded_acts(b, k, seed=b, dtype=dtype)
+    x[1, 3], x[b - 1, k - 1], x[2] = float("inf"), float("nan"), x[2] * 500
+    x = x.cuda()
+    set_option("STREAM_MAX_ROWS", "32")
+    for bs in (None, bias):
+        announce("swiglu stage of the GEMM", dtype, b, n, k, bs is not None)
+        gu = _C.ternary_linear_tiled_forward(x, pairs, scale, bs, k, n, natural_from_pairs=True)
+        want = _C.swiglu(gu[:, :n // 2], gu[:, n // 2:])
+        got = _C.ternary_linear_tiled_forward(x, pairs, scale, bs, k, n, swiglu_pairs=True)
+        assert got.shape == (b, n // 2)
+        same = (got == want) | (got.isnan() & want.isnan())
+        assert bool(same.all()), int((~same).sum())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_ternary_swiglu_decode_uses_the_output_stage(oracle, dtype):
     from bittorch_amd.nn import TernarySwiGLU
     d, ffn = 256, 704
