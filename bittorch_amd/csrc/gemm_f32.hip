@@ -70,7 +70,9 @@ struct GemmF32Params {
     const uint8_t* W;
     int64_t M, C, NC;    // NC: output columns
     int tiles_m, tiles_n;
-    int per_xcd;         // workgroups per XCD (grid = 8 * per_xcd)
+    int per_xcd;         // tiles per XCD
+    int fine_from;       // REM: an XCD's tiles from this one on are shared by `parts` workgroups each
+    int parts;           // 2 or 4
     int wsteps;          // B_TILED: 64-wide steps of the copy
     int tiles16;         // B_TILED: as in tiles16_arg
     int ldw;             // bytes of a W_T row
@@ -87,16 +89,22 @@ constexpr uint32_t LUT_BF16_HALF = 0x00BF3F00u;
 // A wave works on a tile of 64 rows x 64 NG columns.  KS = 1: the four waves of a workgroup are a 2 x 2 block of such tiles.
 // KS > 1: all KS waves of a workgroup work on one tile, each on its run of the contraction, and add their sums through LDS
 // (pairwise, always in the same order): for outputs with too few tiles to occupy the chip.
+// REM (KS = 1): a tile of the remainder, the last that would occupy a part of the compute units only, is shared by two workgroups of
+// 64 rows or four of one wave's tile each; their waves take halves or quarters of the contraction and add their sums through LDS.
 // SC: X's columns are scaled (input gradient with one scale per row of W).
 // RN: forward outputs of N % 4 != 0, an instance of its own: asked at run time, every other output paid half a microsecond for
 // the clamped columns and the second way to store (us, fp32, 300 x 4096 x 512 17.9 / 17.0, 4096 x 768 x 768 28.2 / 27.5).  Only
 // the tile of one wave's 64 x 64 outputs gains from the question: with a branch between them the compiler sends each row's
 // stores off by themselves (512 x 2048 x 1032 17.0 without, 16.0 with it; 4096 x 128 x 2048 24.1 / 23.1).
-template <int SRC, int NG, int KS, bool SC, bool RN>
+template <int SRC, int NG, int KS, bool SC, bool RN, bool REM>
 __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(GemmF32Params p) {
     constexpr int TM = (KS == 1) ? 128 : 64, TN = (KS == 1) ? 128 * NG : 64 * NG;  // a workgroup's tile
     // the 8 XCDs each take a contiguous run of tiles, walked in groups of four row tiles (as in gemm_f16.hip)
-    const uint32_t lin = (blockIdx.x & 7u) * (uint32_t)p.per_xcd + (blockIdx.x >> 3);
+    const uint32_t idx = blockIdx.x >> 3;
+    const bool fine = REM && idx >= (uint32_t)p.fine_from;  // (uniform)
+    const uint32_t parts = fine ? (uint32_t)p.parts : 1u, part = fine ? (idx - (uint32_t)p.fine_from) & (parts - 1u) : 0u;
+    const uint32_t in_xcd = fine ? (uint32_t)p.fine_from + ((idx - (uint32_t)p.fine_from) >> (parts >> 1)) : idx;
+    const uint32_t lin = (blockIdx.x & 7u) * (uint32_t)p.per_xcd + in_xcd;
     const uint32_t tiles_m = (uint32_t)p.tiles_m, tiles_n = (uint32_t)p.tiles_n;
     if (lin >= tiles_m * tiles_n) return;
     constexpr uint32_t GM = 4;
@@ -108,9 +116,13 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i = lane & 15, g = lane >> 4;
-    const int64_t m0 = (int64_t)tm * TM + (KS == 1 ? 64 * (wave >> 1) : 0);
-    const int64_t c0 = (int64_t)tn * TN + (KS == 1 ? 64 * NG * (wave & 1) : 0);
-    if (KS == 1 && (m0 >= p.M || c0 >= p.NC)) return;  // (no barriers below when KS == 1)
+    // which of the tile's four wave tiles, and how many waves share it
+    const int row_half = parts == 1 ? wave >> 1 : parts == 2 ? (int)part : (int)part >> 1, col_half = parts <= 2 ? wave & 1 : (int)part & 1;
+    const int ks = KS > 1 ? KS : (int)parts, k_part = KS > 1 ? wave : parts == 1 ? 0 : parts == 2 ? wave >> 1 : wave;
+    const int64_t m0 = (int64_t)tm * TM + (KS == 1 ? 64 * row_half : 0);
+    const int64_t c0 = (int64_t)tn * TN + (KS == 1 ? 64 * NG * col_half : 0);
+    // (no barriers below for these; of two wave tiles side by side the second may lie past the last column: it loads clamped ones)
+    if (KS == 1 && (m0 >= p.M || (c0 >= p.NC && parts != 2))) return;
 
     // rows and columns past the end repeat the last one: they only feed outputs that are never stored
     const uint8_t* a_base = (const uint8_t*)(p.X + m0 * p.C);
@@ -140,9 +152,9 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
     const uint32_t sel_wt = ((uint32_t)(2 * (g & 1) + 1) << 24) | (0x0Cu << 16) | ((uint32_t)(2 * (g & 1)) << 8) | 0x0Cu;
     // this wave's steps of 32: [st0, st1) of the whole ones, and the partial one if it is the last wave
     const int nfull = (int)(p.C / 32), steps = (int)((p.C + 31) / 32);
-    const int run = (KS == 1) ? nfull : (nfull + KS - 1) / KS;
-    const int st0 = (KS == 1) ? 0 : min(wave * run, nfull), st1 = (KS == 1) ? nfull : min(st0 + run, nfull);
-    const bool last = KS == 1 || wave == KS - 1;
+    const int run = (KS == 1) ? (nfull + ks - 1) >> (ks >> 1) : (nfull + KS - 1) / KS;  // (KS == 1: ks is 1, 2 or 4)
+    const int st0 = min(k_part * run, nfull), st1 = min(st0 + run, nfull);
+    const bool last = k_part == ks - 1;
 
     constexpr int BR = (SRC == B_TILED) ? 4 : 2;
     f32x4_u raw[4][2];
@@ -306,11 +318,14 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
                 for (int r = 0; r < 4; r++) bad |= acc[b][t][r] != acc[b][t][r];
         if (__any(bad)) contract(std::true_type{});
     }
-    if constexpr (KS > 1) {
-        // the upper half of the waves hands its sums to the lower half, until wave 0 has them all; NG words of 16 KiB each
-        __shared__ __attribute__((aligned(16))) float xch[KS / 2 * 4096 * NG];
+    if (KS > 1 || fine) {
+        // the upper half of the waves hands its sums to the lower half, until the first wave of a tile has them all; NG words of 16 KiB each
+        constexpr int KW = KS > 1 ? KS : REM ? 4 : 1;
+        __shared__ __attribute__((aligned(16))) float xch[KW > 1 ? KW / 2 * 4096 * NG : 1];
+        const int least = KS > 1 || parts == 4 ? 1 : 2;  // (parts == 2: waves 2 and 3 are the other halves of waves 0 and 1)
 #pragma unroll
-        for (int half = KS / 2; half >= 1; half /= 2) {
+        for (int half = KW / 2; half >= 1; half /= 2) {
+            if (half < least) break;  // (uniform)
             if (wave >= half && wave < 2 * half) {
 #pragma unroll
                 for (int b = 0; b < 4; b++)
@@ -328,7 +343,7 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
             }
             __syncthreads();
         }
-        if (wave != 0) return;
+        if (wave >= least) return;
     }
 
 #pragma unroll
@@ -384,6 +399,17 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
     }
 }
 
+// Into how many workgroups a tile of the remainder is shared (KS = 1): the tiles beyond one, two ... for every compute unit of an XCD
+// where they are at most half as many as compute units.  A shared tile saves half or three quarters of its steps at 1.2 us each and
+// costs 4 us for the sums' way through LDS.  (The plan is made without regard to it: where one with the contraction over four waves
+// was the cheaper, its sums are shorter ones too.)  us, before / now: 16384 x 768 x 768 forward 67.4 / 55.8, input gradient 75.1 / 64.7;
+// 9000 x 2304 x 768 90.9 / 80.6.
+static int gemm_f32_parts(int64_t tiles, int64_t steps) {
+    const int64_t cus = gemm_compute_units() / 8, per_xcd = ceil_div(tiles, 8), rem = per_xcd % cus;
+    if (per_xcd < cus || rem == 0 || 2 * rem > cus) return 1;
+    const int parts = 4 * rem > cus ? 2 : 4;
+    return 1.2 * (double)steps * (1.0 - 1.0 / parts) > 4.0 ? parts : 1;
+}
 template <int SRC, int NG, int KS, bool SC, bool RN>
 static int launch_gemm_f32_cfg(GemmF32Params p, const char* who, hipStream_t st) {
     p.tiles_m = (int)ceil_div(p.M, KS == 1 ? 128 : 64);
@@ -394,7 +420,17 @@ static int launch_gemm_f32_cfg(GemmF32Params p, const char* who, hipStream_t st)
         return BT_ERR_INVALID;
     }
     p.per_xcd = (int)ceil_div(total, 8);
-    hipLaunchKernelGGL((gemm_f32_kernel<SRC, NG, KS, SC, RN>), dim3((unsigned)(p.per_xcd * 8)), dim3(KS == 1 ? 256 : 64 * KS), 0, st, p);
+    p.parts = KS == 1 ? gemm_f32_parts(total, ceil_div(p.C, 32)) : 1;
+    const int rem = p.parts > 1 ? p.per_xcd % (int)(gemm_compute_units() / 8) : 0;
+    p.fine_from = p.per_xcd - rem;
+    const dim3 grid((unsigned)(8 * (p.fine_from + p.parts * rem))), block(KS == 1 ? 256 : 64 * KS);
+    if constexpr (KS == 1) {
+        if (rem > 0) {
+            hipLaunchKernelGGL((gemm_f32_kernel<SRC, NG, KS, SC, RN, true>), grid, block, 0, st, p);
+            return check_launch(who);
+        }
+    }
+    hipLaunchKernelGGL((gemm_f32_kernel<SRC, NG, KS, SC, RN, false>), grid, block, 0, st, p);
     return check_launch(who);
 }
 // Which split of the work?  0: tiles of 64 x 128 per wave, 1: the same with the contraction over the four waves of a

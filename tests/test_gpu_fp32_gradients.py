@@ -256,3 +256,24 @@ def test_fp32_forward_without_a_workspace(m, n, k):
     norm = _C.ternary_linear_tiled_forward(x, tiled, scale, None, k, n, norm=(None, 1e-5))
     xn = torch.nn.functional.rms_norm(x, (k,), None, 1e-5)
     assert torch.allclose(norm, (xn.double() @ (tern.double() * scale.double()[:, None]).t()).float(), rtol=1e-4, atol=1e-5)
+
+
+@gpu
+@pytest.mark.parametrize("m,n,k", [(33700, 250, 200), (33792, 120, 196), (49000, 256, 232), (34000, 510, 254)])
+def test_fp32_remainder_tiles_shared_by_waves(m, n, k):
+    """33 tiles of 128 x 256 an XCD leave one, 48 leave sixteen: each is shared by four or two workgroups whose waves split the
+    contraction.  Rows that end inside the last tile, one wave tile of columns, column halves past the end, a partial step."""
+    from bittorch_amd import _C
+    announce("fp32 remainder tiles", m, n, k)
+    x, dy, packed, scale, tern = _case(m, n, k)
+    _close(_C.linear_grad_input(dy, packed, scale, k), dy, tern * scale[:, None], _three_terms(n))
+    for y in (_C.ternary_linear_packed_forward(x, packed, scale, None, k),
+              _C.ternary_linear_tiled_forward(x, _C.retile_weights(packed, k), scale, None, k, n)):
+        _close(y, x, tern.t(), _three_terms(k), scale.double()[None, :])
+    bad = dy.clone()
+    bad[m - 1, 0], bad[5, n - 1], bad[m // 2, 1] = float("inf"), float("nan"), float("-inf")
+    got, want = _C.linear_grad_input(bad, packed, scale, k), (bad * scale) @ tern
+    rows = [m - 1, 5, m // 2]
+    for r in rows:
+        assert torch.equal(got[r].isnan(), want[r].isnan()) and torch.equal(got[r].isinf(), want[r].isinf())
+    assert torch.isfinite(got[[0, 6, m - 2]]).all()
