@@ -32,7 +32,7 @@ int check_launch(const char* what) {
 // ---- run-time options (bt_common.h) -----------------------------------------------------------------------------------
 static const char* const kOptionNames[OPT_COUNT] = {
     "STREAM_MAX_ROWS", "GEMM_LONG_EPILOGUE", "GEMM_TAIL_SPLIT", "GROUP_WALK", "GROUP_NACC",
-    "GROUP_UNITS", "PLANES_NACC", "ROWOP_GENERIC", "STREAM_CFG", "NO_PLANES",
+    "GROUP_UNITS", "PLANES_NACC", "ROWOP_GENERIC", "STREAM_CFG", "ROWS_CFG", "NO_PLANES",
 };
 struct OptionSlot {
     char text[2][48];              // two buffers, so that a reader never sees one being rewritten by the next override
@@ -89,6 +89,10 @@ bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, co
 double gemm_f16_cost(int64_t M, int64_t N, int64_t K);
 int launch_gemm_f16(int mode, const void* X, const uint8_t* W_T, int w_layout, const Epilogue& epi, void* Y, int64_t M,
                     int64_t N, int64_t K, hipStream_t st, int64_t Kw = 0, int epi_op = 0);
+bool rows_f16_supported(int64_t N, int64_t K, const void* X);
+double rows_f16_cost(int64_t M, int64_t N, int64_t K);
+int launch_rows_f16(int mode, const void* X, const uint8_t* W, int w_layout, const Epilogue& epi, void* Y, int64_t M, int64_t N,
+                    int64_t K, int epi_op, hipStream_t st);
 int launch_pad_rows(const void* X, int64_t B, int64_t K, void* P, hipStream_t st);
 bool gemm_f32_shape_ok(int64_t N, int64_t K);
 bool gemm_f32_supported(int64_t N, int64_t K, const void* X, const void* Y);
@@ -190,6 +194,18 @@ static bool prefers_stream(int64_t B, int64_t N, int64_t K, bool int8, bool tile
     const double wgs = (double)(ceil_div(B, 16) * ceil_div(N, int8 ? 128 : 64));
     const double t_stream = 4.0 + work * (int8 ? 2.2e-9 : 5.0e-9) + wgs * (int8 ? 0.003 : 0.004);
     return t_stream < (int8 ? gemm_i8_cost(B, N, K, tiled, operand_order) : gemm_f16_cost(B, N, K));
+}
+
+// A third choice for 16-bit rows on tiled weights: the kernel for a few tens of rows (rows_f16.hip), from 33 on (up to 32 the
+// row-major and the tiled weights give the same bits, on the streaming kernel).  That kernel's price of a long K, which a few
+// workgroups walk alone, is added here.  us, bf16, streaming or GEMM / this: 48 x 7680 x 2560 12.4 / 7.1, 128 x 7680 x 2560 16.2 / 10.6,
+// 256 x 2560 x 2560 16.6 / 9.1, 128 x 2560 x 6912 22.6 / 14.5, 77 x 4096 x 11008 31.4 / 20.4, 64 x 11008 x 4096 19.9 / 14.8; the other
+// way 128 x 11008 x 4096 23.0 / 27.9, 192 x 16384 x 1024 12.0 / 16.9.
+static bool prefers_rows(int64_t B, int64_t N, int64_t K) {
+    if (option(OPT_ROWS_CFG)) return true;
+    if (B <= 32 || option(OPT_STREAM_MAX_ROWS)) return false;
+    const double stream = 4.0 + (double)B * (double)N * (double)K * 5.0e-9 + (double)(ceil_div(B, 16) * ceil_div(N, 64)) * 0.004;
+    return rows_f16_cost(B, N, K) < std::min(std::max(stream, 4.2 + 0.0011 * (double)K), 0.95 * gemm_f16_cost(B, N, K));
 }
 
 // The same choice for fp32 activations: the streaming kernel on three bf16 planes (split in a launch of its own, about 3 us)
@@ -381,6 +397,8 @@ static int packed_forward_impl(const char* who, const void* X, int x_dtype, cons
             const void* rows = X;
             int64_t Kr = K;  // values of a row of them
             if ((rc = pad_rows_if(X, x_dtype, B, K, workspace, workspace_bytes, st, &rows, &Kr))) return rc;
+            if (prefers_rows(B, N, K) && rows_f16_supported(N, Kr, rows))
+                return launch_rows_f16(mode, rows, W_T, w_layout, epi, Y, B, N, Kr, epi_op, st);
             if (!prefers_stream(B, N, K, false, true) && gemm_f16_supported(N, Kr, rows, W_T, Y, true))
                 return launch_gemm_f16(mode, rows, W_T, w_layout, epi, Y, B, N, Kr, st, K, epi_op);
             return launch_stream(mode, rows, 2, nullptr, W_T, w_layout, epi, Y, x_dtype, nullptr, B, N, Kr, 1,

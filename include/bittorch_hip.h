@@ -62,7 +62,7 @@ const char* bt_last_error(void);
 /*
  * Run-time options.  The library has a small set of documented switches (kernel choice for tests, benchmarks and
  * tuning runs): STREAM_MAX_ROWS, GEMM_LONG_EPILOGUE, GEMM_TAIL_SPLIT, GROUP_WALK, GROUP_NACC, GROUP_UNITS,
- * PLANES_NACC, ROWOP_GENERIC, STREAM_CFG, NO_PLANES.  Each takes its initial value from the environment variable
+ * PLANES_NACC, ROWOP_GENERIC, STREAM_CFG, ROWS_CFG, NO_PLANES.  Each takes its initial value from the environment variable
  * BITTORCH_<NAME>, read once per process on the first call that consults an option; bt_set_option overrides it from
  * then on (value NULL: not set; name NULL: every option not set).  `name` may carry the BITTORCH_ prefix.  Not to be
  * called while another thread is inside the library.  BITTORCH_KERNEL (auto | generic) is not one of them: like the

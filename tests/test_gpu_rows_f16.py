@@ -1,0 +1,78 @@
+"""The 16-bit kernel for a few tens of rows (rows_f16.hip), which the forward on decode-tiled weights takes from 33 rows on."""
+import pytest
+import torch
+
+from conftest import announce
+from _util import set_option
+
+pytestmark = pytest.mark.gpu
+TILES = ["2,2", "2,4", "3,4", "4,4", "5,4"]
+
+
+def _case(m, n, k, dtype, pairs=False):
+    from bittorch_amd import _C
+    g = torch.Generator("cuda").manual_seed(m * 7 + n * 3 + k)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    packed, scale, tern = _C.ternary_quantize_pack(r(n, k) * 0.02, 0.05, True, True, True)
+    return r(m, k).to(dtype), packed, scale, tern.double(), r(n) * 0.1, r(m, n).to(dtype)
+
+
+def _bound(x, tern, scale, bias, dtype):
+    """|sum| off by a rounding of fp32 each for K products (in any order, parts added up), the scale and the bias, then one of the
+    output's type: 2^-11 or 2^-8 of the value."""
+    value = (x.double() @ tern.t()) * scale.double() + bias.double()
+    mags = (x.double().abs() @ tern.abs().t()) * scale.double() + bias.double().abs()
+    fp32 = (x.shape[1] + 12) * 2.0 ** -24 * mags
+    return fp32 + 2.0 ** (-11 if dtype == torch.float16 else -8) * (value.abs() + fp32) + 2.0 ** -25  # (2^-25: half of fp16's smallest)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("m,n,k", [(33, 64, 64), (80, 65, 8), (81, 48, 72), (47, 1030, 1000), (130, 100, 576), (64, 16, 4096), (100, 257, 640)])
+def test_products_against_float64(m, n, k, tile):
+    """Rows and columns that end inside a tile, a last tile of columns past the matrix, fewer steps than waves, one and two steps more
+    than the loads that are on their way, a partial step."""
+    from bittorch_amd import _C
+    set_option("ROWS_CFG", tile)
+    for dtype in (torch.float16, torch.bfloat16):
+        announce("few rows", tile, m, n, k, dtype)
+        x, packed, scale, tern, bias, res = _case(m, n, k, dtype)
+        tiled = _C.retile_weights(packed, k)
+        got = _C.ternary_linear_tiled_forward(x, tiled, scale, bias, k, n)
+        err = (got.double() - ((x.double() @ tern.t()) * scale.double() + bias.double())).abs()
+        assert bool((err <= _bound(x, tern, scale, bias, dtype)).all()), float(err.max())
+        assert torch.equal(_C.ternary_linear_tiled_forward(x, tiled, scale, bias, k, n, residual=res), got + res)
+        assert torch.equal(_C.ternary_linear_tiled_forward(x, tiled, scale[:1], None, k, n),
+                           _C.ternary_linear_tiled_forward(x, tiled, scale[:1].expand(n).contiguous(), None, k, n))
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("m,n,k", [(33, 96, 100), (82, 160, 512), (64, 32, 1096)])
+def test_gate_up_pairs(m, n, k, tile):
+    """A pair-ordered copy read in natural order gives the natural copy's bits, and the SwiGLU output stage the SwiGLU kernel's;
+    infinities and NaN stay in their rows (K = 100: rows that are padded)."""
+    from bittorch_amd import _C
+    set_option("ROWS_CFG", tile)
+    for dtype in (torch.float16, torch.bfloat16):
+        announce("few rows, pairs", tile, m, n, k, dtype)
+        x, packed, scale, tern, bias, _ = _case(m, n, k, dtype)
+        x[1, k - 1], x[m - 1, 0], x[2] = float("inf"), float("nan"), x[2] * 500
+        natural, pairs = _C.retile_weights(packed, k), _C.retile_weights(packed, k, True)
+        want = _C.ternary_linear_tiled_forward(x, natural, scale, bias, k, n)
+        got = _C.ternary_linear_tiled_forward(x, pairs, scale, bias, k, n, natural_from_pairs=True)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+        assert bool(torch.isfinite(want[[0] + list(range(3, m - 1))]).all()) and bool((~torch.isfinite(want[1])).all())
+        h, ref = _C.ternary_linear_tiled_forward(x, pairs, scale, bias, k, n, swiglu_pairs=True), _C.swiglu(want[:, :n // 2], want[:, n // 2:])
+        assert bool(((h == ref) | (h.isnan() & ref.isnan())).all())
+
+
+def test_choice_by_size():
+    """From 33 rows on the forward's results are this kernel's where it is the cheaper one, and up to 32 rows the row-major weights'."""
+    from bittorch_amd import _C
+    for m, n, k, tile in ((77, 7680, 2560, "3,4"), (64, 2560, 2560, "2,2"), (128, 7680, 2560, "4,4")):
+        x, packed, scale, _, bias, _ = _case(m, n, k, torch.bfloat16)
+        tiled = _C.retile_weights(packed, k)
+        got = _C.ternary_linear_tiled_forward(x, tiled, scale, bias, k, n)
+        set_option("ROWS_CFG", tile)
+        assert torch.equal(got, _C.ternary_linear_tiled_forward(x, tiled, scale, bias, k, n))
+        set_option("ROWS_CFG", None)
+        assert torch.equal(_C.ternary_linear_tiled_forward(x[:32], tiled, scale, bias, k, n), _C.ternary_linear_packed_forward(x[:32], packed, scale, bias, k))
