@@ -7,6 +7,9 @@ the fused quantize+pack kernel and the int8 pipeline stages.  Tensors are
 passed to the library as raw device pointers; outputs and scratch are
 allocated here with torch so the library itself never allocates.
 
+The functions of small calls first ask ``_calls`` (``csrc/calls.cpp``), which does the same in native code for
+an ordinary call and returns None for any other.
+
 Importing this module raises ``ImportError`` when the library is not built.
 """
 
@@ -23,6 +26,7 @@ from torch import Tensor
 from . import _lib
 
 _L = _lib.load()  # ImportError here == "extension not available"
+_N = _lib.load_calls()
 
 _DT = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 _INT8_OUT = 3
@@ -194,6 +198,10 @@ def ternary_linear_packed_forward(X: Tensor, W_T: Tensor, scale: Tensor,
     ``residual`` (additive, not in the reference): a tensor of the output's shape and dtype
     added in the kernel's epilogue with the two roundings of ``linear(x) + residual``.
     """
+    if residual is None:
+        y = _N.packed_forward(X, W_T, scale, bias, X.shape[-1] if in_features < 0 and X.dim() > 0 else in_features)
+        if y is not None:
+            return y
     if in_features < 0:
         in_features = X.shape[-1]
     K, N = _packed_checks(X, W_T, scale, bias, in_features)
@@ -313,6 +321,9 @@ def ternary_linear_tiled_forward(X: Tensor, W_tiled: Tensor, scale: Tensor, bias
     output is the MLP's hidden vector ``swiglu(gate(x), up(x))`` ``[*, N/2]``, formed in the kernel's output stage.
     ``natural_from_pairs``: the same pair-ordered copy read as an ordinary linear layer (output ``[*, N]`` in natural
     column order, bit-identical to a natural-order copy's)."""
+    y = _N.tiled_forward(X, W_tiled, scale, bias, in_features, out_features, residual, norm, swiglu_up, swiglu_pairs, natural_from_pairs)
+    if y is not None:
+        return y
     _check(not (swiglu_pairs and natural_from_pairs), "swiglu_pairs and natural_from_pairs exclude each other")
     _check(not natural_from_pairs or out_features % 32 == 0, "a pair-ordered copy has N % 32 == 0")
     _check(not swiglu_pairs or (residual is None and swiglu_up is None and out_features % 32 == 0),
@@ -466,6 +477,10 @@ def ternary_gemm_int8_tiled(Q: Tensor, s_x: Tensor, W_tiled: Tensor, scale: Tens
                             out_dtype: torch.dtype = torch.float32, return_acc: bool = False,
                             residual: Optional[Tensor] = None, q_operand_order: bool = False):
     """:func:`ternary_gemm_int8` on the decode-tiled copy of the weights (same results bit for bit)."""
+    if not return_acc:
+        y = _N.gemm_i8_tiled(Q, s_x, W_tiled, scale, bias, in_features, out_features, out_dtype, residual, q_operand_order)
+        if y is not None:
+            return y
     _check(Q.dim() == 2 and Q.dtype == torch.int8 and Q.numel() > 0, "Q must be 2D int8")
     K, N = Q.shape[-1], out_features
     _check(K == in_features, "input K doesn't match in_features")
@@ -501,6 +516,10 @@ def ternary_linear_tensor_core_forward(X: Tensor, W_T: Tensor, scale: Tensor,
     packed kernel.  version 2: per-row int8 activations, int8 MFMA, int32
     accumulators (``:349-657`` with the whole-row activation scale).
     """
+    if version == 2:
+        y = _N.tensor_core_forward(X, W_T, scale, bias, X.shape[-1] if in_features < 0 and X.dim() > 0 else in_features)
+        if y is not None:
+            return y
     _check(X.dim() == 2, "X must be 2D")
     _check(version in (1, 2), "version must be 1 (V1 float) or 2 (V2 mma.sync)")
     if in_features < 0:
@@ -538,6 +557,10 @@ def ternary_quantize_pack(weight: Tensor, threshold_factor: float = 0.05, per_ch
     exactly what ``quant.ternary_quantize`` returns.  ``as_half=True`` (fp32 weights): the results for ``weight.half()``,
     rounded as the weights are read.
     """
+    if want_packed and not want_tern:
+        out = _N.quantize_pack(weight, threshold_factor, per_channel, as_half)
+        if out is not None:
+            return out
     _check(weight.dim() == 2, "weight must be 2D [N, K]")
     _check(not as_half or weight.dtype == torch.float32, "as_half takes fp32 weights")
     _check(weight.is_cuda, "All tensors must be CUDA")
@@ -657,6 +680,10 @@ def swiglu(gate: Tensor, up: Tensor, store: bool = True, quantize: bool = False,
     :func:`ternary_gemm_int8` -- ``(h, Q, s_x)`` when both are asked for.  ``gate`` and ``up`` may
     be column slices of one wider matrix (the output of a fused gate/up projection).  ``return_rowsum`` (with
     ``quantize``) appends the rows' sums of ``Q`` (int32), which :func:`ternary_gemm_int8_fields` needs."""
+    if quantize and not store and not return_rowsum:
+        out = _N.swiglu_int8(gate, up, operand_order)
+        if out is not None:
+            return out
     _check(gate.shape == up.shape and gate.dtype == up.dtype, "gate and up must match in shape and dtype")
     _check(gate.dim() >= 1 and gate.numel() > 0, "gate is empty")
     _check(gate.dtype in _DT, "gate must be float32, float16 or bfloat16")
@@ -687,6 +714,10 @@ def rmsnorm(x: Tensor, weight: Optional[Tensor] = None, eps: float = 1e-6, store
     """RMSNorm over the last dimension, ``(x * rsqrt(mean(x^2) + eps)) * weight``; with
     ``quantize`` also (or only, ``store=False``) the per-row int8 form of the result, and with ``return_rowsum``
     the rows' sums of that form appended (int32)."""
+    if quantize and not store and not return_rowsum:
+        out = _N.rmsnorm_int8(x, weight, eps, operand_order)
+        if out is not None:
+            return out
     _check(x.dim() >= 1 and x.numel() > 0, "x is empty")
     _check(x.dtype in _DT, "x must be float32, float16 or bfloat16")
     K = x.shape[-1]
@@ -718,6 +749,10 @@ def unpack_dequant(W_T: Tensor, in_features: int, scale: Optional[Tensor] = None
                    out_dtype: torch.dtype = torch.float32) -> Tensor:
     """Dense ``[N, K]`` weights from packed ``W_T``: ``decode * scale[:, None]``
     (``out_dtype`` float) or the plain ternary values (``out_dtype=torch.int8``)."""
+    if scale is not None and out_dtype != torch.int8:
+        out = _N.unpack_dequant(W_T, in_features, scale, out_dtype)
+        if out is not None:
+            return out
     _check(W_T.dim() == 2 and W_T.dtype == torch.uint8, "W_T must be 2D uint8")
     _check(W_T.shape[0] == (in_features + 3) // 4, "K_bytes doesn't match ceil(K/4)")
     _check(_all_cuda(W_T, scale), "All tensors must be CUDA")
@@ -742,6 +777,9 @@ def unpack_dequant(W_T: Tensor, in_features: int, scale: Optional[Tensor] = None
 def linear_grad_input(dY: Tensor, W_T: Tensor, scale: Tensor, in_features: int) -> Tensor:
     """Input gradient of an fp32 packed layer, ``(dY * scale) @ decode(W_T)`` ``[M, K]`` (``dY`` ``[M, N]`` fp32,
     ``scale`` fp32 ``[N]`` or one entry)."""
+    out = _N.grad_input(dY, W_T, scale, in_features)
+    if out is not None:
+        return out
     _check(dY.dim() == 2 and dY.dtype == torch.float32 and dY.numel() > 0, "dY must be 2D fp32")
     _check(W_T.dim() == 2 and W_T.dtype == torch.uint8 and W_T.shape[0] == (in_features + 3) // 4
            and W_T.shape[1] == dY.shape[1], "W_T must be uint8 [ceil(K/4), N]")
@@ -759,6 +797,9 @@ def linear_grad_input(dY: Tensor, W_T: Tensor, scale: Tensor, in_features: int) 
 def linear_grad_weight(dY: Tensor, X: Tensor, scale: Tensor, want_bias: bool = False) -> Tuple[Tensor, Optional[Tensor]]:
     """Weight gradient under the straight-through estimator, ``scale[:, None] * (dY.T @ X)`` ``[N, K]``, and with
     ``want_bias`` the bias gradient ``dY.sum(0)`` from the same pass (all fp32, N and K at least 4)."""
+    out = _N.grad_weight(dY, X, scale, want_bias)
+    if out is not None:
+        return out
     _check(dY.dim() == 2 and X.dim() == 2 and dY.shape[0] == X.shape[0] and dY.numel() > 0 and X.numel() > 0,
            "dY [M, N] and X [M, K] must be 2D with the same rows")
     _check(dY.dtype == X.dtype == scale.dtype == torch.float32, "dY, X and scale must be fp32")
@@ -778,6 +819,9 @@ def linear_grad_weight(dY: Tensor, X: Tensor, scale: Tensor, want_bias: bool = F
 def linear_grad_weight_16(dY: Tensor, X: Tensor, scale: Tensor, out_dtype: torch.dtype) -> Tensor:
     """Weight gradient of a 16-bit layer, ``scale[:, None] * (dY.T @ X)`` ``[N, K]`` in their dtype or fp32, with the roundings
     of the unfused operations (``dY`` ``[M, N]``, ``X`` ``[M, K]``, N and K multiples of 8)."""
+    out = _N.grad_weight_16(dY, X, scale, out_dtype)
+    if out is not None:
+        return out
     _check(dY.dim() == 2 and X.dim() == 2 and dY.shape[0] == X.shape[0] and dY.numel() > 0 and X.numel() > 0,
            "dY [M, N] and X [M, K] must be 2D with the same rows")
     _check(dY.dtype == X.dtype and dY.dtype in (torch.float16, torch.bfloat16), "dY and X must be fp16 or bf16")

@@ -80,6 +80,7 @@ SIGNATURES = {
 }
 
 _lib: Optional[ctypes.CDLL] = None
+_calls = None
 
 
 def load() -> ctypes.CDLL:
@@ -106,6 +107,24 @@ def load() -> ctypes.CDLL:
         raise ImportError(f"{LIB_PATH} has ABI {lib.bt_abi_version()}, expected {ABI_VERSION}; rebuild it")
     _lib = lib
     return lib
+
+
+def load_calls():
+    """``_hip/_calls.so``, the native host side of the calls (``csrc/calls.cpp``), bound to the loaded library."""
+    global _calls
+    if _calls is None:
+        import importlib.util
+
+        path = os.path.join(_HERE, "_hip", "_calls.so")
+        if not os.path.exists(path):
+            raise ImportError(f"{path} is missing: build it with `python -m bittorch_amd.build`")
+        lib = load()
+        spec = importlib.util.spec_from_file_location("bittorch_amd._hip._calls", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        module.bind({name: ctypes.cast(getattr(lib, name), _vp).value for name in module.names()})
+        _calls = module
+    return _calls
 
 
 def last_error() -> str:

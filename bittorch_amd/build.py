@@ -1,4 +1,5 @@
-"""Builds ``_hip/libbittorch_hip.so`` (the C-ABI HIP library) with hipcc for gfx950.
+"""Builds ``_hip/libbittorch_hip.so`` (the C-ABI HIP library) with hipcc for gfx950, and ``_hip/_calls.so`` (the host side of the
+torch calls) with g++.
 
 Usage: ``python -m bittorch_amd.build``.  The library has no torch dependency;
 hipcc cross-compiles it on a machine without a GPU.
@@ -47,8 +48,28 @@ def _hipcc() -> str:
     return exe
 
 
+def build_calls() -> str:
+    """Compile ``csrc/calls.cpp`` (host code only) against the installed torch into ``_hip/_calls.so``; returns its path."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    out = os.path.join(OUT_DIR, "_calls.so")
+    libs = library_paths()
+    cmd = [shutil.which("g++") or "g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-I{p}" for p in include_paths()), f"-I{sysconfig.get_paths()['include']}",
+           f"-I{os.path.join(os.environ.get('ROCM_PATH', '/opt/rocm'), 'include')}", os.path.join(CSRC, "calls.cpp"), "-o", out,
+           *(f"-L{p}" for p in libs), *(f"-Wl,-rpath,{p}" for p in libs), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on calls.cpp:\n{res.stdout}\n{res.stderr}")
+    return out
+
+
 def build(verbose: bool = False, extra_flags=()) -> str:
-    """Compile every kernel source and link the shared library; returns its path."""
+    """Compile every kernel source and link the shared library, and the native host side of the calls; returns the library's path."""
     os.makedirs(OUT_DIR, exist_ok=True)
     hipcc = _hipcc()
     objs = []
@@ -65,7 +86,9 @@ def build(verbose: bool = False, extra_flags=()) -> str:
         return obj
 
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
+        calls = pool.submit(build_calls)
         objs = list(pool.map(compile_one, SOURCES))
+        calls.result()
     cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:

@@ -35,6 +35,13 @@ from ..quant.ternary_packed import pack_ternary_transposed, unpack_ternary_trans
 # From this many rows an int8 call with row sums takes the prefill GEMM on the field-layout copy (prepare_prefill):
 # below it the routing between the streaming kernel and the tiled GEMM on the decode-tiled copy does as well or better.
 PREFILL_ROWS = 384
+_TILED_DTYPES = frozenset((torch.float16, torch.bfloat16, torch.float32, torch.int8))
+
+
+def _generic_kernel_asked() -> bool:
+    """``BITTORCH_KERNEL=generic``, read on every call."""
+    from .. import _C
+    return _C._N.generic_kernel_asked()
 
 
 class TernaryLinearInference(nn.Module):
@@ -226,14 +233,18 @@ class TernaryLinearInference(nn.Module):
         (the SwiGLU output stage: pair-ordered copy)."""
         if not (self.decode_tiled and x.is_cuda):
             return None
+        here = self.__dict__
+        if here["_tiled"] is not None and here["_tile_order"] == order and "weight_packed" not in here["_buffers"] \
+                and x.dtype in _TILED_DTYPES and not _generic_kernel_asked():
+            return here["_tiled"]  # (what is asked below, for a layer that holds the copy alone)
         if order == "gate_up_pairs":
             if self._tile_order != order:
                 return None
         elif self._tile_order != "natural" and x.dtype == torch.int8:
             return None  # the int8 entry point reads natural-order copies only
-        if os.environ.get("BITTORCH_KERNEL") == "generic":  # the shape-generic kernel reads weight_packed
+        if _generic_kernel_asked():  # the shape-generic kernel reads weight_packed
             return None
-        if x.dtype not in (torch.float16, torch.bfloat16, torch.float32, torch.int8):
+        if x.dtype not in _TILED_DTYPES:
             return None
         kb = (self.in_features + 3) // 4
         if ((self.out_features + 15) // 16) * ((kb + 15) // 16) * 256 >= 2 ** 32:  # beyond the kernels' 32-bit offsets
@@ -325,7 +336,7 @@ class TernaryLinearInference(nn.Module):
         field-layout copy where ``prepare_prefill`` built one; the result does not depend on it."""
         rows = q.numel() // max(q.shape[-1], 1)
         fields = self._prefill_copy() if (q_rowsum is not None and rows >= PREFILL_ROWS and q.is_cuda) else None
-        if fields is not None and os.environ.get("BITTORCH_KERNEL") != "generic":
+        if fields is not None and not _generic_kernel_asked():
             from .. import _C
             y = _C.ternary_gemm_int8_fields(q.reshape(-1, q.shape[-1]), s_x.reshape(-1), q_rowsum.reshape(-1), fields,
                                             self.scale, self.bias, self.in_features, self.out_features, out_dtype, False,
