@@ -89,10 +89,10 @@ bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, co
 double gemm_f16_cost(int64_t M, int64_t N, int64_t K);
 int launch_gemm_f16(int mode, const void* X, const uint8_t* W_T, int w_layout, const Epilogue& epi, void* Y, int64_t M,
                     int64_t N, int64_t K, hipStream_t st, int64_t Kw = 0, int epi_op = 0);
-bool rows_f16_supported(int64_t N, int64_t K, const void* X);
-double rows_f16_cost(int64_t M, int64_t N, int64_t K);
-int launch_rows_f16(int mode, const void* X, const uint8_t* W, int w_layout, const Epilogue& epi, void* Y, int64_t M, int64_t N,
-                    int64_t K, int epi_op, hipStream_t st);
+bool few_rows_supported(int64_t N, int64_t row_bytes, const void* X, const void* W, bool tiled);
+double few_rows_cost(bool i8, bool rows, int64_t M, int64_t N, int64_t K);
+int launch_few_rows(int mode, const void* X, const float* s_x, const uint8_t* W, int w_layout, const Epilogue& epi, void* Y, int y_dtype,
+                    int32_t* acc_out, int64_t M, int64_t N, int64_t K, int epi_op, hipStream_t st, int64_t Kw = 0);
 int launch_pad_rows(const void* X, int64_t B, int64_t K, void* P, hipStream_t st);
 bool gemm_f32_shape_ok(int64_t N, int64_t K);
 bool gemm_f32_supported(int64_t N, int64_t K, const void* X, const void* Y);
@@ -196,16 +196,30 @@ static bool prefers_stream(int64_t B, int64_t N, int64_t K, bool int8, bool tile
     return t_stream < (int8 ? gemm_i8_cost(B, N, K, tiled, operand_order) : gemm_f16_cost(B, N, K));
 }
 
-// A third choice for 16-bit rows on tiled weights: the kernel for a few tens of rows (rows_f16.hip), from 33 on (up to 32 the
-// row-major and the tiled weights give the same bits, on the streaming kernel).  That kernel's price of a long K, which a few
-// workgroups walk alone, is added here.  us, bf16, streaming or GEMM / this: 48 x 7680 x 2560 12.4 / 7.1, 128 x 7680 x 2560 16.2 / 10.6,
-// 256 x 2560 x 2560 16.6 / 9.1, 128 x 2560 x 6912 22.6 / 14.5, 77 x 4096 x 11008 31.4 / 20.4, 64 x 11008 x 4096 19.9 / 14.8; the other
-// way 128 x 11008 x 4096 23.0 / 27.9, 192 x 16384 x 1024 12.0 / 16.9.
-static bool prefers_rows(int64_t B, int64_t N, int64_t K) {
+// A third choice for 16-bit rows, and int8 rows in operand order: the kernel for a few tens of rows (few_rows.hip).  The streaming
+// kernel's price of a long K, which a few workgroups walk alone, is added here.
+//   16-bit, from 33 rows on (up to 32 the row-major and the tiled weights give the same bits, on the streaming kernel).  us, bf16,
+//          streaming or GEMM / this: 48 x 7680 x 2560 12.4 / 7.1, 128 x 7680 x 2560 16.2 / 10.5, 256 x 2560 x 2560 16.6 / 8.9, 128 x 2560 x
+//          6912 22.6 / 13.9, 77 x 4096 x 11008 31.4 / 19.6, 64 x 11008 x 4096 19.9 / 14.8, row-major 192 x 4096 x 11008 57.5 / 24.2; the
+//          other way 128 x 11008 x 4096 23.0 / 27.9, 192 x 16384 x 1024 12.0 / 16.9
+//   int8   (exact sums: any number of rows).  Row-major weights with the quantizer: 32 x 4096 x 11008 20.8 / 15.4, 128 x 7680 x 2560
+//          16.9 / 13.0, 256 x 4096 x 11008 35.9 / 26.1; tiled: 96 x 7680 x 2560 11.7 / 8.7, 256 x 2560 x 6912 21.6 / 14.1.  Up to 16 rows
+//          it wins where 64 columns each are enough workgroups, 16 x 11008 x 4096 10.5 / 9.7, 16 x 16384 x 1024 8.9 / 7.3, not 8 x 4096 x
+//          4096 8.6 / 9.3; tiled 16 x 7680 x 2560 5.7 / 5.3, 8 x 7680 x 2560 5.1 / 5.3
+static bool prefers_rows(bool i8, bool row_major, int64_t B, int64_t N, int64_t K) {
     if (option(OPT_ROWS_CFG)) return true;
-    if (B <= 32 || option(OPT_STREAM_MAX_ROWS)) return false;
-    const double stream = 4.0 + (double)B * (double)N * (double)K * 5.0e-9 + (double)(ceil_div(B, 16) * ceil_div(N, 64)) * 0.004;
-    return rows_f16_cost(B, N, K) < std::min(std::max(stream, 4.2 + 0.0011 * (double)K), 0.95 * gemm_f16_cost(B, N, K));
+    if (option(OPT_STREAM_MAX_ROWS)) return false;
+    const double work = (double)B * (double)N * (double)K, blocks = (double)ceil_div(B, 16);
+    if (ceil_div(B, 16) * ceil_div(N, 64) < 64) return false;  // (narrow matrices: the streaming kernel cuts them finer; int8 32 x 1000 x 3000 8.8 / 10.5)
+    if (!i8) {
+        if (B <= 32) return false;
+        const double stream = std::max(4.0 + work * 5.0e-9 + blocks * (double)ceil_div(N, 64) * 0.004, 4.2 + 0.0011 * (double)K);
+        return few_rows_cost(false, row_major, B, N, K) < std::min(stream, 0.95 * gemm_f16_cost(B, N, K));
+    }
+    if (B <= 16) return B > (row_major ? 1 : 8) && ceil_div(N, 64) >= 100;
+    const double stream = std::max(4.0 + work * 2.2e-9 + blocks * (double)ceil_div(N, 128) * 0.003, 4.0 + (row_major ? 0.0012 : 0.00058) * (double)K);
+    const double us = few_rows_cost(true, row_major, B, N, K);
+    return us < stream && (B <= 32 || us < 0.9 * gemm_i8_cost(B, N, K, !row_major, true));
 }
 
 // The same choice for fp32 activations: the streaming kernel on three bf16 planes (split in a launch of its own, about 3 us)
@@ -397,8 +411,8 @@ static int packed_forward_impl(const char* who, const void* X, int x_dtype, cons
             const void* rows = X;
             int64_t Kr = K;  // values of a row of them
             if ((rc = pad_rows_if(X, x_dtype, B, K, workspace, workspace_bytes, st, &rows, &Kr))) return rc;
-            if (prefers_rows(B, N, K) && rows_f16_supported(N, Kr, rows))
-                return launch_rows_f16(mode, rows, W_T, w_layout, epi, Y, B, N, Kr, epi_op, st);
+            if (prefers_rows(false, false, B, N, K) && few_rows_supported(N, 2 * Kr, rows, W_T, true))
+                return launch_few_rows(mode, rows, nullptr, W_T, w_layout, epi, Y, x_dtype, nullptr, B, N, Kr, epi_op, st, K);
             if (!prefers_stream(B, N, K, false, true) && gemm_f16_supported(N, Kr, rows, W_T, Y, true))
                 return launch_gemm_f16(mode, rows, W_T, w_layout, epi, Y, B, N, Kr, st, K, epi_op);
             return launch_stream(mode, rows, 2, nullptr, W_T, w_layout, epi, Y, x_dtype, nullptr, B, N, Kr, 1,
@@ -433,6 +447,8 @@ static int packed_forward_impl(const char* who, const void* X, int x_dtype, cons
         const void* rows = X;
         int64_t Kr = K;
         if ((rc = pad_rows_if(X, x_dtype, B, K, workspace, workspace_bytes, st, &rows, &Kr))) return rc;
+        if (prefers_rows(false, true, B, N, K) && few_rows_supported(N, 2 * Kr, rows, W_T, false))
+            return launch_few_rows(mode, rows, nullptr, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, x_dtype, nullptr, B, N, Kr, 0, st, K);
         if (!prefers_stream(B, N, K, false) && gemm_f16_supported(N, Kr, rows, W_T, Y, false))
             return launch_gemm_f16(mode, rows, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, B, N, Kr, st, K);
         return launch_stream(mode, rows, 2, nullptr, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, x_dtype, nullptr, B, N, Kr, 1, Q_ROW_MAJOR, 0, nullptr, 0.0f, 0, st, K);
@@ -556,11 +572,15 @@ static int gemm_i8_impl(const char* who, const int8_t* Q, int q_layout, const fl
             return BT_ERR_INVALID;
         }
         const bool oo = q_layout == Q_OPERAND_ORDER;
+        if (oo && prefers_rows(true, false, B, N, K) && few_rows_supported(N, K, Q, W_T, true))
+            return launch_few_rows(MODE_I8, Q, s_x, W_T, w_layout, epi, Y, y_dtype, acc_out, B, N, K, 0, st, Kw);
         if (!prefers_stream(B, N, K, true, true, oo) && gemm_i8_supported_tiled(N, K, Q, oo))
             return launch_gemm_i8(Q, q_layout, s_x, nullptr, W_T, w_layout, epi, Y, y_dtype, acc_out, B, N, K, st, Kw);
         return launch_stream(MODE_I8, Q, 1, s_x, W_T, w_layout, epi, Y, y_dtype, acc_out, B, N, K, 1, q_layout, 0, nullptr,
                              0.0f, 0, st, Kw);
     }
+    if (q_layout == Q_OPERAND_ORDER && prefers_rows(true, true, B, N, K) && few_rows_supported(N, K, Q, W_T, false) && stream_supported(N, K, W_T))
+        return launch_few_rows(MODE_I8, Q, s_x, W_T, W_LAYOUT_ROW_MAJOR, epi, Y, y_dtype, acc_out, B, N, K, 0, st, Kw);
     // decode-shape batches, and any batch whose N the tiled kernel's 4-column
     // vector accesses cannot take, stream the weights once per 16 rows
     if (prefers_stream(B, N, K, true, false, q_layout == Q_OPERAND_ORDER) || !gemm_i8_supported(N, K, Q, W_T)) {

@@ -1,4 +1,4 @@
-"""The 16-bit kernel for a few tens of rows (rows_f16.hip), which the forward on decode-tiled weights takes from 33 rows on."""
+"""The kernel for a few tens of rows (few_rows.hip): 16-bit rows from 33 on, int8 rows in operand order."""
 import pytest
 import torch
 
@@ -41,6 +41,8 @@ def test_products_against_float64(m, n, k, tile):
         err = (got.double() - ((x.double() @ tern.t()) * scale.double() + bias.double())).abs()
         assert bool((err <= _bound(x, tern, scale, bias, dtype)).all()), float(err.max())
         assert torch.equal(_C.ternary_linear_tiled_forward(x, tiled, scale, bias, k, n, residual=res), got + res)
+        if n % 4 == 0:  # row-major weights: the same sums
+            assert torch.equal(_C.ternary_linear_packed_forward(x, packed, scale, bias, k, residual=res), got + res)
         assert torch.equal(_C.ternary_linear_tiled_forward(x, tiled, scale[:1], None, k, n),
                            _C.ternary_linear_tiled_forward(x, tiled, scale[:1].expand(n).contiguous(), None, k, n))
 
@@ -63,6 +65,46 @@ def test_gate_up_pairs(m, n, k, tile):
         assert bool(torch.isfinite(want[[0] + list(range(3, m - 1))]).all()) and bool((~torch.isfinite(want[1])).all())
         h, ref = _C.ternary_linear_tiled_forward(x, pairs, scale, bias, k, n, swiglu_pairs=True), _C.swiglu(want[:, :n // 2], want[:, n // 2:])
         assert bool(((h == ref) | (h.isnan() & ref.isnan())).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 64, 64), (2, 100, 192), (17, 64, 144), (33, 257, 80), (47, 1028, 1024), (80, 48, 16), (81, 160, 1168),
+                                   (130, 96, 2064)])
+def test_int8_accumulators_and_outputs(m, n, k):
+    """The exact integers and the streaming kernel's outputs, bit for bit, on tiled and on row-major weights: rows and columns that end
+    inside a tile, fewer steps than waves, K of half a step more, every output type, residual."""
+    from bittorch_amd import _C
+    x, packed, scale, tern, bias, res = _case(m, n, k, torch.bfloat16)
+    tiled = _C.retile_weights(packed, k)
+    q, sx = _C.act_quant_int8(x)
+    qo, _ = _C.act_quant_int8(x, operand_order=True)
+    want_acc = 127 * (q.cpu().double() @ tern.cpu().t()).to(torch.int32)
+    for dtype in (torch.float32, torch.float16, torch.bfloat16):
+        for r in (None, res.to(dtype)):
+            set_option("ROWS_CFG", None)
+            set_option("STREAM_MAX_ROWS", "2000000")
+            want, acc = _C.ternary_gemm_int8_tiled(qo, sx, tiled, scale, bias, k, n, dtype, True, r, True)
+            assert torch.equal(acc.cpu(), want_acc)
+            set_option("STREAM_MAX_ROWS", None)
+            for tile in ("1,4", "2,4", "3,4", "4,4", "5,4"):
+                announce("few int8 rows", tile, m, n, k, dtype)
+                set_option("ROWS_CFG", tile)
+                for y, a in (_C.ternary_gemm_int8_tiled(qo, sx, tiled, scale, bias, k, n, dtype, True, r, True),
+                             _C.ternary_gemm_int8(qo, sx, packed, scale, bias, k, dtype, True, r, True)):
+                    assert torch.equal(a.cpu(), want_acc) and torch.equal(y, want)
+
+
+@pytest.mark.parametrize("m,n,k", [(3, 64, 100), (40, 128, 8), (70, 64, 1290), (16, 7680, 130)])
+def test_int8_rows_that_are_padded(m, n, k):
+    """K that is no multiple of 16: rows of Q longer than the weights' K, on row-major weights whose last rows then do not exist."""
+    from bittorch_amd import _C
+    x, packed, scale, _, bias, _ = _case(m, n, k, torch.bfloat16)
+    set_option("STREAM_MAX_ROWS", "2000000")
+    want = _C.ternary_linear_tensor_core_forward(x, packed, scale, bias, k, 2)
+    set_option("STREAM_MAX_ROWS", None)
+    for tile in ("1,4", "2,4", "5,4"):
+        announce("few padded int8 rows", tile, m, n, k)
+        set_option("ROWS_CFG", tile)
+        assert torch.equal(_C.ternary_linear_tensor_core_forward(x, packed, scale, bias, k, 2), want)
 
 
 def test_choice_by_size():
