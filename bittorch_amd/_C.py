@@ -506,6 +506,41 @@ def ternary_gemm_int8_tiled(Q: Tensor, s_x: Tensor, W_tiled: Tensor, scale: Tens
     return (y, acc) if return_acc else y
 
 
+def swiglu_int8_tiled_pays(rows: int, in_features: int, out_features: int) -> bool:
+    """Whether :func:`ternary_swiglu_int8_tiled` is the faster way for this size."""
+    return bool(_L.bt_swiglu_i8_tiled_pays(rows, out_features, in_features))
+
+
+def ternary_swiglu_int8_tiled(Q: Tensor, s_x: Tensor, W_tiled: Tensor, scale: Tensor, bias: Optional[Tensor],
+                              in_features: int, out_features: int, out_dtype: torch.dtype) -> Tensor:
+    """``silu(gate) * up`` ``[B, N / 2]`` of the projections ``[gate | up]`` that :func:`ternary_gemm_int8_tiled` makes of the
+    same arguments, bit for bit what :func:`swiglu` makes of its output: the product is formed in the GEMM's output stage.
+    ``Q`` in operand order, a copy in natural order, ``N % 32 == 0`` and a 16-bit ``out_dtype``."""
+    h = _N.swiglu_i8_tiled(Q, s_x, W_tiled, scale, bias, in_features, out_features, out_dtype)
+    if h is not None:
+        return h
+    _check(Q.dim() == 2 and Q.dtype == torch.int8 and Q.numel() > 0, "Q must be 2D int8")
+    K, N = Q.shape[-1], out_features
+    _check(K == in_features, "input K doesn't match in_features")
+    _tiled_checks(W_tiled, N, K)
+    _check(scale.dim() == 1 and scale.shape[0] in (N, 1), "scale size doesn't match N")
+    _check(bias is None or (bias.dim() == 1 and bias.shape[0] == N), "bias shape mismatch")
+    _check(s_x.dtype == torch.float32 and s_x.numel() == Q.shape[0], "s_x must be fp32 [B]")
+    _check(_all_cuda(Q, s_x, W_tiled, scale, bias), "All tensors must be CUDA")
+    _check(out_dtype in (torch.float16, torch.bfloat16) and N % 32 == 0, "out_dtype must be float16 or bfloat16, and N a multiple of 32")
+    q = Q.contiguous()
+    s_x = s_x.contiguous()
+    scale = _prep_vec(scale, s_x)
+    bias = None if bias is None else _prep_vec(bias, s_x)
+    B = q.shape[0]
+    h = torch.empty((B, N // 2), dtype=out_dtype, device=q.device)
+    with _on(q):
+        _status(_L.bt_ternary_swiglu_i8_tiled(
+            q.data_ptr(), s_x.data_ptr(), W_tiled.data_ptr(), scale.data_ptr(), _dt(scale, "scale"), scale.numel(), _ptr(bias),
+            0 if bias is None else _dt(bias, "bias"), h.data_ptr(), _DT[out_dtype], B, N, K, _stream(q)))
+    return h
+
+
 def ternary_linear_tensor_core_forward(X: Tensor, W_T: Tensor, scale: Tensor,
                                        bias: Optional[Tensor] = None, in_features: int = -1,
                                        version: int = 1) -> Tensor:
@@ -589,6 +624,10 @@ def act_quant_int8(X: Tensor, operand_order: bool = False, return_rowsum: bool =
     int8 GEMMs feed the matrix cores; such a ``Q`` must go to :func:`ternary_gemm_int8` with
     ``q_operand_order=True``.  ``return_rowsum=True`` adds the rows' sums of ``Q`` (int32 ``[B]``), which
     :func:`ternary_gemm_int8_fields` needs."""
+    if not return_rowsum:
+        out = _N.act_quant_int8(X, operand_order)
+        if out is not None:
+            return out
     _check(X.dim() == 2 and X.numel() > 0, "X must be 2D and non-empty")
     _check(X.is_cuda, "All tensors must be CUDA")
     x = X.contiguous()

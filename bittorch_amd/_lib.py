@@ -71,6 +71,8 @@ SIGNATURES = {
                                                _i64, _vp, _int, _vp, _int, _vp, _i64, _i64, _i64, _vp, _sz, _vp]),
     "bt_ternary_gemm_i8_tiled": (_int, [_vp, _int, _vp, _vp, _vp, _int, _i64, _vp, _int, _vp, _vp, _int, _vp,
                                         _i64, _i64, _i64, _vp]),
+    "bt_ternary_swiglu_i8_tiled": (_int, [_vp, _vp, _vp, _vp, _int, _i64, _vp, _int, _vp, _int, _i64, _i64, _i64, _vp]),
+    "bt_swiglu_i8_tiled_pays": (_int, [_i64, _i64, _i64]),
     "bt_act_quant_i8_rowsum": (_int, [_vp, _int, _i64, _i64, _vp, _vp, _vp, _int, _vp]),
     "bt_swiglu_rowsum": (_int, [_vp, _i64, _vp, _i64, _int, _i64, _i64, _vp, _vp, _vp, _vp, _int, _vp]),
     "bt_rmsnorm_rowsum": (_int, [_vp, _i64, _vp, ctypes.c_float, _int, _i64, _i64, _vp, _vp, _vp, _vp, _int, _vp]),

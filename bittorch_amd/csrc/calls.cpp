@@ -34,7 +34,8 @@ namespace {
     X(bt_packed_forward_fused_workspace_bytes) X(bt_tensor_core_workspace_bytes) X(bt_linear_grad_weight_workspace_bytes)      \
     X(bt_linear_grad_weight_16_workspace_bytes) X(bt_ternary_linear_tiled_forward) X(bt_ternary_linear_packed_forward)         \
     X(bt_ternary_linear_tensor_core_forward) X(bt_quantize_pack) X(bt_ternary_linear_grad_input) X(bt_linear_grad_weight)      \
-    X(bt_linear_grad_weight_16) X(bt_unpack_dequant) X(bt_swiglu) X(bt_rmsnorm) X(bt_ternary_gemm_i8_tiled)
+    X(bt_linear_grad_weight_16) X(bt_unpack_dequant) X(bt_swiglu) X(bt_rmsnorm) X(bt_ternary_gemm_i8_tiled) \
+    X(bt_ternary_swiglu_i8_tiled) X(bt_act_quant_i8_layout)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
     BT_FUNCTIONS(X)
@@ -383,6 +384,34 @@ PyObject* gemm_i8_tiled(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     END_HANDLE_TH_ERRORS
 }
 
+// swiglu_i8_tiled(Q [B, K] in operand order, s_x, W_tiled, scale, bias, in_features, out_features, dtype) -> [B, N / 2]
+PyObject* swiglu_i8_tiled(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    int device;
+    int64_t K, N;
+    ORDINARY(n_args == 8 && here(a[0], &device) && as_int(a[5], &K) && as_int(a[6], &N) && K > 0 && N > 0 && N % 32 == 0);
+    const at::Tensor *q = plain(a[0], device), *sx = plain(a[1], device), *w = plain(a[2], device), *scale = vec(a[3], N, true, device);
+    ORDINARY(q && q->scalar_type() == at::kChar && q->dim() == 2 && q->size(1) == K && sx && sx->scalar_type() == at::kFloat &&
+             sx->numel() == q->size(0) && scale);
+    ORDINARY(w && w->scalar_type() == at::kByte && w->dim() == 1 && (size_t)w->numel() == lib.bt_tiled_weights_bytes(N, K));
+    ORDINARY(THPDtype_Check(a[7]));
+    const at::ScalarType dtype = reinterpret_cast<THPDtype*>(a[7])->scalar_type;
+    ORDINARY(dtype == at::kHalf || dtype == at::kBFloat16);
+    const int64_t B = q->size(0);
+    const at::Tensor* bias = nullptr;
+    if (a[4] != Py_None) ORDINARY((bias = vec(a[4], N, false, device)));
+    at::Tensor h = output({B, N / 2}, dtype, *q);
+    void* st = stream_of(device);
+    call([&] {
+        return lib.bt_ternary_swiglu_i8_tiled((const int8_t*)q->const_data_ptr(), (const float*)sx->const_data_ptr(), (const uint8_t*)w->const_data_ptr(),
+                                              scale->const_data_ptr(), tag(scale->scalar_type()), scale->numel(),
+                                              bias ? bias->const_data_ptr() : nullptr, bias ? tag(bias->scalar_type()) : 0, h.data_ptr(), tag(dtype),
+                                              B, N, K, st);
+    });
+    return THPVariable_Wrap(std::move(h));
+    END_HANDLE_TH_ERRORS
+}
+
 // grad_weight_16(dY, X, scale, out_dtype)
 PyObject* grad_weight_16(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     HANDLE_TH_ERRORS
@@ -417,6 +446,24 @@ PyObject* int8_rows(at::Tensor q, at::Tensor s) {
     PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(std::move(q)));
     PyTuple_SET_ITEM(out, 1, THPVariable_Wrap(std::move(s)));
     return out;
+}
+
+// act_quant_int8(x [B, K], operand_order) -> (Q, s_x)
+PyObject* act_quant_int8(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    int device;
+    bool oo;
+    ORDINARY(n_args == 2);
+    const at::Tensor* x = rows_of(a[0], &device);
+    ORDINARY(x && x->dim() == 2 && as_bool(a[1], &oo));
+    const int64_t B = x->size(0), K = x->size(1);
+    at::Tensor q = output({B, K}, at::kChar, *x), s = output({B}, at::kFloat, *x);
+    void* st = stream_of(device);
+    call([&] {
+        return lib.bt_act_quant_i8_layout(x->const_data_ptr(), tag(x->scalar_type()), B, K, (int8_t*)q.data_ptr(), (float*)s.data_ptr(), oo ? 1 : 0, st);
+    });
+    return int8_rows(std::move(q), std::move(s));
+    END_HANDLE_TH_ERRORS
 }
 
 // rmsnorm_int8(x [B, K], weight, eps, operand_order) -> (Q, s_x)
@@ -528,7 +575,7 @@ PyObject* names(PyObject*, PyObject* const*, Py_ssize_t) {
 #define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {METHOD(bind), METHOD(names), METHOD(tiled_forward), METHOD(packed_forward), METHOD(tensor_core_forward),
                          METHOD(quantize_pack), METHOD(grad_input), METHOD(grad_weight),
-                         METHOD(grad_weight_16), METHOD(unpack_dequant), METHOD(rmsnorm_int8), METHOD(swiglu_int8), METHOD(gemm_i8_tiled),
+                         METHOD(grad_weight_16), METHOD(unpack_dequant), METHOD(rmsnorm_int8), METHOD(swiglu_int8), METHOD(gemm_i8_tiled), METHOD(swiglu_i8_tiled), METHOD(act_quant_int8),
                          METHOD(generic_kernel_asked), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_calls", "Native host side of small calls (csrc/calls.cpp)", -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -116,6 +116,9 @@ bool planes_bf16_wide(int64_t N, int64_t K);
 int launch_planes_bf16_wide(const void* X, const uint8_t* W, const Epilogue& epi, void* Y, int64_t N, int64_t K, hipStream_t st);
 bool gemm_i8_supported_tiled(int64_t N, int64_t K, const void* Q, bool operand_order);
 double gemm_i8_cost(int64_t M, int64_t N, int64_t K, bool tiled, bool operand_order);
+int gemm_i8_dma_rows(int64_t M, int64_t N, int64_t K, bool tiled, bool fields);
+int launch_gemm_i8_swiglu(const int8_t* Q, const float* s_x, const uint8_t* W_tiled, const Epilogue& epi, void* Y, int y_dtype,
+                          int64_t M, int64_t N, int64_t K, hipStream_t st);
 int launch_gemm_i8(const int8_t* Q, int q_layout, const float* s_x, const int32_t* q_rowsum, const uint8_t* W_T, int w_layout,
                    const Epilogue& epi, void* Y, int y_dtype, int32_t* acc_out, int64_t M, int64_t N, int64_t K,
                    hipStream_t st, int64_t Kw = 0);
@@ -1045,6 +1048,42 @@ extern "C" int bt_ternary_gemm_i8_tiled(const int8_t* Q, int q_layout, const flo
                                         int64_t B, int64_t N, int64_t K, void* stream) {
     return gemm_i8_impl("bt_ternary_gemm_i8_tiled", Q, q_layout, s_x, W_tiled, W_LAYOUT_TILED, scale, scale_dtype,
                         scale_len, bias, bias_dtype, residual, Y, y_dtype, acc_out, B, N, K, stream);
+}
+
+static bool swiglu_i8_ok(int64_t N, int64_t K, const void* Q, const void* W_tiled, const void* Y) {
+    return N % 32 == 0 && K <= kMaxKInt8 && fast_path_ok(Y, N, K) && stream_supported_tiled(N, K, W_tiled) && gemm_i8_supported_tiled(N, K, Q, true);
+}
+
+extern "C" int bt_ternary_swiglu_i8_tiled(const int8_t* Q, const float* s_x, const uint8_t* W_tiled, const void* scale, int scale_dtype,
+                                          int64_t scale_len, const void* bias, int bias_dtype, void* Y, int y_dtype, int64_t B,
+                                          int64_t N, int64_t K, void* stream) {
+    const char* who = "bt_ternary_swiglu_i8_tiled";
+    int rc = check_shape(who, Q, W_tiled, Y, y_dtype, B, N, K);
+    if (rc) return rc;
+    if (!s_x || y_dtype == BT_F32) {
+        set_error("%s: s_x is null, or Y is not of a 16-bit type", who);
+        return BT_ERR_INVALID;
+    }
+    if ((rc = check_q_layout(who, Q_OPERAND_ORDER, K, Q, nullptr))) return rc;
+    if (!swiglu_i8_ok(N, K, Q, W_tiled, Y)) {
+        set_error("%s: N %% 32 == 0, K up to %lld, 16-byte aligned Q and Y and a 256-byte aligned copy below 4 GiB are needed", who,
+                  (long long)kMaxKInt8);
+        return BT_ERR_INVALID;
+    }
+    Epilogue epi;
+    rc = make_epilogue(who, scale, scale_dtype, scale_len, bias, bias_dtype, N, &epi);
+    if (rc) return rc;
+    return launch_gemm_i8_swiglu(Q, s_x, W_tiled, epi, Y, y_dtype, B, N, K, (hipStream_t)stream);
+}
+
+// Where the tiled GEMM would run anyway.  gate|up, SwiGLU and quantization / this and the quantizer, us, bf16: 4096 x 13824 x 2560
+// 152.5 / 144.2, 2048 x 22016 x 4096 177.5 / 172.1, 1000 x 5632 x 1024 20.7 / 17.8, 512 x 13824 x 2560 29.0 / 26.4, 256 x 8192 x 1536
+// 12.6 / 12.0.  Few rows are cheaper on the streaming kernel or few_rows_kernel (64 x 5632 x 1024 8.0 / 10.3), and up to 256 rows also on
+// gemm_i8_kernel where that is the choice (256 x 22016 x 4096 31.2 / 33.4, but 384 x 13824 x 2560 26.9 / 24.9).
+extern "C" int bt_swiglu_i8_tiled_pays(int64_t B, int64_t N, int64_t K) {
+    if (B <= 0 || N <= 0 || K <= 0 || N % 32 != 0 || K % 16 != 0) return 0;
+    if (prefers_rows(true, false, B, N, K) || prefers_stream(B, N, K, true, true, true)) return 0;
+    return B > 256 || gemm_i8_dma_rows(B, N, K, true, false) != 0;
 }
 
 // ---- the prefill-only field layout of the tiled copy ----------------------------------------------------------------

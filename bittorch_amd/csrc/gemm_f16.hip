@@ -150,31 +150,7 @@ __device__ __forceinline__ void fd_epilogue_swiglu(const GemmFParams& p, const v
                 if constexpr (MODE == MODE_BF16) a *= 0.5f;  // weights were decoded as +-2.0
                 y[t][r] = round_to_dtype(epi_float(a, ws[t], bs[t]), YDT);
             }
-        float gate[8], up[8];
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                gate[2 * r + t] = y[t][r];
-                up[2 * r + t] = y[2 + t][r];
-            }
-        swiglu8<YDT>(gate, up);
-        // lanes 2 i and 2 i + 1 hold neighbouring columns: the even one takes two of the rows, the odd one the other two
-        uint32_t d[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const uint16_t h0 = YDT == BT_F16 ? f32_to_f16_bits(gate[2 * r]) : f32_to_bf16_bits(gate[2 * r]);
-            const uint16_t h1 = YDT == BT_F16 ? f32_to_f16_bits(gate[2 * r + 1]) : f32_to_bf16_bits(gate[2 * r + 1]);
-            d[r] = (uint32_t)h0 | ((uint32_t)h1 << 16);
-        }
-        const bool odd = threadIdx.x & 1;
-#pragma unroll
-        for (int r = 0; r < 2; r++) {
-            const uint32_t keep = odd ? d[2 + r] : d[r], give = odd ? d[r] : d[2 + r];
-            const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give, 0xB1, 0xf, 0xf, true);
-            char* at = row + r * row_bytes + lane_off + (odd ? 2 * (uint32_t)row_bytes - 4u : 0u);
-            if (16 * mb + 4 * g + r + (odd ? 2 : 0) < rows_left) st2_nt(at, odd ? got : keep, odd ? keep : got);
-        }
+        swiglu_store16<YDT>(row, row_bytes, lane_off, rows_left - 16 * mb, g, y);
         row += 16 * row_bytes;
         __builtin_amdgcn_sched_barrier(0);
     }

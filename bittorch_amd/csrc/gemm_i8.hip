@@ -501,7 +501,7 @@ bool gemm_i8_supported(int64_t N, int64_t K, const void* Q, const void* W_T) {
 
 // gemm_i8_dma.hip
 int gemm_i8_dma_rows(int64_t M, int64_t N, int64_t K, bool tiled, bool fields);
-int launch_gemm_i8_dma(const GemmParams& p, int rows, bool tiled, bool fields, hipStream_t st);
+int launch_gemm_i8_dma(const GemmParams& p, int rows, bool tiled, bool fields, bool swiglu, hipStream_t st);
 
 // One launch over column tiles [tile_n0, tile_n0 + tiles_n) in tiles of 32 * NB rows.
 template <int NB>
@@ -551,7 +551,7 @@ int launch_gemm_i8(const int8_t* Q, int q_layout, const float* s_x, const int32_
     const bool qoo = q_layout == Q_OPERAND_ORDER, tiled = layout_tiled(w_layout), fields = layout_fields(w_layout);
     const int64_t tiles_n = ceil_div(N, G_BN);
     const int dma_nb = qoo ? gemm_i8_dma_rows(M, N, K, tiled, fields) : 0;  // (gemm_i8_dma.hip)
-    if (dma_nb) return launch_gemm_i8_dma(p, dma_nb, tiled, fields, st);
+    if (dma_nb) return launch_gemm_i8_dma(p, dma_nb, tiled, fields, false, st);
     // the column tiles of a mostly empty last round in finer tiles, a launch of their own behind the whole tiles
     // (gemm_split; same sums, same bits)
     const GemmSplit sp = gemm_split(M, N, tiled && K % G_BK == 0 && !tuning_env("BITTORCH_GEMM_INPHASE"));
@@ -564,6 +564,19 @@ int launch_gemm_i8(const int8_t* Q, int q_layout, const float* s_x, const int32_
                           : launch_gemm_i8_part<2>(p, (int)(tiles_n - sp.cols), (int)sp.cols, qoo, tiled, fields, st);
     }
     return launch_gemm_i8_part<4>(p, 0, (int)tiles_n, qoo, tiled, fields, st);
+}
+
+// The GEMM with the SwiGLU output stage: Q in operand order, a natural-order tiled copy of [gate | up] (N % 32 == 0), Y [M, N / 2] of 16 bits
+int launch_gemm_i8_swiglu(const int8_t* Q, const float* s_x, const uint8_t* W_tiled, const Epilogue& epi, void* Y, int y_dtype,
+                          int64_t M, int64_t N, int64_t K, hipStream_t st) {
+    GemmParams p = {};
+    p.Q = Q; p.s_x = s_x; p.W_T = W_tiled; p.Y = Y; p.epi = epi;
+    p.M = M; p.N = N; p.K = K; p.Kb = ceil_div(K, 4);
+    p.y_dtype = y_dtype;
+    p.wsteps = (int)ceil_div(p.Kb, 16);
+    p.tiles16 = (int)(N / 16);
+    const int rows = gemm_i8_dma_rows(M, N, K, true, false);
+    return launch_gemm_i8_dma(p, rows ? rows : 4, true, false, true, st);  // (0: one tile of 128 rows for each compute unit at most)
 }
 
 }  // namespace bt

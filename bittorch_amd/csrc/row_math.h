@@ -61,6 +61,37 @@ __device__ __forceinline__ void swiglu8(float (&g)[8], const float (&u)[8]) {
 #pragma unroll
     for (int i = 0; i < 8; i++) g[i] = swiglu_value(g[i], u[i], DT);
 }
+// The SwiGLU output stage of the tiled GEMMs, for 16 rows of a tile: y[t][r] are a lane's projections of row 4 g + r, rounded to DT,
+// t = 0, 1 those of the gate's columns c, c + 1 and t = 2, 3 the same columns of up.  It stores what the SwiGLU row kernel makes of
+// stored projections, by the same element arithmetic.  Lanes 2 i and 2 i + 1 hold neighbouring columns: the even one stores two
+// of the rows, the odd one the other two, in 8 bytes each.  left: rows that exist; lane_off: of row 4 g, column c.
+template <int DT>
+__device__ __forceinline__ void swiglu_store16(char* row, int64_t row_bytes, uint32_t lane_off, int left, int g, const float (&y)[4][4]) {
+    float gate[8], up[8];
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            gate[2 * r + t] = y[t][r];
+            up[2 * r + t] = y[2 + t][r];
+        }
+    swiglu8<DT>(gate, up);
+    uint32_t d[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const uint16_t h0 = DT == BT_F16 ? f32_to_f16_bits(gate[2 * r]) : f32_to_bf16_bits(gate[2 * r]);
+        const uint16_t h1 = DT == BT_F16 ? f32_to_f16_bits(gate[2 * r + 1]) : f32_to_bf16_bits(gate[2 * r + 1]);
+        d[r] = (uint32_t)h0 | ((uint32_t)h1 << 16);
+    }
+    const bool odd = threadIdx.x & 1;
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const uint32_t keep = odd ? d[2 + r] : d[r], give = odd ? d[r] : d[2 + r];
+        const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give, 0xB1, 0xf, 0xf, true);
+        char* at = row + r * row_bytes + lane_off + (odd ? 2 * (uint32_t)row_bytes - 4u : 0u);
+        if (4 * g + r + (odd ? 2 : 0) < left) st2_nt(at, odd ? got : keep, odd ? keep : got);
+    }
+}
 __device__ __forceinline__ float rmsnorm_value(float x, float r, float w, int dt) {
     return round_to_dtype(__fmul_rn(__fmul_rn(x, r), w), dt);
 }

@@ -356,6 +356,22 @@ class TernaryLinearInference(nn.Module):
         return ternary_linear_int8(q, s_x, self._row_major_for_call(), self.scale, self.in_features, self.bias,
                                    out_dtype, residual, q_operand_order)
 
+    def forward_int8_swiglu(self, q: Tensor, s_x: Tensor, out_dtype: torch.dtype) -> Optional[Tensor]:
+        """For a layer whose columns are ``[gate | up]``: ``swiglu(gate, up)`` ``(*, N/2)`` of what :meth:`forward_int8` makes of ``q``
+        in operand order, formed in the GEMM's output stage; None for a call that is not served that way (the activation type,
+        the weight copies that the layer holds) or not faster so."""
+        if out_dtype == torch.float32 or not q.is_cuda:
+            return None
+        from .. import _C
+        if not _C.swiglu_int8_tiled_pays(q.numel() // max(q.shape[-1], 1), self.in_features, self.out_features):
+            return None
+        tiled = self._tiled_for(q)
+        if tiled is None:
+            return None
+        h = _C.ternary_swiglu_int8_tiled(q.reshape(-1, q.shape[-1]), s_x.reshape(-1), tiled, self.scale, self.bias, self.in_features,
+                                         self.out_features, out_dtype)
+        return h.reshape(*q.shape[:-1], h.shape[-1])
+
     def extra_repr(self) -> str:
         dense = 4 * self.out_features * self.in_features
         ratio = dense / (self.packed_size_bytes + 2 * self.scale.numel())

@@ -113,6 +113,11 @@ class TernarySwiGLU(nn.Module):
             q, s, *rs = fused.act_quant_int8(x, oo1, return_rowsum=want)
         else:
             q, s, *rs = fused.rmsnorm(x, norm_weight, eps, store=False, quantize=True, operand_order=oo1, return_rowsum=want)
-        g, u = self._gate_up_int8(q, s, x.dtype, oo1, rs[0] if rs else None)
-        q2, s2, *rs2 = fused.swiglu(g, u, store=False, quantize=True, operand_order=oo2, return_rowsum=want)
+        # prefill: the SwiGLU product leaves the gate|up GEMM's own output stage where that pays (same bits)
+        h = self.gate_up.forward_int8_swiglu(q, s, x.dtype) if self.gate_up is not None and oo1 and oo2 and not rs else None
+        if h is not None:
+            q2, s2, *rs2 = fused.act_quant_int8(h, oo2)
+        else:
+            g, u = self._gate_up_int8(q, s, x.dtype, oo1, rs[0] if rs else None)
+            q2, s2, *rs2 = fused.swiglu(g, u, store=False, quantize=True, operand_order=oo2, return_rowsum=want)
         return self.down.forward_int8(q2, s2, x.dtype, residual, oo2, rs2[0] if rs2 else None)

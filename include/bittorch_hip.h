@@ -272,6 +272,9 @@ int bt_ternary_linear_packed_forward_fused(const void* X, int64_t ld_x, int x_dt
  *     to the same call on a natural-order copy.  With the two, one pair-ordered copy serves every call of a fused
  *     [gate | up] layer in 16-bit and fp32 activations (the int8 entry point reads natural-order copies only).
  *   bt_ternary_gemm_i8_tiled: bt_ternary_gemm_i8_res on the tiled copy (same remark).
+ *   bt_ternary_swiglu_i8_tiled: for [gate | up] on a natural-order copy (N % 32 == 0) and Q in operand order, Y [B, N/2]
+ *     of a 16-bit type is what bt_swiglu makes of bt_ternary_gemm_i8_tiled's outputs, bit for bit: the product is formed in the
+ *     output stage of the tiled GEMM.  bt_swiglu_i8_tiled_pays: 1 where that is the faster way for this size (0 else).
  *   A tall int8 batch on the tiled copy may take two kernel launches on the stream instead of one (row-major
  *   activations: the column tiles of a mostly empty last round of 128 x 256 tiles run as tiles of 64 or 32 rows
  *   behind the whole tiles): same results, nothing for the caller to do; both are captured by a HIP graph like any other.
@@ -291,6 +294,10 @@ int bt_ternary_gemm_i8_tiled(const int8_t* Q, int q_layout, const float* s_x, co
                              const void* scale, int scale_dtype, int64_t scale_len, const void* bias,
                              int bias_dtype, const void* residual, void* Y, int y_dtype, int32_t* acc_out,
                              int64_t B, int64_t N, int64_t K, void* stream);
+int bt_ternary_swiglu_i8_tiled(const int8_t* Q, const float* s_x, const uint8_t* W_tiled, const void* scale,
+                               int scale_dtype, int64_t scale_len, const void* bias, int bias_dtype, void* Y,
+                               int y_dtype, int64_t B, int64_t N, int64_t K, void* stream);
+int bt_swiglu_i8_tiled_pays(int64_t B, int64_t N, int64_t K);
 
 /*
  * A prefill-only second form of the tiled copy, for the matrix-core int8 GEMM alone (no counterpart in the

@@ -620,6 +620,74 @@ def test_swiglu_output_stage_of_the_tiled_gemm(oracle, dtype, b, n, k):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,n,k", [(33, 96, 112), (70, 64, 1536), (1, 32, 16), (40, 8192, 4096), (300, 8192, 1600), (500, 320, 1040),
+                                   (512, 8192, 1024), (1000, 13824, 512), (2048, 11008, 256), (1700, 10240, 144)])
+def test_swiglu_output_stage_of_the_int8_gemm(oracle, dtype, b, n, k):
+    """Bit for bit what the SwiGLU kernel makes of the int8 GEMM's stored projections, as int8 too: tiles of 32, 64 and 128 rows and
+    the finer ones of a remainder, one and two groups of waves, a last wave of 16 of its 32 columns, K past whole stages, one scale
+    for all columns, overflowing projections and NaN."""
+    from bittorch_amd import _C
+    _, wt = _packed(oracle, n, k, seed=7)
+    tiled = _C.retile_weights(wt, k)
+    g = torch.Generator().manual_seed(n)
+    scale = (torch.rand(n, generator=g) + 0.5).cuda() * 0.05
+    bias = (torch.randn(n, generator=g) * 0.1).to(dtype).cuda()
+    x = seeded_acts(b, k, seed=b)
+    x[0], x[b // 2] = x[0] * 3e5, x[b // 2] * 500
+    q, s_x = _C.act_quant_int8(x.cuda(), True)
+    s_x[b - 1] = float("nan")
+    for sc, bs in ((scale, None), (scale, bias), (scale[:1], bias)):
+        announce("swiglu stage of the int8 GEMM", dtype, b, n, k, sc.numel(), bs is not None)
+        gu = _C.ternary_gemm_int8_tiled(q, s_x, tiled, sc, bs, k, n, dtype, q_operand_order=True)
+        want = _C.swiglu(gu[:, :n // 2], gu[:, n // 2:])
+        got = _C.ternary_swiglu_int8_tiled(q, s_x, tiled, sc, bs, k, n, dtype)
+        assert got.shape == (b, n // 2)
+        same = (got == want) | (got.isnan() & want.isnan())
+        assert bool(same.all()), int((~same).sum())
+        oo = n % 32 == 0
+        want_q, want_s = _C.swiglu(gu[:, :n // 2], gu[:, n // 2:], False, True, oo)
+        got_q, got_s = _C.act_quant_int8(got, oo)
+        assert torch.equal(got_q, want_q) and torch.equal(got_s, want_s)
+    if b == 33:
+        with pytest.raises(RuntimeError):
+            _C.ternary_swiglu_int8_tiled(q, s_x, tiled, scale, None, k, n, torch.float32)
+        with pytest.raises(RuntimeError):
+            _C.ternary_swiglu_int8_tiled(q, s_x, tiled, scale[:16], None, k, n, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,d,ffn", [((2, 600), 512, 2752), (1200, 256, 1040), (1500, 512, 1000)])
+def test_int8_mlp_on_the_output_stage(oracle, dtype, rows, d, ffn, monkeypatch):
+    """``TernarySwiGLU`` in int8 arithmetic gives the same bits with and without the GEMM's SwiGLU output stage, leading dimensions,
+    captured calls, fp32 and an ffn that it does not take included."""
+    from bittorch_amd import _C
+    from bittorch_amd.nn import TernarySwiGLU
+    mlp = TernarySwiGLU(_layer(oracle, ffn, d, seed=1), _layer(oracle, ffn, d, seed=2), _layer(oracle, d, ffn, seed=3),
+                        compute="int8", fuse_gate_up=True)
+    for L in (mlp.gate_up, mlp.down):
+        L.scale.mul_(0.05)
+        L.prepare_decode()
+    nw = (torch.rand(d) + 0.5).to(dtype).cuda()
+    lead = rows if isinstance(rows, tuple) else (rows,)
+    x = seeded_acts(int(np.prod(lead)), d, seed=5, dtype=dtype).reshape(*lead, d).cuda()
+    got = {}
+    for pays in (False, True):
+        announce("int8 MLP", dtype, rows, d, ffn, pays)
+        monkeypatch.setattr(_C, "swiglu_int8_tiled_pays", lambda *a: pays and ffn % 16 == 0)
+        got[pays] = (mlp(x, nw, 1e-5, x), mlp(x))
+        assert got[pays][0].shape == x.shape
+    assert torch.equal(got[False][0], got[True][0]) and torch.equal(got[False][1], got[True][1])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = mlp(x, nw, 1e-5, x)
+    want = got[True][0].clone()
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_ternary_swiglu_decode_uses_the_output_stage(oracle, dtype):
     from bittorch_amd.nn import TernarySwiGLU
     d, ffn = 256, 704
