@@ -210,6 +210,7 @@ static bool prefers_stream(int64_t B, int64_t N, int64_t K, bool int8, bool tile
 //          it wins where 64 columns each are enough workgroups, 16 x 11008 x 4096 10.5 / 9.7, 16 x 16384 x 1024 8.9 / 7.3, not 8 x 4096 x
 //          4096 8.6 / 9.3; tiled 16 x 7680 x 2560 5.7 / 5.3, 8 x 7680 x 2560 5.1 / 5.3
 static bool prefers_rows(bool i8, bool row_major, int64_t B, int64_t N, int64_t K) {
+    if (B > 65535ll * 16) return false;  // its grid.y is the row blocks; the others slice such a call or walk it in grid.x
     if (option(OPT_ROWS_CFG)) return true;
     if (option(OPT_STREAM_MAX_ROWS)) return false;
     const double work = (double)B * (double)N * (double)K, blocks = (double)ceil_div(B, 16);

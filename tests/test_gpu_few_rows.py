@@ -118,3 +118,17 @@ def test_choice_by_size():
         assert torch.equal(got, _C.ternary_linear_tiled_forward(x, tiled, scale, bias, k, n))
         set_option("ROWS_CFG", None)
         assert torch.equal(_C.ternary_linear_tiled_forward(x[:32], tiled, scale, bias, k, n), _C.ternary_linear_packed_forward(x[:32], packed, scale, bias, k))
+
+
+def test_more_rows_than_its_grid_has_blocks():
+    """65535 blocks of 32 rows and a few rows more: served by a kernel that slices such a call, whatever ROWS_CFG asks for."""
+    from bittorch_amd import _C
+    m, n, k = 65535 * 32 + 17, 64, 16
+    x, packed, scale, tern, bias, _ = _case(m, n, k, torch.bfloat16)
+    tiled = _C.retile_weights(packed, k)
+    want, bound = (x.double() @ tern.t()) * scale.double() + bias.double(), _bound(x, tern, scale, bias, torch.bfloat16)
+    for option in (None, "2,2"):
+        announce("few rows, tall", option, m, n, k)
+        set_option("ROWS_CFG", option)
+        got = _C.ternary_linear_tiled_forward(x, tiled, scale, bias, k, n)
+        assert bool(((got.double() - want).abs() <= bound).all())
