@@ -7,7 +7,7 @@
 // (fp32 accumulation of exact products; the summation order differs from the reference's
 // sequential loop, which the 16-bit output tolerance covers).
 //
-// A 256-thread workgroup (4 waves) owns a tile of 32 NB x 256 outputs, wave w columns 64 w .. +63 over the whole of K; two
+// A 256-thread workgroup (4 waves) owns a tile of 16 NR x 256 outputs, wave w columns 64 w .. +63 over the whole of K; two
 // workgroups share a compute unit, so that one's MFMAs run while the other waits, starts, drains or stores (a 512-thread
 // workgroup that split K over the two waves of a SIMD: 6.9 us a round of tiles with nothing beside it, fp16 / bf16 row-major
 // weights, 4096 x 11008 x 4096 338 -> 260 us, tiled 300 -> 257; 16384 x 768 x 768 30 -> 21.5; 512 x 4096 x 4096 49 -> 31).
@@ -52,7 +52,7 @@ struct GemmFParams {
 static_assert(offsetof(GemmFParams, Y) == 64, "first argument line as laid out above");
 
 // Stages of activations in LDS; of weights one fewer, since a wave has its own in registers half a stage before it needs them.
-// One group of four waves: 56, 44, 36 KiB; two groups: 64 (NB = 2), 56 (NB = 1).
+// NB: 32 rows of them.  One group of four waves: 56, 44, 36 KiB; two groups: 64 (NB = 2), 56 (NB = 1).
 constexpr int fd_stages(int NB, int KG) { return NB == 4 || (NB == 2 && KG == 2) ? 3 : NB == 2 || KG == 2 ? 4 : 5; }
 constexpr int fd_group_bytes(int NB, int KG) { return fd_stages(NB, KG) * NB * 4096 + (fd_stages(NB, KG) - 1) * 4096; }
 
@@ -156,14 +156,15 @@ __device__ __forceinline__ void fd_epilogue_swiglu(const GemmFParams& p, const v
     }
 }
 
-// One tile of 32 NB rows.  TAIL: K is not a multiple of 64 (of 8 it is): the lanes whose k lies past
+// One tile of 16 NR rows (48: a wave stages 64, the last ones repeated).  TAIL: K is not a multiple of 64 (of 8 it is): the lanes whose k lies past
 // the end load something of their own row or column instead and their activations are zeroed on the way to the MFMAs.
-// KG = 2: two groups of four waves, each on its run of the stages; they add their sums through LDS and store half the rows each.
+// KG = 2: two groups of four waves, each on its run of the stages; they add their sums through LDS and store half the rows each
+// (of 48: 32 and 16).
 // SW: the SwiGLU output stage on a copy in gate/up pair order (stored tiles 2 i, 2 i + 1 are 16 columns of the gate and the same of up):
 // a lane takes two columns of either, so that no sum changes lanes.
-template <int MODE, int SRC, int NB, int KG, bool TAIL, bool RN, bool SW>
+template <int MODE, int SRC, int NR, int KG, bool TAIL, bool RN, bool SW>
 __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_t m0, const int tile_n, uint8_t* lds_all) {
-    constexpr int BM = 32 * NB, A_BYTES = NB * 4096, NST = fd_stages(NB, KG), W_AT = NST * A_BYTES;
+    constexpr int NB = (NR + 1) / 2, BM = 16 * NR, A_BYTES = NB * 4096, NST = fd_stages(NB, KG), W_AT = NST * A_BYTES;
     constexpr int A_LOADS = NB, W_LOADS = SRC == W_ROWS ? 4 : 1, LOADS = A_LOADS + W_LOADS;
     const int lane = threadIdx.x & 63;
     const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = wave_all & 3, group = KG == 1 ? 0 : wave_all >> 2;
@@ -241,14 +242,14 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
         w_into = next_wbuf(w_into);
     };
 
-    v4f acc[2 * NB][4];
+    v4f acc[NR][4];
 #pragma unroll
-    for (int mb = 0; mb < 2 * NB; mb++)
+    for (int mb = 0; mb < NR; mb++)
 #pragma unroll
         for (int t = 0; t < 4; t++) acc[mb][t] = v4f{0.f, 0.f, 0.f, 0.f};
 
     // two sets of fragments: the halves of a sub-step (NB = 4) or whole sub-steps
-    constexpr int RB = NB == 4 ? 4 : 2 * NB;
+    constexpr int RB = NB == 4 ? 4 : NR;
     u32x4 a_x[RB], a_y[RB], b0[4], b1[4];
     uint32_t raw[4];
     // lane (j, g): k = 16 g + 8 sub .. +7 of row 16 mb + j
@@ -322,7 +323,7 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
     for (int s = 0; s < mine; s++) {
         const uint32_t nxt = next_buf(buf);
         auto run_mfma = [&](int c, const u32x4 (&a)[RB], const u32x4 (&b)[4], int mb0) {
-            if (c % SL != 0) return;
+            if (c % SL != 0 || c >= 4 * SL * RB) return;
             const int i = (c / SL) >> 2, t = (c / SL) & 3;
             mfma(a[i], b[t], acc[mb0 + i][t]);
         };
@@ -462,8 +463,9 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
         for (int i = 0; i < NB; i++)
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                mine_at[64 * (4 * i + t)] = group ? acc[i][t] : acc[NB + i][t];
-                sums[i][t] = group ? acc[NB + i][t] : acc[i][t];
+                const int other = NB + i < NR ? NB + i : NR - 1;  // (48 rows: the last block twice, stored once)
+                mine_at[64 * (4 * i + t)] = group ? acc[i][t] : acc[other][t];
+                sums[i][t] = group ? acc[other][t] : acc[i][t];
             }
         __syncthreads();
 #pragma unroll
@@ -475,15 +477,15 @@ __device__ __forceinline__ void gemm_f16_tile(const GemmFParams& p, const int64_
     }
 }
 
-// NB: tiles of 32 NB rows.  NF > 0: an XCD's tiles from p.fine_from on are computed in tiles of 32 NF rows.
-template <int MODE, int SRC, int NB, int NF, int KG, bool TAIL, bool RN, bool SW>
-__global__ __launch_bounds__(256 * KG, KG == 2 || NB == 4 ? 2 : NB == 2 ? 3 : 4) void gemm_f16_kernel(GemmFParams p) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[KG * fd_group_bytes(NB, KG)];
+// NR: tiles of 16 NR rows.  NF > 0: an XCD's tiles from p.fine_from on are computed in tiles of 16 NF rows.
+template <int MODE, int SRC, int NR, int NF, int KG, bool TAIL, bool RN, bool SW>
+__global__ __launch_bounds__(256 * KG, KG == 2 || NR == 8 ? 2 : NR == 4 ? 3 : 4) void gemm_f16_kernel(GemmFParams p) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds[KG * fd_group_bytes((NR + 1) / 2, KG)];
     // XCD-aware tile order: the 8 XCDs each take a contiguous run of tiles, walked in groups of four row tiles, so that one
     // XCD's L2 holds a compact block of rows and columns
     const uint32_t idx = blockIdx.x >> 3;
     const bool fine = NF > 0 && idx >= (uint32_t)p.fine_from;  // (uniform)
-    const uint32_t parts = NF > 0 ? NB / (NF > 0 ? NF : 1) : 1, f = fine ? idx - (uint32_t)p.fine_from : 0u;
+    const uint32_t parts = NF > 0 ? NR / (NF > 0 ? NF : 1) : 1, f = fine ? idx - (uint32_t)p.fine_from : 0u;
     const uint32_t in_xcd = fine ? (uint32_t)p.fine_from + f / parts : idx;
     const uint32_t lin = (blockIdx.x & 7u) * (uint32_t)p.per_xcd + in_xcd;
     const uint32_t tiles_m = (uint32_t)p.tiles_m, tiles_n = (uint32_t)p.tiles_n;
@@ -494,15 +496,15 @@ __global__ __launch_bounds__(256 * KG, KG == 2 || NB == 4 ? 2 : NB == 2 ? 3 : 4)
     const uint32_t gm = (tiles_m - first_m < GM) ? tiles_m - first_m : GM;
     const uint32_t in_group = lin - group * GM * tiles_n;
     const uint32_t tn = (gm == GM) ? in_group / GM : in_group / gm;
-    const int64_t m0 = (int64_t)(first_m + (in_group - tn * gm)) * (32 * NB);
+    const int64_t m0 = (int64_t)(first_m + (in_group - tn * gm)) * (16 * NR);
     if constexpr (NF > 0) {
         if (fine) {
-            const int64_t mf = m0 + (int64_t)(f % parts) * (32 * NF);
+            const int64_t mf = m0 + (int64_t)(f % parts) * (16 * NF);
             if (mf < p.M) gemm_f16_tile<MODE, SRC, NF, 1, TAIL, RN, SW>(p, mf, (int)tn, lds);
             return;
         }
     }
-    gemm_f16_tile<MODE, SRC, NB, KG, TAIL, RN, SW>(p, m0, (int)tn, lds);
+    gemm_f16_tile<MODE, SRC, NR, KG, TAIL, RN, SW>(p, m0, (int)tn, lds);
 }
 
 // X and Y are read and written in 16- and 8-byte pieces; 32-bit byte offsets span a tile's rows of X, 16 rows of Y and, for
@@ -521,23 +523,27 @@ bool gemm_f16_supported(int64_t N, int64_t K, const void* X, const void* W_T, co
 // the other tiles' waves for company (1000 x 13824 x 2560 66.9 / 81.2).
 static bool f16_splits_k(int64_t stages) { return stages >= 24; }
 
-// Rows of the tiles in units of 32, and what the launch takes in microseconds.  Up to one tile of 32, then of 64 rows for each
-// compute unit the launch is one tile deep; beyond that a compute unit's run of tiles is priced.  Measured (tiles of 128 / 64 /
+// Rows of the tiles in units of 16, and what the launch takes in microseconds.  Up to one tile of 32, then of 48 (where two groups of
+// waves share it), then of 64 rows for each compute unit the launch is one tile deep; beyond that a compute unit's run of tiles is priced.  Measured (tiles of 128 / 64 /
 // 32 rows, us, row-major weights): M = 512, 1024, 1536, 2048, 3072, 4096 with N = K = 4096 30 / 30 / 25, 33 / 31 / 40,
 // 49 / 49 / 53, 52 / 54 / 75, 89 / 81 / 107, 95 / 106 / 139; 1000 x 13824 x 2560 60 / 66 / 81; 1000 x 2560 x 6912 66 / 45 / 62;
 // 16384 x 768 x 768 21 / 20 / 26; 4096 x 11008 x 4096 (the last round in halves) 251 / 264 / 333.
+// Tiles of 48 rows, us, decode-tiled / row-major bf16, those of 64 / 48 rows: 1000 x 2560 x 6912 45.1 / 43.7, 42.3 / 41.0; 1200 x 2560 x
+// 6912 43.1 / 40.5, 42.4 / 39.7; 832 x 2560 x 2560 19.8 / 18.3; 768 x 4096 x 4096 29.0 / 26.7; 384 x 8192 x 8192 50.0 / 47.3; 350 x 8192 x
+// 1536 14.5 / 13.5 (a stage has a quarter fewer MFMAs, its loads and decode are the same).
 static int gemm_f16_plan(int64_t M, int64_t N, int64_t K, double* us) {
     const int64_t C = gemm_compute_units(), tn = ceil_div(N, F_BN);
     const int64_t t4 = ceil_div(M, 128) * tn, t2 = ceil_div(M, 64) * tn, t1 = ceil_div(M, 32) * tn;
     const bool whole = gemm_whole_tiles(), split = f16_splits_k(ceil_div(K, F_BK));
-    if (t1 <= C && !whole) { *us = split ? 5.7 + 0.0042 * (double)K : 4.0 + 0.0055 * (double)K; return 1; }
-    if (t2 <= C && !whole) { *us = split ? 6.0 + 0.0056 * (double)K : 5.0 + 0.0065 * (double)K; return 2; }
+    if (t1 <= C && !whole) { *us = split ? 5.7 + 0.0042 * (double)K : 4.0 + 0.0055 * (double)K; return 2; }
+    if (split && ceil_div(M, 48) * tn <= C && !whole) { *us = 5.9 + 0.0049 * (double)K; return 3; }
+    if (t2 <= C && !whole) { *us = split ? 6.0 + 0.0056 * (double)K : 5.0 + 0.0065 * (double)K; return 4; }
     const int parts = gemm_dma_parts(t4);
     const double n4 = parts == 1 ? (double)ceil_div(t4, C) : (double)(2 * (t4 / (2 * C))) + (parts == 2 ? 1.2 : 0.6);
     const double p4 = n4 * (2.0 + 0.0113 * (double)K), p2 = (double)ceil_div(t2, C) * (1.3 + 0.0062 * (double)K);
     const bool half = p2 < p4 && !whole;
     *us = 4.0 + (half ? p2 : p4);
-    return half ? 2 : 4;
+    return half ? 4 : 8;
 }
 double gemm_f16_cost(int64_t M, int64_t N, int64_t K) {
     double us;
@@ -545,59 +551,59 @@ double gemm_f16_cost(int64_t M, int64_t N, int64_t K) {
     return us;
 }
 
-template <int MODE, int SRC, int NB, bool TAIL, bool RN = false, bool SW = false>
+template <int MODE, int SRC, int NR, bool TAIL, bool RN = false, bool SW = false>
 static int launch_gemm_f16_cfg(GemmFParams p, hipStream_t st) {
     const char* who = SRC == W_TILES ? "bt_ternary_linear_tiled_forward" : "bt_ternary_linear_packed_forward";
     p.tiles_n = (int)ceil_div(p.N, F_BN);
-    p.tiles_m = (int)ceil_div(p.M, 32 * NB);
+    p.tiles_m = (int)ceil_div(p.M, 16 * NR);
     const int64_t total = (int64_t)p.tiles_m * p.tiles_n;
     if (total >= (1ll << 29)) {
-        set_error("%s: %lld tiles of %d x 256 outputs are more than one launch takes", who, (long long)total, 32 * NB);
+        set_error("%s: %lld tiles of %d x 256 outputs are more than one launch takes", who, (long long)total, 16 * NR);
         return BT_ERR_INVALID;
     }
     p.per_xcd = (int)ceil_div(total, 8);
     p.fine_from = p.per_xcd;
     const dim3 block(256);
-    if constexpr (NB == 4) {
+    if constexpr (NR == 8) {
         const int parts = gemm_dma_parts(total);
         if (parts > 1) {
             const int rem = p.per_xcd % (int)(2 * gemm_compute_units() / 8);
             p.fine_from = p.per_xcd - rem;
             const dim3 grid((unsigned)(8 * (p.fine_from + parts * rem)));
-            if (parts == 2) hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 4, 2, 1, TAIL, RN, SW>), grid, block, 0, st, p);
-            else hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 4, 1, 1, TAIL, RN, SW>), grid, block, 0, st, p);
+            if (parts == 2) hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 8, 4, 1, TAIL, RN, SW>), grid, block, 0, st, p);
+            else hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, 8, 2, 1, TAIL, RN, SW>), grid, block, 0, st, p);
             return check_launch(who);
         }
     }
-    if constexpr (NB != 4) {
-        if (total <= gemm_compute_units() && f16_splits_k(p.wstages)) {
-            hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, NB, 0, 2, TAIL, RN, SW>), dim3((unsigned)(8 * p.per_xcd)), dim3(512), 0, st, p);
+    if constexpr (NR != 8) {
+        if (NR == 3 || (total <= gemm_compute_units() && f16_splits_k(p.wstages))) {
+            hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, NR, 0, 2, TAIL, RN, SW>), dim3((unsigned)(8 * p.per_xcd)), dim3(512), 0, st, p);
             return check_launch(who);
         }
     }
-    hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, NB, 0, 1, TAIL, RN, SW>), dim3((unsigned)(8 * p.per_xcd)), block, 0, st, p);
+    if constexpr (NR != 3) hipLaunchKernelGGL((gemm_f16_kernel<MODE, SRC, NR, 0, 1, TAIL, RN, SW>), dim3((unsigned)(8 * p.per_xcd)), block, 0, st, p);
     return check_launch(who);
 }
-template <int MODE, int SRC, int NB>
+template <int MODE, int SRC, int NR>
 static int launch_gemm_f16_src(const GemmFParams& p, int epi_op, hipStream_t st) {
     if constexpr (SRC == W_TILES) {
         if (epi_op == EPI_SWIGLU_PAIRS)
-            return p.K % F_BK != 0 ? launch_gemm_f16_cfg<MODE, SRC, NB, true, false, true>(p, st)
-                                   : launch_gemm_f16_cfg<MODE, SRC, NB, false, false, true>(p, st);
+            return p.K % F_BK != 0 ? launch_gemm_f16_cfg<MODE, SRC, NR, true, false, true>(p, st)
+                                   : launch_gemm_f16_cfg<MODE, SRC, NR, false, false, true>(p, st);
         // (rows of any length come with K of any length: one instance)
-        if (p.N % 4 != 0) return launch_gemm_f16_cfg<MODE, SRC, NB, true, true>(p, st);
+        if (p.N % 4 != 0) return launch_gemm_f16_cfg<MODE, SRC, NR, true, true>(p, st);
     }
-    return p.K % F_BK != 0 ? launch_gemm_f16_cfg<MODE, SRC, NB, true>(p, st) : launch_gemm_f16_cfg<MODE, SRC, NB, false>(p, st);
+    return p.K % F_BK != 0 ? launch_gemm_f16_cfg<MODE, SRC, NR, true>(p, st) : launch_gemm_f16_cfg<MODE, SRC, NR, false>(p, st);
 }
-template <int MODE, int NB>
+template <int MODE, int NR>
 static int launch_gemm_f16_mode(const GemmFParams& p, int src, int epi_op, hipStream_t st) {
-    return src == W_TILES ? launch_gemm_f16_src<MODE, W_TILES, NB>(p, epi_op, st)
-         : src == W_ROWS16 ? launch_gemm_f16_src<MODE, W_ROWS16, NB>(p, 0, st) : launch_gemm_f16_src<MODE, W_ROWS, NB>(p, 0, st);
+    return src == W_TILES ? launch_gemm_f16_src<MODE, W_TILES, NR>(p, epi_op, st)
+         : src == W_ROWS16 ? launch_gemm_f16_src<MODE, W_ROWS16, NR>(p, 0, st) : launch_gemm_f16_src<MODE, W_ROWS, NR>(p, 0, st);
 }
 template <int MODE>
 static int launch_gemm_f16_rows(const GemmFParams& p, int rows, int src, int epi_op, hipStream_t st) {
-    return rows == 4 ? launch_gemm_f16_mode<MODE, 4>(p, src, epi_op, st)
-         : rows == 2 ? launch_gemm_f16_mode<MODE, 2>(p, src, epi_op, st) : launch_gemm_f16_mode<MODE, 1>(p, src, epi_op, st);
+    return rows == 8 ? launch_gemm_f16_mode<MODE, 8>(p, src, epi_op, st) : rows == 4 ? launch_gemm_f16_mode<MODE, 4>(p, src, epi_op, st)
+         : rows == 3 ? launch_gemm_f16_mode<MODE, 3>(p, src, epi_op, st) : launch_gemm_f16_mode<MODE, 2>(p, src, epi_op, st);
 }
 // epi_op: 0, or EPI_SWIGLU_PAIRS (w_layout W_LAYOUT_TILED in pair order, N % 32 == 0, no residual; Y is [M, N / 2])
 // Kw: the weights' K where the rows of X are longer (zeros behind it; 0: K)

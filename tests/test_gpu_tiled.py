@@ -821,3 +821,25 @@ def test_row_major_fallback_keeps_its_promises(oracle):
     want = _layer(oracle, 256, 256, seed=3, decode_tiled=False).forward_int8(q, sx)
     assert torch.equal(b.forward_int8(q, sx), want)   # outside a capture: rebuilt, both copies held from here on
     assert b.keep_row_major and b._has_row_major()
+
+
+@pytest.mark.parametrize("m,n,k", [(1000, 2560, 1536), (1200, 2560, 1480), (821, 2559, 1500), (993, 2336, 1544)])
+def test_tiles_of_48_rows(m, n, k):
+    """Launches of one 48-row tile for each compute unit: last tiles of 1, 5, 33, 40 and 48 rows, an odd number of stages, a partial one, N of any
+    length; row-major weights give the same bits, the SwiGLU stage the row kernel's, and a residual its two roundings."""
+    from bittorch_amd import _C
+    from test_gpu_few_rows import _bound, _case
+    for dtype in (torch.float16, torch.bfloat16):
+        announce("48-row tiles", m, n, k, dtype)
+        x, packed, scale, tern, bias, res = _case(m, n, k, dtype)
+        natural = _C.retile_weights(packed, k)
+        got = _C.ternary_linear_tiled_forward(x, natural, scale, bias, k, n)
+        err = (got.double() - ((x.double() @ tern.t()) * scale.double() + bias.double())).abs()
+        assert bool((err <= _bound(x, tern, scale, bias, dtype)).all()), float(err.max())
+        assert torch.equal(_C.ternary_linear_tiled_forward(x, natural, scale, bias, k, n, residual=res), got + res)
+        if n % 4 == 0:
+            assert torch.equal(_C.ternary_linear_packed_forward(x, packed, scale, bias, k), got)
+        if n % 32 == 0:
+            pairs = _C.retile_weights(packed, k, True)
+            h = _C.ternary_linear_tiled_forward(x, pairs, scale, bias, k, n, swiglu_pairs=True)
+            assert torch.equal(h, _C.swiglu(got[:, :n // 2], got[:, n // 2:]))
