@@ -315,8 +315,8 @@ def ternary_linear_tiled_forward(X: Tensor, W_tiled: Tensor, scale: Tensor, bias
                                  natural_from_pairs: bool = False) -> Tensor:
     """:func:`ternary_linear_packed_forward` / ``_fused`` on the decode-tiled copy of the weights: the same results
     bit for bit up to 32 rows and in the tiled GEMMs; a larger batch on the streaming kernel may split K among its waves
-    differently on the two layouts, and one of a few tens of 16-bit rows has a kernel that reads tiled weights alone: fp32 sums
-    that differ in their last bits.
+    differently on the two layouts, and the kernel for a few tens of 16-bit rows, priced for each layout by itself, may serve one
+    alone: fp32 sums that differ in their last bits.
     ``swiglu_pairs`` (copy built with ``gate_up_pairs=True``): the layer's columns are ``[gate | up]`` and the
     output is the MLP's hidden vector ``swiglu(gate(x), up(x))`` ``[*, N/2]``, formed in the kernel's output stage.
     ``natural_from_pairs``: the same pair-ordered copy read as an ordinary linear layer (output ``[*, N]`` in natural
