@@ -71,8 +71,7 @@ struct GemmF32Params {
     int64_t M, C, NC;    // NC: output columns
     int tiles_m, tiles_n;
     int per_xcd;         // tiles per XCD
-    int fine_from;       // REM: an XCD's tiles from this one on are shared by `parts` workgroups each
-    int parts;           // 2 or 4
+    int fine_from;       // PARTS > 1: an XCD's tiles from this one on are shared by PARTS workgroups each
     int wsteps;          // B_TILED: 64-wide steps of the copy
     int tiles16;         // B_TILED: as in tiles16_arg
     int ldw;             // bytes of a W_T row
@@ -86,49 +85,24 @@ struct GemmF32Params {
 // bf16 +-0.5: the weights' value here, so that the low byte is zero and a sum cannot overflow before it is doubled
 constexpr uint32_t LUT_BF16_HALF = 0x00BF3F00u;
 
-// A wave works on a tile of 64 rows x 64 NG columns.  KS = 1: the four waves of a workgroup are a 2 x 2 block of such tiles.
+// A wave works on a tile of 16 NB rows x 64 NG columns, from row m0 and column c0 on (NB = 4, but for shared tiles).
 // KS > 1: all KS waves of a workgroup work on one tile, each on its run of the contraction, and add their sums through LDS
 // (pairwise, always in the same order): for outputs with too few tiles to occupy the chip.
-// REM (KS = 1): a tile of the remainder, the last that would occupy a part of the compute units only, is shared by two workgroups of
-// 64 rows or four of one wave's tile each; their waves take halves or quarters of the contraction and add their sums through LDS.
 // SC: X's columns are scaled (input gradient with one scale per row of W).
 // RN: forward outputs of N % 4 != 0, an instance of its own: asked at run time, every other output paid half a microsecond for
 // the clamped columns and the second way to store (us, fp32, 300 x 4096 x 512 17.9 / 17.0, 4096 x 768 x 768 28.2 / 27.5).  Only
 // the tile of one wave's 64 x 64 outputs gains from the question: with a branch between them the compiler sends each row's
 // stores off by themselves (512 x 2048 x 1032 17.0 without, 16.0 with it; 4096 x 128 x 2048 24.1 / 23.1).
-template <int SRC, int NG, int KS, bool SC, bool RN, bool REM>
-__global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(GemmF32Params p) {
-    constexpr int TM = (KS == 1) ? 128 : 64, TN = (KS == 1) ? 128 * NG : 64 * NG;  // a workgroup's tile
-    // the 8 XCDs each take a contiguous run of tiles, walked in groups of four row tiles (as in gemm_f16.hip)
-    const uint32_t idx = blockIdx.x >> 3;
-    const bool fine = REM && idx >= (uint32_t)p.fine_from;  // (uniform)
-    const uint32_t parts = fine ? (uint32_t)p.parts : 1u, part = fine ? (idx - (uint32_t)p.fine_from) & (parts - 1u) : 0u;
-    const uint32_t in_xcd = fine ? (uint32_t)p.fine_from + ((idx - (uint32_t)p.fine_from) >> (parts >> 1)) : idx;
-    const uint32_t lin = (blockIdx.x & 7u) * (uint32_t)p.per_xcd + in_xcd;
-    const uint32_t tiles_m = (uint32_t)p.tiles_m, tiles_n = (uint32_t)p.tiles_n;
-    if (lin >= tiles_m * tiles_n) return;
-    constexpr uint32_t GM = 4;
-    const uint32_t group = lin / (GM * tiles_n), first_m = group * GM;
-    const uint32_t gm = (tiles_m - first_m < GM) ? tiles_m - first_m : GM;
-    const uint32_t in_group = lin - group * GM * tiles_n;
-    const uint32_t tn = (gm == GM) ? in_group / GM : in_group / gm;
-    const uint32_t tm = first_m + (in_group - tn * gm);
-
+template <int SRC, int NG, int NB, int KS, bool SC, bool RN>
+__device__ __forceinline__ void gemm_f32_tile(const GemmF32Params& p, const int64_t m0, const int64_t c0) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i = lane & 15, g = lane >> 4;
-    // which of the tile's four wave tiles, and how many waves share it
-    const int row_half = parts == 1 ? wave >> 1 : parts == 2 ? (int)part : (int)part >> 1, col_half = parts <= 2 ? wave & 1 : (int)part & 1;
-    const int ks = KS > 1 ? KS : (int)parts, k_part = KS > 1 ? wave : parts == 1 ? 0 : parts == 2 ? wave >> 1 : wave;
-    const int64_t m0 = (int64_t)tm * TM + (KS == 1 ? 64 * row_half : 0);
-    const int64_t c0 = (int64_t)tn * TN + (KS == 1 ? 64 * NG * col_half : 0);
-    // (no barriers below for these; of two wave tiles side by side the second may lie past the last column: it loads clamped ones)
-    if (KS == 1 && (m0 >= p.M || (c0 >= p.NC && parts != 2))) return;
 
     // rows and columns past the end repeat the last one: they only feed outputs that are never stored
     const uint8_t* a_base = (const uint8_t*)(p.X + m0 * p.C);
-    uint32_t a_off[4];
+    uint32_t a_off[NB];
 #pragma unroll
-    for (int b = 0; b < 4; b++) {
+    for (int b = 0; b < NB; b++) {
         const int64_t left = p.M - 1 - m0;
         const uint32_t r = (uint32_t)((16 * b + i < left) ? 16 * b + i : left);
         a_off[b] = (r * (uint32_t)p.C + 8u * g) * 4u;
@@ -152,12 +126,12 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
     const uint32_t sel_wt = ((uint32_t)(2 * (g & 1) + 1) << 24) | (0x0Cu << 16) | ((uint32_t)(2 * (g & 1)) << 8) | 0x0Cu;
     // this wave's steps of 32: [st0, st1) of the whole ones, and the partial one if it is the last wave
     const int nfull = (int)(p.C / 32), steps = (int)((p.C + 31) / 32);
-    const int run = (KS == 1) ? (nfull + ks - 1) >> (ks >> 1) : (nfull + KS - 1) / KS;  // (KS == 1: ks is 1, 2 or 4)
-    const int st0 = min(k_part * run, nfull), st1 = min(st0 + run, nfull);
-    const bool last = k_part == ks - 1;
+    const int run = (KS == 1) ? nfull : (nfull + KS - 1) / KS;
+    const int st0 = (KS == 1) ? 0 : min(wave * run, nfull), st1 = (KS == 1) ? nfull : min(st0 + run, nfull);
+    const bool last = KS == 1 || wave == KS - 1;
 
     constexpr int BR = (SRC == B_TILED) ? 4 : 2;
-    f32x4_u raw[4][2];
+    f32x4_u raw[NB][2];
     uint32_t braw[NG][BR];
     f32x4_u sc[2];
 
@@ -221,7 +195,7 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
         }
     };
 
-    v4f acc[4][4 * NG];
+    v4f acc[NB][4 * NG];
     u32x4 pl[2][3];  // the planes of two row blocks: one in the MFMAs, the next being split
     auto split = [&](int b, const f32x4_u (&scn)[2], auto any) __attribute__((always_inline)) {
         float x[8];
@@ -276,8 +250,8 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
         if (more) load_a(0, nx, false);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int b = 0; b < 4; b++) {
-            if (b < 3) {
+        for (int b = 0; b < NB; b++) {
+            if (b < NB - 1) {
                 split(b + 1, scn, any);
                 if (more) load_a(b + 1, nx, false);
             }
@@ -290,19 +264,19 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
     };
     auto contract = [&](auto any) __attribute__((always_inline)) {
 #pragma unroll
-        for (int b = 0; b < 4; b++)
+        for (int b = 0; b < NB; b++)
 #pragma unroll
             for (int t = 0; t < 4 * NG; t++) acc[b][t] = v4f{0.f, 0.f, 0.f, 0.f};
         if (st0 < st1) {
             load_w(st0, false);
 #pragma unroll
-            for (int b = 0; b < 4; b++) load_a(b, st0, false);
+            for (int b = 0; b < NB; b++) load_a(b, st0, false);
             for (int s = st0; s < st1; s++) step(s + 1 < st1 ? s + 1 : s, true, any);  // (past the end: the last one again, never used)
         }
         if (last && nfull < steps) {
             load_w(nfull, true);
 #pragma unroll
-            for (int b = 0; b < 4; b++) load_a(b, nfull, true);
+            for (int b = 0; b < NB; b++) load_a(b, nfull, true);
             step(0, false, any);
         }
     };
@@ -311,39 +285,36 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
         // a non-finite value has no finite terms and left a NaN in its row: once more, with such values as they are
         bool bad = false;
 #pragma unroll
-        for (int b = 0; b < 4; b++)
+        for (int b = 0; b < NB; b++)
 #pragma unroll
             for (int t = 0; t < 4 * NG; t++)
 #pragma unroll
                 for (int r = 0; r < 4; r++) bad |= acc[b][t][r] != acc[b][t][r];
         if (__any(bad)) contract(std::true_type{});
     }
-    if (KS > 1 || fine) {
-        // the upper half of the waves hands its sums to the lower half, until the first wave of a tile has them all; NG words of 16 KiB each
-        constexpr int KW = KS > 1 ? KS : REM ? 4 : 1;
-        __shared__ __attribute__((aligned(16))) float xch[KW > 1 ? KW / 2 * 4096 * NG : 1];
-        const int least = KS > 1 || parts == 4 ? 1 : 2;  // (parts == 2: waves 2 and 3 are the other halves of waves 0 and 1)
+    if constexpr (KS > 1) {
+        // the upper half of the waves hands its sums to the lower half, until wave 0 has them all; NG words of 16 KiB each
+        __shared__ __attribute__((aligned(16))) float xch[KS / 2 * 4096 * NG];
 #pragma unroll
-        for (int half = KW / 2; half >= 1; half /= 2) {
-            if (half < least) break;  // (uniform)
+        for (int half = KS / 2; half >= 1; half /= 2) {
             if (wave >= half && wave < 2 * half) {
 #pragma unroll
-                for (int b = 0; b < 4; b++)
+                for (int b = 0; b < NB; b++)
 #pragma unroll
                     for (int t = 0; t < 4 * NG; t++)
-                        *(v4f*)(xch + ((((wave - half) * 4 + b) * 4 * NG + t) * 64 + lane) * 4) = acc[b][t];
+                        *(v4f*)(xch + ((((wave - half) * NB + b) * 4 * NG + t) * 64 + lane) * 4) = acc[b][t];
             }
             __syncthreads();
             if (wave < half) {
 #pragma unroll
-                for (int b = 0; b < 4; b++)
+                for (int b = 0; b < NB; b++)
 #pragma unroll
                     for (int t = 0; t < 4 * NG; t++)
-                        acc[b][t] += *(const v4f*)(xch + (((wave * 4 + b) * 4 * NG + t) * 64 + lane) * 4);
+                        acc[b][t] += *(const v4f*)(xch + (((wave * NB + b) * 4 * NG + t) * 64 + lane) * 4);
             }
             __syncthreads();
         }
-        if (wave >= least) return;
+        if (wave != 0) return;
     }
 
 #pragma unroll
@@ -360,7 +331,7 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
             }
         }
 #pragma unroll
-        for (int b = 0; b < 4; b++) {
+        for (int b = 0; b < NB; b++) {
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int64_t m = m0 + 16 * b + 4 * g + r;
@@ -399,11 +370,47 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
     }
 }
 
+// KS = 1: the four waves of a workgroup are a 2 x 2 block of tiles of 64 rows.  KS > 1: see gemm_f32_tile.
+// PARTS > 1 (KS = 1): a tile of the remainder, the last that would occupy a part of the compute units only, is shared by PARTS
+// workgroups, whose waves take 32 or 16 rows each over the whole contraction: every output is the same chain of products as in a
+// tile of its own, so that a row's bits do not depend on where it lies in the call.
+template <int SRC, int NG, int KS, bool SC, bool RN, int PARTS>
+__global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(GemmF32Params p) {
+    constexpr int TM = (KS == 1) ? 128 : 64, TN = (KS == 1) ? 128 * NG : 64 * NG;  // a workgroup's tile
+    // the 8 XCDs each take a contiguous run of tiles, walked in groups of four row tiles (as in gemm_f16.hip)
+    const uint32_t idx = blockIdx.x >> 3;
+    const bool fine = PARTS > 1 && idx >= (uint32_t)p.fine_from;  // (uniform)
+    const uint32_t f = fine ? idx - (uint32_t)p.fine_from : 0u, part = f % (uint32_t)PARTS;
+    const uint32_t lin = (blockIdx.x & 7u) * (uint32_t)p.per_xcd + (fine ? (uint32_t)p.fine_from + f / (uint32_t)PARTS : idx);
+    const uint32_t tiles_m = (uint32_t)p.tiles_m, tiles_n = (uint32_t)p.tiles_n;
+    if (lin >= tiles_m * tiles_n) return;
+    constexpr uint32_t GM = 4;
+    const uint32_t group = lin / (GM * tiles_n), first_m = group * GM;
+    const uint32_t gm = (tiles_m - first_m < GM) ? tiles_m - first_m : GM;
+    const uint32_t in_group = lin - group * GM * tiles_n;
+    const uint32_t tn = (gm == GM) ? in_group / GM : in_group / gm;
+    const uint32_t tm = first_m + (in_group - tn * gm);
+
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t c0 = (int64_t)tn * TN + (KS == 1 ? 64 * NG * (wave & 1) : 0);
+    if constexpr (PARTS > 1) {
+        if (fine) {
+            constexpr int NB = 4 / PARTS;
+            const int64_t m0 = (int64_t)tm * TM + 16 * NB * (2 * (int)part + (wave >> 1));
+            if (m0 < p.M && c0 < p.NC) gemm_f32_tile<SRC, NG, NB, KS, SC, RN>(p, m0, c0);
+            return;
+        }
+    }
+    const int64_t m0 = (int64_t)tm * TM + (KS == 1 ? 64 * (wave >> 1) : 0);
+    if (KS == 1 && (m0 >= p.M || c0 >= p.NC)) return;  // (no barriers in a tile when KS == 1)
+    gemm_f32_tile<SRC, NG, 4, KS, SC, RN>(p, m0, c0);
+}
+
 // Into how many workgroups a tile of the remainder is shared (KS = 1): the tiles beyond one, two ... for every compute unit of an XCD
-// where they are at most half as many as compute units.  A shared tile saves half or three quarters of its steps at 1.2 us each and
-// costs 4 us for the sums' way through LDS.  (The plan is made without regard to it: where one with the contraction over four waves
-// was the cheaper, its sums are shorter ones too.)  us, before / now: 16384 x 768 x 768 forward 67.4 / 55.8, input gradient 75.1 / 64.7;
-// 9000 x 2304 x 768 90.9 / 80.6.
+// where they are at most half as many as compute units, so that half or three quarters of such a tile's time are saved.  (The plan is
+// made without regard to it.)  us, tiles of their own / shared: 16384 x 768 x 768 forward 68.8 / 61.0, input gradient 70.9 / 65.5; 9000 x
+// 2304 x 768 forward 93.5 / 86.5; four workgroups, 33792 x 256 x 1024 input gradient 71.5 / 63.6.  Less than 4 us of steps at 1.2 us each
+// are not missed: 16384 x 768 x 192 23.9 / 23.8, 49000 x 256 x 160 22.0 / 22.2.
 static int gemm_f32_parts(int64_t tiles, int64_t steps) {
     const int64_t cus = gemm_compute_units() / 8, per_xcd = ceil_div(tiles, 8), rem = per_xcd % cus;
     if (per_xcd < cus || rem == 0 || 2 * rem > cus) return 1;
@@ -420,17 +427,16 @@ static int launch_gemm_f32_cfg(GemmF32Params p, const char* who, hipStream_t st)
         return BT_ERR_INVALID;
     }
     p.per_xcd = (int)ceil_div(total, 8);
-    p.parts = KS == 1 ? gemm_f32_parts(total, ceil_div(p.C, 32)) : 1;
-    const int rem = p.parts > 1 ? p.per_xcd % (int)(gemm_compute_units() / 8) : 0;
+    const int parts = KS == 1 ? gemm_f32_parts(total, ceil_div(p.C, 32)) : 1;
+    const int rem = parts > 1 ? p.per_xcd % (int)(gemm_compute_units() / 8) : 0;
     p.fine_from = p.per_xcd - rem;
-    const dim3 grid((unsigned)(8 * (p.fine_from + p.parts * rem))), block(KS == 1 ? 256 : 64 * KS);
+    const dim3 grid((unsigned)(8 * (p.fine_from + parts * rem))), block(KS == 1 ? 256 : 64 * KS);
     if constexpr (KS == 1) {
-        if (rem > 0) {
-            hipLaunchKernelGGL((gemm_f32_kernel<SRC, NG, KS, SC, RN, true>), grid, block, 0, st, p);
-            return check_launch(who);
-        }
+        if (parts == 2) hipLaunchKernelGGL((gemm_f32_kernel<SRC, NG, KS, SC, RN, 2>), grid, block, 0, st, p);
+        if (parts == 4) hipLaunchKernelGGL((gemm_f32_kernel<SRC, NG, KS, SC, RN, 4>), grid, block, 0, st, p);
+        if (parts > 1) return check_launch(who);
     }
-    hipLaunchKernelGGL((gemm_f32_kernel<SRC, NG, KS, SC, RN, false>), grid, block, 0, st, p);
+    hipLaunchKernelGGL((gemm_f32_kernel<SRC, NG, KS, SC, RN, 1>), grid, block, 0, st, p);
     return check_launch(who);
 }
 // Which split of the work?  0: tiles of 64 x 128 per wave, 1: the same with the contraction over the four waves of a

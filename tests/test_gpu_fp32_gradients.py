@@ -259,10 +259,12 @@ def test_fp32_forward_without_a_workspace(m, n, k):
 
 
 @gpu
-@pytest.mark.parametrize("m,n,k", [(33700, 250, 200), (33792, 120, 196), (49000, 256, 232), (34000, 510, 254)])
-def test_fp32_remainder_tiles_shared_by_waves(m, n, k):
-    """33 tiles of 128 x 256 an XCD leave one, 48 leave sixteen: each is shared by four or two workgroups whose waves split the
-    contraction.  Rows that end inside the last tile, one wave tile of columns, column halves past the end, a partial step."""
+@pytest.mark.parametrize("m,n,k", [(33700, 250, 200), (33792, 120, 196), (49000, 256, 232), (34000, 510, 254), (49000, 120, 256),
+                                   (49000, 118, 256), (49000, 256, 118)])
+def test_fp32_remainder_tiles_shared_by_workgroups(m, n, k):
+    """33 tiles of 128 x 256 an XCD leave one, 48 leave sixteen: each is shared by four or two workgroups of 32 or 64 rows.  Rows that
+    end inside the last tile, the right half of the columns past the end (forward and input gradient, both numbers of workgroups,
+    N % 4 != 0 too), a partial step."""
     from bittorch_amd import _C
     announce("fp32 remainder tiles", m, n, k)
     x, dy, packed, scale, tern = _case(m, n, k)
@@ -277,3 +279,17 @@ def test_fp32_remainder_tiles_shared_by_waves(m, n, k):
     for r in rows:
         assert torch.equal(got[r].isnan(), want[r].isnan()) and torch.equal(got[r].isinf(), want[r].isinf())
     assert torch.isfinite(got[[0, 6, m - 2]]).all()
+
+
+@gpu
+@pytest.mark.parametrize("m,n,k", [(33792, 120, 224), (49000, 256, 232), (49000, 118, 256), (16384, 768, 768)])
+def test_fp32_rows_are_summed_alike_wherever_they_lie(m, n, k):
+    """Equal rows of a call have equal bits, in tiles of their own and in shared ones, forward and input gradient."""
+    from bittorch_amd import _C
+    announce("fp32 equal rows", m, n, k)
+    x, dy, packed, scale, _ = _case(m, n, k)
+    place = torch.arange(m, device="cuda") % 8
+    x, dy = x[:8][place].contiguous(), dy[:8][place].contiguous()
+    for y in (_C.linear_grad_input(dy, packed, scale, k), _C.ternary_linear_packed_forward(x, packed, scale, None, k),
+              _C.ternary_linear_tiled_forward(x, _C.retile_weights(packed, k), scale, None, k, n)):
+        assert torch.equal(y, y[:8][place])
