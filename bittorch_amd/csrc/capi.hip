@@ -1051,6 +1051,7 @@ extern "C" int bt_ternary_gemm_i8_tiled(const int8_t* Q, int q_layout, const flo
                         scale_len, bias, bias_dtype, residual, Y, y_dtype, acc_out, B, N, K, stream);
 }
 
+// What the SwiGLU output stage of the tiled int8 GEMM takes (null pointers: of the sizes alone).
 static bool swiglu_i8_ok(int64_t N, int64_t K, const void* Q, const void* W_tiled, const void* Y) {
     return N % 32 == 0 && K <= kMaxKInt8 && fast_path_ok(Y, N, K) && stream_supported_tiled(N, K, W_tiled) && gemm_i8_supported_tiled(N, K, Q, true);
 }
@@ -1082,7 +1083,7 @@ extern "C" int bt_ternary_swiglu_i8_tiled(const int8_t* Q, const float* s_x, con
 // 12.6 / 12.0.  Few rows are cheaper on the streaming kernel or few_rows_kernel (64 x 5632 x 1024 8.0 / 10.3), and up to 256 rows also on
 // gemm_i8_kernel where that is the choice (256 x 22016 x 4096 31.2 / 33.4, but 384 x 13824 x 2560 26.9 / 24.9).
 extern "C" int bt_swiglu_i8_tiled_pays(int64_t B, int64_t N, int64_t K) {
-    if (B <= 0 || N <= 0 || K <= 0 || N % 32 != 0 || K % 16 != 0) return 0;
+    if (B <= 0 || N <= 0 || K <= 0 || !swiglu_i8_ok(N, K, nullptr, nullptr, nullptr)) return 0;
     if (prefers_rows(true, false, B, N, K) || prefers_stream(B, N, K, true, true, true)) return 0;
     return B > 256 || gemm_i8_dma_rows(B, N, K, true, false) != 0;
 }

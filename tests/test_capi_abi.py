@@ -85,6 +85,19 @@ def test_tensor_core_forward_refuses_misaligned_weights_of_any_size(n, k):
     assert "16-byte aligned" in _lib.last_error()
 
 
+@pytest.mark.parametrize("n,k,taken", [(13824, 2560, True), (2 ** 26 - 32, 128, True), (2 ** 26, 128, False), (13824 + 16, 2560, False),
+                                       (13824, 2568, False), (1024, 132096, True), (1024, 132112, False), (2 ** 20, 16384, False)])
+def test_int8_swiglu_stage_pays_only_where_it_is_taken(n, k, taken):
+    """From 2^26 columns, 132097 values or 4 GiB of weights on, and for N % 32 or K % 16 != 0, the call is refused, so it pays nowhere."""
+    from bittorch_amd import _lib
+    lib = _lib.load()
+    rows = 100000
+    assert lib.bt_swiglu_i8_tiled_pays(rows, n, k) == int(taken)
+    if not taken:
+        addr = 1 << 20  # (never read: the call ends before any launch)
+        assert lib.bt_ternary_swiglu_i8_tiled(addr, addr, addr, addr, 0, 1, None, 0, addr, 2, rows, n, k, None) == -1
+
+
 def test_extension_probes_are_truthful():
     import bittorch_amd as bt
     from bittorch_amd.nn.ternary_linear import _cuda_kernel_available
