@@ -14,6 +14,7 @@ from typing import Optional
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # BITTORCH_HIP_LIBRARY points at another build of the library (A/B comparisons)
 LIB_PATH = os.environ.get("BITTORCH_HIP_LIBRARY") or os.path.join(_HERE, "_hip", "libbittorch_hip.so")
+CALLS_PATH = os.path.join(_HERE, "_hip", "_calls.so")
 
 ABI_VERSION = 2
 
@@ -93,7 +94,7 @@ def load() -> ctypes.CDLL:
     if not os.path.exists(LIB_PATH):
         raise ImportError(
             f"{LIB_PATH} is missing: build it with `python -m bittorch_amd.build` "
-            "(needs hipcc; cross-compiles for gfx950 without a GPU)")
+            "(needs hipcc, and for the native host side of the calls g++ and torch's headers; cross-compiles for gfx950 without a GPU)")
     try:
         lib = ctypes.CDLL(LIB_PATH)
     except OSError as exc:  # e.g. libamdhip64 not found
@@ -111,22 +112,60 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+def calls_build() -> str:
+    """This build of torch and this Python, as ``_calls.so`` names them."""
+    import sys
+
+    import torch
+    return f"torch {torch.__version__} {torch.version.git_version}, python {sys.version_info[0]}.{sys.version_info[1]}"
+
+
+class _PythonCalls:
+    """In the place of ``_calls.so``: no call is an ordinary one, so the functions of ``_C`` do all of them."""
+
+    @staticmethod
+    def generic_kernel_asked() -> bool:
+        return os.environ.get("BITTORCH_KERNEL") == "generic"
+
+    def __getattr__(self, name: str):
+        return lambda *args: None
+
+
 def load_calls():
-    """``_hip/_calls.so``, the native host side of the calls (``csrc/calls.cpp``), bound to the loaded library."""
+    """``_hip/_calls.so``, the native host side of the calls (``csrc/calls.cpp``), bound to the loaded library.  Where it is missing,
+    does not load or was compiled against something else, a stand-in that leaves every call to Python, with a warning: the results are
+    the same, small calls take about twice as long."""
     global _calls
     if _calls is None:
-        import importlib.util
-
-        path = os.path.join(_HERE, "_hip", "_calls.so")
-        if not os.path.exists(path):
-            raise ImportError(f"{path} is missing: build it with `python -m bittorch_amd.build`")
         lib = load()
-        spec = importlib.util.spec_from_file_location("bittorch_amd._hip._calls", path)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-        module.bind({name: ctypes.cast(getattr(lib, name), _vp).value for name in module.names()})
-        _calls = module
+        try:
+            _calls = _native_calls(lib, CALLS_PATH)
+        except ImportError as exc:
+            import warnings
+
+            warnings.warn(f"{exc}; small calls run in Python until `python -m bittorch_amd.build` has built it (g++, torch's headers)",
+                          RuntimeWarning, stacklevel=2)
+            _calls = _PythonCalls()
     return _calls
+
+
+def _native_calls(lib: ctypes.CDLL, path: str):
+    import importlib.util
+
+    if not os.path.exists(path):
+        raise ImportError(f"{path} is missing")
+    spec = importlib.util.spec_from_file_location("bittorch_amd._hip._calls", path)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    # (asked for before anything else of it is called)
+    got, want = getattr(module, "stamp", lambda: "an unknown build")(), f"abi {ABI_VERSION}, {calls_build()}"
+    if got != want:
+        raise ImportError(f"{path} was compiled against {got}, not {want}")
+    try:
+        module.bind({name: ctypes.cast(getattr(lib, name), _vp).value for name in module.names()})
+    except AttributeError as exc:
+        raise ImportError(f"{path} wants a function that the library does not export ({exc})") from exc
+    return module
 
 
 def last_error() -> str:

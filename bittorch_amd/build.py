@@ -49,16 +49,30 @@ def _hipcc() -> str:
 
 
 def build_calls() -> str:
-    """Compile ``csrc/calls.cpp`` (host code only) against the installed torch into ``_hip/_calls.so``; returns its path."""
+    """Compile ``csrc/calls.cpp`` (host code only) against the installed torch into ``_hip/_calls.so``; returns its path.  Needs g++ and
+    torch with its headers.  Raises, and leaves no earlier one in its place, where it cannot be built."""
     import sysconfig
 
-    import torch
-    from torch.utils.cpp_extension import include_paths, library_paths
-
     out = os.path.join(OUT_DIR, "_calls.so")
+    if os.path.exists(out):
+        os.remove(out)
+    gxx = shutil.which("g++")
+    if gxx is None:
+        raise RuntimeError("g++ not found; _calls.so cannot be built")
+    try:
+        import torch
+        from torch.utils.cpp_extension import include_paths, library_paths
+    except ImportError as exc:
+        raise RuntimeError(f"torch cannot be imported ({exc}); _calls.so cannot be built") from exc
+
+    try:
+        from ._lib import calls_build
+    except ImportError:  # (this file run by its path)
+        from _lib import calls_build
+
     libs = library_paths()
-    cmd = [shutil.which("g++") or "g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+    cmd = [gxx, "-O2", "-fPIC", "-shared", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DBT_CALLS_BUILD="{calls_build()}"',
            *(f"-I{p}" for p in include_paths()), f"-I{sysconfig.get_paths()['include']}",
            f"-I{os.path.join(os.environ.get('ROCM_PATH', '/opt/rocm'), 'include')}", os.path.join(CSRC, "calls.cpp"), "-o", out,
            *(f"-L{p}" for p in libs), *(f"-Wl,-rpath,{p}" for p in libs), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
@@ -68,8 +82,9 @@ def build_calls() -> str:
     return out
 
 
-def build(verbose: bool = False, extra_flags=()) -> str:
-    """Compile every kernel source and link the shared library, and the native host side of the calls; returns the library's path."""
+def build(verbose: bool = False, extra_flags=(), need_calls: bool = False) -> str:
+    """Compile every kernel source and link the shared library, and the native host side of the calls; returns the library's path.
+    The library is complete without the latter (``need_calls`` says that it has to be there): small calls then take longer."""
     os.makedirs(OUT_DIR, exist_ok=True)
     hipcc = _hipcc()
     objs = []
@@ -88,11 +103,16 @@ def build(verbose: bool = False, extra_flags=()) -> str:
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
         calls = pool.submit(build_calls)
         objs = list(pool.map(compile_one, SOURCES))
-        calls.result()
     cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc link failed:\n{res.stdout}\n{res.stderr}")
+    try:
+        calls.result()
+    except Exception as exc:
+        if need_calls:
+            raise
+        print(f"{LIB_PATH} is built, the native host side of its calls is not (they run in Python): {exc}", file=sys.stderr)
     return LIB_PATH
 
 

@@ -536,6 +536,12 @@ PyObject* generic_kernel_asked(PyObject*, PyObject* const*, Py_ssize_t) {
     return PyBool_FromLong(env && !std::strcmp(env, "generic"));
 }
 
+// stamp(): what this file was compiled against.  Its accessors are inlined from torch's headers and its calls typed by
+// bittorch_hip.h, so _lib.py binds it to that build of torch and that ABI alone.
+#define BT_TEXT(x) #x
+#define BT_TEXT_OF(x) BT_TEXT(x)
+PyObject* stamp(PyObject*, PyObject* const*, Py_ssize_t) { return PyUnicode_FromString("abi " BT_TEXT_OF(BT_ABI_VERSION) ", " BT_CALLS_BUILD); }
+
 // bind({name: address}): the library's functions
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     if (n_args != 1 || !PyDict_Check(a[0])) {
@@ -573,7 +579,7 @@ PyObject* names(PyObject*, PyObject* const*, Py_ssize_t) {
 }
 
 #define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(name)), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {METHOD(bind), METHOD(names), METHOD(tiled_forward), METHOD(packed_forward), METHOD(tensor_core_forward),
+PyMethodDef methods[] = {METHOD(bind), METHOD(names), METHOD(stamp), METHOD(tiled_forward), METHOD(packed_forward), METHOD(tensor_core_forward),
                          METHOD(quantize_pack), METHOD(grad_input), METHOD(grad_weight),
                          METHOD(grad_weight_16), METHOD(unpack_dequant), METHOD(rmsnorm_int8), METHOD(swiglu_int8), METHOD(gemm_i8_tiled), METHOD(swiglu_i8_tiled), METHOD(act_quant_int8),
                          METHOD(generic_kernel_asked), {nullptr, nullptr, 0, nullptr}};
