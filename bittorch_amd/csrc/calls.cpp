@@ -23,6 +23,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
+#include <type_traits>
 
 #include "../../include/bittorch_hip.h"
 
@@ -93,14 +94,18 @@ struct Scratch {  // of one call
 };
 void* stream_of(int device) { return c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream(); }
 
-// The library's call without the interpreter lock, as through ctypes.
-template <typename F>
-void call(F f) {
+struct Unlocked {  // the interpreter, until the end of the block however it is left
+    PyThreadState* const state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+// The library's call without the interpreter lock, as through ctypes.  Its arguments are values: what they are read from (tensors, whose
+// accessors may throw and which other threads may point elsewhere) is asked under the lock.
+template <typename... P>
+void call(int (*f)(P...), std::common_type_t<P>... args) {
     int rc;
     {
-        PyThreadState* state = PyEval_SaveThread();
-        rc = f();
-        PyEval_RestoreThread(state);
+        const Unlocked unlocked;
+        rc = f(args...);
     }
     if (rc != 0) {
         const char* text = lib.bt_last_error();
@@ -194,12 +199,10 @@ PyObject* tiled_forward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     at::Tensor y = output(with_last(*x, Ny), x->scalar_type(), *x);
     const Scratch ws(op == 0 && !pairs ? lib.bt_tiled_forward_workspace_bytes(B, N, K, dt) : lib.bt_packed_forward_fused_workspace_bytes(B, N, K, dt), *x);
     void* st = stream_of(device);
-    call([&] {
-        return lib.bt_ternary_linear_tiled_forward(
-            x->const_data_ptr(), K, dt, op, pro ? pro->const_data_ptr() : nullptr, op == 2 ? K : 0, (float)eps, (const uint8_t*)w->const_data_ptr(),
-            scale->const_data_ptr(), tag(scale->scalar_type()), scale->numel(), bias ? bias->const_data_ptr() : nullptr,
-            bias ? tag(bias->scalar_type()) : 0, res ? res->const_data_ptr() : nullptr, epi, y.data_ptr(), B, N, K, ws.ptr(), ws.size(), st);
-    });
+    call(lib.bt_ternary_linear_tiled_forward, x->const_data_ptr(), K, dt, op, pro ? pro->const_data_ptr() : nullptr,
+        op == 2 ? K : 0, (float)eps, (const uint8_t*)w->const_data_ptr(), scale->const_data_ptr(), tag(scale->scalar_type()),
+        scale->numel(), bias ? bias->const_data_ptr() : nullptr, bias ? tag(bias->scalar_type()) : 0,
+        res ? res->const_data_ptr() : nullptr, epi, y.data_ptr(), B, N, K, ws.ptr(), ws.size(), st);
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS
 }
@@ -228,11 +231,9 @@ PyObject* packed_forward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     at::Tensor y = output(with_last(*x, N), x->scalar_type(), *x);
     const Scratch ws(lib.bt_packed_forward_workspace_bytes(B, N, K, dt), *x);
     void* st = stream_of(device);
-    call([&] {
-        return lib.bt_ternary_linear_packed_forward(x->const_data_ptr(), dt, (const uint8_t*)w->const_data_ptr(), scale->const_data_ptr(),
-                                                    tag(scale->scalar_type()), scale->numel(), bias ? bias->const_data_ptr() : nullptr,
-                                                    bias ? tag(bias->scalar_type()) : 0, y.data_ptr(), B, N, K, ws.ptr(), ws.size(), st);
-    });
+    call(lib.bt_ternary_linear_packed_forward, x->const_data_ptr(), dt, (const uint8_t*)w->const_data_ptr(),
+        scale->const_data_ptr(), tag(scale->scalar_type()), scale->numel(), bias ? bias->const_data_ptr() : nullptr,
+        bias ? tag(bias->scalar_type()) : 0, y.data_ptr(), B, N, K, ws.ptr(), ws.size(), st);
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS
 }
@@ -254,12 +255,9 @@ PyObject* tensor_core_forward(PyObject*, PyObject* const* a, Py_ssize_t n_args) 
     at::Tensor y = output({B, N}, x->scalar_type(), *x);
     const Scratch ws(lib.bt_tensor_core_workspace_bytes(B, N, K), *x);
     void* st = stream_of(device);
-    call([&] {
-        return lib.bt_ternary_linear_tensor_core_forward(x->const_data_ptr(), tag(x->scalar_type()), (const uint8_t*)w->const_data_ptr(),
-                                                         scale->const_data_ptr(), tag(scale->scalar_type()), scale->numel(),
-                                                         bias ? bias->const_data_ptr() : nullptr, bias ? tag(bias->scalar_type()) : 0,
-                                                         y.data_ptr(), B, N, K, ws.ptr(), ws.size(), st);
-    });
+    call(lib.bt_ternary_linear_tensor_core_forward, x->const_data_ptr(), tag(x->scalar_type()), (const uint8_t*)w->const_data_ptr(),
+        scale->const_data_ptr(), tag(scale->scalar_type()), scale->numel(), bias ? bias->const_data_ptr() : nullptr,
+        bias ? tag(bias->scalar_type()) : 0, y.data_ptr(), B, N, K, ws.ptr(), ws.size(), st);
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS
 }
@@ -278,10 +276,8 @@ PyObject* quantize_pack(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     at::Tensor packed = output({(K + 3) / 4, N}, at::kByte, *w), scale = output({per_channel ? N : 1}, at::kFloat, *w);
     void* st = stream_of(device);
     constexpr int kF32AsF16 = 4;
-    call([&] {
-        return lib.bt_quantize_pack(w->const_data_ptr(), as_half ? kF32AsF16 : tag(w->scalar_type()), N, K, threshold, per_channel ? 1 : 0,
-                                    (uint8_t*)packed.data_ptr(), (float*)scale.data_ptr(), nullptr, st);
-    });
+    call(lib.bt_quantize_pack, w->const_data_ptr(), as_half ? kF32AsF16 : tag(w->scalar_type()), N, K, threshold,
+        per_channel ? 1 : 0, (uint8_t*)packed.data_ptr(), (float*)scale.data_ptr(), nullptr, st);
     const at::ScalarType dtype = as_half ? at::kHalf : w->scalar_type();
     if (dtype != at::kFloat) scale = scale.to(dtype);
     if (!per_channel) scale = scale.squeeze(0);
@@ -308,10 +304,8 @@ PyObject* grad_input(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     ORDINARY(w && w->size(1) == N && scale && scale->scalar_type() == at::kFloat && (scale->numel() == N || scale->numel() == 1));
     at::Tensor out = output({M, K}, at::kFloat, *dy);
     void* st = stream_of(device);
-    call([&] {
-        return lib.bt_ternary_linear_grad_input((const float*)dy->const_data_ptr(), (const uint8_t*)w->const_data_ptr(),
-                                                (const float*)scale->const_data_ptr(), scale->numel(), (float*)out.data_ptr(), M, N, K, st);
-    });
+    call(lib.bt_ternary_linear_grad_input, (const float*)dy->const_data_ptr(), (const uint8_t*)w->const_data_ptr(),
+        (const float*)scale->const_data_ptr(), scale->numel(), (float*)out.data_ptr(), M, N, K, st);
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
@@ -332,11 +326,9 @@ PyObject* grad_weight(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     if (want_bias) db = output({N}, at::kFloat, *dy);
     const Scratch ws(lib.bt_linear_grad_weight_workspace_bytes(M, N, K), *dy);
     void* st = stream_of(device);
-    call([&] {
-        return lib.bt_linear_grad_weight((const float*)dy->const_data_ptr(), (const float*)x->const_data_ptr(), (const float*)scale->const_data_ptr(),
-                                         scale->numel(), (float*)dw.data_ptr(), want_bias ? (float*)db.data_ptr() : nullptr, M, N, K,
-                                         ws.ptr(), ws.size(), st);
-    });
+    call(lib.bt_linear_grad_weight, (const float*)dy->const_data_ptr(), (const float*)x->const_data_ptr(),
+        (const float*)scale->const_data_ptr(), scale->numel(), (float*)dw.data_ptr(), want_bias ? (float*)db.data_ptr() : nullptr,
+        M, N, K, ws.ptr(), ws.size(), st);
     PyObject* out = PyTuple_New(2);
     if (!out) return nullptr;
     PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(std::move(dw)));
@@ -374,12 +366,10 @@ PyObject* gemm_i8_tiled(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     }
     at::Tensor y = output({B, N}, dtype, *q);
     void* st = stream_of(device);
-    call([&] {
-        return lib.bt_ternary_gemm_i8_tiled((const int8_t*)q->const_data_ptr(), oo ? 1 : 0, (const float*)sx->const_data_ptr(),
-                                            (const uint8_t*)w->const_data_ptr(), scale->const_data_ptr(), tag(scale->scalar_type()), scale->numel(),
-                                            bias ? bias->const_data_ptr() : nullptr, bias ? tag(bias->scalar_type()) : 0,
-                                            res ? res->const_data_ptr() : nullptr, y.data_ptr(), tag(dtype), nullptr, B, N, K, st);
-    });
+    call(lib.bt_ternary_gemm_i8_tiled, (const int8_t*)q->const_data_ptr(), oo ? 1 : 0, (const float*)sx->const_data_ptr(),
+        (const uint8_t*)w->const_data_ptr(), scale->const_data_ptr(), tag(scale->scalar_type()), scale->numel(),
+        bias ? bias->const_data_ptr() : nullptr, bias ? tag(bias->scalar_type()) : 0, res ? res->const_data_ptr() : nullptr,
+        y.data_ptr(), tag(dtype), nullptr, B, N, K, st);
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS
 }
@@ -402,12 +392,9 @@ PyObject* swiglu_i8_tiled(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     if (a[4] != Py_None) ORDINARY((bias = vec(a[4], N, false, device)));
     at::Tensor h = output({B, N / 2}, dtype, *q);
     void* st = stream_of(device);
-    call([&] {
-        return lib.bt_ternary_swiglu_i8_tiled((const int8_t*)q->const_data_ptr(), (const float*)sx->const_data_ptr(), (const uint8_t*)w->const_data_ptr(),
-                                              scale->const_data_ptr(), tag(scale->scalar_type()), scale->numel(),
-                                              bias ? bias->const_data_ptr() : nullptr, bias ? tag(bias->scalar_type()) : 0, h.data_ptr(), tag(dtype),
-                                              B, N, K, st);
-    });
+    call(lib.bt_ternary_swiglu_i8_tiled, (const int8_t*)q->const_data_ptr(), (const float*)sx->const_data_ptr(),
+        (const uint8_t*)w->const_data_ptr(), scale->const_data_ptr(), tag(scale->scalar_type()), scale->numel(),
+        bias ? bias->const_data_ptr() : nullptr, bias ? tag(bias->scalar_type()) : 0, h.data_ptr(), tag(dtype), B, N, K, st);
     return THPVariable_Wrap(std::move(h));
     END_HANDLE_TH_ERRORS
 }
@@ -427,10 +414,8 @@ PyObject* grad_weight_16(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     at::Tensor out = output({N, K}, dtype, *dy);
     const Scratch ws(lib.bt_linear_grad_weight_16_workspace_bytes(M, N, K), *dy);
     void* st = stream_of(device);
-    call([&] {
-        return lib.bt_linear_grad_weight_16(dy->const_data_ptr(), x->const_data_ptr(), tag(dy->scalar_type()), scale->const_data_ptr(),
-                                            tag(scale->scalar_type()), scale->numel(), out.data_ptr(), tag(dtype), M, N, K, ws.ptr(), ws.size(), st);
-    });
+    call(lib.bt_linear_grad_weight_16, dy->const_data_ptr(), x->const_data_ptr(), tag(dy->scalar_type()), scale->const_data_ptr(),
+        tag(scale->scalar_type()), scale->numel(), out.data_ptr(), tag(dtype), M, N, K, ws.ptr(), ws.size(), st);
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
@@ -459,9 +444,8 @@ PyObject* act_quant_int8(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const int64_t B = x->size(0), K = x->size(1);
     at::Tensor q = output({B, K}, at::kChar, *x), s = output({B}, at::kFloat, *x);
     void* st = stream_of(device);
-    call([&] {
-        return lib.bt_act_quant_i8_layout(x->const_data_ptr(), tag(x->scalar_type()), B, K, (int8_t*)q.data_ptr(), (float*)s.data_ptr(), oo ? 1 : 0, st);
-    });
+    call(lib.bt_act_quant_i8_layout, x->const_data_ptr(), tag(x->scalar_type()), B, K, (int8_t*)q.data_ptr(), (float*)s.data_ptr(),
+        oo ? 1 : 0, st);
     return int8_rows(std::move(q), std::move(s));
     END_HANDLE_TH_ERRORS
 }
@@ -483,10 +467,8 @@ PyObject* rmsnorm_int8(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     }
     at::Tensor q = output({B, K}, at::kChar, *x), s = output({B}, at::kFloat, *x);
     void* st = stream_of(device);
-    call([&] {
-        return lib.bt_rmsnorm(x->const_data_ptr(), K, w ? w->const_data_ptr() : nullptr, (float)eps, tag(x->scalar_type()), B, K, nullptr,
-                              (int8_t*)q.data_ptr(), (float*)s.data_ptr(), oo ? 1 : 0, st);
-    });
+    call(lib.bt_rmsnorm, x->const_data_ptr(), K, w ? w->const_data_ptr() : nullptr, (float)eps, tag(x->scalar_type()), B, K,
+        nullptr, (int8_t*)q.data_ptr(), (float*)s.data_ptr(), oo ? 1 : 0, st);
     return int8_rows(std::move(q), std::move(s));
     END_HANDLE_TH_ERRORS
 }
@@ -502,10 +484,8 @@ PyObject* swiglu_int8(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const int64_t B = g->size(0), K = g->size(1);
     at::Tensor q = output({B, K}, at::kChar, *g), s = output({B}, at::kFloat, *g);
     void* st = stream_of(device);
-    call([&] {
-        return lib.bt_swiglu(g->const_data_ptr(), g->stride(0), u->const_data_ptr(), u->stride(0), tag(g->scalar_type()),
-                             B, K, nullptr, (int8_t*)q.data_ptr(), (float*)s.data_ptr(), oo ? 1 : 0, st);
-    });
+    call(lib.bt_swiglu, g->const_data_ptr(), g->stride(0), u->const_data_ptr(), u->stride(0), tag(g->scalar_type()), B, K, nullptr,
+        (int8_t*)q.data_ptr(), (float*)s.data_ptr(), oo ? 1 : 0, st);
     return int8_rows(std::move(q), std::move(s));
     END_HANDLE_TH_ERRORS
 }
@@ -522,10 +502,8 @@ PyObject* unpack_dequant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const at::Tensor scale_f = scale->scalar_type() == at::kFloat ? *scale : scale->detach().to(at::kFloat);
     at::Tensor out = output({w->size(1), K}, dtype, *w);
     void* st = stream_of(device);
-    call([&] {
-        return lib.bt_unpack_dequant((const uint8_t*)w->const_data_ptr(), (const float*)scale_f.const_data_ptr(), scale_f.numel(), out.data_ptr(),
-                                     tag(dtype), w->size(1), K, st);
-    });
+    call(lib.bt_unpack_dequant, (const uint8_t*)w->const_data_ptr(), (const float*)scale_f.const_data_ptr(), scale_f.numel(),
+        out.data_ptr(), tag(dtype), w->size(1), K, st);
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }

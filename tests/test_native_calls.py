@@ -1,6 +1,8 @@
 """The native host side of the calls takes GPU tensors alone, and is bound to the library that is loaded; the package works
 without it."""
 import importlib.util
+import os
+import re
 import types
 
 import pytest
@@ -34,6 +36,15 @@ def test_generic_kernel_is_read_on_every_call(monkeypatch):
     assert not _C._N.generic_kernel_asked()
     monkeypatch.delenv("BITTORCH_KERNEL")
     assert not _C._N.generic_kernel_asked()
+
+
+def test_tensors_are_read_under_the_interpreter_lock():
+    """Between letting go of the lock and taking it back, by a destructor, there is the library's call with values alone."""
+    source = open(os.path.join(build.CSRC, "calls.cpp")).read()
+    assert source.count("PyEval_SaveThread") == source.count("PyEval_RestoreThread") == 1
+    assert re.search(r"~(\w+)\(\) \{ PyEval_RestoreThread\(state\); \}", source)
+    assert re.search(r"const Unlocked unlocked;\s+rc = f\(args\.\.\.\);\s+\}", source) and source.count("Unlocked unlocked") == 1
+    assert not re.search(r"call\(\s*\[", source)  # (a lambda's body would run in there)
 
 
 def test_bound_to_every_function_it_names():
