@@ -107,17 +107,21 @@ def test_int8_rows_that_are_padded(m, n, k):
         assert torch.equal(_C.ternary_linear_tensor_core_forward(x, packed, scale, bias, k, 2), want)
 
 
-def test_choice_by_size():
-    """From 33 rows on the forward's results are this kernel's where it is the cheaper one, and up to 32 rows the row-major weights'."""
+@pytest.mark.parametrize("m,n,k,here", [(77, 7680, 2560, True), (64, 2560, 2560, True), (128, 7680, 2560, True), (192, 16384, 1024, False)])
+def test_choice_by_size(m, n, k, here):
+    """From 33 rows on the forward's results are this kernel's where it is the cheaper one, and not the tiled GEMM's, which sums in another
+    order (its tiles all have the same bits, and so has the streaming kernel on eight waves: not told apart here); up to 32 rows the
+    row-major weights'."""
     from bittorch_amd import _C
-    for m, n, k, tile in ((77, 7680, 2560, "3,4"), (64, 2560, 2560, "2,2"), (128, 7680, 2560, "4,4")):
-        x, packed, scale, _, bias, _ = _case(m, n, k, torch.bfloat16)
-        tiled = _C.retile_weights(packed, k)
-        got = _C.ternary_linear_tiled_forward(x, tiled, scale, bias, k, n)
-        set_option("ROWS_CFG", tile)
-        assert torch.equal(got, _C.ternary_linear_tiled_forward(x, tiled, scale, bias, k, n))
-        set_option("ROWS_CFG", None)
-        assert torch.equal(_C.ternary_linear_tiled_forward(x[:32], tiled, scale, bias, k, n), _C.ternary_linear_packed_forward(x[:32], packed, scale, bias, k))
+    announce("few rows, choice", m, n, k)
+    x, packed, scale, _, bias, _ = _case(m, n, k, torch.bfloat16)
+    tiled = _C.retile_weights(packed, k)
+    got = _C.ternary_linear_tiled_forward(x, tiled, scale, bias, k, n)
+    assert torch.equal(_C.ternary_linear_tiled_forward(x[:32], tiled, scale, bias, k, n), _C.ternary_linear_packed_forward(x[:32], packed, scale, bias, k))
+    for option, value, same in (("ROWS_CFG", "3,4", here), ("STREAM_MAX_ROWS", "1", not here)):
+        set_option(option, value)
+        assert torch.equal(got, _C.ternary_linear_tiled_forward(x, tiled, scale, bias, k, n)) == same
+        set_option(option, None)
 
 
 def test_more_rows_than_its_grid_has_blocks():

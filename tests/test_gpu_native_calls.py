@@ -85,7 +85,7 @@ def test_forwards(monkeypatch, dtype, lead):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_quantizers_gradients_and_int8(monkeypatch, dtype):
     from bittorch_amd import _C
-    n, k, m = 256, 256, 24
+    n, k, m = 320, 256, 24  # (three numbers, so that none stands for another)
     announce("native quantizer and gradients", dtype)
     x, packed, tiled, scale, bias, res, norm = _make(dtype, (m,), n, k)
     w = torch.randn(n, k, device="cuda").to(dtype)
@@ -93,25 +93,88 @@ def test_quantizers_gradients_and_int8(monkeypatch, dtype):
         _both(monkeypatch, lambda: _C.ternary_quantize_pack(w, 0.05, per_channel))
     if dtype == torch.float32:
         _both(monkeypatch, lambda: _C.ternary_quantize_pack(torch.nn.Parameter(w), 0.1, True, as_half=True))
-        _both(monkeypatch, lambda: _C.linear_grad_input(x, packed, scale, k))
+        _both(monkeypatch, lambda: _C.linear_grad_input(res, packed, scale, k))
         for want in (False, True):
-            _both(monkeypatch, lambda: _C.linear_grad_weight(x, res, scale, want))
+            _both(monkeypatch, lambda: _C.linear_grad_weight(res, x, scale, want))
     else:
         for out in (dtype, torch.float32):
-            _both(monkeypatch, lambda: _C.linear_grad_weight_16(x, res, scale, out))
+            _both(monkeypatch, lambda: _C.linear_grad_weight_16(res, x, scale, out))
     for out in (torch.float32, torch.float16, torch.bfloat16):
-        _both(monkeypatch, lambda: _C.unpack_dequant(packed, k, scale.to(dtype), out))
-    q, s = _C.rmsnorm(x, norm, 1e-5, store=False, quantize=True)
+        for sc in (scale.to(dtype), scale[:1].clone()):
+            _both(monkeypatch, lambda: _C.unpack_dequant(packed, k, sc, out))
     for wt in (norm, None):
-        _both(monkeypatch, lambda: _C.rmsnorm(x, wt, 1e-5, store=False, quantize=True, operand_order=True))
+        for order in (False, True):
+            _both(monkeypatch, lambda: _C.rmsnorm(x, wt, 1e-5, store=False, quantize=True, operand_order=order))
     wide = torch.cat([x, x.flip(0)], dim=1)
-    _both(monkeypatch, lambda: _C.swiglu(wide[:, :k], wide[:, k:], store=False, quantize=True))
-    for r in (None, res):
-        _both(monkeypatch, lambda: _C.ternary_gemm_int8_tiled(q, s, tiled, scale, bias, k, n, dtype, residual=r))
+    for order in (False, True):
+        _both(monkeypatch, lambda: _C.swiglu(wide[:, :k], wide[:, k:], store=False, quantize=True, operand_order=order))
+        _both(monkeypatch, lambda: _C.act_quant_int8(x, order))
+        q, s = _C.act_quant_int8(x, order)
+        for r in (None, res):
+            _both(monkeypatch, lambda: _C.ternary_gemm_int8_tiled(q, s, tiled, scale, bias, k, n, dtype, residual=r, q_operand_order=order))
+    if dtype != torch.float32:  # (q in operand order)
+        for sc, b in ((scale, None), (scale[:1].clone(), bias), (scale.to(dtype), bias.to(dtype))):
+            _both(monkeypatch, lambda: _C.ternary_swiglu_int8_tiled(q, s, tiled, sc, b, k, n, dtype))
+
+
+def test_refused_calls_are_refused_alike(monkeypatch):
+    """What each function refuses, with the native module and without it: the same error (none of these reaches a launch)."""
+    from bittorch_amd import _C
+    n, k, m = 64, 128, 6
+    x, packed, tiled, scale, bias, res, norm = _make(torch.bfloat16, (m,), n, k)
+    f, fres = x.float(), res.float()
+    q, s = _C.act_quant_int8(x, True)
+    bf16, fp32 = torch.bfloat16, torch.float32
+    calls = [
+        (_C.ternary_linear_packed_forward, (x, packed, scale, bias, k),
+         [(0, x[:0]), (0, x[:, :-8]), (0, x.int()), (0, x.cpu()), (1, packed[:-1]), (1, packed.to(torch.int8)), (1, packed[0]), (2, scale[:5]),
+          (2, scale[None]), (3, bias[:-1]), (4, k + 1), (4, 0)]),
+        (_C.ternary_linear_tiled_forward, (x, tiled, scale, bias, k, n),
+         [(0, x[:0]), (0, x.int()), (0, x.cpu()), (1, tiled[:-256]), (1, tiled[1:]), (1, tiled.to(torch.int8)), (2, scale[:5]), (3, bias[:-1]),
+          (4, k + 1), (5, n + 16), (5, 0), (5, -1)]),
+        (lambda *a: _C.ternary_linear_tensor_core_forward(*a, 2), (x, packed, scale, bias, k),
+         [(0, x[:0]), (0, x[0]), (0, x.int()), (0, x.cpu()), (1, packed[:-1]), (2, scale[:5]), (3, bias[:-1]), (4, k + 1)]),
+        (_C.ternary_gemm_int8_tiled, (q, s, tiled, scale, bias, k, n, bf16, False, None, True),
+         [(0, q[:0]), (0, q[0]), (0, x), (0, q.cpu()), (1, s[:-1]), (1, s.double()), (2, tiled[:-256]), (3, scale[:5]), (4, bias[:-1]), (5, k + 1),
+          (6, n + 16), (7, torch.int32), (9, res[:-1]), (9, res.float())]),
+        (_C.ternary_swiglu_int8_tiled, (q, s, tiled, scale, bias, k, n, bf16),
+         [(0, q[:0]), (0, x), (0, q.cpu()), (1, s[:-1]), (1, s.double()), (2, tiled[:-256]), (3, scale[:5]), (4, bias[:-1]), (5, k + 1), (6, n - 16),
+          (7, fp32)]),
+        (_C.ternary_quantize_pack, (f,), [(0, f[0]), (0, f[:0]), (0, f.int()), (0, f.cpu())]),
+        (lambda *a: _C.ternary_quantize_pack(*a, as_half=True), (f,), [(0, x)]),
+        (_C.act_quant_int8, (x, True), [(0, x[0]), (0, x[:0]), (0, x.int()), (0, x.cpu()), (0, x[:, :-8].contiguous())]),
+        (lambda *a: _C.rmsnorm(*a, store=False, quantize=True, operand_order=True), (x, norm, 1e-5),
+         [(0, x[:0]), (0, x.int()), (0, x.cpu()), (0, x[:, :-8].contiguous()), (1, norm[:-1]), (1, norm[None])]),
+        (lambda *a: _C.swiglu(*a, store=False, quantize=True, operand_order=True), (x, x),
+         [(0, x[:0]), (0, f), (0, x.cpu()), (1, x[:-1]), (1, f)]),
+        (lambda *a: _C.swiglu(*a, store=False, quantize=True, operand_order=True), (x[:, :40], x[:, :40]), [(0, x[:, :40])]),
+        (_C.unpack_dequant, (packed, k, scale, fp32),
+         [(0, packed[:-1]), (0, packed.to(torch.int8)), (0, packed.cpu()), (1, k + 4), (2, scale[:5]), (3, torch.int32)]),
+        (_C.linear_grad_input, (fres, packed, scale, k),
+         [(0, fres[:0]), (0, fres[0]), (0, res), (0, fres.cpu()), (0, fres[:, :-1]), (1, packed[:-1]), (1, packed.to(torch.int8)), (2, scale[:5]),
+          (2, scale.double()), (3, k + 4)]),
+        (_C.linear_grad_weight, (fres, f, scale), [(0, fres[:0]), (0, res), (0, fres[:-1]), (1, f[0]), (1, x), (1, f.cpu()), (1, f[:, :3].contiguous()), (2, scale[:5]),
+                                                   (2, scale.double())]),
+        (_C.linear_grad_weight_16, (res, x, scale, bf16),
+         [(0, res[:0]), (0, fres), (0, res[:-1]), (0, res.half()), (1, x[0]), (1, x.cpu()), (1, x[:, :-1].contiguous()), (2, scale[:5]), (2, scale.double()),
+          (3, torch.float16)]),
+    ]
+    real = _C._N
+    for i, (call, args, changes) in enumerate(calls):
+        for at, value in changes:
+            announce("refused alike", i, at, tuple(value.shape) if isinstance(value, torch.Tensor) else value)
+            errors = []
+            for module in (real, _AsksNobody()):
+                monkeypatch.setattr(_C, "_N", module)
+                with pytest.raises((RuntimeError, IndexError)) as e:
+                    call(*args[:at], value, *args[at + 1:])
+                errors.append((e.type, str(e.value)))
+            assert errors[0] == errors[1]
+    monkeypatch.setattr(_C, "_N", real)
 
 
 def test_other_calls_go_to_python(monkeypatch):
-    """Strides, alignment, other dtypes and devices, subclasses, modes and transforms: not the native call's."""
+    """Strides, alignment, other dtypes, subclasses and modes: not the native call's."""
     from bittorch_amd import _C
     n, k, m = 64, 128, 6
     x, packed, tiled, scale, bias, res, norm = _make(torch.bfloat16, (m,), n, k)

@@ -823,10 +823,11 @@ def test_row_major_fallback_keeps_its_promises(oracle):
     assert b.keep_row_major and b._has_row_major()
 
 
-@pytest.mark.parametrize("m,n,k", [(1000, 2560, 1536), (1200, 2560, 1480), (821, 2559, 1500), (993, 2336, 1544)])
+@pytest.mark.parametrize("m,n,k", [(1000, 2560, 1536), (1200, 2560, 1480), (821, 2559, 1500), (993, 2336, 1544), (1009, 2560, 1600)])
 def test_tiles_of_48_rows(m, n, k):
-    """Launches of one 48-row tile for each compute unit: last tiles of 1, 5, 33, 40 and 48 rows, an odd number of stages, a partial one, N of any
-    length; row-major weights give the same bits, the SwiGLU stage the row kernel's, and a residual its two roundings."""
+    """Sizes for which the plan is one 48-row tile for each compute unit at most (not asked here: tiles of 64 rows would give the same bits):
+    last tiles of 1, 5, 33, 40 and 48 rows, an odd number of stages, a partial one, N of any length; row-major weights give the same bits,
+    the SwiGLU stage the row kernel's, and a residual its two roundings."""
     from bittorch_amd import _C
     from test_gpu_few_rows import _bound, _case
     for dtype in (torch.float16, torch.bfloat16):
