@@ -43,7 +43,7 @@ enum Option {
     OPT_PLANES_NACC,         // exact GEMV, one matrix per launch: 16-column blocks per workgroup
     OPT_ROWOP_GENERIC,       // 1: SwiGLU / RMSNorm rows on the shape-generic kernel
     OPT_STREAM_CFG,          // "ld,waves": tile width and wave count of the streaming kernel
-    OPT_ROWS_CFG,            // "rb,nacc": 16-bit calls on tiled weights take the kernel for a few tens of rows, tiles of 16 rb x 16 nacc
+    OPT_ROWS_CFG,            // "rb,nacc": 16-bit calls, and int8 ones in operand order, take the kernel for a few tens of rows, tiles of 16 rb x 16 nacc
     OPT_NO_PLANES,           // 1: a single fp16 row takes the 16-bit streaming kernel instead of the exact GEMV
     OPT_COUNT
 };
