@@ -85,7 +85,9 @@ struct GemmF32Params {
 // bf16 +-0.5: the weights' value here, so that the low byte is zero and a sum cannot overflow before it is doubled
 constexpr uint32_t LUT_BF16_HALF = 0x00BF3F00u;
 
-// A wave works on a tile of 16 NB rows x 64 NG columns, from row m0 and column c0 on (NB = 4, but for shared tiles).
+// A wave works on a tile of 16 NB rows x 64 NG columns (NB = 4, but for shared tiles), from row m_at and column c_at on (KS = 1), or tile
+// (tm, tn) (KS > 1).  Parameters by value, and the place of a tile of KS > 1 formed in here: otherwise the compiler orders the output
+// stage so that such launches take a microsecond longer (fp32, 600 x 768 x 3072 29.2 / 30.5, 2000 x 512 x 2048 23.1 / 24.4).
 // KS > 1: all KS waves of a workgroup work on one tile, each on its run of the contraction, and add their sums through LDS
 // (pairwise, always in the same order): for outputs with too few tiles to occupy the chip.
 // SC: X's columns are scaled (input gradient with one scale per row of W).
@@ -94,9 +96,10 @@ constexpr uint32_t LUT_BF16_HALF = 0x00BF3F00u;
 // the tile of one wave's 64 x 64 outputs gains from the question: with a branch between them the compiler sends each row's
 // stores off by themselves (512 x 2048 x 1032 17.0 without, 16.0 with it; 4096 x 128 x 2048 24.1 / 23.1).
 template <int SRC, int NG, int NB, int KS, bool SC, bool RN>
-__device__ __forceinline__ void gemm_f32_tile(const GemmF32Params& p, const int64_t m0, const int64_t c0) {
+__device__ __forceinline__ void gemm_f32_tile(const GemmF32Params p, const int64_t m_at, const int64_t c_at, const uint32_t tm, const uint32_t tn) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i = lane & 15, g = lane >> 4;
+    const int64_t m0 = KS == 1 ? m_at : (int64_t)tm * 64, c0 = KS == 1 ? c_at : (int64_t)tn * (64 * NG);
 
     // rows and columns past the end repeat the last one: they only feed outputs that are never stored
     const uint8_t* a_base = (const uint8_t*)(p.X + m0 * p.C);
@@ -397,13 +400,13 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS, 2) void gemm_f32_kernel(Ge
         if (fine) {
             constexpr int NB = 4 / PARTS;
             const int64_t m0 = (int64_t)tm * TM + 16 * NB * (2 * (int)part + (wave >> 1));
-            if (m0 < p.M && c0 < p.NC) gemm_f32_tile<SRC, NG, NB, KS, SC, RN>(p, m0, c0);
+            if (m0 < p.M && c0 < p.NC) gemm_f32_tile<SRC, NG, NB, KS, SC, RN>(p, m0, c0, tm, tn);
             return;
         }
     }
     const int64_t m0 = (int64_t)tm * TM + (KS == 1 ? 64 * (wave >> 1) : 0);
     if (KS == 1 && (m0 >= p.M || c0 >= p.NC)) return;  // (no barriers in a tile when KS == 1)
-    gemm_f32_tile<SRC, NG, 4, KS, SC, RN>(p, m0, c0);
+    gemm_f32_tile<SRC, NG, 4, KS, SC, RN>(p, m0, c0, tm, tn);
 }
 
 // Into how many workgroups a tile of the remainder is shared (KS = 1): the tiles beyond one, two ... for every compute unit of an XCD

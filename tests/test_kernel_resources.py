@@ -63,10 +63,10 @@ def test_activation_quantizers_keep_their_rows_in_registers(kernels):
 
 
 def test_fp32_gemm_waves_work_alone(kernels):
-    """Where a wave sums the whole contraction (KS = 1) there is no LDS, and the forward's instances keep their sums in registers."""
+    """Where a wave sums the whole contraction (KS = 1) there is no LDS, and the forward's instances keep everything in registers."""
     for name, k in _named(kernels, "gemm_f32_kernel"):
         src, ks = int(name.split("gemm_f32_kernelILi")[1][0]), int(name.split("ELi")[2][0])
         if ks == 1:
             assert k[".group_segment_fixed_size"] == 0, name
-        if src != 2:
-            assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_spill_count"] == 0, name
+            if src != 2:
+                assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_spill_count"] == 0, name
