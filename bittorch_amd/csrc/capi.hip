@@ -206,9 +206,12 @@ static bool prefers_stream(int64_t B, int64_t N, int64_t K, bool int8, bool tile
 //          6912 22.6 / 13.9, 77 x 4096 x 11008 31.4 / 19.6, 64 x 11008 x 4096 19.9 / 14.8, row-major 192 x 4096 x 11008 57.5 / 24.2; the
 //          other way 128 x 11008 x 4096 23.0 / 27.9, 192 x 16384 x 1024 12.0 / 16.9
 //   int8   (exact sums: any number of rows).  Row-major weights with the quantizer: 32 x 4096 x 11008 20.8 / 15.4, 128 x 7680 x 2560
-//          16.9 / 13.0, 256 x 4096 x 11008 35.9 / 26.1; tiled: 96 x 7680 x 2560 11.7 / 8.7, 256 x 2560 x 6912 21.6 / 14.1.  Up to 16 rows
-//          it wins where 64 columns each are enough workgroups, 16 x 11008 x 4096 10.5 / 9.7, 16 x 16384 x 1024 8.9 / 7.3, not 8 x 4096 x
-//          4096 8.6 / 9.3; tiled 16 x 7680 x 2560 5.7 / 5.3, 8 x 7680 x 2560 5.1 / 5.3
+//          16.9 / 13.0, 256 x 4096 x 11008 35.9 / 26.1; up to 16 rows it wins where 64 columns each are enough workgroups, 16 x 11008 x
+//          4096 10.5 / 9.7, 16 x 16384 x 1024 8.9 / 7.3, not 8 x 4096 x 4096 8.6 / 9.3.  Tiled weights stream better, so that its price is
+//          compared with prices of the streaming kernel and of the GEMM alone, fitted to calls on weights that lie in no L2: 16 x 7680 x 1024
+//          5.5 / 4.9, 16 x 11008 x 2560 7.2 / 6.5, 48 x 4096 x 4096 7.2 / 6.5, 96 x 7680 x 2560 11.7 / 8.7; the other way, and there this
+//          kernel is not taken: 9 x 7680 x 4096 5.8 / 6.9, 16 x 7680 x 11008 10.8 / 12.8, 32 x 4096 x 4096 6.1 / 6.5, 224 x 6400 x 11008
+//          30.2 / 47.0, 96 x 16384 x 11008 30.2 / 39.0, 384 x 4096 x 11008 30.0 / 35.5
 static bool prefers_rows(bool i8, bool row_major, int64_t B, int64_t N, int64_t K) {
     if (B > 65535ll * 16) return false;  // its grid.y is the row blocks; the others slice such a call or walk it in grid.x
     if (option(OPT_ROWS_CFG)) return true;
@@ -220,10 +223,15 @@ static bool prefers_rows(bool i8, bool row_major, int64_t B, int64_t N, int64_t 
         const double stream = std::max(4.0 + work * 5.0e-9 + blocks * (double)ceil_div(N, 64) * 0.004, 4.2 + 0.0011 * (double)K);
         return few_rows_cost(false, row_major, B, N, K) < std::min(stream, 0.95 * gemm_f16_cost(B, N, K));
     }
-    if (B <= 16) return B > (row_major ? 1 : 8) && ceil_div(N, 64) >= 100;
-    const double stream = std::max(4.0 + work * 2.2e-9 + blocks * (double)ceil_div(N, 128) * 0.003, 4.0 + (row_major ? 0.0012 : 0.00058) * (double)K);
-    const double us = few_rows_cost(true, row_major, B, N, K);
-    return us < stream && (B <= 32 || us < 0.9 * gemm_i8_cost(B, N, K, !row_major, true));
+    if (B <= 16 && (B <= (row_major ? 1 : 8) || ceil_div(N, 64) < 100)) return false;
+    const double us = few_rows_cost(true, row_major, B, N, K), wgs = blocks * (double)ceil_div(N, 128), k = (double)K;
+    if (row_major) {
+        const double stream = std::max(4.0 + work * 2.2e-9 + wgs * 0.003, 4.0 + 0.0012 * k);
+        return B <= 16 || (us < stream && (B <= 32 || us < 0.9 * gemm_i8_cost(B, N, K, false, true)));
+    }
+    if (B <= 16) return us < 0.97 * (3.8 + 0.0143 * wgs + 0.00021 * k + 3.8e-6 * wgs * k);
+    if (B > 32 && !prefers_stream(B, N, K, true, true, true)) return us < 0.85 * gemm_i8_cost(B, N, K, true, true);  // (priced with the quantizer)
+    return us < (B <= 32 ? 0.94 : 1.0) * (4.55 + 0.0067 * wgs + 0.00024 * k + 4.1e-6 * wgs * k);
 }
 
 // The same choice for fp32 activations: the streaming kernel on three bf16 planes (split in a launch of its own, about 3 us)

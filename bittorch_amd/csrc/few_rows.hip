@@ -259,16 +259,24 @@ __global__ __launch_bounds__(64 * ROWS_WAVES, 2) void few_rows_kernel(RowsParams
 // 77 x 11008 x 4096 23.4 / 22.6 / 25.6 / 18.5 / 20.5; 64 x 4096 x 4096 8.6 / 10.7 / 12.2 / 15.0 / 7.3.  int8 rows are half the bytes and
 // bound by the decode and the chain of a step, 0.5 us and 0.2 a row block; 16 x 64 / 32 x 64 / 48 x 64 / 64 x 64 / 80 x 64, us, tiled:
 // 64 x 7680 x 2560 7.8 / 6.9 / 8.5 / 9.3 / 10.8, 128 x 4096 x 11008 19.3 / 14.9 / 18.4 / 20.1 / 24.7, 16 x 11008 x 4096 6.6 / 7.4 / 8.5 / 9.5 / 11.3.
+// On tiled int8 weights, from memory, such a launch takes 2 to 14 % longer than that, the more the fuller the chip is.
 struct RowsPlan {
     int rb, nacc;
     double us;
 };
+// Column tiles of an XCD where consecutive ones lie on one XCD, or 0: in launch order
+static int rows_per_xcd(int64_t tiles, int64_t blocks) { return blocks > 1 && tiles % 8 != 0 && tiles < 64 ? 0 : (int)ceil_div(tiles, 8); }
 static RowsPlan few_rows_plan(bool i8, bool rows, int64_t M, int64_t N, int64_t row_bytes) {
     const int64_t C = gemm_compute_units();
     const double steps = (double)ceil_div(ceil_div(row_bytes, 128), ROWS_WAVES);
     auto price = [&](int rb, int nacc) {
-        const double rounds = (double)ceil_div(ceil_div(M, 16 * rb) * ceil_div(N, 16 * nacc), C);
-        if (i8) return (0.2 + 0.8 * rounds) * (2.7 + 0.65 * rb + steps * (0.5 + 0.2 * rb));
+        const int64_t blocks = ceil_div(M, 16 * rb), tiles = ceil_div(N, 16 * nacc), per_xcd = rows_per_xcd(tiles, blocks);
+        const double rounds = (double)ceil_div(blocks * tiles, C);
+        if (i8) {
+            // (an XCD's workgroups are on its own compute units: of 5 x 100 some have 65 for 32, three rounds; 224 x 6400 x 11008 47 us)
+            const double turns = per_xcd ? (double)ceil_div(per_xcd * blocks, C / 8) : rounds, full = (double)(blocks * tiles) / ((double)C * turns);
+            return (0.2 + 0.8 * turns) * (2.7 + 0.65 * rb + steps * (0.5 + 0.2 * rb)) * (rows ? 1.0 : 1.02 + 0.12 * full);
+        }
         return 2.6 + rounds * (rounds > 1 ? 1.45 : 1.0) * (0.7 + steps * ROWS_WAVES * (2048.0 * rb + 256.0 * nacc) / 66000.0);
     };
     static const int cfg[6][2] = {{2, 2}, {1, 4}, {2, 4}, {3, 4}, {4, 4}, {5, 4}};
@@ -293,7 +301,7 @@ template <int MODE, bool ROWS, int RB, int NACC, bool SW>
 static int launch_rows_cfg(RowsParams p, hipStream_t st) {
     const int64_t blocks = ceil_div(p.M, 16 * RB);
     p.tiles = (int)ceil_div(p.N, 16 * NACC);
-    p.per_xcd = blocks > 1 && p.tiles % 8 != 0 && p.tiles < 64 ? 0 : (int)ceil_div(p.tiles, 8);
+    p.per_xcd = rows_per_xcd(p.tiles, blocks);
     const dim3 grid((unsigned)(p.per_xcd ? 8 * p.per_xcd : p.tiles), (unsigned)blocks), block(64 * ROWS_WAVES);
     const bool tail = p.row_bytes % 128 != 0 || 4 * p.Kb * (MODE == MODE_I8 ? 1 : 2) < p.row_bytes;
     if (tail) hipLaunchKernelGGL((few_rows_kernel<MODE, ROWS, RB, NACC, SW, true>), grid, block, 0, st, p);

@@ -98,6 +98,16 @@ def test_int8_swiglu_stage_pays_only_where_it_is_taken(n, k, taken):
         assert lib.bt_ternary_swiglu_i8_tiled(addr, addr, addr, addr, 0, 1, None, 0, addr, 2, rows, n, k, None) == -1
 
 
+@pytest.mark.parametrize("m,n,k", [(224, 6400, 11008), (224, 6400, 8192), (384, 4096, 11008), (192, 7680, 11008)])
+def test_int8_rows_on_tiled_weights_take_the_gemm_where_it_is_faster(m, n, k):
+    """The tiled GEMM (and with it its SwiGLU stage), not the kernel for a few tens of rows: us 30 / 47, 24 / 36, 30 / 35, 31 / 35.  The other
+    way round 96 x 7680 x 2560, which that kernel serves in 8.7 us for 11.7."""
+    from bittorch_amd import _lib
+    lib = _lib.load()
+    assert lib.bt_swiglu_i8_tiled_pays(m, n, k) == 1
+    assert lib.bt_swiglu_i8_tiled_pays(96, 7680, 2560) == 0
+
+
 def test_extension_probes_are_truthful():
     import bittorch_amd as bt
     from bittorch_amd.nn.ternary_linear import _cuda_kernel_available
