@@ -49,6 +49,9 @@ enum Option {
 };
 const char* option(Option o);  // the option's text, or nullptr when it is not set (capi.hip)
 
+// Activation rows of more bytes than this are in no XCD's L2 as a whole (few_rows.hip, and the rule in capi.hip)
+constexpr double ROWS_L2_BYTES = 4194304.0;
+
 // A/B switches of experiment builds (-DBT_TUNING): compiled out of the product library.
 #ifdef BT_TUNING
 static inline const char* tuning_env(const char* name) { return getenv(name); }

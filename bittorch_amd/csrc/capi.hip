@@ -217,17 +217,20 @@ static bool prefers_rows(bool i8, bool row_major, int64_t B, int64_t N, int64_t 
     if (option(OPT_ROWS_CFG)) return true;
     if (option(OPT_STREAM_MAX_ROWS)) return false;
     const double work = (double)B * (double)N * (double)K, blocks = (double)ceil_div(B, 16);
+    // Rows that no L2 holds have a price of their own in few_rows_cost, which those of the streaming kernel lack: us, measured / priced, bf16
+    // 600 x 256 x 6912 20.7 / 11.8, 1000 x 256 x 11008 19.9 / 16.3 (here 13.9 and 21.1).
+    const double beyond = (i8 ? 1.0 : 2.0) * (double)B * (double)K > ROWS_L2_BYTES ? 1.25 : 1.0;
     if (ceil_div(B, 16) * ceil_div(N, 64) < 64) return false;  // (narrow matrices: the streaming kernel cuts them finer; int8 32 x 1000 x 3000 8.8 / 10.5)
     if (!i8) {
         if (B <= 32) return false;
         const double stream = std::max(4.0 + work * 5.0e-9 + blocks * (double)ceil_div(N, 64) * 0.004, 4.2 + 0.0011 * (double)K);
-        return few_rows_cost(false, row_major, B, N, K) < std::min(stream, 0.95 * gemm_f16_cost(B, N, K));
+        return few_rows_cost(false, row_major, B, N, K) < std::min(beyond * stream, 0.95 * gemm_f16_cost(B, N, K));
     }
     if (B <= 16 && (B <= (row_major ? 1 : 8) || ceil_div(N, 64) < 100)) return false;
     const double us = few_rows_cost(true, row_major, B, N, K), wgs = blocks * (double)ceil_div(N, 128), k = (double)K;
     if (row_major) {
         const double stream = std::max(4.0 + work * 2.2e-9 + wgs * 0.003, 4.0 + 0.0012 * k);
-        return B <= 16 || (us < stream && (B <= 32 || us < 0.9 * gemm_i8_cost(B, N, K, false, true)));
+        return B <= 16 || (us < beyond * stream && (B <= 32 || us < 0.9 * gemm_i8_cost(B, N, K, false, true)));
     }
     if (B <= 16) return us < 0.97 * (3.8 + 0.0143 * wgs + 0.00021 * k + 3.8e-6 * wgs * k);
     if (B > 32 && !prefers_stream(B, N, K, true, true, true)) return us < 0.85 * gemm_i8_cost(B, N, K, true, true);  // (priced with the quantizer)

@@ -272,12 +272,15 @@ static RowsPlan few_rows_plan(bool i8, bool rows, int64_t M, int64_t N, int64_t 
     auto price = [&](int rb, int nacc) {
         const int64_t blocks = ceil_div(M, 16 * rb), tiles = ceil_div(N, 16 * nacc), per_xcd = rows_per_xcd(tiles, blocks);
         const double rounds = (double)ceil_div(blocks * tiles, C);
+        // Rows that no L2 holds come from behind it, once for each XCD that has a tile of them, at 6 TB/s: 2048 x 512 x 11008 bf16 58 us for
+        // 360 MB, 1000 x 256 x 11008 in tiles of 32 columns 29 us for 176 MB.
+        const double bytes = (double)M * (double)row_bytes, fetch = bytes > ROWS_L2_BYTES ? 2.0 + (double)std::min<int64_t>(tiles, 8) * bytes / 6.5e6 : 0.0;
         if (i8) {
             // (an XCD's workgroups are on its own compute units: of 5 x 100 some have 65 for 32, three rounds; 224 x 6400 x 11008 47 us)
             const double turns = per_xcd ? (double)ceil_div(per_xcd * blocks, C / 8) : rounds, full = (double)(blocks * tiles) / ((double)C * turns);
-            return (0.2 + 0.8 * turns) * (2.7 + 0.65 * rb + steps * (0.5 + 0.2 * rb)) * (rows ? 1.0 : 1.02 + 0.12 * full);
+            return std::max(fetch, (0.2 + 0.8 * turns) * (2.7 + 0.65 * rb + steps * (0.5 + 0.2 * rb)) * (rows ? 1.0 : 1.02 + 0.12 * full));
         }
-        return 2.6 + rounds * (rounds > 1 ? 1.45 : 1.0) * (0.7 + steps * ROWS_WAVES * (2048.0 * rb + 256.0 * nacc) / 66000.0);
+        return std::max(fetch, 2.6 + rounds * (rounds > 1 ? 1.45 : 1.0) * (0.7 + steps * ROWS_WAVES * (2048.0 * rb + 256.0 * nacc) / 66000.0));
     };
     static const int cfg[6][2] = {{2, 2}, {1, 4}, {2, 4}, {3, 4}, {4, 4}, {5, 4}};
     auto has = [&](const int* c) { return c[1] == 2 ? !rows && !i8 : c[0] > 1 || i8; };

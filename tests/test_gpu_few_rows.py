@@ -107,11 +107,11 @@ def test_int8_rows_that_are_padded(m, n, k):
         assert torch.equal(_C.ternary_linear_tensor_core_forward(x, packed, scale, bias, k, 2), want)
 
 
-@pytest.mark.parametrize("m,n,k,here", [(77, 7680, 2560, True), (64, 2560, 2560, True), (128, 7680, 2560, True), (192, 16384, 1024, False)])
+@pytest.mark.parametrize("m,n,k,here", [(77, 7680, 2560, True), (64, 2560, 2560, True), (128, 7680, 2560, True), (192, 16384, 1024, False), (2048, 512, 11008, False)])
 def test_choice_by_size(m, n, k, here):
     """From 33 rows on the forward's results are this kernel's where it is the cheaper one, and not the tiled GEMM's, which sums in another
     order (its tiles all have the same bits, and so has the streaming kernel on eight waves: not told apart here); up to 32 rows the
-    row-major weights'."""
+    row-major weights'.  The last: rows that no L2 holds."""
     from bittorch_amd import _C
     announce("few rows, choice", m, n, k)
     x, packed, scale, _, bias, _ = _case(m, n, k, torch.bfloat16)
